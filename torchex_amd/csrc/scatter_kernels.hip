@@ -62,6 +62,43 @@ namespace {
 constexpr int kMargin = 64;           // staged entries past the tile's end
 constexpr int kNoSeg = 0x7fffffff;    // never a valid seg value
 
+// How a workgroup's threads are dealt to feature rows: `lanes` neighbouring threads (a lane
+// group) cover one row, `groups` lane groups fit in a workgroup; threads beyond the last group
+// only help to stage.  Any number of lanes up to 64 goes: 67 fp32 channels are 17 lanes of four,
+// so 15 groups use 255 threads, where the next power of two (32 lanes, 8 groups) would leave
+// 120 threads idle.  A lane group may straddle two wavefronts: its lanes never exchange
+// registers.  Lane k moves elements k * VEC ..; where VEC does not divide the row, the last
+// lane moves the row's last VEC elements, and the elements it shares with its neighbour are
+// worked out twice, with the same result, and stored twice.  Divisions by the two numbers are
+// multiplications by the rounded-up 2^32-fold reciprocals (exact while n * divisor < 2^32).
+// Measured on 300,007 rows of 67 fp32 channels, mean + max, forward and backward: 293 us with
+// 4-byte lanes (two column blocks of 64, the second with 3 lanes at work), 214 like this (and
+// 178 without the non-temporal hint, below); 200k rows of 131 channels 357 -> 227.
+struct LaneMap {
+    int lanes, groups;
+    unsigned per_lanes, per_groups;  // ceil(2^32 / lanes), ceil(2^32 / groups); 0 stands for a divisor of 1
+};
+__device__ __forceinline__ int div_by(unsigned n, unsigned per) { return per ? (int)__umulhi(n, per) : (int)n; }
+
+// HINT: feature and arg rows on the way in and out, and input-gradient rows, carry the
+// non-temporal hint (each is touched exactly once).  What a hinted access leaves of a 64-byte
+// sector is not merged with the neighbouring row's part in the L2, so rows that do not fill
+// whole sectors go without: us for mean + max, forward and backward, hinted -> not hinted: 2M
+// rows of 40 bytes 447 -> 278, of 32 bytes 333 -> 215, 700k of 268 bytes 438 -> 364, of 262
+// bytes 481 -> 392.  Rows of whole sectors keep it: 1M of 512 bytes 567 -> 625 without, 1M of
+// 128 bytes 167 -> 187 (the stores matter most; hinted loads make no difference up to 128 MB
+// of rows and 2 % at 512 MB).
+template <bool HINT, typename T, int VEC>
+__device__ __forceinline__ Pack<T, VEC> ld_hint(const T *p) {
+    if constexpr (HINT) return ld_stream<T, VEC>(p);
+    else return ld_row<T, VEC>(p);
+}
+template <bool HINT, typename T, int VEC>
+__device__ __forceinline__ void st_hint(T *p, const Pack<T, VEC> &x) {
+    if constexpr (HINT) st_stream<T, VEC>(p, x);
+    else st_row<T, VEC>(p, x);
+}
+
 // ---- the reference's winner among equal maxima (op TXS_MAX_REFTIE) ----------
 // scatter_kernel.cu:131-171 runs B = clamp(up_2n(max_cnt), 32, 1024) threads per
 // voxel; thread tid keeps the LAST maximal row of its residue class (rel % B ==
@@ -95,14 +132,14 @@ constexpr int fwd_min_waves() {
     return (std::is_same<TR, F16>::value && OP == TXS_MAX) ? 6 : 1;
 }
 
-template <class TR, int VEC, int OP>
+template <class TR, int VEC, int OP, bool HINT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(fwd_min_waves<TR, OP>(), 8)))
 void scatter_fwd_kernel(
     const typename TR::raw *__restrict__ feats, const int *__restrict__ perm,
     const int *__restrict__ seg, const int *__restrict__ slot_of,
     typename TR::raw *__restrict__ out, int *__restrict__ arg,
     unsigned long long *__restrict__ scratch, const int *__restrict__ preSum, int N, int C, int U,
-    int lpr_log2, int ref_log2, int chunk) {
+    LaneMap lm, int ref_log2, int T) {
     using raw = typename TR::raw;
     constexpr bool kMax = OP == TXS_MAX || OP == TXS_MAX_REFTIE;
     constexpr bool kRef = OP == TXS_MAX_REFTIE;  // idx[] then holds the winner's staged position, not its row
@@ -113,9 +150,7 @@ void scatter_fwd_kernel(
     using AccT = typename std::conditional<kMax, typename TR::max_t, float>::type;
     constexpr int kEndBit = kSpecialBit;
     extern __shared__ int lds[];
-    const int g_log2 = 8 - lpr_log2;      // kThreads == 256
-    const int G = 1 << g_log2;
-    const int T = G * chunk;              // `chunk` positions per lane group on average
+    const int G = lm.groups;              // T: the tile's positions, a multiple of 64
     const int n_seg_s = T + kMargin + 1;  // positions t0-1 .. t0+T+kMargin-1
     int *seg_s = lds;                     // seg_s[l]: voxel (bit 31: special) at position t0 - 1 + l
     int *pk_s = lds + n_seg_s;            // pk_s[l - 1]: row at position t0 - 1 + l, bit 31 = last row of its run
@@ -174,13 +209,15 @@ void scatter_fwd_kernel(
     const int Tp = b_hi - b_lo;  // rows of the tile's own range: dealt evenly to the lane groups
     if (Tp <= 0) return;         // uniform for the workgroup
 
-    const int gi = (int)threadIdx.x >> lpr_log2;
-    const int lane_in = (int)threadIdx.x & ((1 << lpr_log2) - 1);
-    const int col = ((int)blockIdx.y << lpr_log2 | lane_in) * VEC;
-    const bool live = col < C;
-    auto share_begin = [&](int k) -> int { return b_lo + (int)(((long)k * Tp) >> g_log2); };
-    const int c0 = share_begin(gi), c_end = share_begin(gi + 1);  // this lane group's positions (l)
-    const int ch = (Tp + G - 1) >> g_log2;                          // the largest share
+    const int gi = div_by(threadIdx.x, lm.per_lanes);
+    const int lane_in = (int)threadIdx.x - gi * lm.lanes;
+    const int col_own = ((int)blockIdx.y * lm.lanes + lane_in) * VEC;  // first element that is this lane's alone
+    const int col = min(col_own, C - VEC);                             // first element it moves
+    const bool live = gi < G && col_own < C;
+    auto share_begin = [&](int k) -> int { return b_lo + div_by((unsigned)(k * Tp), lm.per_groups); };
+    const int c0 = share_begin(min(gi, G - 1));  // this lane group's positions (l)
+    const int c_end = share_begin(min(gi, G - 1) + 1);
+    const int ch = div_by((unsigned)(Tp + G - 1), lm.per_groups);  // the largest share
 
     // ids / rows past the staged range are fetched from global memory (only an ordinary run
     // longer than kMargin that crosses the tile's end gets there)
@@ -257,7 +294,7 @@ void scatter_fwd_kernel(
                 for (long p = lo; p < hi; ++p) {
                     const int row = perm ? perm[p] : (int)p;
                     if ((unsigned)row >= (unsigned)N) continue;
-                    Pack<raw, VEC> x = ld<raw, VEC>(feats + (size_t)row * C + col);
+                    Pack<raw, VEC> x = ld_row<raw, VEC>(feats + (size_t)row * C + col);
 #pragma unroll
                     for (int k = 0; k < VEC; ++k)
                         if (ix[k] < 0 && TR::to_f(x.v[k]) == -__builtin_inff()) ix[k] = row;
@@ -302,9 +339,9 @@ void scatter_fwd_kernel(
                     ai.v[k] = ix[k];
                     if (kRef && ix[k] >= 0) ai.v[k] = (kStaged ? pk_s[ix[k] - 1] : pk_at(ix[k])) & kIdMask;
                 }
-                st_stream<int, VEC>(arg + o, ai);
+                st_hint<HINT, int, VEC>(arg + o, ai);
             }
-            st_stream<raw, VEC>(out + o, r);
+            st_hint<HINT, raw, VEC>(out + o, r);
         } else {
             const int slot = slot_of[u];
             if (slot < 0) return;
@@ -316,7 +353,8 @@ void scatter_fwd_kernel(
                         atomicMax(scratch + o, ((unsigned long long)ordered_bits((float)a[k]) << 32) |
                                                    (unsigned long long)(0xffffffffu - low_word(ix[k], u)));
                 } else {
-                    unsafeAtomicAdd(reinterpret_cast<float *>(scratch) + o, (float)a[k]);
+                    // (an element that the neighbouring lane adds as well gets its zero from here)
+                    unsafeAtomicAdd(reinterpret_cast<float *>(scratch) + o, col + k < col_own ? 0.0f : (float)a[k]);
                 }
             }
         }
@@ -429,7 +467,7 @@ void scatter_fwd_kernel(
         const int l_clamp = max(c_end - 1, c0);
         auto issue = [&](Batch &bt, int l) {
 #pragma unroll
-            for (int i = 0; i < kBatch; ++i) bt.v[i] = ld_stream<raw, VEC>(row_ptr(pk_s[min(l + i, l_clamp) - 1] & kIdMask));
+            for (int i = 0; i < kBatch; ++i) bt.v[i] = ld_hint<HINT, raw, VEC>(row_ptr(pk_s[min(l + i, l_clamp) - 1] & kIdMask));
         };
         auto consume_full = [&](const Batch &bt, int l) {
 #pragma unroll
@@ -480,7 +518,7 @@ void scatter_fwd_kernel(
                     for (int l = c_end;; ++l) {
                         const int pk = pk_at(l);
                         if (seg_at(l) == kNoSeg) break;
-                        add_row(std::false_type{}, ld_stream<raw, VEC>(row_ptr(pk & kIdMask)), l, pk);
+                        add_row(std::false_type{}, ld_hint<HINT, raw, VEC>(row_ptr(pk & kIdMask)), l, pk);
                         if (pk < 0) {
                             on_end(std::false_type{}, l);
                             break;
@@ -510,8 +548,8 @@ void scatter_fwd_kernel(
     for (int k = gi - 1; k >= 0; --k) {
         const int k0 = share_begin(k);
         if (k0 == share_begin(k + 1)) continue;  // a lane group without rows
-        const float *cv = carry_v + ((size_t)(k << lpr_log2) + lane_in) * VEC;
-        const int *ci = carry_i + ((size_t)(k << lpr_log2) + lane_in) * VEC;
+        const float *cv = carry_v + (size_t)(k * lm.lanes + lane_in) * VEC;
+        const int *ci = carry_i + (size_t)(k * lm.lanes + lane_in) * VEC;
         AccT b[VEC];
         int bi[VEC];
 #pragma unroll
@@ -601,16 +639,15 @@ __global__ void scatter_finalize_kernel(const typename TR::raw *__restrict__ fea
 // short (measured 1-5 % faster on LiDAR-like occupancy) and 16 when they are long
 // (fewer re-fetches of the same upstream row at chunk borders).
 
-template <class TR, int VEC, int OP, int CHUNK>
+template <class TR, int VEC, int OP, int CHUNK, bool HINT>
 __global__ __launch_bounds__(kThreads) void scatter_bwd_kernel(
     const typename TR::raw *__restrict__ g, const int *__restrict__ arg,
     const int *__restrict__ perm, const int *__restrict__ seg, const int *__restrict__ preSum,
-    typename TR::raw *__restrict__ gin, int N, int C, int U, int lpr_log2) {
+    typename TR::raw *__restrict__ gin, int N, int C, int U, LaneMap lm) {
     using raw = typename TR::raw;
     constexpr int kBatchBwd = sizeof(raw) == 2 ? kBatchBwdHalf : ::kBatchBwd;
     extern __shared__ int lds[];
-    const int G = kThreads >> lpr_log2;
-    const int T = G * CHUNK;
+    const int T = lm.groups * CHUNK;
     int *seg_s = lds;
     int *perm_s = lds + T;
     const long t0l = (long)xcd_block(blockIdx.x, gridDim.x) * T;
@@ -627,9 +664,11 @@ __global__ __launch_bounds__(kThreads) void scatter_bwd_kernel(
     }
     __syncthreads();
 
-    const int col = ((int)blockIdx.y << lpr_log2 | ((int)threadIdx.x & ((1 << lpr_log2) - 1))) * VEC;
-    if (col >= C) return;
-    const int la = ((int)threadIdx.x >> lpr_log2) * CHUNK;
+    const int gi = div_by(threadIdx.x, lm.per_lanes);
+    int col = ((int)blockIdx.y * lm.lanes + (int)threadIdx.x - gi * lm.lanes) * VEC;
+    if (gi >= lm.groups || col >= C) return;
+    col = min(col, C - VEC);
+    const int la = gi * CHUNK;
     const int lb = min(la + CHUNK, N - t0);
     if (la >= lb) return;
 
@@ -659,8 +698,8 @@ __global__ __launch_bounds__(kThreads) void scatter_bwd_kernel(
                 // upstream rows are re-read by the neighbouring chunk when a run
                 // straddles it (keep them cached); an arg row is consumed here and
                 // nowhere else (stream it)
-                bt.gv[i] = ld<raw, VEC>(g + o);
-                if (OP == TXS_MAX) bt.av[i] = ld_stream<int, VEC>(arg + o);
+                bt.gv[i] = ld_row<raw, VEC>(g + o);
+                if (OP == TXS_MAX) bt.av[i] = ld_hint<HINT, int, VEC>(arg + o);
                 if (OP == TXS_MEAN) bt.cnt[i] = preSum[u + 1] - preSum[u];
             }
         }
@@ -692,7 +731,7 @@ __global__ __launch_bounds__(kThreads) void scatter_bwd_kernel(
 #pragma unroll
                 for (int k = 0; k < VEC; ++k) r.v[k] = (aq.v[k] == row) ? q.v[k] : TR::zero();
             }
-            st_stream<raw, VEC>(gin + (size_t)row * C + col, r);
+            st_hint<HINT, raw, VEC>(gin + (size_t)row * C + col, r);
         }
     };
 
@@ -728,55 +767,53 @@ int fwd_chunk_for(long N, long U, int op, int elem) {
     return (elem == 4 && N < 8 * U) ? kChunkShort : kChunk;
 }
 
+bool aligned_to(const void *p, int bytes) { return ((uintptr_t)p % (uintptr_t)bytes) == 0; }
+
 struct Geometry {
     int vec_bytes;  // bytes one lane moves per row
-    int lpr_log2;   // log2(lanes that cover one row slice)
-    int ytiles;     // column tiles when a row is wider than 64 lanes
-    int chunk;      // sorted positions per lane group
+    bool hint;      // rows of whole 64-byte sectors
+    LaneMap lm;
+    int tile;       // sorted positions per workgroup
     unsigned lds_fwd_idx, lds_slots, lds_bwd;  // dynamic LDS: fwd index part (bytes), fwd slot elements, bwd bytes
     dim3 grid;
 };
 
-bool aligned_to(const void *p, int bytes) { return p == nullptr || ((uintptr_t)p % (uintptr_t)bytes) == 0; }
+unsigned reciprocal32(int d) { return d == 1 ? 0u : (unsigned)(((1ULL << 32) + (unsigned)d - 1) / (unsigned)d); }
 
-Geometry make_geometry(long N, long C, int elem, const void *p0, const void *p1, const void *p2,
-                       bool arg_used, const void *parg, int chunk, bool forward = false) {
+Geometry make_geometry(long N, long C, int elem, const void *p0, const void *p1, int chunk, bool forward) {
     Geometry g;
+    g.hint = (C * elem) % 64 == 0 && aligned_to(p0, 64) && aligned_to(p1, 64);
     // bytes per lane and row: 16 for fp32; 8 for the 2-byte types, whose kernels carry
-    // twice the registers per byte (measured 4-12 % faster than 16 on fp16 / bf16)
+    // twice the registers per byte (measured 4-12 % faster than 16 on fp16 / bf16); less only
+    // for rows shorter than that
     int vb = elem == 2 ? kHalfVecBytes : 16;
-    while (vb > elem) {
-        int vec = vb / elem;
-        bool ok = (C * elem) % vb == 0 && aligned_to(p0, vb) && aligned_to(p1, vb) && aligned_to(p2, vb);
-        if (arg_used) ok = ok && aligned_to(parg, vec * 4);
-        if (ok) break;
-        vb >>= 1;
-    }
+    while (vb / elem > C) vb >>= 1;
     g.vec_bytes = vb;
     const long vec = vb / elem;
-    const long lanes = (C + vec - 1) / vec;
-    int l2 = 0;
-    while ((1L << l2) < lanes && l2 < 6) ++l2;
-    g.lpr_log2 = l2;
-    // a tile (lane groups x chunk positions) is a whole number of wavefronts' worth of staged
-    // ids: the forward kernel finds the borders of a tile's range with one ballot each
+    const long lanes = (C + vec - 1) / vec;         // of a row
+    const long ytiles = (lanes + 63) / 64;          // column tiles: a row wider than 64 lanes is dealt to several
+    g.lm.lanes = (int)((lanes + ytiles - 1) / ytiles);
+    g.lm.groups = kThreads / g.lm.lanes;
+    g.lm.per_lanes = reciprocal32(g.lm.lanes);
+    g.lm.per_groups = reciprocal32(g.lm.groups);
     // (forward) a small input gets smaller tiles while that gives the chip more workgroups
     // (below eight per compute unit a tile's fixed costs show: 3-5 % on 200k rows of 256 bytes)
-    while (forward && chunk > 4 && N / ((long)(kThreads >> l2) * chunk) < 2048) chunk /= 2;
-    while (forward && ((long)(kThreads >> l2) * chunk) % 64 != 0) chunk *= 2;
-    g.chunk = chunk;
-    g.ytiles = (int)((lanes + (1L << l2) - 1) >> l2);
-    const long tile = (long)(kThreads >> l2) * chunk;  // sorted positions per workgroup
+    while (forward && chunk > 4 && N / ((long)g.lm.groups * chunk) < 2048) chunk /= 2;
+    long tile = (long)g.lm.groups * chunk;
+    // the forward kernel finds the borders of a tile's range with one wave ballot each: a tile
+    // is a whole number of wavefronts' worth of staged ids (its rows are dealt evenly anyway)
+    if (forward) tile = tile <= 64 ? 64 : (tile + 32) / 64 * 64;
+    g.tile = (int)tile;
     long blocks = (N + tile - 1) / tile;
     blocks = (blocks + 8 * kXcdSpan - 1) / (8 * kXcdSpan) * (8 * kXcdSpan);
     g.lds_fwd_idx = (unsigned)(((2 * (tile + kMargin + 1) + 1 + 3) & ~3L) * sizeof(int));
     g.lds_slots = (unsigned)(2 * kThreads * vec);  // carry cells: a value and a tag per element
     g.lds_bwd = (unsigned)(2 * tile * sizeof(int));
-    g.grid = dim3((unsigned)blocks, (unsigned)g.ytiles, 1);
+    g.grid = dim3((unsigned)blocks, (unsigned)ytiles, 1);
     return g;
 }
 
-template <class TR, int VEC>
+template <class TR, int VEC, bool HINT>
 hipError_t launch_fwd_op(int op, const Geometry &geo, hipStream_t st, const void *feats,
                          const int *perm, const int *seg, const int *preSum, const int *slot_of,
                          void *out, int *arg, void *scratch, int N, int C, int U, int ref_log2) {
@@ -787,8 +824,8 @@ hipError_t launch_fwd_op(int op, const Geometry &geo, hipStream_t st, const void
     dim3 blk(kThreads);
     const unsigned lds8 = geo.lds_fwd_idx + 4 * geo.lds_slots;  // staged ids, then 4-byte carry cells
 #define TXS_FWD_OP(OPC)                                                            \
-    scatter_fwd_kernel<TR, VEC, OPC><<<geo.grid, blk, lds8, st>>>(                 \
-        f, perm, seg, slot_of, o, arg, s, preSum, N, C, U, geo.lpr_log2, ref_log2, geo.chunk);
+    scatter_fwd_kernel<TR, VEC, OPC, HINT><<<geo.grid, blk, lds8, st>>>(                 \
+        f, perm, seg, slot_of, o, arg, s, preSum, N, C, U, geo.lm, ref_log2, geo.tile);
     switch (op) {
         case TXS_SUM: TXS_FWD_OP(TXS_SUM) break;
         case TXS_MEAN: TXS_FWD_OP(TXS_MEAN) break;
@@ -804,18 +841,15 @@ hipError_t launch_fwd(int op, const Geometry &geo, hipStream_t st, const void *f
                       const int *perm, const int *seg, const int *preSum, const int *slot_of,
                       void *out, int *arg, void *scratch, int N, int C, int U, int ref_log2) {
     constexpr int e = (int)sizeof(typename TR::raw);
-#define TXS_FWD(VB)                                                                              \
-    if (geo.vec_bytes == VB)                                                                     \
-        return launch_fwd_op<TR, (VB) / e>(op, geo, st, feats, perm, seg, preSum, slot_of, out,  \
-                                           arg, scratch, N, C, U, ref_log2);
-    if constexpr (e == 4 || kHalfVecBytes == 16) {
-        TXS_FWD(16)
-    }
-    TXS_FWD(8)
-    TXS_FWD(4)
-    if constexpr (e == 2) {
-        TXS_FWD(2)
-    }
+    constexpr int full = e == 2 ? kHalfVecBytes : 16;  // rows of whole sectors always take full lanes
+#define TXS_FWD(VB, HINT)                                                                              \
+    if (geo.vec_bytes == VB && geo.hint == HINT)                                                       \
+        return launch_fwd_op<TR, (VB) / e, HINT>(op, geo, st, feats, perm, seg, preSum, slot_of, out,  \
+                                                 arg, scratch, N, C, U, ref_log2);
+    TXS_FWD(full, true)
+    TXS_FWD(full, false)
+    TXS_FWD(full / 2, false)
+    TXS_FWD(full / 4, false)
 #undef TXS_FWD
     return hipErrorInvalidValue;
 }
@@ -852,7 +886,7 @@ hipError_t launch_finalize(int op, hipStream_t st, const void *feats, const int 
     return hipGetLastError();
 }
 
-template <class TR, int VEC, int CHUNK>
+template <class TR, int VEC, int CHUNK, bool HINT>
 hipError_t launch_bwd_chunk(int op, const Geometry &geo, hipStream_t st, const void *g, const int *arg,
                             const int *perm, const int *seg, const int *preSum, void *gin, int N,
                             int C, int U) {
@@ -862,46 +896,43 @@ hipError_t launch_bwd_chunk(int op, const Geometry &geo, hipStream_t st, const v
     dim3 blk(kThreads);
     switch (op) {
         case TXS_SUM:
-            scatter_bwd_kernel<TR, VEC, TXS_SUM, CHUNK><<<geo.grid, blk, geo.lds_bwd, st>>>(
-                gi, arg, perm, seg, preSum, go, N, C, U, geo.lpr_log2);
+            scatter_bwd_kernel<TR, VEC, TXS_SUM, CHUNK, HINT><<<geo.grid, blk, geo.lds_bwd, st>>>(
+                gi, arg, perm, seg, preSum, go, N, C, U, geo.lm);
             break;
         case TXS_MEAN:
-            scatter_bwd_kernel<TR, VEC, TXS_MEAN, CHUNK><<<geo.grid, blk, geo.lds_bwd, st>>>(
-                gi, arg, perm, seg, preSum, go, N, C, U, geo.lpr_log2);
+            scatter_bwd_kernel<TR, VEC, TXS_MEAN, CHUNK, HINT><<<geo.grid, blk, geo.lds_bwd, st>>>(
+                gi, arg, perm, seg, preSum, go, N, C, U, geo.lm);
             break;
         default:
-            scatter_bwd_kernel<TR, VEC, TXS_MAX, CHUNK><<<geo.grid, blk, geo.lds_bwd, st>>>(
-                gi, arg, perm, seg, preSum, go, N, C, U, geo.lpr_log2);
+            scatter_bwd_kernel<TR, VEC, TXS_MAX, CHUNK, HINT><<<geo.grid, blk, geo.lds_bwd, st>>>(
+                gi, arg, perm, seg, preSum, go, N, C, U, geo.lm);
             break;
     }
     return hipGetLastError();
 }
 
-template <class TR, int VEC>
-hipError_t launch_bwd_op(int op, const Geometry &geo, hipStream_t st, const void *g, const int *arg,
+template <class TR, int VEC, bool HINT>
+hipError_t launch_bwd_op(int op, int chunk, const Geometry &geo, hipStream_t st, const void *g, const int *arg,
                          const int *perm, const int *seg, const int *preSum, void *gin, int N, int C,
                          int U) {
-    if (geo.chunk == kChunkBwdShort)
-        return launch_bwd_chunk<TR, VEC, kChunkBwdShort>(op, geo, st, g, arg, perm, seg, preSum, gin, N, C, U);
-    return launch_bwd_chunk<TR, VEC, kChunkBwdLong>(op, geo, st, g, arg, perm, seg, preSum, gin, N, C, U);
+    if (chunk == kChunkBwdShort)
+        return launch_bwd_chunk<TR, VEC, kChunkBwdShort, HINT>(op, geo, st, g, arg, perm, seg, preSum, gin, N, C, U);
+    return launch_bwd_chunk<TR, VEC, kChunkBwdLong, HINT>(op, geo, st, g, arg, perm, seg, preSum, gin, N, C, U);
 }
 
 template <class TR>
-hipError_t launch_bwd(int op, const Geometry &geo, hipStream_t st, const void *g, const int *arg,
+hipError_t launch_bwd(int op, int chunk, const Geometry &geo, hipStream_t st, const void *g, const int *arg,
                       const int *perm, const int *seg, const int *preSum, void *gin, int N, int C,
                       int U) {
     constexpr int e = (int)sizeof(typename TR::raw);
-#define TXS_BWD(VB)                                                                               \
-    if (geo.vec_bytes == VB)                                                                      \
-        return launch_bwd_op<TR, (VB) / e>(op, geo, st, g, arg, perm, seg, preSum, gin, N, C, U);
-    if constexpr (e == 4 || kHalfVecBytes == 16) {
-        TXS_BWD(16)
-    }
-    TXS_BWD(8)
-    TXS_BWD(4)
-    if constexpr (e == 2) {
-        TXS_BWD(2)
-    }
+    constexpr int full = e == 2 ? kHalfVecBytes : 16;
+#define TXS_BWD(VB, HINT)                     \
+    if (geo.vec_bytes == VB && geo.hint == HINT) \
+        return launch_bwd_op<TR, (VB) / e, HINT>(op, chunk, geo, st, g, arg, perm, seg, preSum, gin, N, C, U);
+    TXS_BWD(full, true)
+    TXS_BWD(full, false)
+    TXS_BWD(full / 2, false)
+    TXS_BWD(full / 4, false)
 #undef TXS_BWD
     return hipErrorInvalidValue;
 }
@@ -977,7 +1008,7 @@ int scatter_forward_impl(int op, int dtype, const void *feats, const int32_t *un
         if (hipGetLastError() != hipSuccess) return TXS_ERR_LAUNCH;
     }
     if (N > 0) {
-        Geometry geo = make_geometry(N, C, elem, feats, out, nullptr, is_max, arg, fwd_chunk_for(N, U, op, elem), true);
+        Geometry geo = make_geometry(N, C, elem, feats, out, fwd_chunk_for(N, U, op, elem), true);
         if (dtype == TXS_F32)
             e = launch_fwd<F32>(op, geo, st, feats, perm, seg, preSum, slot_of, out, arg, scratch, N, C, U, ref_log2);
         else if (dtype == TXS_F16)
@@ -1041,12 +1072,11 @@ int txs_kernel_name(int backward, int op, int dtype, int64_t num_total, int64_t 
     }
     if (backward) {
         const int chunk = (num_total < (int64_t)kChunkBwdLong * num_unq) ? kChunkBwdShort : kChunkBwdLong;
-        const Geometry geo = make_geometry(num_total, channel, elem, p, p, nullptr, op == TXS_MAX, p, chunk);
+        const Geometry geo = make_geometry(num_total, channel, elem, p, p, chunk, false);
         snprintf(buf, (size_t)buf_len, "scatter_bwd_kernel<%s,%d,%s,%d>", kTypes[dtype], geo.vec_bytes / elem,
                  kOps[op], chunk);
     } else {
-        const bool is_max = op == TXS_MAX || op == TXS_MAX_REFTIE;
-        const Geometry geo = make_geometry(num_total, channel, elem, p, p, nullptr, is_max, p,
+        const Geometry geo = make_geometry(num_total, channel, elem, p, p,
                                            fwd_chunk_for(num_total, num_unq, op, elem), true);
         snprintf(buf, (size_t)buf_len, "scatter_fwd_kernel<%s,%d,%s>", kTypes[dtype], geo.vec_bytes / elem, kOps[op]);
     }
@@ -1098,14 +1128,14 @@ int txs_scatter_backward(int op, int dtype, const void *grad_out, const int32_t 
     const int elem = dtype == TXS_F32 ? 4 : 2;
     // short runs on average -> the short chunk; long runs -> the long one
     const int chunk = ((long)N < (long)kChunkBwdLong * U) ? kChunkBwdShort : kChunkBwdLong;
-    Geometry geo = make_geometry(N, C, elem, grad_out, grad_in, nullptr, op == TXS_MAX, arg, chunk);
+    Geometry geo = make_geometry(N, C, elem, grad_out, grad_in, chunk, false);
     hipError_t e;
     if (dtype == TXS_F32)
-        e = launch_bwd<F32>(op, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
+        e = launch_bwd<F32>(op, chunk, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
     else if (dtype == TXS_F16)
-        e = launch_bwd<F16>(op, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
+        e = launch_bwd<F16>(op, chunk, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
     else
-        e = launch_bwd<BF16>(op, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
+        e = launch_bwd<BF16>(op, chunk, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
     return status_of(e);
 }
 

@@ -34,9 +34,6 @@ namespace {
 #ifndef TXS_BATCH_BWD_HALF
 #define TXS_BATCH_BWD_HALF 8
 #endif
-#ifndef TXS_HALF_VEC_BYTES
-#define TXS_HALF_VEC_BYTES 8
-#endif
 #ifndef TXS_F16_NATIVE_MAX
 #define TXS_F16_NATIVE_MAX 1
 #endif
@@ -52,12 +49,6 @@ namespace {
 #ifndef TXS_FAST_DIV_HALF
 #define TXS_FAST_DIV_HALF 1
 #endif
-#ifndef TXS_NT_LOADS
-#define TXS_NT_LOADS 1
-#endif
-#ifndef TXS_NT_STORES
-#define TXS_NT_STORES 1
-#endif
 
 constexpr int kThreads = 256;        // 4 wavefronts per workgroup
 constexpr int kChunk = TXS_CHUNK;    // sorted positions per lane group (forward)
@@ -71,7 +62,7 @@ constexpr int kBatchHalf = TXS_BATCH_HALF;         // the same for the 2-byte ty
 constexpr int kBatchBwdHalf = TXS_BATCH_BWD_HALF;
 constexpr int kBatchHalfMax = TXS_BATCH_HALF_MAX;  // forward max of fp16
 constexpr int kBatchBf16Max = TXS_BATCH_BF16_MAX;  // forward max of bf16
-constexpr int kHalfVecBytes = TXS_HALF_VEC_BYTES;  // bytes one lane moves per row for fp16 / bf16
+constexpr int kHalfVecBytes = 8;  // bytes one lane moves per row for fp16 / bf16
 constexpr int kHeavyDefault = 64;    // voxels above this many rows use the atomic path
 constexpr int kTableMinRowsPerVoxel = 512;  // table mode needs at least this many rows per voxel on average
 constexpr int kSpecialBit = (int)0x80000000;
@@ -154,36 +145,49 @@ __device__ __forceinline__ void st(T *p, const Pack<T, VEC> &x) {
 // Streaming variants: data touched exactly once (feature rows on the way in,
 // input-gradient rows on the way out) is moved with the non-temporal hint so it
 // does not evict the index arrays and upstream-gradient rows that are re-read.
+//
+// The vectors these move need no more than their element's alignment: gfx950 reads and writes
+// 8 and 16 bytes at any element's address with the same instruction, so a row of 67 floats
+// takes 16-byte lanes like one of 64.
 template <typename T, int VEC>
 struct VecOf {
-    typedef T type __attribute__((ext_vector_type(VEC)));
+    typedef T wide __attribute__((ext_vector_type(VEC)));
+    typedef wide type __attribute__((aligned(sizeof(T))));
 };
 template <typename T>
 struct VecOf<T, 1> {
     typedef T type;
 };
+// a lane's vector at an element's alignment, kept in the caches
+template <typename T, int VEC>
+__device__ __forceinline__ Pack<T, VEC> ld_row(const T *p) {
+    using V = typename VecOf<T, VEC>::type;
+    V v = *reinterpret_cast<const V *>(p);
+    Pack<T, VEC> r;
+    __builtin_memcpy(&r, &v, sizeof(r));
+    return r;
+}
 template <typename T, int VEC>
 __device__ __forceinline__ Pack<T, VEC> ld_stream(const T *p) {
-#if TXS_NT_LOADS
     using V = typename VecOf<T, VEC>::type;
     V v = __builtin_nontemporal_load(reinterpret_cast<const V *>(p));
     Pack<T, VEC> r;
     __builtin_memcpy(&r, &v, sizeof(r));
     return r;
-#else
-    return ld<T, VEC>(p);
-#endif
+}
+template <typename T, int VEC>
+__device__ __forceinline__ void st_row(T *p, const Pack<T, VEC> &x) {
+    using V = typename VecOf<T, VEC>::type;
+    V v;
+    __builtin_memcpy(&v, &x, sizeof(v));
+    *reinterpret_cast<V *>(p) = v;
 }
 template <typename T, int VEC>
 __device__ __forceinline__ void st_stream(T *p, const Pack<T, VEC> &x) {
-#if TXS_NT_STORES
     using V = typename VecOf<T, VEC>::type;
     V v;
     __builtin_memcpy(&v, &x, sizeof(v));
     __builtin_nontemporal_store(v, reinterpret_cast<V *>(p));
-#else
-    st<T, VEC>(p, x);
-#endif
 }
 
 // Workgroups are handed to the 8 XCDs round-robin.  Tiles are dealt to the XCDs
