@@ -1,0 +1,68 @@
+"""Index preparation of ids that fill the bucket kernels' slices in every way: one slice or
+several, voxels with a short, a threshold-sized and a long run of rows in a slice (up to a
+slice that is one voxel), few and many voxels per bucket, grouped rows, empty voxels.  The plan
+is whole numbers with one right answer: a stable sort by voxel."""
+import numpy as np
+import pytest
+import torch
+
+import torchex_amd as T
+from torchex_amd import scatter_ext
+
+pytestmark = pytest.mark.gpu
+
+
+def _ids(kind, U, rng):
+    if kind == "even":            # short runs
+        c = rng.integers(0, 6, U)
+    elif kind == "edges":         # 63, 64, 65 rows, and runs of a slice's length and one off it
+        c = rng.choice([0, 1, 2, 63, 64, 65, 66], U, p=[.3, .3, .3, .025, .025, .025, .025])
+        c[rng.integers(0, U, 3)] = [4095, 4096, 4097]
+    elif kind == "long":          # as many long runs in a slice as fit
+        c = np.zeros(U, np.int64)
+        c[U // 3:U // 3 + 200] = 65
+        c[-1] = 1
+    else:                         # a bucket of many slices, most of it in one voxel
+        c = rng.integers(0, 3, U)
+        c[U // 2] = 40_000
+        c[U // 2 + 1:U // 2 + 40] = 700
+    return np.repeat(np.arange(U), c)
+
+
+@pytest.mark.parametrize("grouped", [False, True])
+@pytest.mark.parametrize("kind", ["even", "edges", "long", "crowded"])
+@pytest.mark.parametrize("U", [300, 2049, 5000, 70_000, 600_000])
+def test_plan_of_slices(U, kind, grouped):
+    rng = np.random.default_rng(U)
+    inv = _ids(kind, U, rng)
+    if not grouped:
+        # long stretches of one voxel in input order too, not only shuffled rows
+        rng.shuffle(inv[: inv.size // 2])
+        inv[inv.size // 2:] = inv[inv.size // 2:][::-1]
+    cnts = np.bincount(inv, minlength=U)
+    data = T.ScatterData(torch.from_numpy(inv).cuda(), torch.from_numpy(cnts).cuda())
+    order = np.argsort(inv, kind="stable")
+    pre = np.concatenate([[0], np.cumsum(cnts)])
+    assert np.array_equal(data.preSum.cpu().numpy(), pre)
+    assert (data.perm is None) == bool((np.diff(inv) >= 0).all())
+    if data.perm is not None:
+        assert np.array_equal(data.perm.cpu().numpy(), order)
+    seg = data.seg.cpu().numpy()
+    assert np.array_equal(seg & 0x7fffffff, inv[order])
+    heavy = cnts > 64 if data.num_heavy else np.zeros(U, bool)
+    assert data.num_heavy == heavy.sum() and data.max_cnt == cnts.max()
+    assert data.num_special == heavy.sum() + (cnts == 0).sum()
+    assert np.array_equal(seg < 0, heavy[inv[order]] | (cnts[inv[order]] == 0))
+    ranks = np.empty(inv.size, np.int64)
+    ranks[order] = np.arange(inv.size) - pre[inv[order]]
+    assert np.array_equal(T.ingroup_inds(torch.from_numpy(inv).cuda()).cpu().numpy(), ranks)
+
+
+def test_wrong_counts_are_refused_in_one_and_in_several_slices():
+    for rows in (3000, 30_000):
+        inv = torch.randint(0, 2500, (rows,), generator=torch.Generator().manual_seed(rows))
+        inv[: rows // 2] = 7
+        cnts = torch.bincount(inv, minlength=2500)
+        cnts[7] += 1
+        with pytest.raises(AssertionError):
+            T.ScatterData(inv.cuda(), cnts.cuda())

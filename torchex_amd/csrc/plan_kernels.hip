@@ -380,18 +380,15 @@ __global__ void seg_from_presum_kernel(const int *__restrict__ preSum, long n, i
 //   (2) exclusive scan of the digit-major histogram;
 //   (3) bucket_scatter_kernel: flags of the whole input, bucket boundaries, and the stable
 //       scatter of (id, row) pairs by bucket (wave-ballot ranking);
-//   (4) bucket_count_kernel: a bucket is cut into slices of 2048 rows (at most 64, longer ones
-//       beyond), one workgroup per slice; each counts its slice's rows per voxel (LOW digit,
+//   (4) bucket_count_kernel: a bucket is cut into slices of 4096 rows (at most 64), one workgroup
+//       per slice; where there are several, each counts its slice's rows per voxel (LOW digit,
 //       <= 11 bits) in LDS and writes the counts out;
-//   (5) bucket_plan_kernel: the same workgroups add up the counts of their bucket's slices
-//       (a voxel's count, and its rows in the slices in front), which at the same time yields
-//       the bucket's share of everything else the plan holds: CSR offsets, per-voxel counts
-//       (checked against the caller's), the special-voxel table and its slots, max_cnt; then
-//       each places its slice by the low digit, stably, writing the flagged per-position ids
-//       next to the permutation.
-// (Measured against one kernel in which every workgroup of a bucket counted the whole bucket:
-// 1M ids of a voxelised sweep 67 -> 63 us, of its pillars 64 -> 57 us, 200k ids 38 -> 41 us
-// (one launch more), and 1.25M ids of which 250k fall into 900 neighbouring voxels 198 -> 101 us.)
+//   (5) bucket_plan_kernel: the same workgroups count their slice again, or add up the counts of
+//       their bucket's slices (a voxel's count, and its rows in the slices in front), which at the
+//       same time yields the bucket's share of everything else the plan holds: CSR offsets,
+//       per-voxel counts (checked against the caller's), the special-voxel table and its slots,
+//       max_cnt; then each places its slice by the low digit, stably, writing the flagged
+//       per-position ids next to the permutation.
 // Ids of at most 11 bits need no low digit: (3) already gives the final order, and the
 // elementwise kernels used by the general sequence finish the plan.
 // Measured alternatives (1M ids of 19 bits, 0.13 ms per plan as built): an 11-bit bucket digit
@@ -413,22 +410,50 @@ int hist_items_for(long n) {
     return n >= 256L * kHistThreads * 16 ? 16 : (n >= 256L * kHistThreads * 8 ? 8 : 4);
 }
 constexpr int kHistWaves = kHistThreads / 64;
-#ifndef TXS_BKT_ITEMS
-#define TXS_BKT_ITEMS 8
-#endif
-#ifndef TXS_BKT_SLICE_CHUNKS
-#define TXS_BKT_SLICE_CHUNKS 1
-#endif
-constexpr int kBktItems = TXS_BKT_ITEMS;
-constexpr int kBktChunk = kThreads * kBktItems;        // 4096 rows per placement round
-constexpr int kBktWaves = kThreads / 64;
-constexpr int kBktSlice = TXS_BKT_SLICE_CHUNKS * kBktChunk;  // rows one workgroup places
-#ifndef TXS_BKT_MAX_SLICES
-#define TXS_BKT_MAX_SLICES 64
-#endif
-constexpr int kBktMaxSlices = TXS_BKT_MAX_SLICES;      // workgroups per bucket at most
-constexpr long kBktGiant = 262144;                     // rows in one bucket beyond which the general sequence runs
+constexpr int kBktThreads = 512;
+constexpr int kBktItems = 8;
+constexpr int kBktWaves = kBktThreads / 64;
+constexpr int kBktSlice = kBktThreads * kBktItems;     // rows one workgroup places
+constexpr int kBktMaxSlices = 64;                      // workgroups per bucket at most
+constexpr long kBktGiant = (long)kBktMaxSlices * kBktSlice;  // rows in one bucket beyond which the general sequence runs
+constexpr int kLongRun = 64;                           // rows of one voxel in a slice beyond which they are ranked by ballots
+constexpr int kMaxLongRuns = kBktSlice / (kLongRun + 1);
+static_assert(kMaxLongRuns < 64 && kBktSlice / 64 == 64, "six bits number a slice's long runs, a wave scans their chunk counts");
 constexpr int kFlagUnsorted = 1, kFlagOutOfRange = 2;
+
+// exclusive scan of one int per thread across a workgroup of WAVES wavefronts
+template <int WAVES>
+__device__ __forceinline__ int wide_exclusive_scan(int x, int *total) {
+    __shared__ int wsum[WAVES];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int inc = wave_inclusive_scan(x);
+    __syncthreads();  // wsum may still be read by a previous call
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    int off = 0, tot = 0;
+#pragma unroll
+    for (int k = 0; k < WAVES; ++k) {
+        const int v = wsum[k];
+        if (k < w) off += v;
+        tot += v;
+    }
+    *total = tot;
+    return off + inc - x;
+}
+
+// Lanes of the wavefront whose `digit` (of `bits` bits) equals this lane's, among those with
+// `valid` set; all 64 lanes take part.
+__device__ __forceinline__ unsigned long long wave_match(int digit, int bits, bool valid) {
+    const unsigned long long all = __ballot(valid);
+    unsigned lo = (unsigned)all, hi = (unsigned)(all >> 32);
+    for (int b = 0; b < bits; ++b) {
+        const unsigned mine = (unsigned)((int)((unsigned)digit << (31 - b)) >> 31);  // the bit in every position
+        const unsigned long long bal = __ballot(mine != 0u);
+        lo &= ~((unsigned)bal ^ mine);
+        hi &= ~((unsigned)(bal >> 32) ^ mine);
+    }
+    return ((unsigned long long)hi << 32) | lo;
+}
 
 // hist: [high_bins][n_tiles] digit-major (the order its exclusive scan needs); tile_flags: [n_tiles]
 template <int ITEMS>
@@ -487,10 +512,12 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
     const int *__restrict__ hist, const int *__restrict__ tile_flags, int n_tiles, long giant,
     int *__restrict__ bucket_start, int *__restrict__ stats, int *__restrict__ out_keys,
     int *__restrict__ out_rows, int2 *__restrict__ out_pairs) {
-    extern __shared__ int wcount[];  // [kHistWaves][bins], then base[bins]
+    // [bins] base_s: first destination of this tile's rows, per digit; then the larger of
+    // [kHistWaves][bins] wave counts and the tile's staged (id, row) pairs
+    extern __shared__ __align__(8) int lds_base[];
     __shared__ int s_flags;
     const int bins = 1 << high_bits;
-    int *base_s = wcount + kHistWaves * bins;  // first destination of this tile's rows, per digit
+    int *base_s = lds_base, *lds_scatter = lds_base + bins, *wcount = lds_scatter;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const unsigned long long lanes_below = (1ull << lane) - 1ull;
     if (threadIdx.x == 0) s_flags = 0;
@@ -536,7 +563,7 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
         return;
     }
 
-    // ---- stable ranking inside the tile and the scatter
+    // ---- stable ranking inside the tile
     const long wbase = tile0 + (long)w * (64 * ITEMS);
     int key[ITEMS], lrank[ITEMS];
 #pragma unroll
@@ -549,42 +576,70 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
         const bool valid = key[it] >= 0;
+        const unsigned long long mask = wave_match(valid ? key[it] >> low_bits : 0, high_bits, valid);
+        // rows of the same bucket in front of this one among the wave's 64, and the group's size
+        lrank[it] = __popcll(mask & lanes_below) | (__popcll(mask) << 8);
+    }
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+        const bool valid = key[it] >= 0;
         const int digit = valid ? (key[it] >> low_bits) : 0;
-        unsigned long long mask = __ballot(valid);
-        for (int b = 0; b < high_bits; ++b) {
-            const bool bit = (digit >> b) & 1;
-            const unsigned long long bal = __ballot(bit);
-            mask &= bit ? bal : ~bal;
-        }
-        const int below = __popcll(mask & lanes_below);
+        const int below = lrank[it] & 255, group = lrank[it] >> 8;
         const int prev = wc[digit];
         __builtin_amdgcn_wave_barrier();
-        if (valid && below == 0) wc[digit] = prev + __popcll(mask);
+        if (valid && below == 0) wc[digit] = prev + group;
         __builtin_amdgcn_wave_barrier();
         lrank[it] = prev + below;
     }
     __syncthreads();
-#pragma unroll
-    for (int it = 0; it < ITEMS; ++it) {
-        if (key[it] < 0) continue;
-        const long i = wbase + (long)it * 64 + lane;
-        const int dg = key[it] >> low_bits;
-        int before = base_s[dg];
-        for (int k = 0; k < w; ++k) before += wcount[k * bins + dg];
-        const long dst = (long)before + lrank[it];
-        if (dst >= 0 && dst < n) {
-            if (out_pairs) {
-                out_pairs[dst] = make_int2(key[it], (int)i);
-            } else {
-                out_keys[dst] = key[it];
-                out_rows[dst] = (int)i;
+    // ---- the tile's rows in bucket order: wcount[k][d] becomes the place, inside the tile, of
+    // the first row that wave k has for bucket d, base_s[d] the step from there to its destination
+    int total = 0;
+    {
+        const int per = (bins + kHistThreads - 1) / kHistThreads;
+        const int d0 = (int)threadIdx.x * per;
+        int mine = 0;
+        for (int d = d0; d < min(d0 + per, bins); ++d)
+            for (int k = 0; k < kHistWaves; ++k) mine += wcount[k * bins + d];
+        int run = wide_exclusive_scan<kHistWaves>(mine, &total);
+        for (int d = d0; d < min(d0 + per, bins); ++d) {
+            base_s[d] -= run;
+            for (int k = 0; k < kHistWaves; ++k) {
+                const int c = wcount[k * bins + d];
+                wcount[k * bins + d] = run;
+                run += c;
             }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it)
+        if (key[it] >= 0) lrank[it] += wcount[w * bins + (key[it] >> low_bits)];
+    __syncthreads();
+    // ---- through LDS (over the wave counts, which are done with): the tile's rows leave in
+    // bucket order, so that neighbouring lanes write neighbouring addresses.  Written straight
+    // from the ranking, every 8-byte pair was a memory request of its own.  (4M ids in
+    // 1024 buckets: 37.6 -> 28.5 us; 1M ids, whose tiles hold four rows per bucket only: 15.2 -> 15.6)
+    int2 *stage = reinterpret_cast<int2 *>(lds_scatter);
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it)
+        if (key[it] >= 0) stage[lrank[it]] = make_int2(key[it], (int)(wbase + (long)it * 64 + lane));
+    __syncthreads();
+    for (int p = threadIdx.x; p < total; p += kHistThreads) {
+        const int2 kr = stage[p];
+        const long dst = (long)base_s[kr.x >> low_bits] + p;
+        if (dst < 0 || dst >= n) continue;
+        if (out_pairs) {
+            out_pairs[dst] = kr;
+        } else {
+            out_keys[dst] = kr.x;
+            out_rows[dst] = kr.y;
         }
     }
 }
 
 // Rows of bucket b that slice j of it covers.  A bucket is cut into slices of kBktSlice rows,
-// at most kBktMaxSlices of them (longer slices beyond that).
+// at most kBktMaxSlices of them (the call goes to the general sequence where that is not enough).
 struct BucketSlice {
     long s, e;        // the bucket's rows [s, e) in bucket order
     long my_s, my_e;  // the slice's rows
@@ -597,24 +652,20 @@ __device__ __forceinline__ BucketSlice bucket_slice(long s, long e, int j) {
     BucketSlice r;
     r.s = s;
     r.e = e;
-    const long nb = r.e - r.s;
-    r.nsl = slices_of(nb);
-    long slice = kBktSlice;
-    if (nb > (long)kBktMaxSlices * kBktSlice)
-        slice = ((nb + kBktMaxSlices - 1) / kBktMaxSlices + kBktChunk - 1) / kBktChunk * kBktChunk;
-    r.my_s = r.s + (long)j * slice;
-    r.my_e = min(r.e, r.my_s + slice);
+    r.nsl = slices_of(e - s);
+    r.my_s = s + (long)j * kBktSlice;
+    r.my_e = min(e, r.my_s + kBktSlice);
     return r;
 }
 
 // Workgroup g serves slice j of bucket b; (b, j) follows from the bucket sizes and is kept with
 // the bucket's bounds in wg_pick[g] = (b, j, start, end) (b = -1: no work) for the kernel that
-// follows, which so learns its work from one load.  Each workgroup
-// counts the rows of ITS slice per voxel (low digit) and writes the counts to part_hist[g][*]:
-// the slices of a bucket sit in consecutive workgroups, so the next kernel gets a voxel's count in
-// the whole bucket, and in the slices in front of its own, from at most kBktMaxSlices short
-// reads instead of every workgroup of a crowded bucket counting all of its rows.
-__global__ __launch_bounds__(kThreads) void bucket_count_kernel(
+// follows, which so learns its work from one load.  Where a bucket has several slices, each
+// workgroup counts the rows of ITS slice per voxel (low digit) and writes the counts to
+// part_hist[g][*]: the slices of a bucket sit in consecutive workgroups, so the next kernel gets a
+// voxel's count in the whole bucket, and in the slices in front of its own, from at most
+// kBktMaxSlices short reads instead of every workgroup of a crowded bucket counting all of its rows.
+__global__ __launch_bounds__(kBktThreads) void bucket_count_kernel(
     const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U, int low_bits, int high_bins,
     const int *__restrict__ bucket_start, const int *__restrict__ stats, int4 *__restrict__ wg_pick,
     int *__restrict__ part_hist) {
@@ -625,13 +676,13 @@ __global__ __launch_bounds__(kThreads) void bucket_count_kernel(
     {
         if (threadIdx.x == 0) s_pick[0] = -1;
         int carried = 0;
-        for (int bb0 = 0; bb0 < high_bins; bb0 += kThreads) {
+        for (int bb0 = 0; bb0 < high_bins; bb0 += kBktThreads) {
             const int bb = bb0 + (int)threadIdx.x;
             int nsl = 0;
             if (bb < high_bins && ((long)bb << low_bits) < (long)U)
                 nsl = slices_of((long)bucket_start[bb + 1] - bucket_start[bb]);
             int total;
-            const int first = carried + block_exclusive_scan(nsl, &total);  // (synchronises the workgroup)
+            const int first = carried + wide_exclusive_scan<kBktWaves>(nsl, &total);  // (synchronises the workgroup)
             if ((int)blockIdx.x >= first && (int)blockIdx.x < first + nsl) {
                 s_pick[0] = bb;
                 s_pick[1] = (int)blockIdx.x - first;
@@ -650,138 +701,165 @@ __global__ __launch_bounds__(kThreads) void bucket_count_kernel(
     const int *keys = packed ? pairs1 : inv;
     const BucketSlice sl = bucket_slice(bucket_start[b], bucket_start[b + 1], j);
     if (threadIdx.x == 0) wg_pick[blockIdx.x] = make_int4(b, j, (int)sl.s, (int)sl.e);
-    for (int k = threadIdx.x; k < low_bins; k += kThreads) cnt_s[k] = 0;
+    if (sl.nsl == 1) return;  // (uniform) the next kernel counts the bucket itself
+    for (int k = threadIdx.x; k < low_bins; k += kBktThreads) cnt_s[k] = 0;
     __syncthreads();
-    for (long i0 = sl.my_s; i0 < sl.my_e; i0 += (long)kThreads * kBktItems) {
-        int v[kBktItems];
+    int v[kBktItems];
 #pragma unroll
-        for (int it = 0; it < kBktItems; ++it) {
-            const long i = i0 + (long)it * kThreads + threadIdx.x;
-            v[it] = i < sl.my_e ? kread(keys, i, packed) : -1;
-        }
+    for (int it = 0; it < kBktItems; ++it) {
+        const long i = sl.my_s + (long)it * kBktThreads + threadIdx.x;
+        v[it] = i < sl.my_e ? kread(keys, i, packed) : -1;
+    }
 #pragma unroll
-        for (int it = 0; it < kBktItems; ++it) {
-            const int d = v[it] - u_lo;
-            if (v[it] >= 0 && (unsigned)d < (unsigned)low_bins) atomicAdd(&cnt_s[d], 1);
-        }
+    for (int it = 0; it < kBktItems; ++it) {
+        const int d = v[it] - u_lo;
+        if (v[it] >= 0 && (unsigned)d < (unsigned)low_bins) atomicAdd(&cnt_s[d], 1);
     }
     __syncthreads();
     int *mine = part_hist + (long)blockIdx.x * low_bins;
-    for (int k = threadIdx.x; k < low_bins; k += kThreads) mine[k] = cnt_s[k];
+    for (int k = threadIdx.x; k < low_bins; k += kBktThreads) mine[k] = cnt_s[k];
 }
 
-__global__ __launch_bounds__(kThreads) void bucket_plan_kernel(
+// One slice: its rows are counted per voxel by LDS atomics, whose returned values put them, voxel
+// by voxel, into LDS in whatever order the atomics ran; each row then finds its place among its
+// voxel's rows of the slice by counting the smaller row numbers there (rows ascend along a bucket,
+// so that is the stable order).  That costs as many reads as the voxel has rows in the slice: runs
+// above kLongRun rows (at most kMaxLongRuns of them in a slice) are ranked by wave ballots on a
+// six-bit number instead, with a count per run and 64 rows in input order.  Rows leave in voxel
+// order, neighbouring lanes to neighbouring addresses.
+// What bounds it is the chain of dependent steps inside a workgroup, far more than bytes: 50 KB of
+// LDS keep 24 waves on a compute unit (the ballots on all 11 bits that this replaces needed a count
+// per wave and voxel as well, left 12, and wrote every row as a request of its own).  4M ids of four
+// sweeps (1.3M voxels, 64 MB moved): 103 -> 45 us; 1M ids, ranks only: 31 -> 21.5 us.
+__global__ __launch_bounds__(kBktThreads) void bucket_plan_kernel(
     const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U,
-    int low_bits, int high_bins, const int *__restrict__ bucket_start, int heavy_threshold,
+    int low_bits, const int *__restrict__ bucket_start, int heavy_threshold,
     const long long *__restrict__ unq_cnts, int *__restrict__ perm, int *__restrict__ seg,
     int *__restrict__ preSum, int *__restrict__ slot_of, int *__restrict__ heavy_ids,
     int *__restrict__ stats, const int4 *__restrict__ wg_pick, const int *__restrict__ part_hist,
     long long *__restrict__ ranks) {
     // ranks != NULL: the caller wants the rank of every row inside its voxel and nothing else
-    // (ingroup_inds): off[] then counts from the voxel's first row instead of the bucket's,
-    // and the placement writes ranks[row] in place of the permutation and the ids
+    // (ingroup_inds): the placement writes ranks[row] in place of the permutation and the ids
     const bool rank_mode = ranks != nullptr;
-    extern __shared__ int wc[];  // [kBktWaves][low_bins], tot[low_bins], off[low_bins]
-    __shared__ int s_red[kBktWaves], s_bad[kBktWaves];
+    constexpr int kBins = 1 << kBucketLowBitsMax;
+    __shared__ int row_s[kBktSlice];              // the slice's rows in voxel order; before that, its bucket's counts
+    __shared__ unsigned short dig_s[kBktSlice];   // their voxels (low digits)
+    __shared__ int first_s[kBins + 1];            // the slice's counts, then the first place of every voxel in row_s
+    __shared__ int step_s[kBins];                 // rows of the voxel in front of this slice, then place -> destination
+    __shared__ unsigned char mark_s[kBins];       // bits 0-5: number of a long run + 1 (0: short); bit 7: heavy voxel
+    __shared__ unsigned short chunk_s[kMaxLongRuns][64];  // a long run's rows per 64 rows of the slice
+    __shared__ int s_red[kBktWaves], s_bad[kBktWaves], s_long;
+    static_assert(kBins <= kBktSlice, "the bucket's counts share the rows' space");
+    int *tot = row_s;
     const int low_bins = 1 << low_bits;
-    int *tot = wc + kBktWaves * low_bins;
-    int *off = tot + low_bins;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const unsigned long long lanes_below = (1ull << lane) - 1ull;
     if (stats[TXS_STAT_NEED_GENERAL] != 0) return;
-    (void)high_bins;
     const int4 pick = wg_pick[blockIdx.x];
     const int b = pick.x, j = pick.y;
     if (b < 0) return;
     const int u_lo = b << low_bits;
     const int u_hi = min(U, u_lo + low_bins);
     const bool unsorted = stats[TXS_STAT_UNSORTED] != 0;
-    const bool packed = unsorted;
     const BucketSlice sl = bucket_slice(pick.z, pick.w, j);
     const long s = sl.s, e = sl.e, my_s = sl.my_s, my_e = sl.my_e;
 
-    // Everything the workgroup reads from memory is requested here, in one go: the first
-    // round of the slice's rows, the caller's counts of this bucket's voxels (first slice
-    // only; compared once the kernel's own counts are complete), and the per-slice counts.
-    auto load_round = [&](long c0, int (&key)[kBktItems], int (&row)[kBktItems]) {
-        const long wbase = c0 + (long)w * (64 * kBktItems);
+    // Everything the workgroup reads from memory is requested here, in one go: the slice's rows
+    // and the caller's counts of this bucket's voxels (first slice only; compared once the
+    // kernel's own counts are complete).
+    int dig[kBktItems], row[kBktItems];
 #pragma unroll
-        for (int it = 0; it < kBktItems; ++it) {
-            const long i = wbase + (long)it * 64 + lane;
-            int v = -1;
-            row[it] = (int)i;
-            if (i < my_e) {
-                if (packed) {
-                    const int2 kr = reinterpret_cast<const int2 *>(pairs1)[i];
-                    v = kr.x;
-                    row[it] = kr.y;
-                } else {
-                    v = inv[i];
-                }
+    for (int it = 0; it < kBktItems; ++it) {
+        const long i = my_s + (long)it * kBktThreads + threadIdx.x;
+        int v = -1;
+        row[it] = (int)i;
+        if (i < my_e) {
+            if (unsorted) {
+                const int2 kr = reinterpret_cast<const int2 *>(pairs1)[i];
+                v = kr.x;
+                row[it] = kr.y;
+            } else {
+                v = inv[i];
             }
-            key[it] = (i < my_e && (unsigned)(v - u_lo) < (unsigned)low_bins) ? v : -1;
         }
-    };
-    int key0[kBktItems], row0[kBktItems];
-    load_round(my_s, key0, row0);
-    constexpr int kCntPer = (1 << kBucketLowBitsMax) / kThreads;
+        dig[it] = (i < my_e && (unsigned)(v - u_lo) < (unsigned)low_bins) ? v - u_lo : -1;
+    }
+    constexpr int kCntPer = kBins / kBktThreads;
     long long given[kCntPer];
     const bool check_counts = j == 0 && unq_cnts != nullptr;
     if (check_counts) {
 #pragma unroll
         for (int k = 0; k < kCntPer; ++k) {
-            const int d = k * kThreads + (int)threadIdx.x;
+            const int d = k * kBktThreads + (int)threadIdx.x;
             given[k] = (d < low_bins && u_lo + d < u_hi) ? unq_cnts[u_lo + d] : -1;
         }
     }
-    // ---- counts of the bucket's voxels, and of the rows in front of this slice: sums over the
-    // per-slice counts of the bucket's workgroups (blockIdx.x - j is the bucket's first), eight
-    // loads in flight per thread
-    for (int k = threadIdx.x; k < (kBktWaves + 2) * low_bins; k += kThreads) wc[k] = 0;
+    for (int k = threadIdx.x; k < low_bins; k += kBktThreads) {
+        tot[k] = 0;
+        first_s[k] = 0;
+        step_s[k] = 0;
+    }
+    if (threadIdx.x == 0) s_long = 0;
     __syncthreads();
-    {
+    // ---- the slice's rows per voxel; a row's turn among them, for now in any order
+    int turn[kBktItems];
+#pragma unroll
+    for (int it = 0; it < kBktItems; ++it) turn[it] = dig[it] >= 0 ? atomicAdd(&first_s[dig[it]], 1) : 0;
+    // ---- several slices: counts of the bucket's voxels, and of the rows in front of this slice, as
+    // sums over the per-slice counts of the bucket's workgroups (blockIdx.x - j is the bucket's
+    // first), eight loads in flight per thread
+    if (sl.nsl > 1) {
         const int *first = part_hist + ((long)blockIdx.x - j) * low_bins;
         const int total = sl.nsl << low_bits;
         constexpr int kGather = 8;
-        for (int i0 = threadIdx.x; i0 < total; i0 += kThreads * kGather) {
+        for (int i0 = threadIdx.x; i0 < total; i0 += kBktThreads * kGather) {
             int c[kGather];
 #pragma unroll
             for (int q = 0; q < kGather; ++q) {
-                const int i = i0 + q * kThreads;
+                const int i = i0 + q * kBktThreads;
                 c[q] = i < total ? first[i] : 0;
             }
 #pragma unroll
             for (int q = 0; q < kGather; ++q) {
-                const int i = i0 + q * kThreads;
+                const int i = i0 + q * kBktThreads;
                 if (c[q] == 0) continue;
                 const int d = i & (low_bins - 1), k = i >> low_bits;
                 atomicAdd(&tot[d], c[q]);
-                if (k < j) atomicAdd(&off[d], c[q]);
+                if (k < j) atomicAdd(&step_s[d], c[q]);
             }
         }
     }
     __syncthreads();
-    // ---- exclusive scan over the voxels of the bucket: a run of consecutive voxels per thread
-    const int per = (low_bins + kThreads - 1) / kThreads;
-    const int d0 = threadIdx.x * per;
-    int mine = 0;
-    for (int k = 0; k < per; ++k)
-        if (d0 + k < low_bins) mine += tot[d0 + k];
-    int total;
-    int run = block_exclusive_scan(mine, &total);
-    // off[d] becomes the bucket-relative position of the slice's first row of voxel d
-    for (int k = 0; k < per; ++k) {
-        const int d = d0 + k;
-        if (d >= low_bins) break;
-        const int c = tot[d];
-        const int excl = run;
-        run += c;
-        if (!rank_mode) off[d] += excl;
+    // ---- exclusive scans over the voxels of the bucket, a run of consecutive voxels per thread:
+    // of the slice's counts and (the same where there is one slice) of the bucket's
+    const int per = (low_bins + kBktThreads - 1) / kBktThreads;
+    const int d0 = (int)threadIdx.x * per, d1 = min(d0 + per, low_bins);
+    int mine = 0, mine_all = 0;
+    for (int d = d0; d < d1; ++d) {
+        mine += first_s[d];
+        if (sl.nsl > 1) mine_all += tot[d];
+    }
+    int placed, ignored;
+    int run = wide_exclusive_scan<kBktWaves>(mine, &placed);
+    int run_all = sl.nsl > 1 ? wide_exclusive_scan<kBktWaves>(mine_all, &ignored) : run;
+    for (int d = d0; d < d1; ++d) {
+        const int c = first_s[d];
+        const int c_all = sl.nsl > 1 ? tot[d] : c;
+        if (sl.nsl == 1) tot[d] = c;
+        int mark = c_all > heavy_threshold ? 128 : 0;
+        if (c > kLongRun) mark |= 1 + atomicAdd(&s_long, 1);
+        mark_s[d] = (unsigned char)mark;
+        first_s[d] = run;
+        // ranks count from the voxel's first row, positions from the bucket's start
+        step_s[d] += (rank_mode ? 0 : (int)s + run_all) - run;
         if (j == 0 && u_lo + d < u_hi) {
-            preSum[u_lo + d] = (int)s + excl;
+            preSum[u_lo + d] = (int)s + run_all;
             if (u_lo + d == U - 1) preSum[U] = (int)n;
         }
+        run += c;
+        run_all += c_all;
     }
+    if (threadIdx.x == 0) first_s[low_bins] = placed;
     __syncthreads();
     // ---- statistics, special voxels and their slots (first slice only; as plan_special_kernel)
     if (j == 0 && slot_of != nullptr) {
@@ -790,11 +868,11 @@ __global__ __launch_bounds__(kThreads) void bucket_plan_kernel(
         if (check_counts) {
 #pragma unroll
             for (int k = 0; k < kCntPer; ++k) {
-                const int d = k * kThreads + (int)threadIdx.x;
+                const int d = k * kBktThreads + (int)threadIdx.x;
                 if (d < low_bins && u_lo + d < u_hi) mismatch |= given[k] != (long long)tot[d];
             }
         }
-        for (int dd = 0; dd < low_bins; dd += kThreads) {
+        for (int dd = 0; dd < low_bins; dd += kBktThreads) {
             const int d = dd + (int)threadIdx.x;
             const int u = u_lo + d;
             const bool in = d < low_bins && u < u_hi;
@@ -829,7 +907,7 @@ __global__ __launch_bounds__(kThreads) void bucket_plan_kernel(
             s_red[w] = wmax;
             s_bad[w] = any_mismatch;
         }
-        __syncthreads();
+        __syncthreads();  // (also: the last read of tot, whose space the rows take next)
         if (threadIdx.x == 0) {
             int m = 0, bad = 0;
             for (int k = 0; k < kBktWaves; ++k) {
@@ -841,67 +919,66 @@ __global__ __launch_bounds__(kThreads) void bucket_plan_kernel(
         }
     }
 
-    // ---- stable placement of the slice by the low digit, round after round
-    for (long c0 = my_s; c0 < my_e; c0 += kBktChunk) {
-        int key[kBktItems], row[kBktItems], lrank[kBktItems];
-        volatile int *mywc = wc + w * low_bins;
-        if (c0 == my_s) {
-#pragma unroll
-            for (int it = 0; it < kBktItems; ++it) {
-                key[it] = key0[it];
-                row[it] = row0[it];
-            }
-        } else {
-            load_round(c0, key, row);
+    // what is known of a row once its place p in voxel order is: p's destination
+    auto put = [&](int d, int p, int row_i) {
+        const long dst = (long)step_s[d] + p;
+        if (rank_mode) {
+            if ((unsigned)row_i < (unsigned)n) ranks[row_i] = dst;
+        } else if (unsorted && dst >= s && dst < e) {
+            perm[dst] = row_i;
         }
+    };
+    // ---- long runs: straight from the registers, ranked by 64 rows in input order at a time
+    const int n_long = s_long;  // (uniform)
+    if (n_long > 0) {
+        for (int k = threadIdx.x; k < n_long * 64; k += kBktThreads) (&chunk_s[0][0])[k] = 0;
+        __syncthreads();
 #pragma unroll
         for (int it = 0; it < kBktItems; ++it) {
-            const bool valid = key[it] >= 0;
-            const int digit = valid ? key[it] - u_lo : 0;
-            unsigned long long mask = __ballot(valid);
-            for (int bb = 0; bb < low_bits; ++bb) {
-                const bool bit = (digit >> bb) & 1;
-                const unsigned long long bal = __ballot(bit);
-                mask &= bit ? bal : ~bal;
-            }
+            const int id = dig[it] >= 0 ? (mark_s[dig[it]] & 63) : 0;
+            const unsigned long long mask = wave_match(id, 6, id > 0);
             const int below = __popcll(mask & lanes_below);
-            const int prev = mywc[digit];
-            __builtin_amdgcn_wave_barrier();
-            if (valid && below == 0) mywc[digit] = prev + __popcll(mask);
-            __builtin_amdgcn_wave_barrier();
-            lrank[it] = prev + below;
-        }
-        __syncthreads();
-        // destination = slice-start position of the voxel + rows of the voxel that the waves
-        // in front of this one hold in this pass + rank inside the wave; the per-voxel
-        // bookkeeping is done per ROW (a few LDS operations each), never per voxel: a pass
-        // has fewer rows than a bucket can have voxel-times-wave counters
-        long dst[kBktItems];
-#pragma unroll
-        for (int it = 0; it < kBktItems; ++it) {
-            dst[it] = -1;
-            if (key[it] < 0) continue;
-            const int dg = key[it] - u_lo;
-            int before = off[dg];
-            for (int k = 0; k < w; ++k) before += wc[k * low_bins + dg];
-            dst[it] = s + before + lrank[it];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < kBktItems; ++it) {
-            if (key[it] < 0) continue;
-            const int dg = key[it] - u_lo;
-            atomicAdd(&off[dg], 1);       // the next pass starts behind this pass's rows
-            wc[w * low_bins + dg] = 0;    // (every row of the group stores the same zero)
-            if (rank_mode) {
-                if ((unsigned)row[it] < (unsigned)n) ranks[row[it]] = (long long)(dst[it] - s);
-            } else if (dst[it] >= s && dst[it] < e) {
-                const int c = tot[dg];
-                seg[dst[it]] = key[it] | (c > heavy_threshold ? kSpecialBit : 0);
-                if (unsorted) perm[dst[it]] = row[it];
+            if (id > 0) {
+                turn[it] = below;
+                if (below == 0) chunk_s[id - 1][it * kBktWaves + w] = (unsigned short)__popcll(mask);
             }
         }
         __syncthreads();
+        for (int k = w; k < n_long; k += kBktWaves) {
+            const int c = chunk_s[k][lane];
+            chunk_s[k][lane] = (unsigned short)(wave_inclusive_scan(c) - c);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < kBktItems; ++it) {
+            const int id = dig[it] >= 0 ? (mark_s[dig[it]] & 63) : 0;
+            if (id > 0) put(dig[it], first_s[dig[it]] + chunk_s[id - 1][it * kBktWaves + w] + turn[it], row[it]);
+        }
+    }
+    // ---- short runs: into voxel order, then by the number of smaller rows in the run
+#pragma unroll
+    for (int it = 0; it < kBktItems; ++it) {
+        if (dig[it] < 0) continue;
+        // (a long run's rows are placed already: any of its places will do for its ids)
+        const int id = mark_s[dig[it]] & 63;
+        const int p = first_s[dig[it]] +
+                      (id > 0 ? chunk_s[id - 1][it * kBktWaves + w] + turn[it] : turn[it]);
+        row_s[p] = row[it];
+        dig_s[p] = (unsigned short)dig[it];
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < placed; p += kBktThreads) {
+        const int d = dig_s[p];
+        const int mark = mark_s[d];
+        if (!rank_mode) {
+            const long dst = (long)step_s[d] + p;
+            if (dst >= s && dst < e) seg[dst] = (u_lo + d) | ((mark & 128) ? kSpecialBit : 0);
+        }
+        if ((mark & 63) != 0 || (!rank_mode && !unsorted)) continue;
+        const int a = first_s[d], z = first_s[d + 1], row_i = row_s[p];
+        int smaller = 0;
+        for (int q = a; q < z; ++q) smaller += row_s[q] < row_i;
+        put(d, a + smaller, row_i);
     }
 }
 
@@ -1183,7 +1260,8 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
                                                               n_tiles);
     // one entry more than the histogram: it receives the total, the end of the last bucket
     if (exclusive_scan(hist, used, hist, used + 1, scan_ws, st) != hipSuccess) return TXS_ERR_LAUNCH;
-    const size_t lds_scatter = (size_t)(kHistWaves + 1) * high_bins * sizeof(int);
+    const size_t lds_scatter = (size_t)high_bins * sizeof(int) +
+                               max((size_t)kHistWaves * high_bins * sizeof(int), (size_t)tile * sizeof(int2));
     if (low_bits == 0) {
         // a bucket is a voxel: the scatter already gives the final order
         scatter_kernel<<<dim3(n_tiles), dim3(kHistThreads), lds_scatter, st>>>(
@@ -1204,11 +1282,10 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
         unq_inv, n, U, low_bits, high_bits, hist, tile_flags, n_tiles, giant, bucket_start, stats, nullptr,
         nullptr, reinterpret_cast<int2 *>(pairs1));
     const int low_bins = 1 << low_bits;
-    const size_t lds = (size_t)(kBktWaves + 2) * low_bins * sizeof(int);
-    bucket_count_kernel<<<dim3((unsigned)groups), dim3(kThreads), (size_t)low_bins * sizeof(int), st>>>(
+    bucket_count_kernel<<<dim3((unsigned)groups), dim3(kBktThreads), (size_t)low_bins * sizeof(int), st>>>(
         unq_inv, pairs1, n, U, low_bits, high_bins, bucket_start, stats, reinterpret_cast<int4 *>(wg_pick), part_hist);
-    bucket_plan_kernel<<<dim3((unsigned)groups), dim3(kThreads), lds, st>>>(
-        unq_inv, pairs1, n, U, low_bits, high_bins, bucket_start, heavy_threshold,
+    bucket_plan_kernel<<<dim3((unsigned)groups), dim3(kBktThreads), 0, st>>>(
+        unq_inv, pairs1, n, U, low_bits, bucket_start, heavy_threshold,
         (const long long *)unq_cnts, perm, seg, preSum, slot_of, heavy_ids, stats,
         reinterpret_cast<const int4 *>(wg_pick), part_hist, ranks);
     return status_of(hipGetLastError());
