@@ -336,6 +336,34 @@ int txs_grid_hash_build(const int32_t *keys, const int32_t *values, int64_t num_
 int txs_grid_hash_probe(const int32_t *keys, int64_t num_keys, const int32_t *table,
                         int64_t table_size, int32_t *out_values, void *stream);
 
+/* The same hash over the distinct rows of voxel coordinates (what GridHash of
+ * torchex/operator_py/grid_hash.py:59-104 builds from torch.unique(coors, dim=0)), in three
+ * calls with a read-back after the first two:
+ *   txs_coor_max: the largest coordinate per axis, as txs_coor_max_parts() partial triples
+ *     (int64 [parts, 3]) for the host to fold; dims = largest + 1.
+ *   txs_coor_bitmap_count: occupancy bitmap of the linear keys (x * dims[1] + y) * dims[2] + z
+ *     (cut to 32 bits) and its scanned population counts.  bitmap_ws: int32 array of
+ *     txs_unique_bitmap_workspace_len(dims[0] * dims[1] * dims[2]) entries, 16-byte aligned; its
+ *     entries [off, off + 2), off = txs_coor_bitmap_count_offset(key bound), then hold the number
+ *     of distinct keys and a flag, nonzero if a key lies outside [0, key bound).
+ *   txs_grid_hash_index: table int32 [table_size, 2] (a power of two >= num_unq) of (key, rank of
+ *     the key among the distinct keys); valid [table_size] 1 for occupied slots; valid_table
+ *     int32 [num_unq, 2] the occupied slots in slot order; index_ws: int32 array of
+ *     txs_grid_hash_index_workspace_len entries.
+ * coors: int32 or int64 [num_total, 3], num_total > 0.  txs_grid_hash_probe_coors probes with
+ * coordinates linearised the same way (in their own integer type, then cut to 32 bits). */
+int txs_coor_max_parts(void);
+int txs_coor_max(const void *coors, int coor_is_int64, int64_t num_total, int64_t *parts, void *stream);
+int64_t txs_coor_bitmap_count_offset(int64_t key_bound);
+int txs_coor_bitmap_count(const void *coors, int coor_is_int64, int64_t num_total, const int64_t *dims,
+                          int32_t *bitmap_ws, void *stream);
+int64_t txs_grid_hash_index_workspace_len(int64_t num_unq, int64_t table_size);
+int txs_grid_hash_index(const int32_t *bitmap_ws, int64_t key_bound, int64_t num_unq, int32_t *table,
+                        int64_t table_size, int32_t *index_ws, unsigned char *valid, int32_t *valid_table,
+                        void *stream);
+int txs_grid_hash_probe_coors(const void *coors, int coor_is_int64, int64_t num_coors, int64_t dim1, int64_t dim2,
+                              const int32_t *table, int64_t table_size, int32_t *out_values, void *stream);
+
 /* ---- the hot path --------------------------------------------------------- */
 
 /* Forward reduction.  Replaces scatter_sum_launcher / scatter_max_launcher

@@ -103,19 +103,40 @@ __global__ void unique_finish_kernel(const int *__restrict__ ks, const int *__re
 // inside its word.  That is the inverse torch.unique returns (ids ascend with the keys),
 // found without sorting the keys.
 
-__global__ void bytemap_clear_kernel(uint4 *__restrict__ map16, long n16) {
+// Where the keys come from: an array of them, or voxel coordinates [n, 3], linearised here
+// (x-major, and cut to 32 bits before the range check, as a caller who stores int32 keys would).
+template <typename K>
+struct FlatKeys {
+    const K *p;
+    __device__ __forceinline__ long operator()(long i) const { return (long)p[i]; }
+};
+template <typename K>
+struct CoorKeys {
+    const K *p;
+    long s0, s1;  // strides of x and y in the key
+    __device__ __forceinline__ long operator()(long i) const {
+        const K *c = p + 3 * i;
+        return (long)(int)(unsigned)((unsigned long)c[0] * (unsigned long)s0 + (unsigned long)c[1] * (unsigned long)s1 +
+                                     (unsigned long)c[2]);
+    }
+};
+
+// bad (may be NULL): an int cleared along with the map
+__global__ void bytemap_clear_kernel(uint4 *__restrict__ map16, long n16, int *__restrict__ bad) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n16) map16[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (bad && i == 0) bad[0] = 0;
 }
 
-template <typename K>
-__global__ void bytemap_mark_kernel(const K *__restrict__ keys, long n, long key_bound,
-                                    unsigned char *__restrict__ map, int *__restrict__ stats) {
+// bad: set to 1 if a key lies outside [0, key_bound)
+template <class Keys>
+__global__ void bytemap_mark_kernel(Keys keys, long n, long key_bound, unsigned char *__restrict__ map,
+                                    int *__restrict__ bad) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const long k = (long)keys[i];
+    const long k = keys(i);
     if (k < 0 || k >= key_bound) {
-        stats[TXS_STAT_OUT_OF_RANGE] = 1;
+        bad[0] = 1;
         return;
     }
     map[k] = 1;
@@ -450,6 +471,7 @@ __device__ __forceinline__ int grid_hash_slot(int key, int probe_i, int table_si
     return (int)(((k & mask) + (unsigned long long)probe_i * (k * 2ull + 1ull)) & mask);
 }
 
+// values == NULL: key number i gets the value i
 __global__ void grid_hash_build_kernel(const int *__restrict__ keys, const int *__restrict__ values,
                                        unsigned long long *__restrict__ table, int table_size, long n,
                                        int *__restrict__ fail) {
@@ -457,7 +479,7 @@ __global__ void grid_hash_build_kernel(const int *__restrict__ keys, const int *
     if (i >= n) return;
     const int key = keys[i];
     const unsigned long long word =
-        ((unsigned long long)(unsigned)values[i] << 32) | (unsigned long long)(unsigned)key;
+        ((unsigned long long)(unsigned)(values ? values[i] : (int)i) << 32) | (unsigned long long)(unsigned)key;
     const unsigned long long empty = ~0ull;  // (-1, -1)
     for (int t = 0; key >= 0 && t < table_size; ++t) {
         const int s = grid_hash_slot(key, t, table_size);
@@ -466,27 +488,152 @@ __global__ void grid_hash_build_kernel(const int *__restrict__ keys, const int *
     if (fail) fail[0] = 1;  // table full or key negative (the reference asserts)
 }
 
-__global__ void grid_hash_probe_kernel(const int *__restrict__ keys,
-                                       const unsigned long long *__restrict__ table, int table_size,
-                                       long n, int *__restrict__ out) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int key = keys[i];
-    int v = -1;
+__device__ __forceinline__ int grid_hash_find(int key, const unsigned long long *__restrict__ table, int table_size) {
     for (int t = 0; key >= 0 && t < table_size; ++t) {
-        const int s = grid_hash_slot(key, t, table_size);
-        const unsigned long long word = table[s];
+        const unsigned long long word = table[grid_hash_slot(key, t, table_size)];
         const int slot_key = (int)(unsigned)(word & 0xffffffffull);
-        if (slot_key == key) {
-            v = (int)(unsigned)(word >> 32);
-            break;
-        }
+        if (slot_key == key) return (int)(unsigned)(word >> 32);
         // An empty slot on the probe sequence proves the key was never inserted
         // (no deletions).  The reference keeps scanning all table_size slots
         // before giving up (functions.cuh:54-63), with the same answer.
         if (slot_key == -1) break;
     }
-    out[i] = v;
+    return -1;
+}
+
+template <class Keys>
+__global__ void grid_hash_probe_kernel(Keys keys, const unsigned long long *__restrict__ table, int table_size,
+                                       long n, int *__restrict__ out) {
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = grid_hash_find((int)keys(i), table, table_size);
+}
+
+// ---- a hash of the distinct voxel coordinates -------------------------------------
+// From the occupancy map of the coordinates' grid (as above: distinct keys in ascending order
+// without a sort), so that the coordinates are read twice, once for the grid's extents and once
+// to mark the map, and never stored as keys.  300k rows of a sweep, 146k of them
+// distinct in 16.7M cells, built and probed with another 300k: 307 us of kernels in 44 launches
+// (the sort's plan, the linearised keys and the valid slots by library calls) -> 73 us in 13.
+
+// Largest coordinate per axis, one partial [3] per workgroup (the host folds the few of them).
+constexpr int kCoorMaxParts = 128;
+template <typename K>
+__global__ __launch_bounds__(kThreads) void coor_max_kernel(const K *__restrict__ coors, long n,
+                                                            long long *__restrict__ parts) {
+    __shared__ long long s_max[kThreads / 64][3];
+    long long m[3] = {(long long)coors[0], (long long)coors[1], (long long)coors[2]};
+    for (long i = (long)blockIdx.x * kThreads + threadIdx.x; i < n; i += (long)kCoorMaxParts * kThreads) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) m[a] = max(m[a], (long long)coors[3 * i + a]);
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) m[a] = max(m[a], (long long)__shfl_xor(m[a], d, 64));
+        if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6][a] = m[a];
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        long long x = s_max[0][threadIdx.x];
+        for (int k = 1; k < kThreads / 64; ++k) x = max(x, s_max[k][threadIdx.x]);
+        parts[blockIdx.x * 3 + threadIdx.x] = x;
+    }
+}
+
+// the distinct keys in ascending order (from the bitmap), and the table's slots emptied
+__global__ void grid_hash_prepare_kernel(const unsigned *__restrict__ bm, const int *__restrict__ base, long words,
+                                         int num_unq, int *__restrict__ unq_keys,
+                                         unsigned long long *__restrict__ table, long table_size) {
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < table_size) table[i] = ~0ull;
+    if (i >= words) return;
+    unsigned m = bm[i];
+    for (int r = base[i]; m && r < num_unq; ++r) {
+        unq_keys[r] = (int)(i * 32 + __builtin_ctz(m));
+        m &= m - 1u;
+    }
+}
+
+// Occupied slots: a byte per slot, and the occupied ones' (key, value) words in slot order.  Two
+// launches: occupied slots per tile, then their words behind those of the tiles in front.
+constexpr int kValidItems = 8;
+constexpr int kValidTile = kThreads * kValidItems;
+constexpr int kValidSumTiles = 1024;  // up to this many tiles the second launch adds up the tiles in front itself
+__global__ __launch_bounds__(kThreads) void grid_hash_valid_kernel(const unsigned long long *__restrict__ table,
+                                                                   long table_size, unsigned char *__restrict__ valid,
+                                                                   int *__restrict__ tile_sums) {
+    const long base = (long)blockIdx.x * kValidTile;
+    int c = 0;
+#pragma unroll
+    for (int k = 0; k < kValidItems; ++k) {
+        const long i = base + (long)k * kThreads + threadIdx.x;
+        if (i >= table_size) continue;
+        const bool used = (int)(unsigned)(table[i] & 0xffffffffull) != -1;
+        valid[i] = used ? 1 : 0;
+        c += used;
+    }
+    int total;
+    block_exclusive_scan(c, &total);
+    if (threadIdx.x == 0) tile_sums[blockIdx.x] = total;
+}
+__global__ __launch_bounds__(kThreads) void grid_hash_compact_kernel(const unsigned long long *__restrict__ table,
+                                                                     long table_size, const int *__restrict__ tile_offs,
+                                                                     int offsets_ready,
+                                                                     unsigned long long *__restrict__ out, long n_out) {
+    const long base = (long)blockIdx.x * kValidTile + (long)threadIdx.x * kValidItems;
+    unsigned long long word[kValidItems];
+    int c = 0;
+#pragma unroll
+    for (int k = 0; k < kValidItems; ++k) {
+        word[k] = base + k < table_size ? table[base + k] : ~0ull;
+        c += (int)(unsigned)(word[k] & 0xffffffffull) != -1;
+    }
+    int off;
+    if (offsets_ready) {
+        off = tile_offs[blockIdx.x];
+    } else {
+        int part = 0;
+        for (int t = threadIdx.x; t < (int)blockIdx.x; t += kThreads) part += tile_offs[t];
+        block_exclusive_scan(part, &off);
+    }
+    int total;
+    long at = (long)off + block_exclusive_scan(c, &total);
+#pragma unroll
+    for (int k = 0; k < kValidItems; ++k)
+        if ((int)(unsigned)(word[k] & 0xffffffffull) != -1) {
+            if (at < n_out) out[at] = word[k];
+            ++at;
+        }
+}
+
+// byte map -> bitmap -> scanned population counts of one set of keys.  Layout of the workspace:
+// byte map (8 ints per word), bitmap, scanned counts (words + 1: the last is the number of distinct
+// keys), a flag for a key outside the bound (used where the caller has no other), scan workspace.
+struct BitmapWs {
+    long words;
+    uint4 *map16;
+    unsigned *bm;
+    int *base, *bad, *scan_ws;
+};
+BitmapWs bitmap_ws_of(const int32_t *ws_in, int64_t key_bound) {
+    int32_t *ws = const_cast<int32_t *>(ws_in);
+    BitmapWs r;
+    r.words = (long)((key_bound + 31) / 32);
+    r.map16 = reinterpret_cast<uint4 *>(ws);
+    r.bm = reinterpret_cast<unsigned *>(ws + 8 * r.words);
+    r.base = ws + 9 * r.words;
+    r.bad = r.base + r.words + 1;
+    r.scan_ws = r.bad + 1;
+    return r;
+}
+template <class Keys>
+int bitmap_count(Keys keys, long n, int64_t key_bound, const BitmapWs &b, int *clear_flag, int *bad, hipStream_t st) {
+    bytemap_clear_kernel<<<dim3(blocks_for(2 * b.words)), dim3(kThreads), 0, st>>>(b.map16, 2 * b.words, clear_flag);
+    bytemap_mark_kernel<Keys><<<dim3(blocks_for(n)), dim3(kThreads), 0, st>>>(
+        keys, n, (long)key_bound, reinterpret_cast<unsigned char *>(b.map16), bad);
+    bytemap_pack_kernel<<<dim3(blocks_for(b.words)), dim3(kThreads), 0, st>>>(b.map16, b.words, b.bm, b.base);
+    if (exclusive_scan(b.base, b.words, b.base, b.words + 1, b.scan_ws, st) != hipSuccess) return TXS_ERR_LAUNCH;
+    return status_of(hipGetLastError());
 }
 
 }  // namespace
@@ -511,8 +658,8 @@ int txs_voxel_keys(const float *points, int64_t num_total, int64_t point_stride,
 int64_t txs_unique_bitmap_workspace_len(int64_t key_bound) {
     if (key_bound <= 0 || key_bound > (1LL << 31)) return -1;
     const int64_t words = (key_bound + 31) / 32;
-    // byte map (32 bytes per word), bitmap, scanned counts, scan workspace
-    return 8 * words + words + (words + 1) + scan_tiles(words + 1) + 17;
+    // byte map (32 bytes per word), bitmap, scanned counts, range flag, scan workspace
+    return 8 * words + words + (words + 1) + 1 + scan_tiles(words + 1) + 17;
 }
 
 int txs_unique_bitmap_count(const void *keys, int key_is_int64, int64_t num_total, int64_t key_bound,
@@ -521,23 +668,84 @@ int txs_unique_bitmap_count(const void *keys, int key_is_int64, int64_t num_tota
     if (num_total == 0) return TXS_OK;
     if (!keys || !bitmap_ws || ((uintptr_t)bitmap_ws & 15u) != 0) return TXS_ERR_INVALID_ARG;
     hipStream_t st = (hipStream_t)stream;
-    const long n = num_total;
-    const long words = (long)((key_bound + 31) / 32);
-    uint4 *map16 = reinterpret_cast<uint4 *>(bitmap_ws);
-    unsigned char *map = reinterpret_cast<unsigned char *>(bitmap_ws);
-    unsigned *bm = reinterpret_cast<unsigned *>(bitmap_ws + 8 * words);
-    int *base = bitmap_ws + 9 * words;
-    int *scan_ws = base + words + 1;
-    bytemap_clear_kernel<<<dim3(blocks_for(2 * words)), dim3(kThreads), 0, st>>>(map16, 2 * words);
-    if (key_is_int64)
-        bytemap_mark_kernel<long long><<<dim3(blocks_for(n)), dim3(kThreads), 0, st>>>(
-            static_cast<const long long *>(keys), n, (long)key_bound, map, stats);
+    const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
+    int *bad = stats + TXS_STAT_OUT_OF_RANGE;
+    const int rc = key_is_int64
+                       ? bitmap_count(FlatKeys<long long>{static_cast<const long long *>(keys)}, num_total, key_bound, b,
+                                      nullptr, bad, st)
+                       : bitmap_count(FlatKeys<int>{static_cast<const int *>(keys)}, num_total, key_bound, b, nullptr,
+                                      bad, st);
+    if (rc != TXS_OK) return rc;
+    bitmap_total_kernel<<<dim3(1), dim3(64), 0, st>>>(b.base, b.words, stats);
+    return status_of(hipGetLastError());
+}
+
+int txs_coor_max_parts(void) { return kCoorMaxParts; }
+
+int txs_coor_max(const void *coors, int coor_is_int64, int64_t num_total, int64_t *parts, void *stream) {
+    if (!fits_i32(num_total) || num_total == 0 || !coors || !parts) return TXS_ERR_INVALID_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    if (coor_is_int64)
+        coor_max_kernel<long long><<<dim3(kCoorMaxParts), dim3(kThreads), 0, st>>>(
+            static_cast<const long long *>(coors), num_total, (long long *)parts);
     else
-        bytemap_mark_kernel<int><<<dim3(blocks_for(n)), dim3(kThreads), 0, st>>>(
-            static_cast<const int *>(keys), n, (long)key_bound, map, stats);
-    bytemap_pack_kernel<<<dim3(blocks_for(words)), dim3(kThreads), 0, st>>>(map16, words, bm, base);
-    if (exclusive_scan(base, words, base, words + 1, scan_ws, st) != hipSuccess) return TXS_ERR_LAUNCH;
-    bitmap_total_kernel<<<dim3(1), dim3(64), 0, st>>>(base, words, stats);
+        coor_max_kernel<int><<<dim3(kCoorMaxParts), dim3(kThreads), 0, st>>>(static_cast<const int *>(coors), num_total,
+                                                                            (long long *)parts);
+    return status_of(hipGetLastError());
+}
+
+int64_t txs_coor_bitmap_count_offset(int64_t key_bound) {
+    return key_bound <= 0 || key_bound > (1LL << 31) ? -1 : 10 * ((key_bound + 31) / 32);
+}
+
+int txs_coor_bitmap_count(const void *coors, int coor_is_int64, int64_t num_total, const int64_t *dims,
+                          int32_t *bitmap_ws, void *stream) {
+    if (!fits_i32(num_total) || num_total == 0 || !coors || !dims || !bitmap_ws || ((uintptr_t)bitmap_ws & 15u) != 0)
+        return TXS_ERR_INVALID_ARG;
+    int64_t key_bound = 1;
+    for (int a = 0; a < 3; ++a) {
+        if (dims[a] <= 0 || dims[a] > (1LL << 31) / key_bound) return TXS_ERR_INVALID_ARG;
+        key_bound *= dims[a];
+    }
+    hipStream_t st = (hipStream_t)stream;
+    const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
+    const long s0 = (long)(dims[1] * dims[2]), s1 = (long)dims[2];
+    if (coor_is_int64)
+        return bitmap_count(CoorKeys<long long>{static_cast<const long long *>(coors), s0, s1}, num_total, key_bound, b,
+                            b.bad, b.bad, st);
+    return bitmap_count(CoorKeys<int>{static_cast<const int *>(coors), s0, s1}, num_total, key_bound, b, b.bad, b.bad, st);
+}
+
+int64_t txs_grid_hash_index_workspace_len(int64_t num_unq, int64_t table_size) {
+    if (!fits_i32(num_unq) || !fits_i32(table_size)) return -1;
+    const int64_t tiles = (table_size + kValidTile - 1) / kValidTile;
+    return num_unq + tiles + scan_tiles(tiles) + 17;
+}
+
+int txs_grid_hash_index(const int32_t *bitmap_ws, int64_t key_bound, int64_t num_unq, int32_t *table,
+                        int64_t table_size, int32_t *index_ws, unsigned char *valid, int32_t *valid_table,
+                        void *stream) {
+    if (key_bound <= 0 || key_bound > (1LL << 31) || !fits_i32(num_unq) || num_unq == 0 || !fits_i32(table_size) ||
+        num_unq > table_size || (table_size & (table_size - 1)) != 0)
+        return TXS_ERR_INVALID_ARG;
+    if (!bitmap_ws || !table || !index_ws || !valid || !valid_table || (((uintptr_t)table | (uintptr_t)valid_table) & 7) != 0)
+        return TXS_ERR_INVALID_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
+    auto slots = reinterpret_cast<unsigned long long *>(table);
+    int *unq_keys = index_ws, *tile_sums = index_ws + num_unq;
+    const long span = b.words > table_size ? b.words : (long)table_size;
+    grid_hash_prepare_kernel<<<dim3(blocks_for(span)), dim3(kThreads), 0, st>>>(b.bm, b.base, b.words, (int)num_unq,
+                                                                               unq_keys, slots, table_size);
+    grid_hash_build_kernel<<<dim3(blocks_for(num_unq)), dim3(kThreads), 0, st>>>(unq_keys, nullptr, slots,
+                                                                                (int)table_size, num_unq, nullptr);
+    const long tiles = (table_size + kValidTile - 1) / kValidTile;
+    grid_hash_valid_kernel<<<dim3((unsigned)tiles), dim3(kThreads), 0, st>>>(slots, table_size, valid, tile_sums);
+    const bool few = tiles <= kValidSumTiles;
+    if (!few && exclusive_scan(tile_sums, tiles, tile_sums, tiles, tile_sums + tiles, st) != hipSuccess)
+        return TXS_ERR_LAUNCH;
+    grid_hash_compact_kernel<<<dim3((unsigned)tiles), dim3(kThreads), 0, st>>>(
+        slots, table_size, tile_sums, !few, reinterpret_cast<unsigned long long *>(valid_table), num_unq);
     return status_of(hipGetLastError());
 }
 
@@ -548,9 +756,10 @@ int txs_unique_bitmap_assign(const void *keys, int key_is_int64, int64_t num_tot
     if (!keys || !bitmap_ws || !unq_inv || !unq_keys) return TXS_ERR_INVALID_ARG;
     hipStream_t st = (hipStream_t)stream;
     const long n = num_total;
-    const long words = (long)((key_bound + 31) / 32);
-    const unsigned *bm = reinterpret_cast<const unsigned *>(bitmap_ws + 8 * words);
-    const int *base = bitmap_ws + 9 * words;
+    const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
+    const long words = b.words;
+    const unsigned *bm = b.bm;
+    const int *base = b.base;
     const long span = n > words ? n : words;
     if (key_is_int64)
         bitmap_assign_kernel<long long><<<dim3(blocks_for(span)), dim3(kThreads), 0, st>>>(
@@ -696,7 +905,26 @@ int txs_grid_hash_probe(const int32_t *keys, int64_t num_keys, const int32_t *ta
     if (num_keys == 0) return TXS_OK;
     if (!keys || !out_values) return TXS_ERR_INVALID_ARG;
     grid_hash_probe_kernel<<<dim3(blocks_for(num_keys)), dim3(kThreads), 0, (hipStream_t)stream>>>(
-        keys, (const unsigned long long *)table, (int)table_size, num_keys, out_values);
+        FlatKeys<int>{keys}, (const unsigned long long *)table, (int)table_size, num_keys, out_values);
+    return status_of(hipGetLastError());
+}
+
+int txs_grid_hash_probe_coors(const void *coors, int coor_is_int64, int64_t num_coors, int64_t dim1, int64_t dim2,
+                              const int32_t *table, int64_t table_size, int32_t *out_values, void *stream) {
+    if (!fits_i32(num_coors) || !fits_i32(table_size) || table_size <= 0 || !table) return TXS_ERR_INVALID_ARG;
+    if ((table_size & (table_size - 1)) != 0 || ((uintptr_t)table & 7) != 0) return TXS_ERR_INVALID_ARG;
+    if (num_coors == 0) return TXS_OK;
+    if (!coors || !out_values) return TXS_ERR_INVALID_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    const dim3 grid(blocks_for(num_coors)), blk(kThreads);
+    const long s0 = (long)(dim1 * dim2), s1 = (long)dim2;
+    auto slots = (const unsigned long long *)table;
+    if (coor_is_int64)
+        grid_hash_probe_kernel<<<grid, blk, 0, st>>>(CoorKeys<long long>{static_cast<const long long *>(coors), s0, s1},
+                                                     slots, (int)table_size, num_coors, out_values);
+    else
+        grid_hash_probe_kernel<<<grid, blk, 0, st>>>(CoorKeys<int>{static_cast<const int *>(coors), s0, s1}, slots,
+                                                     (int)table_size, num_coors, out_values);
     return status_of(hipGetLastError());
 }
 

@@ -224,6 +224,12 @@ std::tuple<Tensor, Tensor, Tensor> voxel_keys(const Tensor &points, std::vector<
     return {coors, keys, stats};
 }
 
+// What is cheaper than sorting the keys: an occupancy map of all possible keys.  Its cost is that
+// of clearing and packing key_bound bytes, the sort's that of 4 passes of 4 launches over N keys.
+bool bitmap_is_cheaper(int64_t N, int64_t key_bound) {
+    return key_bound <= (int64_t(1) << 28) && key_bound <= 64 * N;
+}
+
 // torch.unique(keys, return_inverse=True, return_counts=True) fused with the
 // scatter plan: one sort, one host synchronisation.
 // returns (unq_keys, unq_inv, unq_cnts, preSum, perm | None, seg, slot_of, heavy_ids, stats)
@@ -245,7 +251,7 @@ unique_plan(const Tensor &keys_in, int64_t key_bound, int64_t heavy_threshold, c
     // map (no sort of the keys), then the index preparation of those ids.  `stats` is read
     // twice: the number of distinct keys, which sizes the plan (fetched while the ids are
     // still being written), and the plan's own figures.
-    if (N > 0 && key_bound <= (int64_t(1) << 28) && key_bound <= 64 * N) {
+    if (N > 0 && bitmap_is_cheaper(N, key_bound)) {
         const int is64 = keys_in.scalar_type() == at::kLong;
         Tensor inv = at::empty({N}, i32), unq = at::empty({std::min(N, key_bound)}, i32);
         Tensor bws = at::empty({txs_unique_bitmap_workspace_len(key_bound)}, i32);
@@ -529,6 +535,70 @@ Tensor grid_hash_probe(const Tensor &coors, const Tensor &table) {
     check_status(txs_grid_hash_probe(i32p(coors), coors.numel(), table.data_ptr<int32_t>(), table.size(0),
                                      i32w(out), cur_stream(coors)),
                  "grid_hash_probe");
+    return out;
+}
+
+void check_coors(const Tensor &coors) {
+    check_dev(coors, "coors");
+    TORCH_CHECK(coors.dim() == 2 && coors.size(1) == 3, "coors must be [N, 3]");
+    TORCH_CHECK(coors.scalar_type() == at::kInt || coors.scalar_type() == at::kLong, "coors must be int32 or int64");
+}
+
+// GridHash of distinct voxel coordinates: (dims, table | None, valid_mask | None, valid_table | None).
+// The tables are None where the coordinates' grid is not for the occupancy map (too large for the
+// number of rows, or not a grid at all): the caller then sorts the keys.  Two host
+// synchronisations: the grid's extents, and the number of distinct coordinates.
+std::tuple<std::vector<int64_t>, OptTensor, OptTensor, OptTensor> grid_hash_index(const Tensor &coors) {
+    check_coors(coors);
+    TORCH_CHECK(coors.size(0) > 0, "coors must not be empty");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(coors.device());
+    const int64_t N = coors.size(0);
+    const int is64 = coors.scalar_type() == at::kLong;
+    void *st = cur_stream(coors);
+    const auto i32 = coors.options().dtype(at::kInt);
+    const int64_t num_parts = txs_coor_max_parts();
+    Tensor parts = at::empty({num_parts, 3}, coors.options().dtype(at::kLong));
+    check_status(txs_coor_max(coors.data_ptr(), is64, N, parts.data_ptr<int64_t>(), st), "coor_max");
+    const Tensor parts_host = parts.cpu();
+    const int64_t *ph = parts_host.data_ptr<int64_t>();
+    std::vector<int64_t> dims(ph, ph + 3);
+    for (int64_t k = 1; k < num_parts; ++k)
+        for (int a = 0; a < 3; ++a) dims[a] = std::max(dims[a], ph[3 * k + a]);
+    int64_t bound = 1;
+    bool grid = true;
+    for (int a = 0; a < 3; ++a) {
+        if (dims[a] < std::numeric_limits<int64_t>::max()) ++dims[a];
+        grid = grid && dims[a] > 0 && dims[a] <= (int64_t(1) << 28) / bound;
+        if (grid) bound *= dims[a];
+    }
+    if (!grid || !bitmap_is_cheaper(N, bound)) return {dims, std::nullopt, std::nullopt, std::nullopt};
+    Tensor bws = at::empty({txs_unique_bitmap_workspace_len(bound)}, i32);
+    check_status(txs_coor_bitmap_count(coors.data_ptr(), is64, N, dims.data(), i32w(bws), st), "coor_bitmap_count");
+    const Tensor found = bws.narrow(0, txs_coor_bitmap_count_offset(bound), 2).cpu();
+    const int64_t U = found.data_ptr<int32_t>()[0];
+    TORCH_CHECK(found.data_ptr<int32_t>()[1] == 0, "keys (or points) outside the grid: keys must be in [0, ", bound, ")");
+    const int64_t size = up_2n_host(U);
+    Tensor table = at::empty({size, 2}, i32), valid_table = at::empty({U, 2}, i32);
+    Tensor valid = at::empty({size}, coors.options().dtype(at::kBool));
+    Tensor iws = at::empty({txs_grid_hash_index_workspace_len(U, size)}, i32);
+    check_status(txs_grid_hash_index(i32p(bws), bound, U, i32w(table), size, i32w(iws),
+                                     static_cast<unsigned char *>(valid.data_ptr()), i32w(valid_table), st),
+                 "grid_hash_index");
+    return {dims, table, valid, valid_table};
+}
+
+// probe_table with voxel coordinates [N, 3]; dim1, dim2: the grid's second and third extent
+Tensor grid_hash_probe_coors(const Tensor &coors, int64_t dim1, int64_t dim2, const Tensor &table) {
+    check_coors(coors);
+    check_i32(table, "table");
+    TORCH_CHECK(table.dim() == 2 && table.size(1) == 2, "table must be [size, 2]");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(coors.device());
+    Tensor out = at::empty({coors.size(0)}, table.options());
+    check_status(txs_grid_hash_probe_coors(coors.numel() ? coors.data_ptr() : nullptr,
+                                           coors.scalar_type() == at::kLong, coors.size(0), dim1, dim2,
+                                           table.data_ptr<int32_t>(), table.size(0),
+                                           out.numel() ? i32w(out) : nullptr, cur_stream(coors)),
+                 "grid_hash_probe_coors");
     return out;
 }
 
@@ -909,6 +979,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                      "kernel_name");
         return std::string(buf);
     }, "kernel_name(backward, op, like, num_total, num_unq, table_allowed): the kernel a call on `like`-shaped rows launches");
+    m.def("grid_hash_index", &grid_hash_index,
+          "grid_hash_index(coors [N, 3]) -> (dims, table, valid_mask, valid_table); the last three None where the keys are to be sorted",
+          pybind11::arg("coors"));
+    m.def("grid_hash_probe_coors", &grid_hash_probe_coors, "grid_hash_probe_coors(coors [N, 3], dim1, dim2, table) -> values",
+          pybind11::arg("coors"), pybind11::arg("dim1"), pybind11::arg("dim2"), pybind11::arg("table"));
     m.attr("PATH_AUTO") = (int)TXS_PATH_AUTO;
     m.attr("PATH_VOXEL_ORDER") = (int)TXS_PATH_VOXEL_ORDER;
     m.attr("PATH_TABLE") = (int)TXS_PATH_TABLE;

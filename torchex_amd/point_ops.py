@@ -54,6 +54,9 @@ def grid_hash_probe(coors, table):
     return scatter_ext.grid_hash_probe(coors.contiguous(), table.contiguous())
 
 
+_COOR_DTYPES = (torch.int32, torch.int64)   # what the kernels linearise themselves
+
+
 def _flatten_3dim_coors(coors, sizes):
     # grid_hash.py:7-15
     x, y, z = coors[:, 0], coors[:, 1], coors[:, 2]
@@ -66,19 +69,40 @@ class GridHash:
     integer keys) in sorted order, ``probe(coors)`` returns their indices.
 
     The reference makes the rows unique with ``torch.unique(coors, dim=0)``; here the keys
-    are linearised first and made unique by the same single radix sort that serves the
-    scatter plan, which orders them identically (row-lexicographic == linear key order).
+    are linearised first and made unique by an occupancy map of the grid, or by the radix sort
+    that serves the scatter plan where the grid is too large for its rows; both order them
+    identically (row-lexicographic == linear key order).
     """
 
     def __init__(self, coors, debug=False):
+        table = None
         if coors.ndim == 1:
             self.dim_size = None
             keys = coors
         else:
             assert coors.ndim == 2 and coors.size(1) == 3
-            self.dim_size = tuple(int(v) + 1 for v in coors.amax(0).tolist())   # grid_hash.py:17-23
+            if coors.is_cuda and coors.dtype in _COOR_DTYPES and coors.numel() > 0:
+                dims, table, valid_mask, valid_table = scatter_ext.grid_hash_index(coors.contiguous())
+            else:
+                dims = [int(v) + 1 for v in coors.amax(0).tolist()]   # grid_hash.py:17-23
+            self.dim_size = tuple(dims)
             assert self.dim_size[0] * self.dim_size[1] * self.dim_size[2] < 2 ** 31
-            keys = _flatten_3dim_coors(coors.long(), self.dim_size)
+            keys = None if table is not None else _flatten_3dim_coors(coors.long(), self.dim_size)
+        if table is not None:
+            self.table, self.valid_mask, self.valid_table = table, valid_mask, valid_table
+            count = len(valid_table)
+        else:
+            count = self._index_keys(keys)
+        if debug:
+            assert self.valid_mask.sum() == count
+            assert self.valid_table[:, 1].max() + 1 == count
+            assert count == len(torch.unique(self.valid_table[:, 1]))
+            if not self.valid_mask.all():
+                assert (self.table[~self.valid_mask, 0] == -1).all()
+
+    def _index_keys(self, keys):
+        """The table from linear keys: flat ones, or those of a grid too large for an
+        occupancy map of all of it.  Returns how many of them are distinct."""
         if keys.numel() == 0:
             raise ValueError("GridHash needs at least one coordinate")
         bound = int(keys.max()) + 1 if self.dim_size is None else \
@@ -90,16 +114,14 @@ class GridHash:
         self.table = grid_hash_build(unq_keys, values)
         self.valid_mask = self.table[:, 0] != -1
         self.valid_table = self.table[self.valid_mask]
-        if debug:
-            assert self.valid_mask.sum() == len(unq_keys)
-            assert self.valid_table[:, 1].max() + 1 == len(unq_keys)
-            assert len(self.valid_table[:, 1]) == len(torch.unique(self.valid_table[:, 1]))
-            if not self.valid_mask.all():
-                assert (self.table[~self.valid_mask, 0] == -1).all()
+        return len(unq_keys)
 
     def probe(self, coors):
         if coors.ndim == 2:
             assert coors.size(1) == 3
+            if coors.is_cuda and coors.dtype in _COOR_DTYPES and coors.device == self.table.device:
+                return scatter_ext.grid_hash_probe_coors(coors.contiguous(), self.dim_size[1], self.dim_size[2],
+                                                         self.table)
             coors = _flatten_3dim_coors(coors, self.dim_size)
         else:
             assert coors.ndim == 1
