@@ -267,6 +267,20 @@ int txs_unique_bitmap_assign(const void *keys, int key_is_int64, int64_t num_tot
                              int32_t *unq_keys, void *stream);
 int64_t txs_unique_bitmap_workspace_len(int64_t key_bound);
 
+/* The triple by occupancy map and the plan of its unq_inv, queued in one go: the number of
+ * distinct keys stays on the device until the caller reads `stats`.  Everything that has an entry
+ * per voxel holds min(num_total, key_bound) of them (preSum one more), of which the first U are
+ * written.  stats: TXS_STATS_LEN + 2 ints, not initialised; entry TXS_STATS_LEN receives U, the next
+ * one is nonzero if a key lies outside [0, key_bound) (the rest is then not valid).  key_flag: NULL,
+ * or a device int that already tells of a key outside the bound and to which this call adds.
+ * plan_ws: txs_plan_workspace_len(num_total, min(num_total, key_bound)) entries.  Where
+ * stats[NEED_GENERAL] is set, the caller runs txs_plan_build_general on unq_inv and U and takes the
+ * counts from the offsets.  num_total > 0; the rest as for the functions above and txs_plan_build. */
+int txs_unique_plan(const void *keys, int key_is_int64, int64_t num_total, int64_t key_bound,
+                    int32_t *key_flag, int32_t *bitmap_ws, int32_t heavy_threshold, int32_t *plan_ws,
+                    int32_t *unq_inv, int32_t *unq_keys, int64_t *unq_cnts, int32_t *perm, int32_t *seg,
+                    int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream);
+
 /* unq_cnts[u] = preSum[u + 1] - preSum[u] as int64: the counts torch.unique(...,
  * return_counts=True) returns, which ScatterData keeps (scatter_op.py:14-17). */
 int txs_counts_from_presum(const int32_t *preSum, int64_t num_unq, int64_t *unq_cnts, void *stream);

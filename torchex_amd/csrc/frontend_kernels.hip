@@ -142,18 +142,37 @@ __global__ void bytemap_mark_kernel(Keys keys, long n, long key_bound, unsigned 
     map[k] = 1;
 }
 
-// 32 map bytes (each 0 or 1) -> one bitmap word and its population count
-__global__ void bytemap_pack_kernel(const uint4 *__restrict__ map16, long words, unsigned *__restrict__ bm,
-                                    int *__restrict__ cnt) {
-    const long w = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= words) return;
-    const uint4 lo = map16[2 * w], hi = map16[2 * w + 1];
+// 32 map bytes (each 0 or 1) -> one bitmap word and its population count, and the sums of the
+// counts over the tiles of the scan that follows (a workgroup per tile)
+constexpr int kPackThreads = 1024;
+__global__ __launch_bounds__(kPackThreads) void bytemap_pack_kernel(const uint4 *__restrict__ map16, long words,
+                                                                    unsigned *__restrict__ bm, int *__restrict__ cnt,
+                                                                    int *__restrict__ tile_sums) {
+    constexpr int kItems = txs_detail::kScanTileItems / kPackThreads;
+    __shared__ int s_sum[kPackThreads / 64];
     // bytes b0..b3 of a word, each 0 or 1 -> bits 0..3: (x * 0x10204080) >> 28 leaves b0 + 2 b1 + 4 b2 + 8 b3
     auto nib = [](unsigned x) -> unsigned { return ((x * 0x10204080u) >> 28) & 15u; };
-    const unsigned word = nib(lo.x) | (nib(lo.y) << 4) | (nib(lo.z) << 8) | (nib(lo.w) << 12) | (nib(hi.x) << 16) |
-                          (nib(hi.y) << 20) | (nib(hi.z) << 24) | (nib(hi.w) << 28);
-    bm[w] = word;
-    cnt[w] = __popc(word);
+    int sum = 0;
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+        const long w = (long)blockIdx.x * txs_detail::kScanTileItems + it * kPackThreads + threadIdx.x;
+        if (w >= words) continue;
+        const uint4 lo = map16[2 * w], hi = map16[2 * w + 1];
+        const unsigned word = nib(lo.x) | (nib(lo.y) << 4) | (nib(lo.z) << 8) | (nib(lo.w) << 12) | (nib(hi.x) << 16) |
+                              (nib(hi.y) << 20) | (nib(hi.z) << 24) | (nib(hi.w) << 28);
+        bm[w] = word;
+        const int c = __popc(word);
+        cnt[w] = c;
+        sum += c;
+    }
+    sum = wave_inclusive_scan(sum);
+    if ((threadIdx.x & 63) == 63) s_sum[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int t = 0;
+        for (int k = 0; k < kPackThreads / 64; ++k) t += s_sum[k];
+        tile_sums[blockIdx.x] = t;
+    }
 }
 
 // base: exclusive scan of the population counts, words + 1 entries (the last is the total)
@@ -164,8 +183,13 @@ __global__ void bitmap_total_kernel(const int *__restrict__ base, long words, in
 template <typename K>
 __global__ void bitmap_assign_kernel(const K *__restrict__ keys, long n, long key_bound,
                                      const unsigned *__restrict__ bm, const int *__restrict__ base,
-                                     long words, int *__restrict__ inv, int *__restrict__ unq_keys) {
+                                     long words, int *__restrict__ inv, int *__restrict__ unq_keys,
+                                     const int *__restrict__ bad, int *__restrict__ found) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (found && i == 0) {  // the number of distinct keys, and whether one lies outside the bound
+        found[0] = base[words];
+        found[1] = bad[0];
+    }
     if (i < n) {
         const long k = (long)keys[i];
         int id = 0;
@@ -631,8 +655,10 @@ int bitmap_count(Keys keys, long n, int64_t key_bound, const BitmapWs &b, int *c
     bytemap_clear_kernel<<<dim3(blocks_for(2 * b.words)), dim3(kThreads), 0, st>>>(b.map16, 2 * b.words, clear_flag);
     bytemap_mark_kernel<Keys><<<dim3(blocks_for(n)), dim3(kThreads), 0, st>>>(
         keys, n, (long)key_bound, reinterpret_cast<unsigned char *>(b.map16), bad);
-    bytemap_pack_kernel<<<dim3(blocks_for(b.words)), dim3(kThreads), 0, st>>>(b.map16, b.words, b.bm, b.base);
-    if (exclusive_scan(b.base, b.words, b.base, b.words + 1, b.scan_ws, st) != hipSuccess) return TXS_ERR_LAUNCH;
+    bytemap_pack_kernel<<<dim3((unsigned)scan_tiles(b.words + 1)), dim3(kPackThreads), 0, st>>>(b.map16, b.words, b.bm,
+                                                                                               b.base, b.scan_ws);
+    if (txs_detail::scan_from_tile_sums(b.base, b.words, b.base, b.words + 1, b.scan_ws, st) != hipSuccess)
+        return TXS_ERR_LAUNCH;
     return status_of(hipGetLastError());
 }
 
@@ -763,11 +789,43 @@ int txs_unique_bitmap_assign(const void *keys, int key_is_int64, int64_t num_tot
     const long span = n > words ? n : words;
     if (key_is_int64)
         bitmap_assign_kernel<long long><<<dim3(blocks_for(span)), dim3(kThreads), 0, st>>>(
-            static_cast<const long long *>(keys), n, (long)key_bound, bm, base, words, unq_inv, unq_keys);
+            static_cast<const long long *>(keys), n, (long)key_bound, bm, base, words, unq_inv, unq_keys, nullptr, nullptr);
     else
         bitmap_assign_kernel<int><<<dim3(blocks_for(span)), dim3(kThreads), 0, st>>>(
-            static_cast<const int *>(keys), n, (long)key_bound, bm, base, words, unq_inv, unq_keys);
+            static_cast<const int *>(keys), n, (long)key_bound, bm, base, words, unq_inv, unq_keys, nullptr, nullptr);
     return status_of(hipGetLastError());
+}
+
+int txs_unique_plan(const void *keys, int key_is_int64, int64_t num_total, int64_t key_bound, int32_t *key_flag,
+                    int32_t *bitmap_ws, int32_t heavy_threshold, int32_t *plan_ws, int32_t *unq_inv,
+                    int32_t *unq_keys, int64_t *unq_cnts, int32_t *perm, int32_t *seg, int32_t *preSum,
+                    int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream) {
+    if (!fits_i32(num_total) || num_total == 0 || key_bound <= 0 || key_bound > (1LL << 31)) return TXS_ERR_INVALID_ARG;
+    if (!keys || !bitmap_ws || ((uintptr_t)bitmap_ws & 15u) != 0 || !unq_inv || !unq_keys || !unq_cnts || !slot_of ||
+        !heavy_ids || !stats)
+        return TXS_ERR_INVALID_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    const long n = num_total;
+    const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
+    int *bad = key_flag ? key_flag : b.bad, *clear_flag = key_flag ? nullptr : b.bad;
+    int *found = stats + TXS_STATS_LEN;
+    const dim3 grid(blocks_for(n > b.words ? n : b.words)), blk(kThreads);
+    int rc;
+    if (key_is_int64) {
+        auto k = static_cast<const long long *>(keys);
+        rc = bitmap_count(FlatKeys<long long>{k}, n, key_bound, b, clear_flag, bad, st);
+        bitmap_assign_kernel<long long><<<grid, blk, 0, st>>>(k, n, (long)key_bound, b.bm, b.base, b.words, unq_inv,
+                                                              unq_keys, bad, found);
+    } else {
+        auto k = static_cast<const int *>(keys);
+        rc = bitmap_count(FlatKeys<int>{k}, n, key_bound, b, clear_flag, bad, st);
+        bitmap_assign_kernel<int><<<grid, blk, 0, st>>>(k, n, (long)key_bound, b.bm, b.base, b.words, unq_inv, unq_keys,
+                                                        bad, found);
+    }
+    if (rc != TXS_OK || hipGetLastError() != hipSuccess) return TXS_ERR_LAUNCH;
+    const int64_t most = num_total < key_bound ? num_total : key_bound;
+    return txs_detail::plan_build(unq_inv, num_total, most, heavy_threshold, nullptr, plan_ws, perm, seg, preSum,
+                                  slot_of, heavy_ids, stats, nullptr, b.base + b.words, (long long *)unq_cnts, stream);
 }
 
 int txs_counts_from_presum(const int32_t *preSum, int64_t num_unq, int64_t *unq_cnts, void *stream) {
@@ -810,7 +868,8 @@ int txs_group_ranks(const int32_t *group_ids, int64_t num_total, int64_t num_gro
     // the bucket kernels rank while they place; any other route leaves a plan to rank from
     const bool fused = txs_detail::plan_writes_ranks(num_total, num_groups);
     const int rc = txs_detail::plan_build(group_ids, num_total, num_groups, heavy, nullptr, plan_ws, perm, seg, preSum,
-                                          nullptr, nullptr, stats, fused ? (long long *)out : nullptr, stream);
+                                          nullptr, nullptr, stats, fused ? (long long *)out : nullptr, nullptr, nullptr,
+                                          stream);
     if (rc != TXS_OK || fused) return rc;
     ingroup_inds_auto_kernel<<<dim3(blocks_for(num_total)), dim3(kThreads), 0, (hipStream_t)stream>>>(
         seg, perm, preSum, stats, num_total, (int)num_groups, (long long *)out);

@@ -102,6 +102,7 @@ __global__ __launch_bounds__(kGapBlock) void presum_gap_blocks_kernel(const int 
 
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kThreads * kScanItems;
+static_assert(kScanTile == txs_detail::kScanTileItems, "producers of tile sums use the same tile");
 constexpr int kScanFusedTiles = 1024;  // up to this many tiles the apply kernel sums the tile totals itself
 
 __global__ __launch_bounds__(kThreads) void scan_tile_sums_kernel(const int *__restrict__ in,
@@ -175,8 +176,14 @@ long scan_tiles(long n_out) { return (n_out + kScanTile - 1) / kScanTile; }
 hipError_t exclusive_scan(const int *in, long n_in, int *out, long n_out, int *ws,
                           hipStream_t st) {
     if (n_out <= 0) return hipSuccess;
-    long tiles = scan_tiles(n_out);
+    const long tiles = scan_tiles(n_out);
     scan_tile_sums_kernel<<<dim3((unsigned)tiles), dim3(kThreads), 0, st>>>(in, n_in, ws);
+    return scan_from_tile_sums(in, n_in, out, n_out, ws, st);
+}
+
+hipError_t scan_from_tile_sums(const int *in, long n_in, int *out, long n_out, int *ws, hipStream_t st) {
+    if (n_out <= 0) return hipSuccess;
+    const long tiles = scan_tiles(n_out);
     const int few = tiles <= kScanFusedTiles;
     if (!few) scan_tile_offsets_kernel<<<dim3(1), dim3(kThreads), 0, st>>>(ws, tiles);
     scan_apply_kernel<<<dim3((unsigned)tiles), dim3(kThreads), 0, st>>>(in, n_in, out, n_out, ws, !few);
@@ -666,9 +673,11 @@ __device__ __forceinline__ BucketSlice bucket_slice(long s, long e, int j) {
 // voxel's count in the whole bucket, and in the slices in front of its own, from at most
 // kBktMaxSlices short reads instead of every workgroup of a crowded bucket counting all of its rows.
 __global__ __launch_bounds__(kBktThreads) void bucket_count_kernel(
-    const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U, int low_bits, int high_bins,
+    const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U_arg, int low_bits, int high_bins,
     const int *__restrict__ bucket_start, const int *__restrict__ stats, int4 *__restrict__ wg_pick,
-    int *__restrict__ part_hist) {
+    int *__restrict__ part_hist, const int *__restrict__ num_unq_dev) {
+    // the voxel count may only be known on the device (unique path): U_arg is then an upper bound
+    const int U = num_unq_dev ? min(U_arg, *num_unq_dev) : U_arg;
     extern __shared__ int cnt_s[];  // [low_bins]
     __shared__ int s_pick[2];
     const int low_bins = 1 << low_bits;
@@ -732,12 +741,13 @@ __global__ __launch_bounds__(kBktThreads) void bucket_count_kernel(
 // per wave and voxel as well, left 12, and wrote every row as a request of its own).  4M ids of four
 // sweeps (1.3M voxels, 64 MB moved): 103 -> 45 us; 1M ids, ranks only: 31 -> 21.5 us.
 __global__ __launch_bounds__(kBktThreads) void bucket_plan_kernel(
-    const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U,
-    int low_bits, const int *__restrict__ bucket_start, int heavy_threshold,
+    const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U_arg,
+    int low_bits, int heavy_threshold,
     const long long *__restrict__ unq_cnts, int *__restrict__ perm, int *__restrict__ seg,
     int *__restrict__ preSum, int *__restrict__ slot_of, int *__restrict__ heavy_ids,
     int *__restrict__ stats, const int4 *__restrict__ wg_pick, const int *__restrict__ part_hist,
-    long long *__restrict__ ranks) {
+    long long *__restrict__ ranks, const int *__restrict__ num_unq_dev, long long *__restrict__ cnts_out) {
+    const int U = num_unq_dev ? min(U_arg, *num_unq_dev) : U_arg;
     // ranks != NULL: the caller wants the rank of every row inside its voxel and nothing else
     // (ingroup_inds): the placement writes ranks[row] in place of the permutation and the ids
     const bool rank_mode = ranks != nullptr;
@@ -854,6 +864,7 @@ __global__ __launch_bounds__(kBktThreads) void bucket_plan_kernel(
         step_s[d] += (rank_mode ? 0 : (int)s + run_all) - run;
         if (j == 0 && u_lo + d < u_hi) {
             preSum[u_lo + d] = (int)s + run_all;
+            if (cnts_out) cnts_out[u_lo + d] = (long long)c_all;
             if (u_lo + d == U - 1) preSum[U] = (int)n;
         }
         run += c;
@@ -1001,6 +1012,11 @@ __global__ void demote_heavy_kernel(const int *__restrict__ preSum, int *__restr
     for (int p = lo + (int)threadIdx.x; p < hi; p += (int)blockDim.x) seg[p] &= kIdMask;
     if (threadIdx.x == 0) slot_of[u] = -1;
 }
+
+int plan_general(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
+                 const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum,
+                 int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, const int *num_unq_dev, long long *cnts_out,
+                 void *stream);
 
 int radix_bits(int64_t U) {
     int bits = 1;
@@ -1160,6 +1176,26 @@ int64_t txs_plan_workspace_len(int64_t num_total, int64_t num_unq) {
 int txs_plan_build_general(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
                            const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg,
                            int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream) {
+    return plan_general(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum, slot_of,
+                        heavy_ids, stats, nullptr, nullptr, stream);
+}
+
+int txs_plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
+                   const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum,
+                   int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream) {
+    return txs_detail::plan_build(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum,
+                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, stream);
+}
+
+}  // extern "C"
+
+namespace {
+
+// num_unq_dev, cnts_out: as for txs_plan_special
+int plan_general(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
+                 const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum,
+                 int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, const int *num_unq_dev, long long *cnts_out,
+                 void *stream) {
     if (!fits_i32(num_total) || !fits_i32(num_unq) || !stats || !preSum || heavy_threshold < kChunk)
         return TXS_ERR_INVALID_ARG;
     const long n = num_total;
@@ -1172,20 +1208,13 @@ int txs_plan_build_general(const int32_t *unq_inv, int64_t num_total, int64_t nu
     if (rc == TXS_OK) rc = txs_plan_presum(seg, U > 0 ? n : 0, U, preSum, stream);
     if (slot_of == nullptr) return rc;  // order and offsets only
     if (rc == TXS_OK)
-        rc = txs_plan_special(preSum, U, heavy_threshold, unq_cnts, slot_of, heavy_ids, stats, nullptr, nullptr,
-                              stream);
+        rc = txs_plan_special(preSum, U, heavy_threshold, unq_cnts, slot_of, heavy_ids, stats, num_unq_dev,
+                              (int64_t *)cnts_out, stream);
     if (rc == TXS_OK) rc = txs_plan_seg_flag(seg, U > 0 ? n : 0, U, slot_of, stream);
     return rc;
 }
 
-int txs_plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
-                   const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum,
-                   int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream) {
-    return txs_detail::plan_build(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum,
-                                  slot_of, heavy_ids, stats, nullptr, stream);
-}
-
-}  // extern "C"
+}  // namespace
 
 // txs_plan_build, or with `ranks` the in-voxel rank of every row and no special-voxel table.
 // Ranks are written by the bucket kernels only: txs_detail::plan_writes_ranks tells a caller
@@ -1198,7 +1227,7 @@ bool txs_detail::plan_writes_ranks(long num_total, long num_unq) {
 int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
                            const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg,
                            int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids, int32_t *stats,
-                           long long *ranks, void *stream) {
+                           long long *ranks, const int *num_unq_dev, long long *cnts_out, void *stream) {
     if (!fits_i32(num_total) || !fits_i32(num_unq) || !stats || !preSum || heavy_threshold < kChunk)
         return TXS_ERR_INVALID_ARG;
     hipStream_t st = (hipStream_t)stream;
@@ -1209,15 +1238,15 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
     if (((uintptr_t)plan_ws & 7u) != 0) return TXS_ERR_INVALID_ARG;
     if (slot_of == nullptr) heavy_threshold = 0x7fffffff;  // no special voxels: no flag bit in seg
     const int bits = radix_bits(U > 1 ? U : 1);
-    if (n == 0 || U == 0) {
-        // nothing to sort: the general sequence only writes the offsets and the table of
-        // (empty) voxels; it adds to `stats`, which this call promises to initialise itself
+    if (n == 0 || U == 0 || (num_unq_dev && bits > kBucketBitsMax)) {
+        // the general sequence adds to `stats`, which this call promises to initialise itself
+        // where there is nothing to sort, and the unique path always
         stats_clear_kernel<<<dim3(1), dim3(64), 0, st>>>(stats);
         if (hipGetLastError() != hipSuccess) return TXS_ERR_LAUNCH;
     }
     if (n == 0 || U == 0 || bits > kBucketBitsMax)
-        return txs_plan_build_general(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg,
-                                      preSum, slot_of, heavy_ids, stats, stream);
+        return plan_general(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum, slot_of,
+                            heavy_ids, stats, num_unq_dev, cnts_out, stream);
     // ids of up to 11 bits are sorted by the bucket pass alone; beyond that the bucket digit has
     // 9 bits (narrower, and the buckets of a spatially sorted id space get too uneven: a
     // bucket's workgroups each count the whole bucket; wider, and a tile sends too few rows to
@@ -1270,8 +1299,8 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
         int rc = txs_plan_presum(seg, n, U, preSum, stream);
         if (slot_of == nullptr) return rc;
         if (rc == TXS_OK)
-            rc = txs_plan_special(preSum, U, heavy_threshold, unq_cnts, slot_of, heavy_ids, stats, nullptr, nullptr,
-                                  stream);
+            rc = txs_plan_special(preSum, U, heavy_threshold, unq_cnts, slot_of, heavy_ids, stats, num_unq_dev,
+                                  (int64_t *)cnts_out, stream);
         if (rc == TXS_OK) rc = txs_plan_seg_flag(seg, n, U, slot_of, stream);
         return rc;
     }
@@ -1283,10 +1312,10 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
         nullptr, reinterpret_cast<int2 *>(pairs1));
     const int low_bins = 1 << low_bits;
     bucket_count_kernel<<<dim3((unsigned)groups), dim3(kBktThreads), (size_t)low_bins * sizeof(int), st>>>(
-        unq_inv, pairs1, n, U, low_bits, high_bins, bucket_start, stats, reinterpret_cast<int4 *>(wg_pick), part_hist);
+        unq_inv, pairs1, n, U, low_bits, high_bins, bucket_start, stats, reinterpret_cast<int4 *>(wg_pick), part_hist, num_unq_dev);
     bucket_plan_kernel<<<dim3((unsigned)groups), dim3(kBktThreads), 0, st>>>(
-        unq_inv, pairs1, n, U, low_bits, bucket_start, heavy_threshold,
+        unq_inv, pairs1, n, U, low_bits, heavy_threshold,
         (const long long *)unq_cnts, perm, seg, preSum, slot_of, heavy_ids, stats,
-        reinterpret_cast<const int4 *>(wg_pick), part_hist, ranks);
+        reinterpret_cast<const int4 *>(wg_pick), part_hist, ranks, num_unq_dev, cnts_out);
     return status_of(hipGetLastError());
 }

@@ -69,13 +69,14 @@ Tensor empty_i32(int64_t n, const Tensor &like) {
 }
 
 std::vector<int64_t> read_stats(const Tensor &stats) {
+    const int64_t len = stats.numel();
     // the one host synchronisation of index preparation: an asynchronous copy into pinned
     // host memory (from the caching host allocator), then a wait on the stream
-    Tensor h = at::empty({TXS_STATS_LEN}, stats.options().device(at::kCPU).pinned_memory(true));
+    Tensor h = at::empty({len}, stats.options().device(at::kCPU).pinned_memory(true));
     h.copy_(stats, /*non_blocking=*/true);
     c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(stats.device().index()).synchronize();
-    std::vector<int64_t> v(TXS_STATS_LEN);
-    for (int i = 0; i < TXS_STATS_LEN; ++i) v[i] = h.data_ptr<int32_t>()[i];
+    std::vector<int64_t> v(len);
+    for (int64_t i = 0; i < len; ++i) v[i] = h.data_ptr<int32_t>()[i];
     return v;
 }
 
@@ -224,10 +225,13 @@ std::tuple<Tensor, Tensor, Tensor> voxel_keys(const Tensor &points, std::vector<
     return {coors, keys, stats};
 }
 
-// What is cheaper than sorting the keys: an occupancy map of all possible keys.  Its cost is that
-// of clearing and packing key_bound bytes, the sort's that of 4 passes of 4 launches over N keys.
+// What is cheaper than sorting the keys: an occupancy map of all possible keys.  Clearing and
+// packing it costs 10 us per 2^24 keys whatever the rows; the sort is 4 passes of 4 launches, 57 us
+// of launches alone at the smallest.  A frame of 200k points in 16.9M cells, plan included: sort
+// 119 us of kernels in 27 launches, map 75 in 14; in a quarter of a million rows or less the map
+// still wins at 2^25 keys, beyond that a row for every 64 keys is asked for.
 bool bitmap_is_cheaper(int64_t N, int64_t key_bound) {
-    return key_bound <= (int64_t(1) << 28) && key_bound <= 64 * N;
+    return key_bound <= (int64_t(1) << 28) && key_bound <= std::max<int64_t>(64 * N, int64_t(1) << 25);
 }
 
 // torch.unique(keys, return_inverse=True, return_counts=True) fused with the
@@ -244,36 +248,52 @@ unique_plan(const Tensor &keys_in, int64_t key_bound, int64_t heavy_threshold, c
     const int64_t N = keys_in.numel();
     void *st = cur_stream(keys_in);
     const auto i32 = keys_in.options().dtype(at::kInt);
-    Tensor stats = stats_in.has_value() ? *stats_in : at::zeros({TXS_STATS_LEN}, i32);
-    check_i32(stats, "stats");
-    TORCH_CHECK(stats.numel() == TXS_STATS_LEN, "stats must have TXS_STATS_LEN entries");
-    // Keys from a grid that is not much larger than the input: dense ids from an occupancy
-    // map (no sort of the keys), then the index preparation of those ids.  `stats` is read
-    // twice: the number of distinct keys, which sizes the plan (fetched while the ids are
-    // still being written), and the plan's own figures.
-    if (N > 0 && bitmap_is_cheaper(N, key_bound)) {
-        const int is64 = keys_in.scalar_type() == at::kLong;
-        Tensor inv = at::empty({N}, i32), unq = at::empty({std::min(N, key_bound)}, i32);
-        Tensor bws = at::empty({txs_unique_bitmap_workspace_len(key_bound)}, i32);
-        check_status(txs_unique_bitmap_count(keys_in.data_ptr(), is64, N, key_bound, i32w(bws), i32w(stats), st),
-                     "unique_bitmap_count");
-        Tensor h = at::empty({TXS_STATS_LEN}, stats.options().device(at::kCPU).pinned_memory(true));
-        h.copy_(stats, /*non_blocking=*/true);
-        at::cuda::CUDAEvent counted;
-        counted.record(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(keys_in.device().index()));
-        check_status(txs_unique_bitmap_assign(keys_in.data_ptr(), is64, N, key_bound, i32p(bws), i32w(inv), i32w(unq), st),
-                     "unique_bitmap_assign");
-        counted.synchronize();
-        TORCH_CHECK(h.data_ptr<int32_t>()[TXS_STAT_OUT_OF_RANGE] == 0,
-                    "keys (or points) outside the grid: keys must be in [0, ", key_bound, ")");
-        const int64_t U = h.data_ptr<int32_t>()[TXS_STAT_NUM_UNQ];
-        auto [preSum, perm_out, seg, slot_of, heavy_ids, hs] = build_plan(inv, U, heavy_threshold, std::nullopt, false);
-        Tensor cnts = at::empty({U}, keys_in.options().dtype(at::kLong));
-        check_status(txs_counts_from_presum(i32p(preSum), U, U ? cnts.data_ptr<int64_t>() : nullptr, st),
-                     "counts_from_presum");
-        hs[TXS_STAT_NUM_UNQ] = U;
-        return {unq.narrow(0, 0, U), inv, cnts, preSum, perm_out, seg, slot_of, heavy_ids, hs};
+    if (stats_in.has_value()) {
+        check_i32(*stats_in, "stats");
+        TORCH_CHECK(stats_in->numel() == TXS_STATS_LEN, "stats must have TXS_STATS_LEN entries");
     }
+    // Keys from a bounded grid: dense ids from an occupancy map (no sort of the keys), then the
+    // index preparation of those ids.  The number of distinct keys is read back with the plan's own
+    // figures: until then everything is sized for as many as there can be.
+    if (N > 0 && bitmap_is_cheaper(N, key_bound)) {
+        const int64_t most = std::min(N, key_bound);
+        Tensor inv = at::empty({N}, i32), unq = at::empty({most}, i32), seg = at::empty({N}, i32);
+        Tensor perm = at::empty({N}, i32), preSum = at::empty({most + 1}, i32);
+        Tensor slot_of = at::empty({most}, i32), heavy_all = at::empty({most}, i32);
+        Tensor cnts = at::empty({most}, keys_in.options().dtype(at::kLong));
+        Tensor bws = at::empty({txs_unique_bitmap_workspace_len(key_bound)}, i32);
+        Tensor ws = at::empty({txs_plan_workspace_len(N, most)}, i32);
+        Tensor stats = at::empty({TXS_STATS_LEN + 2}, i32);
+        check_status(txs_unique_plan(keys_in.data_ptr(), keys_in.scalar_type() == at::kLong, N, key_bound,
+                                     stats_in.has_value() ? stats_in->data_ptr<int32_t>() + TXS_STAT_OUT_OF_RANGE
+                                                          : nullptr,
+                                     i32w(bws), (int32_t)heavy_threshold, i32w(ws), i32w(inv), i32w(unq),
+                                     cnts.data_ptr<int64_t>(), i32w(perm), i32w(seg), i32w(preSum), i32w(slot_of),
+                                     i32w(heavy_all), i32w(stats), st),
+                     "unique_plan");
+        std::vector<int64_t> hs = read_stats(stats);
+        const int64_t U = hs[TXS_STATS_LEN];
+        TORCH_CHECK(hs[TXS_STATS_LEN + 1] == 0, "keys (or points) outside the grid: keys must be in [0, ", key_bound, ")");
+        if (hs[TXS_STAT_NEED_GENERAL]) {
+            // a few voxels own most of the rows: the bucket kernels stepped aside
+            stats.zero_();
+            check_status(txs_plan_build_general(i32p(inv), N, U, (int32_t)heavy_threshold, nullptr, i32w(ws),
+                                                i32w(perm), i32w(seg), i32w(preSum), i32w(slot_of),
+                                                i32w(heavy_all), i32w(stats), st),
+                         "plan_build_general");
+            check_status(txs_counts_from_presum(i32p(preSum), U, cnts.data_ptr<int64_t>(), st), "counts_from_presum");
+            hs = read_stats(stats);
+        }
+        hs.resize(TXS_STATS_LEN);
+        hs[TXS_STAT_NUM_UNQ] = U;
+        demote_few_heavy(hs, heavy_threshold, preSum, seg, slot_of, heavy_all, stats, N, U, st);
+        OptTensor perm_out;
+        if (hs[TXS_STAT_UNSORTED]) perm_out = perm;
+        // (every voxel owns rows: heavy ones are the only special ones, at the front of the list)
+        return {unq.narrow(0, 0, U), inv, cnts.narrow(0, 0, U), preSum.narrow(0, 0, U + 1), perm_out, seg,
+                slot_of.narrow(0, 0, U), special_list(heavy_all, most, hs), hs};
+    }
+    Tensor stats = stats_in.has_value() ? *stats_in : at::zeros({TXS_STATS_LEN}, i32);
     // int64 keys are narrowed for the sort; one outside int32 is first pinned to a value that
     // stays outside [0, key_bound) (key_bound is below 2^31 - 1), so that the range check on
     // the device flags it instead of seeing its low 32 bits

@@ -271,14 +271,19 @@ long scan_tiles(long n_out);
 // out[i] = sum_{k<i} in[k] for i in [0, n_out), where in[k] = 0 for k >= n_in; in
 // and out may alias.  Three launches on `st`, no inter-block waiting.
 hipError_t exclusive_scan(const int *in, long n_in, int *out, long n_out, int *ws, hipStream_t st);
-
+// The same where ws already holds the sums of the tiles of kScanTileItems inputs.
+constexpr int kScanTileItems = 2048;
+hipError_t scan_from_tile_sums(const int *in, long n_in, int *out, long n_out, int *ws, hipStream_t st);
 
 // txs_plan_build with one more output (plan_kernels.hip): ranks != NULL asks for the rank of
 // every row inside its voxel instead of the permutation and the per-position ids; only the
-// bucket kernels write it, which plan_writes_ranks() predicts from the extents.
+// bucket kernels write it, which plan_writes_ranks() predicts from the extents.  num_unq_dev != NULL:
+// the voxel count, on the device; num_unq is then an upper bound of it, no voxel below it may be
+// empty, and `stats` needs no initialisation.  cnts_out (may be NULL): rows of every voxel.
 int plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
                const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum,
-               int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, long long *ranks, void *stream);
+               int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, long long *ranks, const int *num_unq_dev,
+               long long *cnts_out, void *stream);
 bool plan_writes_ranks(long num_total, long num_unq);
 
 // Row-order "table mode" for inputs with few voxels (table_kernels.hip): whether it
