@@ -187,6 +187,12 @@ int txs_plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq,
                    int32_t heavy_threshold, const int64_t *unq_cnts, int32_t *plan_ws,
                    int32_t *perm, int32_t *seg, int32_t *preSum, int32_t *slot_of,
                    int32_t *heavy_ids, int32_t *stats, void *stream);
+/* The same from int64 ids (the inverse torch.unique returns), cut to 32 bits: unq_inv [num_total]
+ * is an output here. */
+int txs_plan_build_i64(const int64_t *ids, int32_t *unq_inv, int64_t num_total, int64_t num_unq,
+                       int32_t heavy_threshold, const int64_t *unq_cnts, int32_t *plan_ws,
+                       int32_t *perm, int32_t *seg, int32_t *preSum, int32_t *slot_of,
+                       int32_t *heavy_ids, int32_t *stats, void *stream);
 int64_t txs_plan_workspace_len(int64_t num_total, int64_t num_unq);
 /* The same outputs through the general sequence (any number of voxels, any occupancy). */
 int txs_plan_build_general(const int32_t *unq_inv, int64_t num_total, int64_t num_unq,
@@ -306,6 +312,10 @@ int txs_ingroup_inds(const int32_t *seg, const int32_t *perm, const int32_t *pre
 int txs_group_ranks(const int32_t *group_ids, int64_t num_total, int64_t num_groups,
                     int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum, int64_t *out,
                     int32_t *stats, void *stream);
+/* The same from int64 ids, cut to 32 bits: group_ids [num_total] is an output here. */
+int txs_group_ranks_i64(const int64_t *ids, int32_t *group_ids, int64_t num_total, int64_t num_groups,
+                        int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum, int64_t *out,
+                        int32_t *stats, void *stream);
 
 /* Points inside (enlarged) rotated boxes.  Replaces dynamic_point_pool_launcher
  * (torchex/src/dynamic_point_pool/dynamic_point_pool.cpp:20-32, kernels

@@ -17,7 +17,7 @@ def _ids(kind, U, rng):
         c = rng.integers(0, 6, U)
     elif kind == "edges":         # 63, 64, 65 rows, and runs of a slice's length and one off it
         c = rng.choice([0, 1, 2, 63, 64, 65, 66], U, p=[.3, .3, .3, .025, .025, .025, .025])
-        c[rng.integers(0, U, 3)] = [4095, 4096, 4097]
+        c[rng.choice(U, 6, replace=False)] = [2047, 2048, 2049, 4095, 4096, 4097]
     elif kind == "long":          # as many long runs in a slice as fit
         c = np.zeros(U, np.int64)
         c[U // 3:U // 3 + 200] = 65
@@ -53,9 +53,15 @@ def test_plan_of_slices(U, kind, grouped):
     assert data.num_heavy == heavy.sum() and data.max_cnt == cnts.max()
     assert data.num_special == heavy.sum() + (cnts == 0).sum()
     assert np.array_equal(seg < 0, heavy[inv[order]] | (cnts[inv[order]] == 0))
+    # int32 ids take another first kernel than the int64 ones above
+    assert data.unq_inv.dtype == torch.int32 and np.array_equal(data.unq_inv.cpu().numpy(), inv)
+    same = T.ScatterData(torch.from_numpy(inv).int().cuda(), torch.from_numpy(cnts).cuda())
+    assert torch.equal(same.seg, data.seg) and torch.equal(same.preSum, data.preSum)
+    assert (same.perm is None and data.perm is None) or torch.equal(same.perm, data.perm)
     ranks = np.empty(inv.size, np.int64)
     ranks[order] = np.arange(inv.size) - pre[inv[order]]
     assert np.array_equal(T.ingroup_inds(torch.from_numpy(inv).cuda()).cpu().numpy(), ranks)
+    assert np.array_equal(T.ingroup_inds(torch.from_numpy(inv).int().cuda()).cpu().numpy(), ranks)
 
 
 def test_wrong_counts_are_refused_in_one_and_in_several_slices():

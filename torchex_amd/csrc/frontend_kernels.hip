@@ -830,7 +830,8 @@ int txs_unique_plan(const void *keys, int key_is_int64, int64_t num_total, int64
     if (rc != TXS_OK || hipGetLastError() != hipSuccess) return TXS_ERR_LAUNCH;
     const int64_t most = num_total < key_bound ? num_total : key_bound;
     return txs_detail::plan_build(unq_inv, num_total, most, heavy_threshold, nullptr, plan_ws, perm, seg, preSum,
-                                  slot_of, heavy_ids, stats, nullptr, b.base + b.words, (long long *)unq_cnts, stream);
+                                  slot_of, heavy_ids, stats, nullptr, b.base + b.words, (long long *)unq_cnts, nullptr,
+                                  stream);
 }
 
 int txs_counts_from_presum(const int32_t *preSum, int64_t num_unq, int64_t *unq_cnts, void *stream) {
@@ -864,8 +865,9 @@ int txs_unique_runs(const int32_t *sorted_keys, const int32_t *perm, int64_t num
     return status_of(hipGetLastError());
 }
 
-int txs_group_ranks(const int32_t *group_ids, int64_t num_total, int64_t num_groups, int32_t *plan_ws,
-                    int32_t *perm, int32_t *seg, int32_t *preSum, int64_t *out, int32_t *stats, void *stream) {
+static int group_ranks(const long long *ids64, const int32_t *group_ids, int64_t num_total, int64_t num_groups,
+                       int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum, int64_t *out, int32_t *stats,
+                       void *stream) {
     if (!fits_i32(num_total) || !fits_i32(num_groups) || !stats) return TXS_ERR_INVALID_ARG;
     if (num_total == 0) return TXS_OK;
     if (!group_ids || !plan_ws || !perm || !seg || !preSum || !out || num_groups <= 0) return TXS_ERR_INVALID_ARG;
@@ -874,11 +876,24 @@ int txs_group_ranks(const int32_t *group_ids, int64_t num_total, int64_t num_gro
     const bool fused = txs_detail::plan_writes_ranks(num_total, num_groups);
     const int rc = txs_detail::plan_build(group_ids, num_total, num_groups, heavy, nullptr, plan_ws, perm, seg, preSum,
                                           nullptr, nullptr, stats, fused ? (long long *)out : nullptr, nullptr, nullptr,
-                                          stream);
+                                          ids64, stream);
     if (rc != TXS_OK || fused) return rc;
     ingroup_inds_auto_kernel<<<dim3(blocks_for(num_total)), dim3(kThreads), 0, (hipStream_t)stream>>>(
         seg, perm, preSum, stats, num_total, (int)num_groups, (long long *)out);
     return status_of(hipGetLastError());
+}
+
+int txs_group_ranks(const int32_t *group_ids, int64_t num_total, int64_t num_groups, int32_t *plan_ws,
+                    int32_t *perm, int32_t *seg, int32_t *preSum, int64_t *out, int32_t *stats, void *stream) {
+    return group_ranks(nullptr, group_ids, num_total, num_groups, plan_ws, perm, seg, preSum, out, stats, stream);
+}
+
+int txs_group_ranks_i64(const int64_t *ids, int32_t *group_ids, int64_t num_total, int64_t num_groups,
+                        int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum, int64_t *out, int32_t *stats,
+                        void *stream) {
+    if (num_total > 0 && !ids) return TXS_ERR_INVALID_ARG;
+    return group_ranks((const long long *)ids, group_ids, num_total, num_groups, plan_ws, perm, seg, preSum, out, stats,
+                       stream);
 }
 
 int txs_ingroup_inds(const int32_t *seg, const int32_t *perm, const int32_t *preSum,

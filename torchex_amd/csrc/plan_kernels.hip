@@ -463,10 +463,13 @@ __device__ __forceinline__ unsigned long long wave_match(int digit, int bits, bo
 }
 
 // hist: [high_bins][n_tiles] digit-major (the order its exclusive scan needs); tile_flags: [n_tiles]
-template <int ITEMS>
+// K = long long: ids as torch.unique returns them, cut to 32 bits and left in `ids32` for the
+// kernels that follow (a conversion of its own reads and writes them once more: 16 us of 4M ids,
+// 5 us of 1M)
+template <int ITEMS, typename K>
 __global__ __launch_bounds__(kHistThreads) void bucket_hist_kernel(
-    const int *__restrict__ inv, long n, int U, int low_bits, int high_bins, int *__restrict__ hist,
-    int *__restrict__ tile_flags, int n_tiles) {
+    const K *__restrict__ inv, long n, int U, int low_bits, int high_bins, int *__restrict__ hist,
+    int *__restrict__ tile_flags, int n_tiles, int *__restrict__ ids32) {
     __shared__ int h[1 << kBucketLowBitsMax];
     __shared__ int s_flags;
     for (int d = threadIdx.x; d < high_bins; d += kHistThreads) h[d] = 0;
@@ -477,7 +480,8 @@ __global__ __launch_bounds__(kHistThreads) void bucket_hist_kernel(
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
         const long i = base + (long)it * kHistThreads + threadIdx.x;
-        v[it] = i < n ? inv[i] : 0x7fffffff;
+        v[it] = i < n ? (int)inv[i] : 0x7fffffff;
+        if (sizeof(K) == 8 && i < n) ids32[i] = v[it];
     }
     bool bad_range = false, bad_order = false;
 #pragma unroll
@@ -491,7 +495,7 @@ __global__ __launch_bounds__(kHistThreads) void bucket_hist_kernel(
         }
         // neighbour in memory = the next thread's element of the same round
         int nb = __shfl_down(v[it], 1, 64);
-        if ((threadIdx.x & 63) == 63) nb = (i + 1 < n) ? inv[i + 1] : 0x7fffffff;
+        if ((threadIdx.x & 63) == 63) nb = (i + 1 < n) ? (int)inv[i + 1] : 0x7fffffff;
         if (i + 1 < n && nb < v[it]) bad_order = true;
     }
     const int f = (__ballot(bad_order) != 0ull ? kFlagUnsorted : 0) | (__ballot(bad_range) != 0ull ? kFlagOutOfRange : 0);
@@ -499,6 +503,11 @@ __global__ __launch_bounds__(kHistThreads) void bucket_hist_kernel(
     __syncthreads();
     for (int d = threadIdx.x; d < high_bins; d += kHistThreads) hist[(long)d * n_tiles + blockIdx.x] = h[d];
     if (threadIdx.x == 0) tile_flags[blockIdx.x] = s_flags;
+}
+
+__global__ void narrow_ids_kernel(const long long *__restrict__ ids64, long n, int *__restrict__ ids32) {
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) ids32[i] = (int)ids64[i];
 }
 
 // id at position i: of unq_inv itself (rows in order) or of the (id, row) pairs the bucket scatter wrote
@@ -539,14 +548,14 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
     // ---- first destination of this tile's rows per digit (from the scanned histogram), the
     // bucket boundaries (workgroup 0 publishes them) and the test for an overfull bucket
     for (int d = threadIdx.x; d < bins; d += kHistThreads) {
-        const int first = hist[(long)d * n_tiles];
-        const int next = hist[(long)(d + 1) * n_tiles];  // the entry after the last bucket holds the total
         base_s[d] = hist[(long)d * n_tiles + blockIdx.x];
         if (blockIdx.x == 0) {
+            const int first = base_s[d];
+            const int next = hist[(long)(d + 1) * n_tiles];  // the entry after the last bucket holds the total
             bucket_start[d] = first;
             if (d == bins - 1) bucket_start[bins] = next;
+            if ((long)next - first > giant) atomicOr(&s_flags, 4);
         }
-        if ((long)next - first > giant) atomicOr(&s_flags, 4);
     }
     __syncthreads();
     const int flags = s_flags;
@@ -559,7 +568,9 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
             stats[k] = val;
         }
     }
-    if (flags & 4) return;  // the caller re-plans with the general sequence
+    // (where a bucket is overfull the caller re-plans with the general sequence, and what the
+    // workgroups write from here on goes unread: only the first one looks, because two more reads
+    // per bucket in every workgroup cost more than that rare case's wasted scatter)
     const long tile0 = (long)blockIdx.x * (kHistThreads * ITEMS);
     if (!(flags & kFlagUnsorted)) {
         if (out_keys)
@@ -1184,7 +1195,15 @@ int txs_plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, i
                    const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum,
                    int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream) {
     return txs_detail::plan_build(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum,
-                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, stream);
+                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, nullptr, stream);
+}
+
+int txs_plan_build_i64(const int64_t *ids, int32_t *unq_inv, int64_t num_total, int64_t num_unq,
+                       int32_t heavy_threshold, const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg,
+                       int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream) {
+    if (num_total > 0 && !ids) return TXS_ERR_INVALID_ARG;
+    return txs_detail::plan_build(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum,
+                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, (const long long *)ids, stream);
 }
 
 }  // extern "C"
@@ -1227,7 +1246,8 @@ bool txs_detail::plan_writes_ranks(long num_total, long num_unq) {
 int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
                            const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg,
                            int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids, int32_t *stats,
-                           long long *ranks, const int *num_unq_dev, long long *cnts_out, void *stream) {
+                           long long *ranks, const int *num_unq_dev, long long *cnts_out,
+                           const long long *ids64, void *stream) {
     if (!fits_i32(num_total) || !fits_i32(num_unq) || !stats || !preSum || heavy_threshold < kChunk)
         return TXS_ERR_INVALID_ARG;
     hipStream_t st = (hipStream_t)stream;
@@ -1244,9 +1264,12 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
         stats_clear_kernel<<<dim3(1), dim3(64), 0, st>>>(stats);
         if (hipGetLastError() != hipSuccess) return TXS_ERR_LAUNCH;
     }
-    if (n == 0 || U == 0 || bits > kBucketBitsMax)
+    int *ids32 = const_cast<int *>(unq_inv);  // written only where ids64 is given
+    if (n == 0 || U == 0 || bits > kBucketBitsMax) {
+        if (ids64 && n > 0) narrow_ids_kernel<<<dim3(blocks_for(n)), dim3(kThreads), 0, st>>>(ids64, n, ids32);
         return plan_general(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum, slot_of,
                             heavy_ids, stats, num_unq_dev, cnts_out, stream);
+    }
     // ids of up to 11 bits are sorted by the bucket pass alone; beyond that the bucket digit has
     // 9 bits (narrower, and the buckets of a spatially sorted id space get too uneven: a
     // bucket's workgroups each count the whole bucket; wider, and a tile sends too few rows to
@@ -1282,11 +1305,18 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
                 return TXS_ERR_LAUNCH;
         lds_allowed[dev].store(true, std::memory_order_release);
     }
-    auto hist_kernel = items == 16 ? bucket_hist_kernel<16> : (items == 8 ? bucket_hist_kernel<8> : bucket_hist_kernel<4>);
+    auto hist32 = items == 16 ? bucket_hist_kernel<16, int>
+                              : (items == 8 ? bucket_hist_kernel<8, int> : bucket_hist_kernel<4, int>);
+    auto hist64 = items == 16 ? bucket_hist_kernel<16, long long>
+                              : (items == 8 ? bucket_hist_kernel<8, long long> : bucket_hist_kernel<4, long long>);
     auto scatter_kernel =
         items == 16 ? bucket_scatter_kernel<16> : (items == 8 ? bucket_scatter_kernel<8> : bucket_scatter_kernel<4>);
-    hist_kernel<<<dim3(n_tiles), dim3(kHistThreads), 0, st>>>(unq_inv, n, U, low_bits, high_bins, hist, tile_flags,
-                                                              n_tiles);
+    if (ids64)
+        hist64<<<dim3(n_tiles), dim3(kHistThreads), 0, st>>>(ids64, n, U, low_bits, high_bins, hist, tile_flags, n_tiles,
+                                                             ids32);
+    else
+        hist32<<<dim3(n_tiles), dim3(kHistThreads), 0, st>>>(unq_inv, n, U, low_bits, high_bins, hist, tile_flags,
+                                                             n_tiles, nullptr);
     // one entry more than the histogram: it receives the total, the end of the last bucket
     if (exclusive_scan(hist, used, hist, used + 1, scan_ws, st) != hipSuccess) return TXS_ERR_LAUNCH;
     const size_t lds_scatter = (size_t)high_bins * sizeof(int) +

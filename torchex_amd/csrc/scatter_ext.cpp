@@ -112,12 +112,13 @@ void demote_few_heavy(std::vector<int64_t> &hs, int64_t heavy_threshold, const T
 // (extends torchex/operator_py/scatter_op.py:13-21).  Everything is queued on
 // the current stream; the only host synchronisation is the read of `stats`.
 // returns (preSum, perm | None, seg, slot_of, heavy_ids, stats)
+// ids64: the ids as int64; unq_inv then is written from them, not read (not with assume_sorted).
 // assume_sorted: the caller states that unq_inv is non-decreasing (the only order the
 // reference accepts); the sort is then not even queued, and the statement is checked
 // on the device (an unsorted unq_inv raises).
-std::tuple<Tensor, OptTensor, Tensor, Tensor, Tensor, std::vector<int64_t>> build_plan(
-    const Tensor &unq_inv, int64_t num_unq, int64_t heavy_threshold, const OptTensor &unq_cnts,
-    bool assume_sorted) {
+using Plan = std::tuple<Tensor, OptTensor, Tensor, Tensor, Tensor, std::vector<int64_t>>;
+Plan build_plan_from(const Tensor &unq_inv, const int64_t *ids64, int64_t num_unq, int64_t heavy_threshold,
+                     const OptTensor &unq_cnts, bool assume_sorted) {
     check_i32(unq_inv, "unq_inv");
     TORCH_CHECK(unq_inv.dim() == 1, "unq_inv must be 1-D");
     TORCH_CHECK(num_unq >= 0, "num_unq must be non-negative");
@@ -131,7 +132,10 @@ std::tuple<Tensor, OptTensor, Tensor, Tensor, Tensor, std::vector<int64_t>> buil
     c10::hip::HIPGuardMasqueradingAsCUDA guard(unq_inv.device());
     const int64_t N = unq_inv.numel(), U = num_unq;
     void *st = cur_stream(unq_inv);
-    Tensor stats = at::zeros({TXS_STATS_LEN}, unq_inv.options());
+    // (the bucket kernels set every entry themselves; the other sequences add to them)
+    const bool add_to_stats = assume_sorted || U > (int64_t(1) << 22);
+    Tensor stats = add_to_stats ? at::zeros({TXS_STATS_LEN}, unq_inv.options())
+                                : at::empty({TXS_STATS_LEN}, unq_inv.options());
     Tensor seg, perm;
     Tensor preSum = empty_i32(U + 1, unq_inv);
     Tensor slot_of = empty_i32(U, unq_inv);
@@ -150,9 +154,13 @@ std::tuple<Tensor, OptTensor, Tensor, Tensor, Tensor, std::vector<int64_t>> buil
         seg = empty_i32(N, unq_inv);
         perm = empty_i32(N, unq_inv);
         Tensor ws = empty_i32(txs_plan_workspace_len(N, U), unq_inv);
-        check_status(txs_plan_build(i32p(unq_inv), N, U, (int32_t)heavy_threshold, cnts, i32w(ws), i32w(perm),
-                                    i32w(seg), i32w(preSum), i32w(slot_of), i32w(heavy_all), i32w(stats), st),
-                     "plan_build");
+        const int rc =
+            ids64 ? txs_plan_build_i64(ids64, N ? unq_inv.data_ptr<int32_t>() : nullptr, N, U, (int32_t)heavy_threshold,
+                                       cnts, i32w(ws), i32w(perm), i32w(seg), i32w(preSum), i32w(slot_of),
+                                       i32w(heavy_all), i32w(stats), st)
+                  : txs_plan_build(i32p(unq_inv), N, U, (int32_t)heavy_threshold, cnts, i32w(ws), i32w(perm), i32w(seg),
+                                   i32w(preSum), i32w(slot_of), i32w(heavy_all), i32w(stats), st);
+        check_status(rc, "plan_build");
         hs = read_stats(stats);
         if (hs[TXS_STAT_NEED_GENERAL]) {
             // a few voxels own most of the rows: the bucket kernels stepped aside
@@ -173,6 +181,23 @@ std::tuple<Tensor, OptTensor, Tensor, Tensor, Tensor, std::vector<int64_t>> buil
     if (hs[TXS_STAT_UNSORTED]) perm_out = perm;
     Tensor heavy_ids = special_list(heavy_all, U, hs);
     return {preSum, perm_out, seg, slot_of, heavy_ids, hs};
+}
+
+Plan build_plan(const Tensor &unq_inv, int64_t num_unq, int64_t heavy_threshold, const OptTensor &unq_cnts,
+                bool assume_sorted) {
+    return build_plan_from(unq_inv, nullptr, num_unq, heavy_threshold, unq_cnts, assume_sorted);
+}
+
+// the same from int64 ids: (ids as int32, plan)
+std::tuple<Tensor, Plan> build_plan_i64(const Tensor &ids, int64_t num_unq, int64_t heavy_threshold,
+                                        const OptTensor &unq_cnts) {
+    check_dev(ids, "unq_inv");
+    TORCH_CHECK(ids.scalar_type() == at::kLong && ids.dim() == 1, "unq_inv must be int64 and 1-D");
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(ids.device());
+    Tensor inv = empty_i32(ids.numel(), ids);
+    Plan plan = build_plan_from(inv, ids.numel() ? ids.data_ptr<int64_t>() : nullptr, num_unq, heavy_threshold, unq_cnts,
+                                false);
+    return {inv, plan};
 }
 
 // Plan for callers that hold only CSR offsets of already grouped rows.
@@ -355,22 +380,27 @@ void group_ranks_into(const Tensor &ids_in, Tensor &out) {
     TORCH_CHECK(ids_in.scalar_type() == at::kInt || ids_in.scalar_type() == at::kLong,
                 "group_inds must be int32 or int64");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(ids_in.device());
-    Tensor ids = ids_in.reshape({-1}).contiguous();
-    if (ids.scalar_type() != at::kInt) ids = ids.to(at::kInt);
-    const int64_t N = ids.numel();
+    const Tensor flat = ids_in.reshape({-1}).contiguous();
+    const int64_t N = flat.numel();
     if (N == 0) return;
+    // int64 ids are cut to 32 bits by the first kernel that reads them
+    const bool narrow = flat.scalar_type() == at::kLong;
+    Tensor ids = narrow ? at::empty({N}, flat.options().dtype(at::kInt)) : flat;
     void *st = cur_stream(ids);
     // `exact`: U is the true bound of the ids (largest id + 1), not the guess `number of rows`
     auto attempt = [&](int64_t U, bool exact) -> bool {
-        Tensor stats = at::zeros({TXS_STATS_LEN}, ids.options());
+        Tensor stats = U > (int64_t(1) << 22) ? at::zeros({TXS_STATS_LEN}, ids.options())
+                                              : at::empty({TXS_STATS_LEN}, ids.options());
         Tensor seg = empty_i32(N, ids), perm = empty_i32(N, ids);
         Tensor preSum = empty_i32(U + 1, ids);
         Tensor ws = empty_i32(txs_plan_workspace_len(N, U), ids);
         const int32_t heavy = txs_default_heavy_threshold();
         // order and offsets only (no special-voxel table) and the ranks, queued together
-        check_status(txs_group_ranks(i32p(ids), N, U, i32w(ws), i32w(perm), i32w(seg), i32w(preSum),
-                                     out.data_ptr<int64_t>(), i32w(stats), st),
-                     "group_ranks");
+        const int rc = narrow ? txs_group_ranks_i64(flat.data_ptr<int64_t>(), i32w(ids), N, U, i32w(ws), i32w(perm),
+                                                    i32w(seg), i32w(preSum), out.data_ptr<int64_t>(), i32w(stats), st)
+                              : txs_group_ranks(i32p(ids), N, U, i32w(ws), i32w(perm), i32w(seg), i32w(preSum),
+                                                out.data_ptr<int64_t>(), i32w(stats), st);
+        check_status(rc, "group_ranks");
         std::vector<int64_t> hs = read_stats(stats);
         if (hs[TXS_STAT_OUT_OF_RANGE]) return false;
         if (hs[TXS_STAT_NEED_GENERAL]) {
@@ -958,6 +988,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("sum", &sum_ref, "scatter_sum over CSR offsets, in place (HIP)");
     m.def("max", &max_ref, "scatter_max with arg over CSR offsets, in place (HIP)");
     m.def("getPreSum", &get_presum_ref, "CSR offsets from a sorted unq_inv (HIP)");
+    m.def("build_plan_i64", &build_plan_i64,
+          "build_plan_i64(unq_inv int64, num_unq, heavy_threshold, unq_cnts|None) -> (unq_inv int32, build_plan(...))",
+          pybind11::arg("unq_inv"), pybind11::arg("num_unq"), pybind11::arg("heavy_threshold"), pybind11::arg("unq_cnts"));
     m.def("build_plan", &build_plan, "build_plan(unq_inv, num_unq, heavy_threshold, unq_cnts|None, assume_sorted=False)",
           pybind11::arg("unq_inv"), pybind11::arg("num_unq"), pybind11::arg("heavy_threshold"),
           pybind11::arg("unq_cnts"), pybind11::arg("assume_sorted") = false);

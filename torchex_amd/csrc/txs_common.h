@@ -280,10 +280,11 @@ hipError_t scan_from_tile_sums(const int *in, long n_in, int *out, long n_out, i
 // bucket kernels write it, which plan_writes_ranks() predicts from the extents.  num_unq_dev != NULL:
 // the voxel count, on the device; num_unq is then an upper bound of it, no voxel below it may be
 // empty, and `stats` needs no initialisation.  cnts_out (may be NULL): rows of every voxel.
+// ids64 != NULL: the ids come from there, and unq_inv is written (cut to 32 bits), not read.
 int plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
                const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum,
                int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, long long *ranks, const int *num_unq_dev,
-               long long *cnts_out, void *stream);
+               long long *cnts_out, const long long *ids64, void *stream);
 bool plan_writes_ranks(long num_total, long num_unq);
 
 // Row-order "table mode" for inputs with few voxels (table_kernels.hip): whether it

@@ -83,7 +83,6 @@ class ScatterData:
             1, 2), f"unq_inv in ScatterData should be 1 or 2-dims, but got {unq_inv.ndim}-dims"
         assert unq_cnts.ndim in (
             1, 2), f"unq_cnts in ScatterData should be 1 or 2-dims, but got {unq_cnts.ndim}-dims"
-        self.unq_inv = unq_inv.int()
         if unq_cnts.ndim == 1:
             self.unq_cnts = unq_cnts.unsqueeze(-1)
         else:
@@ -92,11 +91,18 @@ class ScatterData:
         if heavy_threshold is None:
             heavy_threshold = scatter_ext.default_heavy_threshold()
         self.heavy_threshold = int(heavy_threshold)
-        flat = self.unq_inv.reshape(-1).contiguous()
         num_unq = self.unq_cnts.shape[0]
         cnts64 = self.unq_cnts.reshape(-1).long().contiguous()
-        (self.preSum, self.perm, self.seg, self.slot_of, self.heavy_ids,
-         stats) = scatter_ext.build_plan(flat, num_unq, self.heavy_threshold, cnts64, bool(assume_sorted))
+        if unq_inv.dtype == torch.int64 and unq_inv.is_cuda and not assume_sorted:
+            # torch.unique's inverse as it comes: the first kernel that reads it narrows it
+            flat, plan = scatter_ext.build_plan_i64(unq_inv.reshape(-1).contiguous(), num_unq,
+                                                    self.heavy_threshold, cnts64)
+            self.unq_inv = flat.reshape(unq_inv.shape)
+        else:
+            self.unq_inv = unq_inv.int()
+            flat = self.unq_inv.reshape(-1).contiguous()
+            plan = scatter_ext.build_plan(flat, num_unq, self.heavy_threshold, cnts64, bool(assume_sorted))
+        self.preSum, self.perm, self.seg, self.slot_of, self.heavy_ids, stats = plan
         # same consistency check as the reference (scatter_op.py:19), made on
         # the recomputed histogram so that a stale unq_cnts is caught too
         assert stats[5] == 0, "unq_cnts is not the histogram of unq_inv"
