@@ -22,3 +22,20 @@ def test_rows_that_fill_no_whole_vectors(C, dtype):
     feats[torch.rand(feats.shape, generator=g) < 0.05] = 1.25    # ties
     data = run_case(f"vectors{C}", feats, inv, cnts, dtype=dtype)
     assert data.num_heavy == 10
+
+
+@pytest.mark.parametrize("N,C,dtype", [(270_000, 3, torch.float32), (600_000, 4, torch.float16),
+                                       (1_100_000, 2, torch.float32), (1_100_000, 13, torch.bfloat16)])
+def test_narrow_rows_with_heavy_voxels_in_large_tiles(N, C, dtype):
+    """The tile grows with the rows (1024 to 4096 positions): heavy voxels that fill many tiles, lie
+    inside one, and end at a tile's edge, between ordinary ones."""
+    g = torch.Generator().manual_seed(N + C)
+    cnts = torch.cat([torch.randint(1, 12, (N // 12,), generator=g), torch.tensor([4096, 4095, 4097, 65, 97, 64, 30_000]),
+                      torch.randint(65, 2000, (40,), generator=g)])
+    cnts = cnts[torch.randperm(cnts.numel(), generator=g)]
+    cnts = torch.cat([cnts, torch.ones(max(0, N - int(cnts.sum())), dtype=torch.long)])
+    inv = torch.repeat_interleave(torch.arange(cnts.numel()), cnts)
+    inv = inv[torch.randperm(inv.numel(), generator=g)]
+    feats = torch.randn((inv.numel(), C), generator=g)
+    data = run_case(f"narrow{N}", feats, inv, cnts, dtype=dtype)
+    assert data.num_heavy >= 40

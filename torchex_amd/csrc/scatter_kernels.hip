@@ -780,7 +780,8 @@ struct Geometry {
 
 unsigned reciprocal32(int d) { return d == 1 ? 0u : (unsigned)(((1ULL << 32) + (unsigned)d - 1) / (unsigned)d); }
 
-Geometry make_geometry(long N, long C, int elem, const void *p0, const void *p1, int chunk, bool forward) {
+Geometry make_geometry(long N, long C, int elem, const void *p0, const void *p1, int chunk, bool forward,
+                       bool heavy = false) {
     Geometry g;
     g.hint = (C * elem) % 64 == 0 && aligned_to(p0, 64) && aligned_to(p1, 64);
     // bytes per lane and row: 16 for fp32; 8 for the 2-byte types, whose kernels carry
@@ -799,6 +800,15 @@ Geometry make_geometry(long N, long C, int elem, const void *p0, const void *p1,
     // (forward) a small input gets smaller tiles while that gives the chip more workgroups
     // (below eight per compute unit a tile's fixed costs show: 3-5 % on 200k rows of 256 bytes)
     while (forward && chunk > 4 && N / ((long)g.lm.groups * chunk) < 2048) chunk /= 2;
+    // Narrow rows (at most four lanes) with heavy voxels: every tile that a heavy voxel reaches into
+    // costs an atomic per element, and neighbouring heavy rows share their cache lines, on which
+    // atomics run one after the other.  The largest tile that still gives every compute unit one:
+    // mean of three fp32 channels over pillars, 316k rows in tiles of 256 / 512 / 1024 / 4096 31.4 /
+    // 26.6 / 19.7 / 27.2 us, 1.6M rows in tiles of 512 / 1024 / 4096 52.6 / 52.1 / 48.8.
+    if (forward && heavy && g.lm.lanes <= 4) {
+        chunk = 4;
+        while (g.lm.groups * chunk * 2 <= 4096 && N / ((long)g.lm.groups * chunk * 2) >= 256) chunk *= 2;
+    }
     long tile = (long)g.lm.groups * chunk;
     // the forward kernel finds the borders of a tile's range with one wave ballot each: a tile
     // is a whole number of wavefronts' worth of staged ids (its rows are dealt evenly anyway)
@@ -1008,7 +1018,7 @@ int scatter_forward_impl(int op, int dtype, const void *feats, const int32_t *un
         if (hipGetLastError() != hipSuccess) return TXS_ERR_LAUNCH;
     }
     if (N > 0) {
-        Geometry geo = make_geometry(N, C, elem, feats, out, fwd_chunk_for(N, U, op, elem), true);
+        Geometry geo = make_geometry(N, C, elem, feats, out, fwd_chunk_for(N, U, op, elem), true, num_heavy > 0);
         if (dtype == TXS_F32)
             e = launch_fwd<F32>(op, geo, st, feats, perm, seg, preSum, slot_of, out, arg, scratch, N, C, U, ref_log2);
         else if (dtype == TXS_F16)
