@@ -805,9 +805,12 @@ Geometry make_geometry(long N, long C, int elem, const void *p0, const void *p1,
     // atomics run one after the other.  The largest tile that still gives every compute unit one:
     // mean of three fp32 channels over pillars, 316k rows in tiles of 256 / 512 / 1024 / 4096 31.4 /
     // 26.6 / 19.7 / 27.2 us, 1.6M rows in tiles of 512 / 1024 / 4096 52.6 / 52.1 / 48.8.
+    // With one lane per row an atomic instruction reaches one element of a row only, and fewer,
+    // larger tiles still pay: four fp32 channels, 316k rows in tiles of 1024 / 4096 30.7 / 28.2 us.
     if (forward && heavy && g.lm.lanes <= 4) {
+        const long least = g.lm.lanes == 1 ? 64 : 256;  // workgroups
         chunk = 4;
-        while (g.lm.groups * chunk * 2 <= 4096 && N / ((long)g.lm.groups * chunk * 2) >= 256) chunk *= 2;
+        while (g.lm.groups * chunk * 2 <= 4096 && N / ((long)g.lm.groups * chunk * 2) >= least) chunk *= 2;
     }
     long tile = (long)g.lm.groups * chunk;
     // the forward kernel finds the borders of a tile's range with one wave ballot each: a tile
