@@ -2,12 +2,14 @@
 several, voxels with a short, a threshold-sized and a long run of rows in a slice (up to a
 slice that is one voxel), few and many voxels per bucket, grouped rows, empty voxels.  The plan
 is whole numbers with one right answer: a stable sort by voxel."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import torchex_amd as T
-from torchex_amd import scatter_ext
+from torchex_amd import _native
 
 pytestmark = pytest.mark.gpu
 
@@ -72,3 +74,26 @@ def test_wrong_counts_are_refused_in_one_and_in_several_slices():
         cnts[7] += 1
         with pytest.raises(AssertionError):
             T.ScatterData(inv.cuda(), cnts.cuda())
+
+
+def test_an_overfull_bucket_leaves_the_rows_alone():
+    """Where one bucket holds more rows than the bucket kernels take, the call only says so: the
+    space the rows would be sorted into is not written."""
+    lib = _native.cabi()
+    vp, i64 = ctypes.c_void_p, ctypes.c_int64
+    N, U = 400_000, 5000
+    rng = np.random.default_rng(1)
+    inv = rng.integers(0, U, N).astype(np.int32)
+    inv[rng.permutation(N)[:300_000]] = 7
+    ids = torch.from_numpy(inv).cuda()
+    lib.txs_plan_workspace_len.restype = i64
+    ws = torch.full((lib.txs_plan_workspace_len(i64(N), i64(U)),), -7, dtype=torch.int32, device="cuda")
+    perm, seg, pre, slot, heavy, stats = (torch.full((n,), -7, dtype=torch.int32, device="cuda")
+                                          for n in (N, N, U + 1, U, U, 16))
+    rc = lib.txs_plan_build(vp(ids.data_ptr()), i64(N), i64(U), ctypes.c_int32(64), vp(0), vp(ws.data_ptr()),
+                            vp(perm.data_ptr()), vp(seg.data_ptr()), vp(pre.data_ptr()), vp(slot.data_ptr()),
+                            vp(heavy.data_ptr()), vp(stats.data_ptr()), vp(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    assert stats[8].item() == 1 and stats[0].item() == 1      # NEED_GENERAL, UNSORTED
+    for t in (ws[:2 * N], perm, seg, pre, slot, heavy):
+        assert (t == -7).all()

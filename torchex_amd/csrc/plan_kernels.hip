@@ -137,9 +137,11 @@ __global__ __launch_bounds__(kThreads) void scan_tile_offsets_kernel(int *__rest
 // With offsets_ready == 0, tile_offs still holds the plain tile sums and the
 // workgroup adds up the ones in front of its own tile itself (cheaper than a
 // launch of its own while there are few tiles).
+// heads (may be NULL): receives every stride-th output on its own, heads[k] = out[k * stride].
 __global__ __launch_bounds__(kThreads) void scan_apply_kernel(const int *in, long n_in, int *out,
                                                               long n_out, const int *tile_offs,
-                                                              int offsets_ready) {
+                                                              int offsets_ready, int *__restrict__ heads,
+                                                              int stride) {
     long base = (long)blockIdx.x * kScanTile + (long)threadIdx.x * kScanItems;
     int x[kScanItems];
     int s = 0;
@@ -159,10 +161,14 @@ __global__ __launch_bounds__(kThreads) void scan_apply_kernel(const int *in, lon
     }
     int tot;
     int run = block_exclusive_scan(s, &tot) + tile_off;
+    long head = heads ? (base + stride - 1) / stride : 0;  // the next one at or after `base`
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         long i = base + k;
-        if (i < n_out) out[i] = run;
+        if (i < n_out) {
+            out[i] = run;
+            if (heads && i == head * stride) heads[head++] = run;
+        }
         run += x[k];
     }
 }
@@ -174,19 +180,20 @@ namespace txs_detail {
 long scan_tiles(long n_out) { return (n_out + kScanTile - 1) / kScanTile; }
 
 hipError_t exclusive_scan(const int *in, long n_in, int *out, long n_out, int *ws,
-                          hipStream_t st) {
+                          hipStream_t st, int *heads, int stride) {
     if (n_out <= 0) return hipSuccess;
     const long tiles = scan_tiles(n_out);
     scan_tile_sums_kernel<<<dim3((unsigned)tiles), dim3(kThreads), 0, st>>>(in, n_in, ws);
-    return scan_from_tile_sums(in, n_in, out, n_out, ws, st);
+    return scan_from_tile_sums(in, n_in, out, n_out, ws, st, heads, stride);
 }
 
-hipError_t scan_from_tile_sums(const int *in, long n_in, int *out, long n_out, int *ws, hipStream_t st) {
+hipError_t scan_from_tile_sums(const int *in, long n_in, int *out, long n_out, int *ws, hipStream_t st, int *heads,
+                               int stride) {
     if (n_out <= 0) return hipSuccess;
     const long tiles = scan_tiles(n_out);
     const int few = tiles <= kScanFusedTiles;
     if (!few) scan_tile_offsets_kernel<<<dim3(1), dim3(kThreads), 0, st>>>(ws, tiles);
-    scan_apply_kernel<<<dim3((unsigned)tiles), dim3(kThreads), 0, st>>>(in, n_in, out, n_out, ws, !few);
+    scan_apply_kernel<<<dim3((unsigned)tiles), dim3(kThreads), 0, st>>>(in, n_in, out, n_out, ws, !few, heads, stride);
     return hipGetLastError();
 }
 
@@ -516,7 +523,7 @@ __device__ __forceinline__ int kread(const int *keys, long i, bool packed) {
 }
 
 // Stable scatter by the high digit.  hist: the exclusive scan of the digit-major tile histograms.
-//   bucket_start [high_bins + 1] (written by workgroup 0): first position of every bucket.
+//   bucket_start [high_bins + 1] (from the scan): first position of every bucket.
 //   stats: zero-filled here (workgroup 0), then UNSORTED / OUT_OF_RANGE of the whole input
 //   and NEED_GENERAL (a bucket above `giant` rows: the bucket kernels step aside).
 // Rows already in order are not moved: out_keys (if given) receives a copy of the ids, and
@@ -526,7 +533,7 @@ template <int ITEMS>
 __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
     const int *__restrict__ inv, long n, int U, int low_bits, int high_bits,
     const int *__restrict__ hist, const int *__restrict__ tile_flags, int n_tiles, long giant,
-    int *__restrict__ bucket_start, int *__restrict__ stats, int *__restrict__ out_keys,
+    const int *__restrict__ bucket_start, int *__restrict__ stats, int *__restrict__ out_keys,
     int *__restrict__ out_rows, int2 *__restrict__ out_pairs) {
     // [bins] base_s: first destination of this tile's rows, per digit; then the larger of
     // [kHistWaves][bins] wave counts and the tile's staged (id, row) pairs
@@ -545,17 +552,12 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
     for (int t = threadIdx.x; t < n_tiles; t += kHistThreads) f |= tile_flags[t];
     if (f) atomicOr(&s_flags, f);
 
-    // ---- first destination of this tile's rows per digit (from the scanned histogram), the
-    // bucket boundaries (workgroup 0 publishes them) and the test for an overfull bucket
+    // ---- first destination of this tile's rows per digit (from the scanned histogram) and the
+    // test for an overfull bucket.  The bucket boundaries lie side by side for it: read from the
+    // histogram, two lines of it per bucket, they cost every workgroup more (1M ids 13.7 -> 15.4 us).
     for (int d = threadIdx.x; d < bins; d += kHistThreads) {
         base_s[d] = hist[(long)d * n_tiles + blockIdx.x];
-        if (blockIdx.x == 0) {
-            const int first = base_s[d];
-            const int next = hist[(long)(d + 1) * n_tiles];  // the entry after the last bucket holds the total
-            bucket_start[d] = first;
-            if (d == bins - 1) bucket_start[bins] = next;
-            if ((long)next - first > giant) atomicOr(&s_flags, 4);
-        }
+        if ((long)bucket_start[d + 1] - bucket_start[d] > giant) atomicOr(&s_flags, 4);
     }
     __syncthreads();
     const int flags = s_flags;
@@ -568,9 +570,7 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
             stats[k] = val;
         }
     }
-    // (where a bucket is overfull the caller re-plans with the general sequence, and what the
-    // workgroups write from here on goes unread: only the first one looks, because two more reads
-    // per bucket in every workgroup cost more than that rare case's wasted scatter)
+    if (flags & 4) return;  // the caller re-plans with the general sequence
     const long tile0 = (long)blockIdx.x * (kHistThreads * ITEMS);
     if (!(flags & kFlagUnsorted)) {
         if (out_keys)
@@ -1317,8 +1317,9 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
     else
         hist32<<<dim3(n_tiles), dim3(kHistThreads), 0, st>>>(unq_inv, n, U, low_bits, high_bins, hist, tile_flags,
                                                              n_tiles, nullptr);
-    // one entry more than the histogram: it receives the total, the end of the last bucket
-    if (exclusive_scan(hist, used, hist, used + 1, scan_ws, st) != hipSuccess) return TXS_ERR_LAUNCH;
+    // one entry more than the histogram: it receives the total, the end of the last bucket.  A
+    // bucket's first entry (that of tile 0) is where it starts.
+    if (exclusive_scan(hist, used, hist, used + 1, scan_ws, st, bucket_start, n_tiles) != hipSuccess) return TXS_ERR_LAUNCH;
     const size_t lds_scatter = (size_t)high_bins * sizeof(int) +
                                max((size_t)kHistWaves * high_bins * sizeof(int), (size_t)tile * sizeof(int2));
     if (low_bits == 0) {

@@ -269,11 +269,14 @@ namespace txs_detail {
 long scan_tiles(long n_out);
 
 // out[i] = sum_{k<i} in[k] for i in [0, n_out), where in[k] = 0 for k >= n_in; in
-// and out may alias.  Three launches on `st`, no inter-block waiting.
-hipError_t exclusive_scan(const int *in, long n_in, int *out, long n_out, int *ws, hipStream_t st);
+// and out may alias.  Three launches on `st`, no inter-block waiting.  heads (may be NULL):
+// heads[k] = out[k * stride] for every k * stride < n_out, side by side.
+hipError_t exclusive_scan(const int *in, long n_in, int *out, long n_out, int *ws, hipStream_t st,
+                          int *heads = nullptr, int stride = 1);
 // The same where ws already holds the sums of the tiles of kScanTileItems inputs.
 constexpr int kScanTileItems = 2048;
-hipError_t scan_from_tile_sums(const int *in, long n_in, int *out, long n_out, int *ws, hipStream_t st);
+hipError_t scan_from_tile_sums(const int *in, long n_in, int *out, long n_out, int *ws, hipStream_t st,
+                               int *heads = nullptr, int stride = 1);
 
 // txs_plan_build with one more output (plan_kernels.hip): ranks != NULL asks for the rank of
 // every row inside its voxel instead of the permutation and the per-position ids; only the
