@@ -1,12 +1,16 @@
 """ScatterData straight from keys by occupancy map, whose number of voxels stays on the device until
-the plan is done, against numpy and against ScatterData of the unique's ids: one voxel to as many as
-rows, ids of up to 11 bits and beyond, crowded buckets that the bucket kernels leave to the general
-sequence, key bounds at a word's edge, on either side of the map's limit, and above 2^22 rows."""
+the plan is done (up to 2^20 rows; counted first beyond), against numpy and against ScatterData of the
+unique's ids: one voxel to as many as rows, ids of up to 11 bits and beyond, voxels of many slices,
+crowded buckets that the bucket kernels leave to the general sequence, key bounds at a word's edge,
+on either side of the map's limit, and row numbers on either side of 2^20 and of 2^22."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import torchex_amd as T
+from torchex_amd import _native
 
 pytestmark = pytest.mark.gpu
 
@@ -15,7 +19,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n,bound,used", [
     (1, 1, 1), (5, 32, 32), (5, 33, 2), (700, 1 << 25, 700), (3000, 4096, 4096), (4000, 1 << 25, 1),
     (20_000, (1 << 25) + 1, 20_000), (60_000, 1 << 24, 1 << 24), (400_000, 1 << 20, 3), (400_000, 1 << 20, 5000),
-    (4_300_000, 1 << 22, 1 << 22),
+    (4_300_000, 1 << 22, 1 << 22), (1 << 20, 1 << 24, 700), ((1 << 20) + 1, 1 << 24, 700),
+    ((1 << 20) + 1, 1 << 24, 1 << 24), (1_000_000, 1 << 23, 2000), (4_300_000, 1 << 23, 90_000),
 ])
 def test_unique_plan(n, bound, used, dtype):
     rng = np.random.default_rng(n + bound)
@@ -23,6 +28,19 @@ def test_unique_plan(n, bound, used, dtype):
     keys[0] = bound - 1
     if n > 1:
         keys[-1] = 0
+    _check(keys, bound, dtype)
+
+
+@pytest.mark.parametrize("n,voxels,rows", [(900_000, 700, 700_000), (900_000, 2048, 500_000),
+                                           (900_000, 2049, 700_000), (500_000, 60_000, 300_000)])
+def test_one_voxel_owns_most_rows(n, voxels, rows):
+    rng = np.random.default_rng(voxels)
+    keys = rng.permutation(1 << 23)[:voxels][np.concatenate([np.full(rows, voxels // 2), np.arange(voxels),
+                                                             rng.integers(0, voxels, n - rows - voxels)])]
+    _check(rng.permutation(keys), 1 << 23, torch.int32)
+
+
+def _check(keys, bound, dtype):
     unq, inv, cnt = np.unique(keys, return_inverse=True, return_counts=True)
     d = T.ScatterData.from_keys(torch.from_numpy(keys).to(dtype).cuda(), bound)
     assert d.num_unq == unq.size and d.unq_cnts.shape == (unq.size, 1) and d.unq_cnts.dtype == torch.int64
@@ -45,3 +63,44 @@ def test_keys_outside_the_bound_are_refused():
             T.ScatterData.from_keys(keys.cuda(), 1000)
     with pytest.raises(RuntimeError):
         T.ScatterData.from_points(torch.tensor([[0.5, 0.5, 0.5], [9.0, 0.5, 0.5]]).cuda(), [1, 1, 1], [0, 0, 0, 2, 2, 2])
+
+
+@pytest.mark.parametrize("n,voxels", [(1_000_000, 2), (1_000_000, 64), (1_000_000, 2000), (1_000_000, 5000)])
+def test_few_voxels_of_a_large_grid_need_no_second_plan(n, voxels):
+    """The digits of the ids are split by the voxels there are, not by the most there could be: the
+    bound's split would put these into one bucket and leave the plan to the general sequence."""
+    lib = _native.cabi()
+    vp, i64, bound = ctypes.c_void_p, ctypes.c_int64, 1 << 24
+    rng = np.random.default_rng(voxels)
+    keys = rng.permutation(bound)[:voxels][rng.integers(0, voxels, n)].astype(np.int32)
+    unq, inv, cnt = np.unique(keys, return_inverse=True, return_counts=True)
+    lib.txs_unique_bitmap_workspace_len.restype = lib.txs_plan_workspace_len.restype = i64
+
+    def i32(m):
+        return torch.empty((m,), dtype=torch.int32, device="cuda")
+    k, bws, ws = torch.from_numpy(keys).cuda(), i32(lib.txs_unique_bitmap_workspace_len(i64(bound))), \
+        i32(lib.txs_plan_workspace_len(i64(n), i64(n)))
+    o_inv, o_unq, perm, seg, pre, slot, heavy, stats = (i32(m) for m in (n, n, n, n, n + 1, n, n, 18))
+    o_cnt = torch.empty((n,), dtype=torch.int64, device="cuda")
+    rc = lib.txs_unique_plan(vp(k.data_ptr()), ctypes.c_int(0), i64(n), i64(bound), vp(0), vp(bws.data_ptr()),
+                             ctypes.c_int32(64), vp(ws.data_ptr()), vp(o_inv.data_ptr()), vp(o_unq.data_ptr()),
+                             vp(o_cnt.data_ptr()), vp(perm.data_ptr()), vp(seg.data_ptr()), vp(pre.data_ptr()),
+                             vp(slot.data_ptr()), vp(heavy.data_ptr()), vp(stats.data_ptr()),
+                             vp(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    st = stats.cpu().numpy()
+    assert st[16] == unq.size and st[17] == 0 and st[8] == 0      # voxels, no key outside, no general sequence
+    assert st[2] == cnt.max() and st[7] == (cnt > 64).sum()
+    assert np.array_equal(o_inv.cpu().numpy(), inv) and np.array_equal(o_cnt.cpu().numpy()[:unq.size], cnt)
+    assert np.array_equal(perm.cpu().numpy(), np.argsort(inv, kind="stable"))
+
+
+def test_what_is_kept_per_voxel_is_bounded():
+    """Up to 2^20 rows the arrays with an entry per voxel may lie in one of an entry per row (20 bytes);
+    beyond that they have their own length."""
+    for n, most in ((1 << 20, 20 << 20), (2_000_000, 64 * 24)):
+        keys = torch.randint(0, 64, (n,), generator=torch.Generator().manual_seed(n))
+        d = T.ScatterData.from_keys((keys * 200_000).cuda(), 1 << 24)
+        kept = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes()
+                for t in (d.unq_cnts, d.preSum, d.slot_of, d.heavy_ids)}
+        assert d.num_unq == 64 and sum(kept.values()) <= most + 64

@@ -428,12 +428,21 @@ constexpr int kBktThreads = 512;
 constexpr int kBktItems = 8;
 constexpr int kBktWaves = kBktThreads / 64;
 constexpr int kBktSlice = kBktThreads * kBktItems;     // rows one workgroup places
-constexpr int kBktMaxSlices = 64;                      // workgroups per bucket at most
-constexpr long kBktGiant = (long)kBktMaxSlices * kBktSlice;  // rows in one bucket beyond which the general sequence runs
+constexpr long kBktGiant = 64L * kBktSlice;            // rows in one bucket beyond which the general sequence runs
 constexpr int kLongRun = 64;                           // rows of one voxel in a slice beyond which they are ranked by ballots
 constexpr int kMaxLongRuns = kBktSlice / (kLongRun + 1);
 static_assert(kMaxLongRuns < 64 && kBktSlice / 64 == 64, "six bits number a slice's long runs, a wave scans their chunk counts");
 constexpr int kFlagUnsorted = 1, kFlagOutOfRange = 2;
+
+// Bits of ids below U, and of them the low digit where the bucket digit may take high_bits.
+__host__ __device__ __forceinline__ int radix_bits(int U) { return U > 2 ? 32 - __builtin_clz((unsigned)(U - 1)) : 1; }
+__device__ __forceinline__ int low_bits_of(int U, int high_bits) { return max(0, radix_bits(U) - high_bits); }
+// The voxel count a kernel works with: num_unq_dev (may be NULL) holds it where the host knows an
+// upper bound only.  The digits are split by this count, not by the bound: ids of 2000 voxels among
+// a million rows would all lie in the first bucket of the bound's split.
+__device__ __forceinline__ int voxel_count(int U_arg, const int *__restrict__ num_unq_dev) {
+    return num_unq_dev ? min(U_arg, *num_unq_dev) : U_arg;
+}
 
 // exclusive scan of one int per thread across a workgroup of WAVES wavefronts
 template <int WAVES>
@@ -475,10 +484,11 @@ __device__ __forceinline__ unsigned long long wave_match(int digit, int bits, bo
 // 5 us of 1M)
 template <int ITEMS, typename K>
 __global__ __launch_bounds__(kHistThreads) void bucket_hist_kernel(
-    const K *__restrict__ inv, long n, int U, int low_bits, int high_bins, int *__restrict__ hist,
-    int *__restrict__ tile_flags, int n_tiles, int *__restrict__ ids32) {
+    const K *__restrict__ inv, long n, int U_arg, int high_bits, int *__restrict__ hist,
+    int *__restrict__ tile_flags, int n_tiles, int *__restrict__ ids32, const int *__restrict__ num_unq_dev) {
     __shared__ int h[1 << kBucketLowBitsMax];
     __shared__ int s_flags;
+    const int U = voxel_count(U_arg, num_unq_dev), low_bits = low_bits_of(U, high_bits), high_bins = 1 << high_bits;
     for (int d = threadIdx.x; d < high_bins; d += kHistThreads) h[d] = 0;
     if (threadIdx.x == 0) s_flags = 0;
     __syncthreads();
@@ -525,20 +535,23 @@ __device__ __forceinline__ int kread(const int *keys, long i, bool packed) {
 // Stable scatter by the high digit.  hist: the exclusive scan of the digit-major tile histograms.
 //   bucket_start [high_bins + 1] (from the scan): first position of every bucket.
 //   stats: zero-filled here (workgroup 0), then UNSORTED / OUT_OF_RANGE of the whole input
-//   and NEED_GENERAL (a bucket above `giant` rows: the bucket kernels step aside).
+//   and NEED_GENERAL (a bucket above kBktGiant rows: the bucket kernels step aside; not where so few
+//   voxels have so many rows that the low digit has next to nothing left).
 // Rows already in order are not moved: out_keys (if given) receives a copy of the ids, and
 // the next kernel reads unq_inv itself.  out_pairs: (id, row) per position, one 8-byte
 // store; or out_keys / out_rows as two arrays when the order is already final.
 template <int ITEMS>
 __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
-    const int *__restrict__ inv, long n, int U, int low_bits, int high_bits,
-    const int *__restrict__ hist, const int *__restrict__ tile_flags, int n_tiles, long giant,
+    const int *__restrict__ inv, long n, int U_arg, int high_bits,
+    const int *__restrict__ hist, const int *__restrict__ tile_flags, int n_tiles,
     const int *__restrict__ bucket_start, int *__restrict__ stats, int *__restrict__ out_keys,
-    int *__restrict__ out_rows, int2 *__restrict__ out_pairs) {
+    int *__restrict__ out_rows, int2 *__restrict__ out_pairs, const int *__restrict__ num_unq_dev) {
     // [bins] base_s: first destination of this tile's rows, per digit; then the larger of
     // [kHistWaves][bins] wave counts and the tile's staged (id, row) pairs
     extern __shared__ __align__(8) int lds_base[];
     __shared__ int s_flags;
+    const int U = voxel_count(U_arg, num_unq_dev), low_bits = low_bits_of(U, high_bits);
+    const bool may_overfill = U > 1 << kBucketLowBitsMax;
     const int bins = 1 << high_bits;
     int *base_s = lds_base, *lds_scatter = lds_base + bins, *wcount = lds_scatter;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -557,7 +570,7 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
     // histogram, two lines of it per bucket, they cost every workgroup more (1M ids 13.7 -> 15.4 us).
     for (int d = threadIdx.x; d < bins; d += kHistThreads) {
         base_s[d] = hist[(long)d * n_tiles + blockIdx.x];
-        if ((long)bucket_start[d + 1] - bucket_start[d] > giant) atomicOr(&s_flags, 4);
+        if (may_overfill && (long)bucket_start[d + 1] - bucket_start[d] > kBktGiant) atomicOr(&s_flags, 4);
     }
     __syncthreads();
     const int flags = s_flags;
@@ -656,15 +669,14 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
     }
 }
 
-// Rows of bucket b that slice j of it covers.  A bucket is cut into slices of kBktSlice rows,
-// at most kBktMaxSlices of them (the call goes to the general sequence where that is not enough).
+// Rows of bucket b that slice j of it covers.  A bucket is cut into slices of kBktSlice rows.
 struct BucketSlice {
     long s, e;        // the bucket's rows [s, e) in bucket order
     long my_s, my_e;  // the slice's rows
     int nsl;          // slices of the bucket
 };
 __device__ __forceinline__ int slices_of(long cnt_b) {
-    return (int)min((long)kBktMaxSlices, max(1L, (cnt_b + kBktSlice - 1) / kBktSlice));
+    return (int)max(1L, (cnt_b + kBktSlice - 1) / kBktSlice);
 }
 __device__ __forceinline__ BucketSlice bucket_slice(long s, long e, int j) {
     BucketSlice r;
@@ -681,14 +693,13 @@ __device__ __forceinline__ BucketSlice bucket_slice(long s, long e, int j) {
 // follows, which so learns its work from one load.  Where a bucket has several slices, each
 // workgroup counts the rows of ITS slice per voxel (low digit) and writes the counts to
 // part_hist[g][*]: the slices of a bucket sit in consecutive workgroups, so the next kernel gets a
-// voxel's count in the whole bucket, and in the slices in front of its own, from at most
-// kBktMaxSlices short reads instead of every workgroup of a crowded bucket counting all of its rows.
+// voxel's count in the whole bucket, and in the slices in front of its own, from one short
+// read per slice instead of every workgroup of a crowded bucket counting all of its rows.
 __global__ __launch_bounds__(kBktThreads) void bucket_count_kernel(
-    const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U_arg, int low_bits, int high_bins,
+    const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U_arg, int high_bits,
     const int *__restrict__ bucket_start, const int *__restrict__ stats, int4 *__restrict__ wg_pick,
     int *__restrict__ part_hist, const int *__restrict__ num_unq_dev) {
-    // the voxel count may only be known on the device (unique path): U_arg is then an upper bound
-    const int U = num_unq_dev ? min(U_arg, *num_unq_dev) : U_arg;
+    const int U = voxel_count(U_arg, num_unq_dev), low_bits = low_bits_of(U, high_bits), high_bins = 1 << high_bits;
     extern __shared__ int cnt_s[];  // [low_bins]
     __shared__ int s_pick[2];
     const int low_bins = 1 << low_bits;
@@ -753,12 +764,12 @@ __global__ __launch_bounds__(kBktThreads) void bucket_count_kernel(
 // sweeps (1.3M voxels, 64 MB moved): 103 -> 45 us; 1M ids, ranks only: 31 -> 21.5 us.
 __global__ __launch_bounds__(kBktThreads) void bucket_plan_kernel(
     const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U_arg,
-    int low_bits, int heavy_threshold,
+    int high_bits, int heavy_threshold,
     const long long *__restrict__ unq_cnts, int *__restrict__ perm, int *__restrict__ seg,
     int *__restrict__ preSum, int *__restrict__ slot_of, int *__restrict__ heavy_ids,
     int *__restrict__ stats, const int4 *__restrict__ wg_pick, const int *__restrict__ part_hist,
     long long *__restrict__ ranks, const int *__restrict__ num_unq_dev, long long *__restrict__ cnts_out) {
-    const int U = num_unq_dev ? min(U_arg, *num_unq_dev) : U_arg;
+    const int U = voxel_count(U_arg, num_unq_dev), low_bits = low_bits_of(U, high_bits);
     // ranks != NULL: the caller wants the rank of every row inside its voxel and nothing else
     // (ingroup_inds): the placement writes ranks[row] in place of the permutation and the ids
     const bool rank_mode = ranks != nullptr;
@@ -1028,12 +1039,6 @@ int plan_general(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int
                  const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum,
                  int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, const int *num_unq_dev, long long *cnts_out,
                  void *stream);
-
-int radix_bits(int64_t U) {
-    int bits = 1;
-    while ((1LL << bits) < U) ++bits;
-    return bits;
-}
 
 }  // namespace
 
@@ -1312,11 +1317,11 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
     auto scatter_kernel =
         items == 16 ? bucket_scatter_kernel<16> : (items == 8 ? bucket_scatter_kernel<8> : bucket_scatter_kernel<4>);
     if (ids64)
-        hist64<<<dim3(n_tiles), dim3(kHistThreads), 0, st>>>(ids64, n, U, low_bits, high_bins, hist, tile_flags, n_tiles,
-                                                             ids32);
+        hist64<<<dim3(n_tiles), dim3(kHistThreads), 0, st>>>(ids64, n, U, high_bits, hist, tile_flags, n_tiles, ids32,
+                                                             num_unq_dev);
     else
-        hist32<<<dim3(n_tiles), dim3(kHistThreads), 0, st>>>(unq_inv, n, U, low_bits, high_bins, hist, tile_flags,
-                                                             n_tiles, nullptr);
+        hist32<<<dim3(n_tiles), dim3(kHistThreads), 0, st>>>(unq_inv, n, U, high_bits, hist, tile_flags, n_tiles, nullptr,
+                                                             num_unq_dev);
     // one entry more than the histogram: it receives the total, the end of the last bucket.  A
     // bucket's first entry (that of tile 0) is where it starts.
     if (exclusive_scan(hist, used, hist, used + 1, scan_ws, st, bucket_start, n_tiles) != hipSuccess) return TXS_ERR_LAUNCH;
@@ -1325,8 +1330,7 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
     if (low_bits == 0) {
         // a bucket is a voxel: the scatter already gives the final order
         scatter_kernel<<<dim3(n_tiles), dim3(kHistThreads), lds_scatter, st>>>(
-            unq_inv, n, U, low_bits, high_bits, hist, tile_flags, n_tiles, n + 1, bucket_start, stats, seg, perm,
-            nullptr);
+            unq_inv, n, U, high_bits, hist, tile_flags, n_tiles, bucket_start, stats, seg, perm, nullptr, num_unq_dev);
         int rc = txs_plan_presum(seg, n, U, preSum, stream);
         if (slot_of == nullptr) return rc;
         if (rc == TXS_OK)
@@ -1337,15 +1341,14 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
     }
     // a bucket so full that its workgroups would run long after all others have finished
     // (only a few voxels holding most of the rows do that) sends the call to the general sequence
-    const long giant = kBktGiant;
     scatter_kernel<<<dim3(n_tiles), dim3(kHistThreads), lds_scatter, st>>>(
-        unq_inv, n, U, low_bits, high_bits, hist, tile_flags, n_tiles, giant, bucket_start, stats, nullptr,
-        nullptr, reinterpret_cast<int2 *>(pairs1));
+        unq_inv, n, U, high_bits, hist, tile_flags, n_tiles, bucket_start, stats, nullptr, nullptr,
+        reinterpret_cast<int2 *>(pairs1), num_unq_dev);
     const int low_bins = 1 << low_bits;
     bucket_count_kernel<<<dim3((unsigned)groups), dim3(kBktThreads), (size_t)low_bins * sizeof(int), st>>>(
-        unq_inv, pairs1, n, U, low_bits, high_bins, bucket_start, stats, reinterpret_cast<int4 *>(wg_pick), part_hist, num_unq_dev);
+        unq_inv, pairs1, n, U, high_bits, bucket_start, stats, reinterpret_cast<int4 *>(wg_pick), part_hist, num_unq_dev);
     bucket_plan_kernel<<<dim3((unsigned)groups), dim3(kBktThreads), 0, st>>>(
-        unq_inv, pairs1, n, U, low_bits, heavy_threshold,
+        unq_inv, pairs1, n, U, high_bits, heavy_threshold,
         (const long long *)unq_cnts, perm, seg, preSum, slot_of, heavy_ids, stats,
         reinterpret_cast<const int4 *>(wg_pick), part_hist, ranks, num_unq_dev, cnts_out);
     return status_of(hipGetLastError());

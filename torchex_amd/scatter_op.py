@@ -124,9 +124,11 @@ class ScatterData:
         """ScatterData straight from voxel keys (any non-negative int ids below
         ``key_bound``, e.g. linear voxel ids): computes what ``torch.unique(keys,
         return_inverse=True, return_counts=True)`` returns -- kept as ``unq_keys``,
-        ``unq_inv``, ``unq_cnts`` -- and the scatter plan, with one host read and ONE sort (of
-        the dense ids an occupancy map gives the keys, or of the keys where their bound is too
-        large for a map), where ``torch.unique`` followed by ``ScatterData(...)`` sorts twice."""
+        ``unq_inv``, ``unq_cnts`` -- and the scatter plan, with ONE sort (of the dense ids an
+        occupancy map gives the keys, or of the keys where their bound is too large for a map),
+        where ``torch.unique`` followed by ``ScatterData(...)`` sorts twice.  The host reads
+        back once, or twice where both the rows and the bound exceed 2^20 or a few neighbouring voxels own
+        most of the rows."""
         _check_tie_rule(max_tie_rule)
         self = cls.__new__(cls)
         if heavy_threshold is None:
