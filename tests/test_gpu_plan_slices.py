@@ -1,6 +1,6 @@
 """Index preparation of ids that fill the bucket kernels' slices in every way: one slice or
-several, voxels with a short, a threshold-sized and a long run of rows in a slice (up to a
-slice that is one voxel), few and many voxels per bucket, grouped rows, empty voxels.  The plan
+several, voxels with a short run of rows in a slice, one at the ballots' limit (24), at the heavy
+threshold (64) and a long one (up to a slice that is one voxel), few and many voxels per bucket, grouped rows, empty voxels.  The plan
 is whole numbers with one right answer: a stable sort by voxel."""
 import ctypes
 
@@ -20,10 +20,13 @@ def _ids(kind, U, rng):
     elif kind == "edges":         # 63, 64, 65 rows, and runs of a slice's length and one off it
         c = rng.choice([0, 1, 2, 63, 64, 65, 66], U, p=[.3, .3, .3, .025, .025, .025, .025])
         c[rng.choice(U, 6, replace=False)] = [2047, 2048, 2049, 4095, 4096, 4097]
-    elif kind == "long":          # as many long runs in a slice as fit
+    elif kind == "long":          # long runs side by side, then as many of them in a slice as fit
         c = np.zeros(U, np.int64)
         c[U // 3:U // 3 + 200] = 65
+        c[U // 3 + 200:U // 3 + 600] = 25
         c[-1] = 1
+    elif kind == "limit":         # runs on either side of the ballots' limit
+        c = rng.choice([0, 1, 23, 24, 25, 26], U)
     else:                         # a bucket of many slices, most of it in one voxel
         c = rng.integers(0, 3, U)
         c[U // 2] = 40_000
@@ -32,7 +35,7 @@ def _ids(kind, U, rng):
 
 
 @pytest.mark.parametrize("grouped", [False, True])
-@pytest.mark.parametrize("kind", ["even", "edges", "long", "crowded"])
+@pytest.mark.parametrize("kind", ["even", "edges", "limit", "long", "crowded"])
 @pytest.mark.parametrize("U", [300, 2049, 5000, 70_000, 600_000])
 def test_plan_of_slices(U, kind, grouped):
     rng = np.random.default_rng(U)

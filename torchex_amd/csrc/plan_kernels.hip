@@ -429,9 +429,13 @@ constexpr int kBktItems = 8;
 constexpr int kBktWaves = kBktThreads / 64;
 constexpr int kBktSlice = kBktThreads * kBktItems;     // rows one workgroup places
 constexpr long kBktGiant = 64L * kBktSlice;            // rows in one bucket beyond which the general sequence runs
-constexpr int kLongRun = 64;                           // rows of one voxel in a slice beyond which they are ranked by ballots
+// Rows of one voxel in a slice beyond which they are ranked by ballots.  bucket_plan_kernel, us, with
+// 64 (and one read at a time) / 63 / 31 / 24 / 21: 1M ids of pillars 37.2 / 29.5 / 22.9 / 22.8 / 22.1, 1M
+// ids of 50 rows per voxel 46.3 / 39.6 / 31.0 / 29.7 / 29.4, of 25 rows 33.7 / 30.3 / 28.4 / 27.7 / 27.8, of 10
+// rows 20.9 / 17.6 / 18.8 / 20.9 / 21.4, of a sweep 21.5 / 19.5 / 20.8 / 21.8 / 21.9.
+constexpr int kLongRun = 24;
 constexpr int kMaxLongRuns = kBktSlice / (kLongRun + 1);
-static_assert(kMaxLongRuns < 64 && kBktSlice / 64 == 64, "six bits number a slice's long runs, a wave scans their chunk counts");
+static_assert(kMaxLongRuns < 256 && kBktSlice / 64 == 64, "eight bits number a slice's long runs, a wave scans their chunk counts");
 constexpr int kFlagUnsorted = 1, kFlagOutOfRange = 2;
 
 // Bits of ids below U, and of them the low digit where the bucket digit may take high_bits.
@@ -754,14 +758,15 @@ __global__ __launch_bounds__(kBktThreads) void bucket_count_kernel(
 // One slice: its rows are counted per voxel by LDS atomics, whose returned values put them, voxel
 // by voxel, into LDS in whatever order the atomics ran; each row then finds its place among its
 // voxel's rows of the slice by counting the smaller row numbers there (rows ascend along a bucket,
-// so that is the stable order).  That costs as many reads as the voxel has rows in the slice: runs
-// above kLongRun rows (at most kMaxLongRuns of them in a slice) are ranked by wave ballots on a
-// six-bit number instead, with a count per run and 64 rows in input order.  Rows leave in voxel
-// order, neighbouring lanes to neighbouring addresses.
-// What bounds it is the chain of dependent steps inside a workgroup, far more than bytes: 50 KB of
+// so that is the stable order).  That costs as many reads, four in flight, as the voxel has rows in
+// the slice: runs above kLongRun rows (at most kMaxLongRuns of them in a slice) are ranked by wave
+// ballots on their number instead, with a count per run and 64 rows in input order.  Rows leave in
+// voxel order, neighbouring lanes to neighbouring addresses.
+// What bounds it is the chain of dependent steps inside a workgroup, far more than bytes: 45 KB of
 // LDS keep 24 waves on a compute unit (the ballots on all 11 bits that this replaces needed a count
-// per wave and voxel as well, left 12, and wrote every row as a request of its own).  4M ids of four
-// sweeps (1.3M voxels, 64 MB moved): 103 -> 45 us; 1M ids, ranks only: 31 -> 21.5 us.
+// per wave and voxel as well, left 12, and wrote every row as a request of its own).  Then -> now, us:
+// 4M ids of four sweeps (1.3M voxels, 64 MB moved) 131 -> 47, 1M of one 26.2 -> 21.8, of pillars 21.9 ->
+// 22.8, 1M ids of 50 / 25 / 10 rows per voxel 27.5 -> 29.7, 23.7 -> 27.7, 28.2 -> 20.9.
 __global__ __launch_bounds__(kBktThreads) void bucket_plan_kernel(
     const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U_arg,
     int high_bits, int heavy_threshold,
@@ -774,15 +779,17 @@ __global__ __launch_bounds__(kBktThreads) void bucket_plan_kernel(
     // (ingroup_inds): the placement writes ranks[row] in place of the permutation and the ids
     const bool rank_mode = ranks != nullptr;
     constexpr int kBins = 1 << kBucketLowBitsMax;
-    __shared__ int row_s[kBktSlice];              // the slice's rows in voxel order; before that, its bucket's counts
-    __shared__ unsigned short dig_s[kBktSlice];   // their voxels (low digits)
+    // one after the other: the bucket's counts; a long run's rows per 64 rows of the slice; the slice's
+    // rows in voxel order and their voxels (low digits)
+    __shared__ int pool_s[kBktSlice + kBktSlice / 2];
     __shared__ int first_s[kBins + 1];            // the slice's counts, then the first place of every voxel in row_s
     __shared__ int step_s[kBins];                 // rows of the voxel in front of this slice, then place -> destination
-    __shared__ unsigned char mark_s[kBins];       // bits 0-5: number of a long run + 1 (0: short); bit 7: heavy voxel
-    __shared__ unsigned short chunk_s[kMaxLongRuns][64];  // a long run's rows per 64 rows of the slice
+    __shared__ unsigned short mark_s[kBins];      // bits 0-7: number of a long run + 1 (0: short); bit 15: heavy voxel
     __shared__ int s_red[kBktWaves], s_bad[kBktWaves], s_long;
-    static_assert(kBins <= kBktSlice, "the bucket's counts share the rows' space");
-    int *tot = row_s;
+    static_assert(kBins <= kBktSlice && kMaxLongRuns * 64 * sizeof(short) <= sizeof(pool_s), "what shares a space fits");
+    int *tot = pool_s, *row_s = pool_s;
+    unsigned short *dig_s = reinterpret_cast<unsigned short *>(pool_s + kBktSlice);
+    auto chunk_s = reinterpret_cast<unsigned short(*)[64]>(pool_s);
     const int low_bins = 1 << low_bits;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const unsigned long long lanes_below = (1ull << lane) - 1ull;
@@ -878,9 +885,9 @@ __global__ __launch_bounds__(kBktThreads) void bucket_plan_kernel(
         const int c = first_s[d];
         const int c_all = sl.nsl > 1 ? tot[d] : c;
         if (sl.nsl == 1) tot[d] = c;
-        int mark = c_all > heavy_threshold ? 128 : 0;
+        int mark = c_all > heavy_threshold ? 0x8000 : 0;
         if (c > kLongRun) mark |= 1 + atomicAdd(&s_long, 1);
-        mark_s[d] = (unsigned char)mark;
+        mark_s[d] = (unsigned short)mark;
         first_s[d] = run;
         // ranks count from the voxel's first row, positions from the bucket's start
         step_s[d] += (rank_mode ? 0 : (int)s + run_all) - run;
@@ -964,12 +971,13 @@ __global__ __launch_bounds__(kBktThreads) void bucket_plan_kernel(
     // ---- long runs: straight from the registers, ranked by 64 rows in input order at a time
     const int n_long = s_long;  // (uniform)
     if (n_long > 0) {
+        const int id_bits = 32 - __builtin_clz((unsigned)n_long);
         for (int k = threadIdx.x; k < n_long * 64; k += kBktThreads) (&chunk_s[0][0])[k] = 0;
         __syncthreads();
 #pragma unroll
         for (int it = 0; it < kBktItems; ++it) {
-            const int id = dig[it] >= 0 ? (mark_s[dig[it]] & 63) : 0;
-            const unsigned long long mask = wave_match(id, 6, id > 0);
+            const int id = dig[it] >= 0 ? (mark_s[dig[it]] & 255) : 0;
+            const unsigned long long mask = wave_match(id, id_bits, id > 0);
             const int below = __popcll(mask & lanes_below);
             if (id > 0) {
                 turn[it] = below;
@@ -984,18 +992,18 @@ __global__ __launch_bounds__(kBktThreads) void bucket_plan_kernel(
         __syncthreads();
 #pragma unroll
         for (int it = 0; it < kBktItems; ++it) {
-            const int id = dig[it] >= 0 ? (mark_s[dig[it]] & 63) : 0;
-            if (id > 0) put(dig[it], first_s[dig[it]] + chunk_s[id - 1][it * kBktWaves + w] + turn[it], row[it]);
+            const int id = dig[it] >= 0 ? (mark_s[dig[it]] & 255) : 0;
+            if (id == 0) continue;
+            turn[it] += chunk_s[id - 1][it * kBktWaves + w];
+            put(dig[it], first_s[dig[it]] + turn[it], row[it]);
         }
+        __syncthreads();  // (the rows take the chunk counts' space)
     }
     // ---- short runs: into voxel order, then by the number of smaller rows in the run
 #pragma unroll
     for (int it = 0; it < kBktItems; ++it) {
         if (dig[it] < 0) continue;
-        // (a long run's rows are placed already: any of its places will do for its ids)
-        const int id = mark_s[dig[it]] & 63;
-        const int p = first_s[dig[it]] +
-                      (id > 0 ? chunk_s[id - 1][it * kBktWaves + w] + turn[it] : turn[it]);
+        const int p = first_s[dig[it]] + turn[it];
         row_s[p] = row[it];
         dig_s[p] = (unsigned short)dig[it];
     }
@@ -1005,12 +1013,18 @@ __global__ __launch_bounds__(kBktThreads) void bucket_plan_kernel(
         const int mark = mark_s[d];
         if (!rank_mode) {
             const long dst = (long)step_s[d] + p;
-            if (dst >= s && dst < e) seg[dst] = (u_lo + d) | ((mark & 128) ? kSpecialBit : 0);
+            if (dst >= s && dst < e) seg[dst] = (u_lo + d) | ((mark & 0x8000) ? kSpecialBit : 0);
         }
-        if ((mark & 63) != 0 || (!rank_mode && !unsorted)) continue;
+        if ((mark & 255) != 0 || (!rank_mode && !unsorted)) continue;
         const int a = first_s[d], z = first_s[d + 1], row_i = row_s[p];
         int smaller = 0;
-        for (int q = a; q < z; ++q) smaller += row_s[q] < row_i;
+        for (int q = a; q < z; q += 4) {
+            int other[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) other[e] = row_s[min(q + e, kBktSlice - 1)];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) smaller += (q + e < z && other[e] < row_i) ? 1 : 0;
+        }
         put(d, a + smaller, row_i);
     }
 }
