@@ -108,6 +108,13 @@ int txs_kernel_name(int backward, int op, int dtype, int64_t num_total, int64_t 
                     int64_t num_unq, int64_t pointer_alignment, int table_allowed, char *buf,
                     int64_t buf_len);
 
+/* How a voxel-order forward call of these extents, with 64-byte aligned tensors, is cut: `lanes`
+ * neighbouring threads of `elements` channels each cover a row (or one of several blocks of
+ * columns of a row wider than 64 lanes), and a workgroup takes `positions` sorted rows.  Host only;
+ * for tests and logs. */
+int txs_forward_tile(int dtype, int64_t num_total, int64_t channel, int64_t num_unq, int64_t num_heavy,
+                     int32_t *lanes, int32_t *elements, int32_t *positions);
+
 /* Default population above which a voxel is reduced through atomics (64), and the
  * smallest heavy_threshold the plan functions accept (16: a smaller one is refused with
  * TXS_ERR_INVALID_ARG). */

@@ -115,6 +115,45 @@ def test_argument_validation_needs_no_gpu():
     assert lib.txs_dpp_workspace_len(i64(200_000), i64(200)) * 4 >= 25 * 200_000 * 2
 
 
+def _tile(dtype, n, c, u, heavy):
+    lanes, elements, positions = (ctypes.c_int32() for _ in range(3))
+    i64 = ctypes.c_int64
+    assert _lib().txs_forward_tile(ctypes.c_int(dtype), i64(n), i64(c), i64(u), i64(heavy), ctypes.byref(lanes),
+                                   ctypes.byref(elements), ctypes.byref(positions)) == 0
+    return lanes.value, elements.value, positions.value
+
+
+def test_forward_tiles_cover_rows_and_fit():
+    for dtype, full in ((0, 4), (1, 4), (2, 4)):
+        for n in (1, 1000, 60_000, 300_000, 1_000_000, 5_000_000):
+            for u in (max(1, n // 100), max(1, n // 10), max(1, n // 3)):
+                for c in list(range(1, 70)) + [127, 128, 131, 255, 256, 257, 300]:
+                    for heavy in (0, 1):
+                        lanes, elements, positions = _tile(dtype, n, c, u, heavy)
+                        blocks = -(-(-(-c // elements)) // lanes)
+                        assert elements <= full and elements <= c and 1 <= lanes <= 64
+                        assert blocks * lanes * elements >= c and (blocks == 1 or c > 64 * elements)
+                        assert positions % 64 == 0 and 64 <= positions <= 8192
+
+
+def test_heavy_voxels_give_narrow_rows_more_lanes_whatever_the_size():
+    """A heavy voxel costs a walk over the lane groups of every tile it reaches into: few channels must
+    neither shrink to one lane per row nor get larger tiles, with one heavy voxel or with thousands."""
+    for dtype in (0, 1, 2):
+        for n in (20_000, 60_000, 300_000, 1_000_000, 5_000_000):
+            for heavy in (1, 100, n // 100):
+                for c in range(1, 21):
+                    lanes, elements, positions = _tile(dtype, n, c, n // 5, heavy)
+                    assert elements == 1 and lanes == c
+                    assert positions <= 16 * (256 // c) + 32 and (positions <= 1088 or n >= 15 * positions)
+                for c in (21, 24, 35, 40):
+                    lanes, elements, positions = _tile(dtype, n, c, n // 5, heavy)
+                    assert elements == 2 and lanes == -(-c // 2) and positions <= 16 * (256 // lanes) + 32
+                # whole sectors, and rows of enough lanes, stay with full vectors
+                for c in (32, 41, 64, 128):
+                    assert _tile(dtype, n, c, n // 5, heavy) == _tile(dtype, n, c, n // 5, 0)
+
+
 def test_package_surface_matches_reference_exports():
     import torchex
     import torchex_amd

@@ -767,6 +767,24 @@ int fwd_chunk_for(long N, long U, int op, int elem) {
     return (elem == 4 && N < 8 * U) ? kChunkShort : kChunk;
 }
 
+// Narrow rows of an input with heavy voxels.  In every tile it reaches into, a heavy voxel costs a
+// walk over the parts its rows left in the tile's lane groups, one after the other, and an atomic
+// per element.  In full vectors a row of 4 floats is one lane: the walk is 256 parts long, and an
+// atomic instruction reaches one element of the row.  So these rows get more lanes: one element
+// each up to kByElementRow elements, two up to kByPairRow (not in rows of whole sectors, which
+// give up the non-temporal hint for it: 2M rows of 32 floats, 100 voxels of 100 rows, mean 61 -> 70
+// us), in tiles of kChunk positions per lane group, less below 16 tiles.
+// Times of one forward, us: full vectors with every lane group a power of two of lanes and tiles of 8
+// or 16 positions per lane group / any number of lanes and tiles of up to 4096 positions for the
+// narrowest rows / this rule:
+//   300k rows, one voxel of 200, the others of 4: mean of 4 / 10 / 16 floats 17 15 15 / 20 17 16 / 13 15 13
+//   300k rows, 100 voxels of 500: max of 3 / 4 / 10 / 16 floats 22 49 20 31 / 24 31 32 24 / 18 18 17 15,
+//     of 20 / 35 floats 25 26 / 32 29 / @20 @35
+//   316k rows of pillars, 949 heavy voxels: mean of 3 / 4 floats 20 29 / 18 27 / 15 15, max of 10 20 / 28 / 16
+//   1.6M rows of pillars, 3452 heavy voxels: mean of 3 / 4 floats 49 82 / 50 62 / 45 41, max of 10 61 / 62 / 45
+//   1M rows, one voxel of 200, the others of 4: mean of 3 / 4 / 16 floats 24 23 27 / 25 32 31 / 25 24 28
+constexpr long kByElementRow = 20, kByPairRow = 40;
+
 bool aligned_to(const void *p, int bytes) { return ((uintptr_t)p % (uintptr_t)bytes) == 0; }
 
 struct Geometry {
@@ -784,11 +802,17 @@ Geometry make_geometry(long N, long C, int elem, const void *p0, const void *p1,
                        bool heavy = false) {
     Geometry g;
     g.hint = (C * elem) % 64 == 0 && aligned_to(p0, 64) && aligned_to(p1, 64);
+    const int most_vec = !(forward && heavy) ? 64 : (C <= kByElementRow ? 1 : (C <= kByPairRow && !g.hint ? 2 : 64));
     // bytes per lane and row: 16 for fp32; 8 for the 2-byte types, whose kernels carry
     // twice the registers per byte (measured 4-12 % faster than 16 on fp16 / bf16); less only
     // for rows shorter than that
     int vb = elem == 2 ? kHalfVecBytes : 16;
     while (vb / elem > C) vb >>= 1;
+    const bool narrow = most_vec * elem <= vb;
+    if (narrow) {
+        vb = most_vec * elem;
+        g.hint = false;  // (only full vectors carry it)
+    }
     g.vec_bytes = vb;
     const long vec = vb / elem;
     const long lanes = (C + vec - 1) / vec;         // of a row
@@ -799,19 +823,8 @@ Geometry make_geometry(long N, long C, int elem, const void *p0, const void *p1,
     g.lm.per_groups = reciprocal32(g.lm.groups);
     // (forward) a small input gets smaller tiles while that gives the chip more workgroups
     // (below eight per compute unit a tile's fixed costs show: 3-5 % on 200k rows of 256 bytes)
-    while (forward && chunk > 4 && N / ((long)g.lm.groups * chunk) < 2048) chunk /= 2;
-    // Narrow rows (at most four lanes) with heavy voxels: every tile that a heavy voxel reaches into
-    // costs an atomic per element, and neighbouring heavy rows share their cache lines, on which
-    // atomics run one after the other.  The largest tile that still gives every compute unit one:
-    // mean of three fp32 channels over pillars, 316k rows in tiles of 256 / 512 / 1024 / 4096 31.4 /
-    // 26.6 / 19.7 / 27.2 us, 1.6M rows in tiles of 512 / 1024 / 4096 52.6 / 52.1 / 48.8.
-    // With one lane per row an atomic instruction reaches one element of a row only, and fewer,
-    // larger tiles still pay: four fp32 channels, 316k rows in tiles of 1024 / 4096 30.7 / 28.2 us.
-    if (forward && heavy && g.lm.lanes <= 4) {
-        const long least = g.lm.lanes == 1 ? 64 : 256;  // workgroups
-        chunk = 4;
-        while (g.lm.groups * chunk * 2 <= 4096 && N / ((long)g.lm.groups * chunk * 2) >= least) chunk *= 2;
-    }
+    if (narrow) chunk = kChunk;
+    while (forward && chunk > 4 && N / ((long)g.lm.groups * chunk) < (narrow ? 16 : 2048)) chunk /= 2;
     long tile = (long)g.lm.groups * chunk;
     // the forward kernel finds the borders of a tile's range with one wave ballot each: a tile
     // is a whole number of wavefronts' worth of staged ids (its rows are dealt evenly anyway)
@@ -1093,6 +1106,21 @@ int txs_kernel_name(int backward, int op, int dtype, int64_t num_total, int64_t 
                                            fwd_chunk_for(num_total, num_unq, op, elem), true);
         snprintf(buf, (size_t)buf_len, "scatter_fwd_kernel<%s,%d,%s>", kTypes[dtype], geo.vec_bytes / elem, kOps[op]);
     }
+    return TXS_OK;
+}
+
+int txs_forward_tile(int dtype, int64_t num_total, int64_t channel, int64_t num_unq, int64_t num_heavy,
+                     int32_t *lanes, int32_t *elements, int32_t *positions) {
+    if (dtype < TXS_F32 || dtype > TXS_BF16) return TXS_ERR_UNSUPPORTED;
+    if (!fits_i32(num_total) || !fits_i32(channel) || !fits_i32(num_unq) || channel < 1 || num_heavy < 0 ||
+        num_heavy > num_unq || !lanes || !elements || !positions)
+        return TXS_ERR_INVALID_ARG;
+    const int elem = dtype == TXS_F32 ? 4 : 2;
+    const Geometry geo = make_geometry(num_total, channel, elem, nullptr, nullptr,
+                                       fwd_chunk_for(num_total, num_unq, TXS_SUM, elem), true, num_heavy > 0);
+    *lanes = geo.lm.lanes;
+    *elements = geo.vec_bytes / elem;
+    *positions = geo.tile;
     return TXS_OK;
 }
 
