@@ -145,13 +145,28 @@ def test_heavy_voxels_give_narrow_rows_more_lanes_whatever_the_size():
                 for c in range(1, 21):
                     lanes, elements, positions = _tile(dtype, n, c, n // 5, heavy)
                     assert elements == 1 and lanes == c
-                    assert positions <= 16 * (256 // c) + 32 and (positions <= 1088 or n >= 15 * positions)
+                    assert positions < 16 * (256 // c) + 64 and (positions <= 1088 or n >= 15 * positions)
                 for c in (21, 24, 35, 40):
                     lanes, elements, positions = _tile(dtype, n, c, n // 5, heavy)
-                    assert elements == 2 and lanes == -(-c // 2) and positions <= 16 * (256 // lanes) + 32
-                # whole sectors, and rows of enough lanes, stay with full vectors
+                    assert elements == 2 and lanes == -(-c // 2) and positions < 16 * (256 // lanes) + 64
+                # whole sectors, and rows of enough lanes, stay with full vectors where the rows fill the chip
                 for c in (32, 41, 64, 128):
-                    assert _tile(dtype, n, c, n // 5, heavy) == _tile(dtype, n, c, n // 5, 0)
+                    assert n < 1_000_000 or _tile(dtype, n, c, n // 5, heavy)[1] == 4
+
+
+def test_few_rows_get_more_lanes_before_smaller_shares():
+    for dtype in (0, 1, 2):
+        # voxels of many rows: a run should lie in few lane groups
+        for n, c in ((60_000, 5), (60_000, 10), (60_000, 13), (300_000, 13), (60_000, 48)):
+            lanes, elements, positions = _tile(dtype, n, c, n // 25, 0)
+            assert elements < 4 and n // positions >= 100 and positions * lanes >= 256 * 4
+        # tiles are rounded up: 21 lane groups of 4 positions are not squeezed into 64
+        assert _tile(dtype, 300_000, 48, 12_000, 0)[2] >= 128
+        # short runs: only the smallest inputs
+        assert _tile(dtype, 20_000, 5, 7000, 0)[1] == 1 and _tile(dtype, 300_000, 5, 100_000, 0)[1] == 4
+        for n in (2_000_000, 4_000_000):
+            for c in (13, 48, 67, 128):
+                assert _tile(dtype, n, c, n // 10, 0)[1] == 4 and _tile(dtype, n, c, n // 3, 0)[1] == 4
 
 
 def test_package_surface_matches_reference_exports():

@@ -31,6 +31,7 @@
 
 #include <stdio.h>
 
+#include <algorithm>
 #include <initializer_list>
 #include <mutex>
 
@@ -758,14 +759,32 @@ __global__ __launch_bounds__(kThreads) void scatter_bwd_kernel(
 // per lane group (fewer tile borders for a run to cross, one atomic row per tile and heavy
 // voxel); short runs of 4-byte elements in tiles of 8 (twice the workgroups, shorter dependent
 // walks: 4 % on the LiDAR sweep, 8 % on 200k rows); everything else in tiles of 16.
-int fwd_chunk_for(long N, long U, int op, int elem) {
-#ifdef TXS_FORCE_FWD_CHUNK
-    return TXS_FORCE_FWD_CHUNK;
-#endif
-    (void)op;
+int fwd_chunk_for(long N, long U, int elem) {
     if (N >= 64 * U) return kChunkLong;
     return (elem == 4 && N < 8 * U) ? kChunkShort : kChunk;
 }
+
+// Sorted positions per lane group of the backward kernel.  Long shares for long runs, unless they leave
+// fewer than 2048 workgroups: mean of 5 / 10 / 13 floats over 60k rows in voxels of 25, shares of 16 / 8:
+// 12.1 10.9 10.3 / 6.6 6.4 6.2 us.
+int bwd_chunk_for(long N, long U, int groups) {
+    return N < (long)kChunkBwdLong * U || N / ((long)groups * kChunkBwdLong) < 2048 ? kChunkBwdShort : kChunkBwdLong;
+}
+
+// Forward, everything but the narrow rows with heavy voxels below: more lanes per row while full
+// vectors leave too few workgroups, then smaller tiles.
+// Voxels of kManyRows rows and more, or heavy ones among them: a run that covers several shares of a tile costs a walk over
+// them, so a lane group should keep many rows: lanes are added, up to 32 per row, while tiles of
+// kChunk positions per lane group are fewer than 1024, and only then tiles shrink, to 8 positions per
+// lane group below 1536 tiles and to 4 below 1024, rounded up to whole wavefronts.  Short runs: lanes
+// up to 16 while tiles of 4 positions are fewer than 256, then tiles shrink below 2048 (below eight
+// workgroups per compute unit a tile's fixed costs show: 3-5 % on 200k rows of 256 bytes).
+// Forward, us, lanes a power of two and vectors that divide the row / full vectors on any number of
+// lanes in tiles rounded to the nearest wavefront / this rule:
+//   300k rows in voxels of 25, max of 48 / 96 2-byte elements 20 22 / 33 29 / 15 21, of 13 13 / 18 / 10
+//   60k rows in voxels of 25, max of 5 / 10 / 13 floats 7.2 8.1 7.2 / 10.6 10.2 9.9 / 6.6 6.2 5.8
+//   20k rows in voxels of 1-3, mean of 5 / 10 floats 4.9 5.1 / 6.0 5.6 / 5.0 5.0
+constexpr long kManyRows = 8;
 
 // Narrow rows of an input with heavy voxels.  In every tile it reaches into, a heavy voxel costs a
 // walk over the parts its rows left in the tile's lane groups, one after the other, and an atomic
@@ -779,7 +798,7 @@ int fwd_chunk_for(long N, long U, int op, int elem) {
 // narrowest rows / this rule:
 //   300k rows, one voxel of 200, the others of 4: mean of 4 / 10 / 16 floats 17 15 15 / 20 17 16 / 13 15 13
 //   300k rows, 100 voxels of 500: max of 3 / 4 / 10 / 16 floats 22 49 20 31 / 24 31 32 24 / 18 18 17 15,
-//     of 20 / 35 floats 25 26 / 32 29 / @20 @35
+//     of 20 / 35 floats 25 26 / 33 29 / 17 24
 //   316k rows of pillars, 949 heavy voxels: mean of 3 / 4 floats 20 29 / 18 27 / 15 15, max of 10 20 / 28 / 16
 //   1.6M rows of pillars, 3452 heavy voxels: mean of 3 / 4 floats 49 82 / 50 62 / 45 41, max of 10 61 / 62 / 45
 //   1M rows, one voxel of 200, the others of 4: mean of 3 / 4 / 16 floats 24 23 27 / 25 32 31 / 25 24 28
@@ -791,6 +810,8 @@ struct Geometry {
     int vec_bytes;  // bytes one lane moves per row
     bool hint;      // rows of whole 64-byte sectors
     LaneMap lm;
+    int ytiles;     // blocks of columns
+    int chunk;      // (backward) sorted positions per lane group
     int tile;       // sorted positions per workgroup
     unsigned lds_fwd_idx, lds_slots, lds_bwd;  // dynamic LDS: fwd index part (bytes), fwd slot elements, bwd bytes
     dim3 grid;
@@ -798,44 +819,67 @@ struct Geometry {
 
 unsigned reciprocal32(int d) { return d == 1 ? 0u : (unsigned)(((1ULL << 32) + (unsigned)d - 1) / (unsigned)d); }
 
-Geometry make_geometry(long N, long C, int elem, const void *p0, const void *p1, int chunk, bool forward,
-                       bool heavy = false) {
-    Geometry g;
-    g.hint = (C * elem) % 64 == 0 && aligned_to(p0, 64) && aligned_to(p1, 64);
-    const int most_vec = !(forward && heavy) ? 64 : (C <= kByElementRow ? 1 : (C <= kByPairRow && !g.hint ? 2 : 64));
-    // bytes per lane and row: 16 for fp32; 8 for the 2-byte types, whose kernels carry
-    // twice the registers per byte (measured 4-12 % faster than 16 on fp16 / bf16); less only
-    // for rows shorter than that
-    int vb = elem == 2 ? kHalfVecBytes : 16;
-    while (vb / elem > C) vb >>= 1;
-    const bool narrow = most_vec * elem <= vb;
-    if (narrow) {
-        vb = most_vec * elem;
-        g.hint = false;  // (only full vectors carry it)
-    }
-    g.vec_bytes = vb;
-    const long vec = vb / elem;
-    const long lanes = (C + vec - 1) / vec;         // of a row
-    const long ytiles = (lanes + 63) / 64;          // column tiles: a row wider than 64 lanes is dealt to several
-    g.lm.lanes = (int)((lanes + ytiles - 1) / ytiles);
+// Lanes of `vec_bytes` each over a row of C elements.
+void deal_lanes(Geometry &g, long C, int elem, int vec_bytes) {
+    g.vec_bytes = vec_bytes;
+    const long vec = vec_bytes / elem;
+    const long lanes = (C + vec - 1) / vec;       // of a row
+    g.ytiles = (int)((lanes + 63) / 64);          // column tiles: a row wider than 64 lanes is dealt to several
+    g.lm.lanes = (int)((lanes + g.ytiles - 1) / g.ytiles);
     g.lm.groups = kThreads / g.lm.lanes;
     g.lm.per_lanes = reciprocal32(g.lm.lanes);
     g.lm.per_groups = reciprocal32(g.lm.groups);
-    // (forward) a small input gets smaller tiles while that gives the chip more workgroups
-    // (below eight per compute unit a tile's fixed costs show: 3-5 % on 200k rows of 256 bytes)
-    if (narrow) chunk = kChunk;
-    while (forward && chunk > 4 && N / ((long)g.lm.groups * chunk) < (narrow ? 16 : 2048)) chunk /= 2;
-    long tile = (long)g.lm.groups * chunk;
-    // the forward kernel finds the borders of a tile's range with one wave ballot each: a tile
-    // is a whole number of wavefronts' worth of staged ids (its rows are dealt evenly anyway)
-    if (forward) tile = tile <= 64 ? 64 : (tile + 32) / 64 * 64;
+}
+
+Geometry make_geometry(long N, long C, long U, int elem, const void *p0, const void *p1, bool forward, bool heavy) {
+    Geometry g;
+    g.hint = (C * elem) % 64 == 0 && aligned_to(p0, 64) && aligned_to(p1, 64);
+    // bytes per lane and row: 16 for fp32; 8 for the 2-byte types, whose kernels carry
+    // twice the registers per byte (measured 4-12 % faster than 16 on fp16 / bf16); less only
+    // for rows shorter than that and where more lanes pay, below
+    const int full = elem == 2 ? kHalfVecBytes : 16;
+    int vb = full;
+    while (vb / elem > C) vb >>= 1;
+    deal_lanes(g, C, elem, vb);
+    long tile;
+    if (!forward) {
+        g.chunk = bwd_chunk_for(N, U, g.lm.groups);
+        tile = (long)g.lm.groups * g.chunk;
+    } else {
+        // a tile is a whole number of wavefronts' worth of staged ids: the kernel finds the borders of
+        // its range with one wave ballot each (its rows are dealt evenly to the lane groups anyway)
+        auto tile_of = [&](int chunk) { return ((long)g.lm.groups * chunk + 63) / 64 * 64; };
+        int chunk = fwd_chunk_for(N, U, elem);
+        const bool many = N >= kManyRows * U || heavy;
+        if (heavy && (C <= kByElementRow || (C <= kByPairRow && !g.hint))) {
+            deal_lanes(g, C, elem, C <= kByElementRow ? elem : 2 * elem);
+            chunk = kChunk;
+            while (chunk > 4 && N / tile_of(chunk) < 16) chunk /= 2;
+            tile = tile_of(chunk);
+        } else {
+            while (g.vec_bytes > elem && N / tile_of(many ? kChunk : 4) < (many ? 1024 : 256)) {
+                Geometry more = g;
+                deal_lanes(more, C, elem, g.vec_bytes / 2);
+                if (more.ytiles > 1 || more.lm.lanes > (many ? 32 : 16)) break;
+                g = more;
+            }
+            if (many) {
+                while (chunk > 4 && N / tile_of(chunk) < (chunk > 8 ? 1536 : 1024)) chunk /= 2;
+                tile = tile_of(chunk);
+            } else {
+                while (chunk > 4 && N / ((long)g.lm.groups * chunk) < 2048) chunk /= 2;
+                tile = std::max(64L, ((long)g.lm.groups * chunk + 32) / 64 * 64);
+            }
+        }
+        if (g.vec_bytes < full) g.hint = false;  // (only full vectors carry it)
+    }
     g.tile = (int)tile;
     long blocks = (N + tile - 1) / tile;
     blocks = (blocks + 8 * kXcdSpan - 1) / (8 * kXcdSpan) * (8 * kXcdSpan);
     g.lds_fwd_idx = (unsigned)(((2 * (tile + kMargin + 1) + 1 + 3) & ~3L) * sizeof(int));
-    g.lds_slots = (unsigned)(2 * kThreads * vec);  // carry cells: a value and a tag per element
+    g.lds_slots = (unsigned)(2 * kThreads * (g.vec_bytes / elem));  // carry cells: a value and a tag per element
     g.lds_bwd = (unsigned)(2 * tile * sizeof(int));
-    g.grid = dim3((unsigned)blocks, (unsigned)ytiles, 1);
+    g.grid = dim3((unsigned)blocks, (unsigned)g.ytiles, 1);
     return g;
 }
 
@@ -938,23 +982,23 @@ hipError_t launch_bwd_chunk(int op, const Geometry &geo, hipStream_t st, const v
 }
 
 template <class TR, int VEC, bool HINT>
-hipError_t launch_bwd_op(int op, int chunk, const Geometry &geo, hipStream_t st, const void *g, const int *arg,
+hipError_t launch_bwd_op(int op, const Geometry &geo, hipStream_t st, const void *g, const int *arg,
                          const int *perm, const int *seg, const int *preSum, void *gin, int N, int C,
                          int U) {
-    if (chunk == kChunkBwdShort)
+    if (geo.chunk == kChunkBwdShort)
         return launch_bwd_chunk<TR, VEC, kChunkBwdShort, HINT>(op, geo, st, g, arg, perm, seg, preSum, gin, N, C, U);
     return launch_bwd_chunk<TR, VEC, kChunkBwdLong, HINT>(op, geo, st, g, arg, perm, seg, preSum, gin, N, C, U);
 }
 
 template <class TR>
-hipError_t launch_bwd(int op, int chunk, const Geometry &geo, hipStream_t st, const void *g, const int *arg,
+hipError_t launch_bwd(int op, const Geometry &geo, hipStream_t st, const void *g, const int *arg,
                       const int *perm, const int *seg, const int *preSum, void *gin, int N, int C,
                       int U) {
     constexpr int e = (int)sizeof(typename TR::raw);
     constexpr int full = e == 2 ? kHalfVecBytes : 16;
 #define TXS_BWD(VB, HINT)                     \
     if (geo.vec_bytes == VB && geo.hint == HINT) \
-        return launch_bwd_op<TR, (VB) / e, HINT>(op, chunk, geo, st, g, arg, perm, seg, preSum, gin, N, C, U);
+        return launch_bwd_op<TR, (VB) / e, HINT>(op, geo, st, g, arg, perm, seg, preSum, gin, N, C, U);
     TXS_BWD(full, true)
     TXS_BWD(full, false)
     TXS_BWD(full / 2, false)
@@ -1034,7 +1078,7 @@ int scatter_forward_impl(int op, int dtype, const void *feats, const int32_t *un
         if (hipGetLastError() != hipSuccess) return TXS_ERR_LAUNCH;
     }
     if (N > 0) {
-        Geometry geo = make_geometry(N, C, elem, feats, out, fwd_chunk_for(N, U, op, elem), true, num_heavy > 0);
+        const Geometry geo = make_geometry(N, C, U, elem, feats, out, true, num_heavy > 0);
         if (dtype == TXS_F32)
             e = launch_fwd<F32>(op, geo, st, feats, perm, seg, preSum, slot_of, out, arg, scratch, N, C, U, ref_log2);
         else if (dtype == TXS_F16)
@@ -1097,13 +1141,11 @@ int txs_kernel_name(int backward, int op, int dtype, int64_t num_total, int64_t 
         }
     }
     if (backward) {
-        const int chunk = (num_total < (int64_t)kChunkBwdLong * num_unq) ? kChunkBwdShort : kChunkBwdLong;
-        const Geometry geo = make_geometry(num_total, channel, elem, p, p, chunk, false);
+        const Geometry geo = make_geometry(num_total, channel, num_unq, elem, p, p, false, false);
         snprintf(buf, (size_t)buf_len, "scatter_bwd_kernel<%s,%d,%s,%d>", kTypes[dtype], geo.vec_bytes / elem,
-                 kOps[op], chunk);
+                 kOps[op], geo.chunk);
     } else {
-        const Geometry geo = make_geometry(num_total, channel, elem, p, p,
-                                           fwd_chunk_for(num_total, num_unq, op, elem), true);
+        const Geometry geo = make_geometry(num_total, channel, num_unq, elem, p, p, true, false);
         snprintf(buf, (size_t)buf_len, "scatter_fwd_kernel<%s,%d,%s>", kTypes[dtype], geo.vec_bytes / elem, kOps[op]);
     }
     return TXS_OK;
@@ -1116,8 +1158,7 @@ int txs_forward_tile(int dtype, int64_t num_total, int64_t channel, int64_t num_
         num_heavy > num_unq || !lanes || !elements || !positions)
         return TXS_ERR_INVALID_ARG;
     const int elem = dtype == TXS_F32 ? 4 : 2;
-    const Geometry geo = make_geometry(num_total, channel, elem, nullptr, nullptr,
-                                       fwd_chunk_for(num_total, num_unq, TXS_SUM, elem), true, num_heavy > 0);
+    const Geometry geo = make_geometry(num_total, channel, num_unq, elem, nullptr, nullptr, true, num_heavy > 0);
     *lanes = geo.lm.lanes;
     *elements = geo.vec_bytes / elem;
     *positions = geo.tile;
@@ -1167,16 +1208,14 @@ int txs_scatter_backward(int op, int dtype, const void *grad_out, const int32_t 
     }
     if (path == TXS_PATH_TABLE) return TXS_ERR_UNSUPPORTED;
     const int elem = dtype == TXS_F32 ? 4 : 2;
-    // short runs on average -> the short chunk; long runs -> the long one
-    const int chunk = ((long)N < (long)kChunkBwdLong * U) ? kChunkBwdShort : kChunkBwdLong;
-    Geometry geo = make_geometry(N, C, elem, grad_out, grad_in, chunk, false);
+    const Geometry geo = make_geometry(N, C, U, elem, grad_out, grad_in, false, false);
     hipError_t e;
     if (dtype == TXS_F32)
-        e = launch_bwd<F32>(op, chunk, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
+        e = launch_bwd<F32>(op, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
     else if (dtype == TXS_F16)
-        e = launch_bwd<F16>(op, chunk, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
+        e = launch_bwd<F16>(op, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
     else
-        e = launch_bwd<BF16>(op, chunk, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
+        e = launch_bwd<BF16>(op, geo, st, grad_out, arg, perm, seg, preSum, grad_in, N, C, U);
     return status_of(e);
 }
 
