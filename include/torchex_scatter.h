@@ -90,7 +90,8 @@ enum {
     TXS_STATS_LEN = 16
 };
 
-/* Library ABI version (8); bumped when a signature or the meaning of an argument changes. */
+/* Library ABI version (10); bumped when an entry point is added or goes, or when a signature or the
+ * meaning of an argument changes. */
 int txs_abi_version(void);
 
 /* Human-readable text for a status code. */

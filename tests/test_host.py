@@ -4,6 +4,7 @@ import ctypes
 import io
 import os
 import re
+import zlib
 from contextlib import redirect_stdout
 
 import numpy as np
@@ -29,6 +30,16 @@ def test_header_symbols_are_exported():
     assert not missing, missing
 
 
+def test_version_changes_with_the_declarations():
+    """A declaration that comes, goes or changes asks for another ABI version: the digest below
+    belongs to version 10."""
+    with open(os.path.join(ROOT, "include", "torchex_scatter.h")) as f:
+        text = re.sub(r"/\*.*?\*/", "", f.read(), flags=re.S)
+    declared = sorted(" ".join(d.split()) for d in re.findall(r"[\w ]+\**\s*\btxs_[a-z_0-9]+\s*\([^;]*\)\s*;", text))
+    assert len(declared) == 48
+    assert (_lib().txs_abi_version(), zlib.crc32("\n".join(declared).encode())) == (10, 4097301585)
+
+
 def test_header_is_plain_c_and_links(tmp_path):
     """The boundary is a C ABI: the header compiles as C11 with no extensions and a C
     program links against the library without any C++ or torch symbol in sight."""
@@ -40,7 +51,7 @@ def test_header_is_plain_c_and_links(tmp_path):
         pytest.skip("no C compiler on this machine")
     src = tmp_path / "abi.c"
     src.write_text('#include "torchex_scatter.h"\n'
-                   'int main(void) { return txs_abi_version() == 9 && txs_chunk_rows() > 0 ? 0 : 1; }\n')
+                   'int main(void) { return txs_abi_version() == 10 && txs_chunk_rows() > 0 ? 0 : 1; }\n')
     inc = os.path.join(ROOT, "include")
     pkg = os.path.join(ROOT, "torchex_amd")
     subprocess.check_call([cc, "-std=c11", "-Wall", "-Wextra", "-pedantic", "-Werror", "-I" + inc,
@@ -53,7 +64,7 @@ def test_header_is_plain_c_and_links(tmp_path):
 
 def test_host_only_entry_points():
     lib = _lib()
-    assert lib.txs_abi_version() == 9
+    assert lib.txs_abi_version() == 10
     lib.txs_status_string.restype = ctypes.c_char_p
     assert lib.txs_status_string(0) == b"ok"
     assert b"invalid" in lib.txs_status_string(1)
