@@ -97,11 +97,13 @@ int txs_abi_version(void);
 /* Human-readable text for a status code. */
 const char *txs_status_string(int status);
 
-/* Name of the kernel instantiation that txs_scatter_forward (backward == 0) or
- * txs_scatter_backward (backward != 0) launches for these extents, as a profiler lists
- * it without namespaces ("scatter_fwd_kernel<F32,4,MAX>": dtype, elements per lane,
- * operator; "scatter_bwd_kernel<F32,4,MAX,8>": the same and the chunk length).  pointer_alignment is
- * the alignment in bytes of the least aligned tensor (16 for ordinary allocations);
+/* Name of the kernel that txs_scatter_forward (backward == 0) or txs_scatter_backward
+ * (backward != 0) launches for these extents without heavy voxels ("scatter_fwd_kernel<F32,4,MAX>":
+ * dtype, elements per lane, operator; "scatter_bwd_kernel<F32,4,MAX,8>": the same and the chunk
+ * length).  Not part of it: the last template argument a profiler lists for these two, whether rows
+ * carry the non-temporal hint; with heavy voxels a forward call may take fewer elements per lane
+ * (txs_forward_tile).  pointer_alignment is the alignment in bytes of the least aligned tensor (16
+ * for ordinary allocations; the table kernels go by it);
  * table_allowed != 0 means the call would be made with TXS_PATH_AUTO, row-order ids and
  * enough scratch ("table_fwd_kernel<F32,4,MAX>" is then reported where table mode applies).
  * For logs and benchmarks; buf needs at least 48 bytes. */

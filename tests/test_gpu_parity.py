@@ -800,9 +800,9 @@ def test_many_rows_few_channels():
     assert torch.equal(x.grad, gup[inv.to(DEV)])
 
 
-def test_misaligned_views_fall_back_to_narrow_vectors():
-    """Tensors whose storage offset breaks 16-byte alignment still work (the launcher picks a
-    narrower per-lane vector)."""
+def test_misaligned_views_give_the_same_results():
+    """Tensors whose storage offset breaks 16-byte alignment still work: the voxel-order kernels read and
+    write full vectors at an element's alignment, without the non-temporal hint."""
     T = tx()
     import scatter_ext
     g = torch.Generator().manual_seed(88)

@@ -1075,7 +1075,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                                      table_allowed, buf, 64),
                      "kernel_name");
         return std::string(buf);
-    }, "kernel_name(backward, op, like, num_total, num_unq, table_allowed): the kernel a call on `like`-shaped rows launches");
+    }, "kernel_name(backward, op, like, num_total, num_unq, table_allowed): the kernel a call on `like`-shaped rows "
+       "without heavy voxels launches");
     m.def("grid_hash_index", &grid_hash_index,
           "grid_hash_index(coors [N, 3]) -> (dims, table, valid_mask, valid_table); the last three None where the keys are to be sorted",
           pybind11::arg("coors"));
