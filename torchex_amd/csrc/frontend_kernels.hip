@@ -542,7 +542,7 @@ __global__ void grid_hash_probe_kernel(Keys keys, const unsigned long long *__re
 // without a sort), so that the coordinates are read twice, once for the grid's extents and once
 // to mark the map, and never stored as keys.  300k rows of a sweep, 146k of them
 // distinct in 16.7M cells, built and probed with another 300k: 307 us of kernels in 44 launches
-// (the sort's plan, the linearised keys and the valid slots by library calls) -> 73 us in 13.
+// (the sort's plan, the linearised keys and the valid slots by library calls) -> 70 us in 12.
 
 // Largest coordinate per axis, one partial [3] per workgroup (the host folds the few of them).
 constexpr int kCoorMaxParts = 128;

@@ -392,11 +392,11 @@ __global__ void seg_from_presum_kernel(const int *__restrict__ preSum, long n, i
 //   (1) bucket_hist_kernel: per tile of 2048 - 8192 rows, the histogram of the HIGH digit of the
 //       voxel id (the "bucket") and the tile's order / range flags;
 //   (2) exclusive scan of the digit-major histogram;
-//   (3) bucket_scatter_kernel: flags of the whole input, bucket boundaries, and the stable
-//       scatter of (id, row) pairs by bucket (wave-ballot ranking);
-//   (4) bucket_count_kernel: a bucket is cut into slices of 4096 rows (at most 64), one workgroup
-//       per slice; where there are several, each counts its slice's rows per voxel (LOW digit,
-//       <= 11 bits) in LDS and writes the counts out;
+//   (3) bucket_scatter_kernel: flags of the whole input and the stable scatter of (id, row) pairs
+//       by bucket (wave-ballot ranking, then through LDS);
+//   (4) bucket_count_kernel: a bucket is cut into slices of 4096 rows, one workgroup per slice;
+//       where there are several, each counts its slice's rows per voxel (LOW digit, <= 11 bits)
+//       in LDS and writes the counts out;
 //   (5) bucket_plan_kernel: the same workgroups count their slice again, or add up the counts of
 //       their bucket's slices (a voxel's count, and its rows in the slices in front), which at the
 //       same time yields the bucket's share of everything else the plan holds: CSR offsets,
@@ -405,11 +405,10 @@ __global__ void seg_from_presum_kernel(const int *__restrict__ preSum, long n, i
 //       per-position ids next to the permutation.
 // Ids of at most 11 bits need no low digit: (3) already gives the final order, and the
 // elementwise kernels used by the general sequence finish the plan.
-// Measured alternatives (1M ids of 19 bits, 0.13 ms per plan as built): an 11-bit bucket digit
-// makes the scatter write 16-byte runs and costs 30 us instead of 20; folding the scan into
-// the scatter (every workgroup adding up the tile histograms itself) saves two launches but
-// costs more than it saves from about 100 tiles on; per-voxel instead of per-row offset
-// bookkeeping in (5) makes no difference.
+// Measured alternatives (1M ids of 19 bits): an 11-bit bucket digit made the scatter, then without
+// staging through LDS, write 16-byte runs and cost 30 us instead of 20; folding the scan into the
+// scatter (every workgroup adding up the tile histograms itself) saves two launches but costs
+// more than it saves from about 100 tiles on.
 
 #ifndef TXS_BUCKET_HIGH_BITS
 #define TXS_BUCKET_HIGH_BITS 9
@@ -1290,10 +1289,10 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
                             heavy_ids, stats, num_unq_dev, cnts_out, stream);
     }
     // ids of up to 11 bits are sorted by the bucket pass alone; beyond that the bucket digit has
-    // 9 bits (narrower, and the buckets of a spatially sorted id space get too uneven: a
-    // bucket's workgroups each count the whole bucket; wider, and a tile sends too few rows to
-    // a bucket for the scatter to write whole cache lines) and the low digit takes the rest,
-    // at most 11
+    // 9 bits (narrower, and the buckets of a spatially sorted id space get too uneven: every
+    // workgroup of a crowded bucket adds up the counts of all its slices, and above kBktGiant rows the
+    // plan is left to the general sequence; wider, and a tile sends too few rows to a bucket for
+    // the scatter to write whole cache lines) and the low digit takes the rest, at most 11
     const int low_bits = bits <= kBucketLowBitsMax ? 0 : min(bits - kBucketHighBits, kBucketLowBitsMax);
     const int high_bits = bits - low_bits;
     const int high_bins = 1 << high_bits;

@@ -253,8 +253,9 @@ std::tuple<Tensor, Tensor, Tensor> voxel_keys(const Tensor &points, std::vector<
 // What is cheaper than sorting the keys: an occupancy map of all possible keys.  Clearing and
 // packing it costs 10 us per 2^24 keys whatever the rows; the sort is 4 passes of 4 launches, 57 us
 // of launches alone at the smallest.  A frame of 200k points in 16.9M cells, plan included: sort
-// 119 us of kernels in 27 launches, map 75 in 14; in a quarter of a million rows or less the map
-// still wins at 2^25 keys, beyond that a row for every 64 keys is asked for.
+// 119 us of kernels in 27 launches, map 75 in 14; in half a million rows (2^25 / 64) or less the map still wins
+// at 2^25 keys (from_keys of 10 / 1000 / 60,000 keys: sort 137 / 140 / 157 us, map 107 / 112 / 113),
+// at the price of 42 MB of scratch; beyond that a row for every 64 keys is asked for.
 bool bitmap_is_cheaper(int64_t N, int64_t key_bound) {
     return key_bound <= (int64_t(1) << 28) && key_bound <= std::max<int64_t>(64 * N, int64_t(1) << 25);
 }

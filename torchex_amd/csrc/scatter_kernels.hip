@@ -3,8 +3,8 @@
 // Design in one paragraph.  Index preparation sorts row ids by voxel id once
 // and stores, for every sorted position j, the row perm[j] and the voxel seg[j].
 // The forward pass is then a segmented reduction over sorted positions: a "lane
-// group" (the lanes that together cover one feature row, each lane owning one
-// 128-bit channel vector) keeps the running sum / max of the current voxel in
+// group" (the lanes that together cover one feature row, each lane owning up to
+// 128 bits of it) keeps the running sum / max of the current voxel in
 // registers and writes a voxel's output row exactly once when its run of equal
 // ids ends.  A workgroup owns a tile of positions whose borders are moved to the
 // next run start, so that an ordinary voxel lies in one tile, and deals the tile's
@@ -47,8 +47,8 @@ namespace {
 
 // ----------------------------------------------------------------- forward --
 //
-// One workgroup owns a tile of G * chunk consecutive sorted positions (G = 256 /
-// (lanes per row) lane groups).  The tile's seg and perm entries (plus one entry
+// One workgroup owns a tile of consecutive sorted positions: chunk of them for each of its G = 256 /
+// (lanes per row) lane groups, rounded to whole wavefronts.  The tile's seg and perm entries (plus one entry
 // before and kMargin after) are staged in LDS by one coalesced load, so the row
 // loads that follow never wait on an index load.  The tile's own range runs from
 // the first run start at or after its first position to the first run start at or
