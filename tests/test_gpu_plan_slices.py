@@ -108,3 +108,31 @@ def test_an_overfull_bucket_leaves_the_rows_alone():
     assert stats[8].item() == 1 and stats[0].item() == 1      # NEED_GENERAL, UNSORTED
     for t in (ws[:2 * N], perm, seg, pre, slot, heavy):
         assert (t == -7).all()
+
+
+@pytest.mark.parametrize("N,U", [
+    (1, 1), (2, 5000), (1023, 2), (1024, 3), (1025, 1 << 20), (3000, (1 << 22) - 1), (1 << 18, 700), ((1 << 18) + 1, 90_000),
+    (5 << 18, 2048), ((5 << 18) + 1, 2049), (1 << 21, 1 << 20), ((1 << 21) + 1, 1_000_003),
+    (1 << 24, 1 << 22), (1 << 24, 1500), ((1 << 24) + 1, 1 << 21), ((1 << 24) + 1, 1500), ((1 << 24) + 4097, 70_000)])
+def test_plan_at_the_edges_of_tiles(N, U):
+    """Row numbers on either side of a tile's length, of every change of it and of the most rows that are
+    sorted in tiles (2^24; beyond, the rows are moved to bucket order), with few and many voxels."""
+    g = torch.Generator().manual_seed(N + U)
+    inv = torch.randint(0, U, (N,), generator=g)
+    inv[N // 2: N // 2 + N // 8] = U // 2     # a crowded bucket, and long runs
+    cnts = torch.bincount(inv, minlength=U)
+    order = torch.sort(inv, stable=True)[1]
+    pre = torch.cat([torch.zeros(1, dtype=torch.long), torch.cumsum(cnts, 0)])
+    data = T.ScatterData(inv.cuda(), cnts.cuda())
+    assert torch.equal(data.preSum.cpu().long(), pre) and data.max_cnt == int(cnts.max())
+    assert (data.perm is None) == bool((inv[1:] >= inv[:-1]).all())
+    assert data.perm is None or torch.equal(data.perm.cpu().long(), order)
+    assert torch.equal((data.seg.cpu() & 0x7fffffff).long(), inv[order])
+    ranks = torch.empty_like(inv)
+    ranks[order] = torch.arange(N) - pre[inv[order]]
+    assert torch.equal(T.ingroup_inds(inv.cuda()).cpu(), ranks)
+    if N > 1:
+        wrong = inv.clone()
+        wrong[N - 1] = U
+        with pytest.raises(RuntimeError):
+            T.ScatterData(wrong.cuda(), cnts.cuda())

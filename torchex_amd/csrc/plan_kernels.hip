@@ -388,53 +388,41 @@ __global__ void seg_from_presum_kernel(const int *__restrict__ preSum, long n, i
 
 // ------------------------------------------------ two-level plan (bucket sort) --
 //
-// For up to 2^22 voxels the whole index preparation is four kernels and a scan:
-//   (1) bucket_hist_kernel: per tile of 2048 - 8192 rows, the histogram of the HIGH digit of the
-//       voxel id (the "bucket") and the tile's order / range flags;
-//   (2) exclusive scan of the digit-major histogram;
-//   (3) bucket_scatter_kernel: flags of the whole input and the stable scatter of (id, row) pairs
-//       by bucket (wave-ballot ranking, then through LDS);
-//   (4) bucket_count_kernel: a bucket is cut into slices of 4096 rows, one workgroup per slice;
-//       where there are several, each counts its slice's rows per voxel (LOW digit, <= 11 bits)
-//       in LDS and writes the counts out;
-//   (5) bucket_plan_kernel: the same workgroups count their slice again, or add up the counts of
-//       their bucket's slices (a voxel's count, and its rows in the slices in front), which at the
-//       same time yields the bucket's share of everything else the plan holds: CSR offsets,
-//       per-voxel counts (checked against the caller's), the special-voxel table and its slots,
-//       max_cnt; then each places its slice by the low digit, stably, writing the flagged
-//       per-position ids next to the permutation.
-// Ids of at most 11 bits need no low digit: (3) already gives the final order, and the
-// elementwise kernels used by the general sequence finish the plan.
-// Measured alternatives (1M ids of 19 bits): an 11-bit bucket digit made the scatter, then without
-// staging through LDS, write 16-byte runs and cost 30 us instead of 20; folding the scan into the
-// scatter (every workgroup adding up the tile histograms itself) saves two launches but costs
-// more than it saves from about 100 tiles on.
+// For up to 2^22 voxels the whole index preparation is four kernels:
+//   (1) tile_sort_kernel: a tile of 1024 - 8192 rows is sorted by the HIGH digit of the voxel id
+//       (the "bucket") in LDS and written back in place of itself, four bytes a row (the LOW digit
+//       and the row's number inside the tile), with the tile's first row of every bucket and its
+//       order / range flags;
+//   (2) bucket_start_kernel: the first rows of a bucket, added up over the tiles, are the rows of all
+//       buckets in front of it: where the bucket starts.  Flags of the whole input;
+//   (3) bucket_count_kernel: a bucket is cut into slices; where one has very many, each is counted
+//       per voxel (low digit, <= 11 bits) by a workgroup and the counts are written out.  Returns
+//       at once for ordinary inputs;
+//   (4) bucket_plan_kernel: a workgroup per slice gathers its rows from the tiles (a short run of
+//       each, found by a scan over the tiles' counts) and counts them, and the bucket's other
+//       slices, per voxel, which at the same time yields the bucket's share of everything else the
+//       plan holds: CSR offsets, per-voxel counts (checked against the caller's), the special-voxel
+//       table and its slots, max_cnt; then it places its slice by the low digit, stably, writing
+//       the flagged per-position ids next to the permutation.
+// No kernel needs the histogram of the whole input before it can write, so that neither a pass
+// over the ids for it nor its scan is there, and every write up to the last kernel's is a stream.
+// Above kTiledRows rows a bucket's runs would lie in too many tiles: the rows are then moved to
+// bucket order, as (id, row) pairs, by bucket_hist_kernel, an exclusive scan of the digit-major
+// histogram and bucket_scatter_kernel, and (3) and (4) read them there.
 
-#ifndef TXS_BUCKET_HIGH_BITS
-#define TXS_BUCKET_HIGH_BITS 9
-#endif
-constexpr int kBucketHighBits = TXS_BUCKET_HIGH_BITS;
+constexpr int kBucketHighBits = 9;      // high digit of the rows moved to bucket order
 constexpr int kBucketLowBitsMax = 11;   // also the largest high digit
 constexpr int kBucketBitsMax = 22;
 constexpr int kHistThreads = 512;
-// rows per tile of the histogram and scatter kernels: 512 * {4, 8, 16}, the largest that still
-// gives every compute unit a tile
-int hist_items_for(long n) {
-    return n >= 256L * kHistThreads * 16 ? 16 : (n >= 256L * kHistThreads * 8 ? 8 : 4);
-}
+// rows per tile of the histogram and scatter kernels: the instances of 4 and 8 items a thread
+// served inputs that tile_sort_kernel takes now
+constexpr int kHistItems = 16;
 constexpr int kHistWaves = kHistThreads / 64;
-constexpr int kBktThreads = 512;
-constexpr int kBktItems = 8;
-constexpr int kBktWaves = kBktThreads / 64;
-constexpr int kBktSlice = kBktThreads * kBktItems;     // rows one workgroup places
-constexpr long kBktGiant = 64L * kBktSlice;            // rows in one bucket beyond which the general sequence runs
-// Rows of one voxel in a slice beyond which they are ranked by ballots.  bucket_plan_kernel, us, with
-// 64 (and one read at a time) / 63 / 31 / 24 / 21: 1M ids of pillars 37.2 / 29.5 / 22.9 / 22.8 / 22.1, 1M
-// ids of 50 rows per voxel 46.3 / 39.6 / 31.0 / 29.7 / 29.4, of 25 rows 33.7 / 30.3 / 28.4 / 27.7 / 27.8, of 10
-// rows 20.9 / 17.6 / 18.8 / 20.9 / 21.4, of a sweep 21.5 / 19.5 / 20.8 / 21.8 / 21.9.
-constexpr int kLongRun = 24;
-constexpr int kMaxLongRuns = kBktSlice / (kLongRun + 1);
-static_assert(kMaxLongRuns < 256 && kBktSlice / 64 == 64, "eight bits number a slice's long runs, a wave scans their chunk counts");
+constexpr int kBktItems = 8;                           // rows of its slice a thread places
+constexpr long kBktGiant = 262144;                     // rows in one bucket beyond which the general sequence runs
+// A bucket of up to this many slices is counted as a whole by each of its workgroups; above, the
+// counts come from bucket_count_kernel.
+constexpr int kSelfSlices = 2;
 constexpr int kFlagUnsorted = 1, kFlagOutOfRange = 2;
 
 // Bits of ids below U, and of them the low digit where the bucket digit may take high_bits.
@@ -446,6 +434,28 @@ __device__ __forceinline__ int low_bits_of(int U, int high_bits) { return max(0,
 __device__ __forceinline__ int voxel_count(int U_arg, const int *__restrict__ num_unq_dev) {
     return num_unq_dev ? min(U_arg, *num_unq_dev) : U_arg;
 }
+
+// How the rows are cut into tiles and the ids into digits, for ids of `bits` bits.
+constexpr int kTileRowsMax = 8192;
+constexpr int kTilesMax = 2048;
+constexpr long kTiledRows = (long)kTileRowsMax * kTilesMax;
+struct TileSplit {
+    int tile_bits;   // log2(rows per tile)
+    int high_bits;
+    int tiles;
+    int pitch;       // entries of a tile's row of first rows: one per bucket, the tile's valid rows, padding
+};
+TileSplit tile_split(long n, int bits) {
+    TileSplit r;
+    r.tile_bits = n <= (1L << 18) ? 10 : (n <= (5L << 18) ? 11 : (n <= (1L << 21) ? 12 : 13));
+    r.high_bits = bits <= kBucketLowBitsMax ? bits : min(max(kBucketHighBits, bits - 10), kBucketLowBitsMax);
+    if (r.high_bits > 10 && r.tile_bits < 11) r.tile_bits = 11;  // (256 threads scan at most 1024 buckets)
+    r.tiles = (int)((n + (1L << r.tile_bits) - 1) >> r.tile_bits);
+    r.pitch = max(1 << r.high_bits, 4) + 4;
+    return r;
+}
+// threads of the workgroups that serve a slice of kBktItems rows per thread
+int slice_threads_for(long n, int low_bits) { return n > (1L << 19) || low_bits > 10 ? 512 : 256; }  // (four voxels a thread)
 
 // exclusive scan of one int per thread across a workgroup of WAVES wavefronts
 template <int WAVES>
@@ -481,11 +491,301 @@ __device__ __forceinline__ unsigned long long wave_match(int digit, int bits, bo
     return ((unsigned long long)hi << 32) | lo;
 }
 
+// Rank of every row among its wave's rows of the same digit (`bits` bits of the key from bit `shift` on, the
+// key's highest ones), in (item, lane) order: turn[k] for the rows with key[k] >= 0.  counts2: the wave's own 16-bit counts, one per digit, zero on entry; the wave's
+// rows per digit on return.  The items advance bit by bit side by side: an item's chain of ballots depends on
+// itself all the way, and one item after the other left the vector units idle for most of it (eight
+// items of eight bits, in a workgroup of 256 threads: 3.1 us, now 2.1).
+template <int COUNT>
+__device__ __forceinline__ void wave_rank(const int (&key)[COUNT], int shift, int bits, unsigned *counts2, int (&turn)[COUNT]) {
+    const int lane = threadIdx.x & 63;
+    const unsigned below_lo = lane < 32 ? (1u << lane) - 1u : 0xffffffffu;
+    const unsigned below_hi = lane < 32 ? 0u : (1u << (lane - 32)) - 1u;
+    unsigned lo[COUNT], hi[COUNT];
+#pragma unroll
+    for (int k = 0; k < COUNT; ++k) {
+        const unsigned long long all = __ballot(key[k] >= 0);
+        lo[k] = (unsigned)all;
+        hi[k] = (unsigned)(all >> 32);
+    }
+#pragma unroll 1
+    for (int b = 0; b < bits; ++b) {
+#pragma unroll
+        for (int k = 0; k < COUNT; ++k) {
+            const unsigned mine = (unsigned)__builtin_amdgcn_sbfe(key[k], shift + b, 1);  // the bit in every position
+            const unsigned long long bal = __ballot(mine != 0u);
+            lo[k] &= ~((unsigned)bal ^ mine);
+            hi[k] &= ~((unsigned)(bal >> 32) ^ mine);
+        }
+    }
+    // The first row of each group adds the group to the count, two 16-bit counts to a word, and hands
+    // the count before it round: the adds of all items are in flight together (LDS serves a wave's
+    // instructions in order, so they count up item by item); the other rows add nothing to a word of
+    // their own, so that no add is under a branch.  The stages are kept apart to bound the registers.
+    __shared__ unsigned sink_s[64];
+    unsigned before[COUNT];
+#pragma unroll
+    for (int k = 0; k < COUNT; ++k) {
+        const int below = __popc(lo[k] & below_lo) + __popc(hi[k] & below_hi), group = __popc(lo[k]) + __popc(hi[k]);
+        const int leader = lo[k] ? __builtin_ctz(lo[k]) : 32 + __builtin_ctz(hi[k] | 0x80000000u);
+        turn[k] = below | leader << 8 | group << 16;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < COUNT; ++k) {
+        const bool first = key[k] >= 0 && (turn[k] & 255) == 0;
+        before[k] = atomicAdd(first ? counts2 + (key[k] >> (shift + 1)) : &sink_s[lane],
+                              first ? (unsigned)(turn[k] >> 16) << ((key[k] >> shift & 1) << 4) : 0u);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < COUNT; ++k)
+        turn[k] = (turn[k] & 255) + (int)((__shfl(before[k], (turn[k] >> 8) & 255, 64) >> ((key[k] >> shift & 1) << 4)) & 0xffffu);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// A tile's rows in bucket order: rows_out[tile's first row + k] = low digit << tile bits | row inside
+// the tile; offs[tile][d] = the tile's rows in buckets below d (d up to the number of buckets).
+// K = long long: ids as torch.unique returns them, cut to 32 bits and left in `ids32` for later readers.
+// stats and ctl are cleared for the kernels that follow.
+// Ranking is by wave ballots on the digit's bits and a 16-bit count per wave and bucket; the rows pass
+// through LDS so that they leave as one stream.
+template <int THREADS, int ITEMS, typename K>
+__global__ __launch_bounds__(THREADS) void tile_sort_kernel(
+    const K *__restrict__ ids, long n, int U_arg, int high_bits, unsigned *__restrict__ rows_out,
+    unsigned short *__restrict__ offs, int pitch, int *__restrict__ tile_flags, int *__restrict__ ids32,
+    int *__restrict__ stats, int *__restrict__ ctl, const int *__restrict__ num_unq_dev) {
+    constexpr int WAVES = THREADS / 64, kRows = THREADS * ITEMS, kTileBits = __builtin_ctz(kRows);
+    // [bins] first place of every bucket, then the larger of [WAVES][bins] counts and the staged rows
+    extern __shared__ __align__(16) uint2 lds_tile[];
+    __shared__ int s_flags;
+    const int U = voxel_count(U_arg, num_unq_dev), low_bits = low_bits_of(U, high_bits);
+    const int quads = max(1 << high_bits, 4) >> 2;  // bins / 4
+    uint2 *first4 = lds_tile, *cnt4 = lds_tile + quads;
+    const unsigned short *first = reinterpret_cast<const unsigned short *>(first4);
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const long tile0 = (long)blockIdx.x * kRows;
+    const long wbase = tile0 + (long)w * (64 * ITEMS);
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < TXS_STATS_LEN) stats[threadIdx.x] = 0;
+        if (threadIdx.x == 0) ctl[0] = 0;
+    }
+    int key[ITEMS];
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+        const long i = wbase + (long)it * 64 + lane;
+        key[it] = i < n ? (int)ids[i] : 0x7fffffff;
+    }
+    // the id behind the wave's rows
+    int behind = 0x7fffffff;
+    if (lane == 63 && wbase + 64 * ITEMS < n) behind = (int)ids[wbase + 64 * ITEMS];
+    if (threadIdx.x == 0) s_flags = 0;
+    for (int k = threadIdx.x; k < WAVES * quads; k += THREADS) cnt4[k] = make_uint2(0u, 0u);
+    __syncthreads();
+    bool bad_range = false, bad_order = false;
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+        const long i = wbase + (long)it * 64 + lane;
+        if (sizeof(K) == 8 && i < n) ids32[i] = key[it];
+        int next = __shfl_down(key[it], 1, 64);
+        const int wrap = it + 1 < ITEMS ? __builtin_amdgcn_readfirstlane(key[it + 1 < ITEMS ? it + 1 : 0]) : behind;
+        if (lane == 63) next = wrap;
+        bad_order |= next < key[it];  // (rows behind the last one compare as the largest id)
+        if ((unsigned)key[it] >= (unsigned)U) {
+            bad_range |= i < n;
+            key[it] = -1;  // out-of-range ids are dropped (and flagged)
+        }
+    }
+    const int f = (__ballot(bad_order) != 0ull ? kFlagUnsorted : 0) | (__ballot(bad_range) != 0ull ? kFlagOutOfRange : 0);
+    if (f && lane == 0) atomicOr(&s_flags, f);
+    int place[ITEMS];
+    wave_rank<ITEMS>(key, low_bits, high_bits, reinterpret_cast<unsigned *>(cnt4 + w * quads), place);
+    __syncthreads();
+    const unsigned short *wc = reinterpret_cast<const unsigned short *>(cnt4 + w * quads);
+    // counts per wave -> rows of the waves in front; totals -> first place of every bucket.  Four
+    // buckets a thread, two 16-bit numbers to a word: no sum passes the tile's 8192 rows.
+    uint2 run = make_uint2(0u, 0u);
+    const int q = threadIdx.x;
+    if (q < quads) {
+#pragma unroll
+        for (int k = 0; k < WAVES; ++k) {
+            const uint2 c = cnt4[k * quads + q];
+            cnt4[k * quads + q] = run;
+            run.x += c.x;
+            run.y += c.y;
+        }
+    }
+    const int c0 = run.x & 0xffff, c1 = run.x >> 16, c2 = run.y & 0xffff, c3 = run.y >> 16;
+    int total;
+    const int at = wide_exclusive_scan<WAVES>(c0 + c1 + c2 + c3, &total);
+    uint2 *offs4 = reinterpret_cast<uint2 *>(offs + (long)blockIdx.x * pitch);
+    if (q < quads) {
+        const uint2 o = make_uint2((unsigned)at | (unsigned)(at + c0) << 16,
+                                   (unsigned)(at + c0 + c1) | (unsigned)(at + c0 + c1 + c2) << 16);
+        first4[q] = o;
+        offs4[q] = o;
+    }
+    if (threadIdx.x == 0) {
+        offs4[quads] = make_uint2((unsigned)total * 0x10001u, (unsigned)total * 0x10001u);
+        tile_flags[blockIdx.x] = s_flags;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) place[it] += (int)first[max(key[it], 0) >> low_bits] + (int)wc[max(key[it], 0) >> low_bits];
+    __syncthreads();
+    unsigned *stage = reinterpret_cast<unsigned *>(cnt4);
+    const unsigned low_mask = (1u << low_bits) - 1u;
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it)
+        if (key[it] >= 0)
+            stage[place[it]] = ((unsigned)key[it] & low_mask) << kTileBits | (unsigned)(w * (64 * ITEMS) + it * 64 + lane);
+    __syncthreads();
+    for (int p = threadIdx.x; p < total; p += THREADS) rows_out[tile0 + p] = stage[p];
+}
+
+// What a plan holds per voxel (any of it may be NULL but preSum; slot_of and heavy_ids go together).
+struct VoxelArgs {
+    int heavy_threshold;
+    const long long *unq_cnts;  // the caller's counts
+    int *preSum, *slot_of, *heavy_ids;
+    long long *cnts_out;
+};
+// Special voxels and their slots, as plan_special_kernel: COUNT consecutive voxels a lane, from `u` on, as
+// far as they lie below `end`.  One atomic per wave and kind.
+template <int COUNT>
+__device__ __forceinline__ void voxel_slots(const VoxelArgs &v, int U, int u, int end, const int (&count)[COUNT],
+                                            int *__restrict__ stats) {
+    const int lane = threadIdx.x & 63;
+    const unsigned long long lanes_below = (1ull << lane) - 1ull;
+    int heavy = 0, empty = 0, heavy_below[COUNT], empty_below[COUNT];  // of the wave; in front of this voxel
+#pragma unroll
+    for (int k = 0; k < COUNT; ++k) {
+        const bool valid = u + k < end;
+        const unsigned long long mh = __ballot(valid && count[k] > v.heavy_threshold), me = __ballot(valid && count[k] == 0);
+        heavy_below[k] = heavy + __popcll(mh & lanes_below);
+        empty_below[k] = empty + __popcll(me & lanes_below);
+        heavy += __popcll(mh);
+        empty += __popcll(me);
+    }
+    int base_h = 0, base_e = 0;
+    if (heavy + empty > 0) {
+        if (lane == 0) {
+            if (heavy) base_h = atomicAdd(&stats[TXS_STAT_NUM_HEAVY], heavy);
+            if (empty) base_e = atomicAdd(&stats[TXS_STAT_NUM_EMPTY], empty);
+            atomicAdd(&stats[TXS_STAT_NUM_SPECIAL], heavy + empty);
+        }
+        base_h = __shfl(base_h, 0, 64);
+        base_e = __shfl(base_e, 0, 64);
+    }
+#pragma unroll
+    for (int k = 0; k < COUNT; ++k) {
+        if (u + k >= end) continue;
+        int slot = -1;
+        if (count[k] > v.heavy_threshold) {
+            slot = base_h + heavy_below[k];
+            if (slot < U) v.heavy_ids[slot] = u + k;
+        } else if (count[k] == 0) {
+            slot = U - 1 - (base_e + empty_below[k]);
+            if (slot >= 0) v.heavy_ids[slot] = u + k;
+        }
+        v.slot_of[u + k] = slot;
+    }
+}
+
+// The same and the rest of it where a bucket is a voxel: a wave of voxels u, those with `in`, whose rows
+// start at `start`.
+__device__ __forceinline__ void bucket_voxel(const VoxelArgs &v, int U, int n, int u, bool in, int start, int rows,
+                                             int *__restrict__ stats) {
+    if (in) {
+        v.preSum[u] = start;
+        if (v.cnts_out) v.cnts_out[u] = (long long)rows;
+        if (u == U - 1) v.preSum[U] = n;
+    }
+    if (v.slot_of == nullptr) return;
+    const int count[1] = {rows};
+    voxel_slots<1>(v, U, u, in ? U : 0, count, stats);
+    const bool mismatch = in && v.unq_cnts && v.unq_cnts[u] != (long long)rows;
+    const int most = wave_max_i32(in ? rows : 0);
+    if (__ballot(mismatch) != 0ull && (threadIdx.x & 63) == 0) stats[TXS_STAT_COUNT_MISMATCH] = 1;
+    if ((threadIdx.x & 63) == 0 && most > 0) atomicMax(&stats[TXS_STAT_MAX_CNT], most);
+}
+__global__ __launch_bounds__(64) void bucket_voxels_kernel(const int *__restrict__ bucket_start, int n, int U_arg,
+                                                           int high_bits, int *__restrict__ stats,
+                                                           const int *__restrict__ num_unq_dev, VoxelArgs v) {
+    const int U = voxel_count(U_arg, num_unq_dev), u = (int)(blockIdx.x * 64 + threadIdx.x);
+    if (low_bits_of(U, high_bits) > 0 || stats[TXS_STAT_NEED_GENERAL] != 0) return;
+    const bool in = u < U;
+    const int start = in ? bucket_start[u] : 0;
+    bucket_voxel(v, U, n, u, in, start, in ? bucket_start[u + 1] - start : 0, stats);
+}
+
+// bucket_start[d] = rows in buckets below d, for d up to the number of buckets: the sum over the tiles
+// of offs[.][d].  A workgroup reads 32 neighbouring columns (a 64-byte sector per tile) and owns the
+// first 30 of them, so that it also sees where each of its buckets ends.
+// Where a bucket is a voxel (ids of at most 11 bits), what the plan holds per voxel is left here too: the
+// statistics take one atomic per 30 voxels, where bucket_plan_kernel's workgroups, one or more per voxel,
+// would queue up for the same few words (index preparation of 1M rows in 1000 Zipf voxels: 88 us with
+// that, 65 so).
+// Sets stats[NEED_GENERAL] for a bucket above kBktGiant rows (the kernels that follow step aside; not
+// where so few voxels have so many rows that the low digit has next to nothing left) and ctl[0] for
+// one of more than kSelfSlices slices; workgroup 0 also the flags of the whole input.
+constexpr int kStartThreads = 1024, kStartColumns = 32, kStartOwned = 30;
+__global__ __launch_bounds__(kStartThreads) void bucket_start_kernel(
+    const unsigned short *__restrict__ offs, int pitch, int n_tiles, int n, int U_arg, int high_bits, int self_rows,
+    const int *__restrict__ tile_flags, int *__restrict__ bucket_start, int *__restrict__ stats,
+    int *__restrict__ ctl, const int *__restrict__ num_unq_dev, VoxelArgs v) {
+    constexpr int kLanes = kStartColumns / 2, kGroups = kStartThreads / kLanes;  // two columns a thread
+    __shared__ int sum_s[kGroups][kStartColumns + 2];
+    __shared__ int start_s[kStartColumns];
+    const int x = threadIdx.x % kLanes, y = threadIdx.x / kLanes;
+    const int word = (int)blockIdx.x * (kStartOwned / 2) + x, words = pitch / 2;
+    const unsigned *offs2 = reinterpret_cast<const unsigned *>(offs);
+    int lo = 0, hi = 0;
+    if (word < words) {
+#pragma unroll 4
+        for (int t = y; t < n_tiles; t += kGroups) {
+            const unsigned two = offs2[(long)t * words + word];
+            lo += (int)(two & 0xffffu);
+            hi += (int)(two >> 16);
+        }
+    }
+    sum_s[y][2 * x] = lo;
+    sum_s[y][2 * x + 1] = hi;
+    if (blockIdx.x == 0) {
+        int f = 0;
+        for (int t = threadIdx.x; t < n_tiles; t += kStartThreads) f |= tile_flags[t];
+        if (f & kFlagUnsorted) stats[TXS_STAT_UNSORTED] = 1;
+        if (f & kFlagOutOfRange) stats[TXS_STAT_OUT_OF_RANGE] = 1;
+    }
+    __syncthreads();
+    // 32 threads per column
+    const int c = threadIdx.x >> 5, part = threadIdx.x & 31;
+    int s = 0;
+    for (int k = part; k < kGroups; k += 32) s += sum_s[k][c];
+#pragma unroll
+    for (int d = 16; d >= 1; d >>= 1) s += __shfl_xor(s, d, 64);
+    if (part == 0) start_s[c] = s;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int col = (int)blockIdx.x * kStartOwned + (int)threadIdx.x;
+    const int bins = 1 << high_bits, U = voxel_count(U_arg, num_unq_dev);
+    const bool owned = threadIdx.x < kStartOwned, bucket = owned && col < bins;
+    const int start = owned ? start_s[threadIdx.x] : 0;
+    const int rows = bucket ? start_s[threadIdx.x + 1] - start : 0;
+    if (owned && col <= bins) bucket_start[col] = start;
+    if (low_bits_of(U, high_bits) > 0) {
+        if (rows > kBktGiant && U > 1 << kBucketLowBitsMax) stats[TXS_STAT_NEED_GENERAL] = 1;
+        if (rows > self_rows) ctl[0] = 1;
+        return;
+    }
+    bucket_voxel(v, U, n, col, bucket && col < U, start, rows, stats);
+}
+
 // hist: [high_bins][n_tiles] digit-major (the order its exclusive scan needs); tile_flags: [n_tiles]
 // K = long long: ids as torch.unique returns them, cut to 32 bits and left in `ids32` for the
 // kernels that follow (a conversion of its own reads and writes them once more: 16 us of 4M ids,
 // 5 us of 1M)
-template <int ITEMS, typename K>
+template <typename K>
 __global__ __launch_bounds__(kHistThreads) void bucket_hist_kernel(
     const K *__restrict__ inv, long n, int U_arg, int high_bits, int *__restrict__ hist,
     int *__restrict__ tile_flags, int n_tiles, int *__restrict__ ids32, const int *__restrict__ num_unq_dev) {
@@ -495,17 +795,17 @@ __global__ __launch_bounds__(kHistThreads) void bucket_hist_kernel(
     for (int d = threadIdx.x; d < high_bins; d += kHistThreads) h[d] = 0;
     if (threadIdx.x == 0) s_flags = 0;
     __syncthreads();
-    const long base = (long)blockIdx.x * (kHistThreads * ITEMS);
-    int v[ITEMS];
+    const long base = (long)blockIdx.x * (kHistThreads * kHistItems);
+    int v[kHistItems];
 #pragma unroll
-    for (int it = 0; it < ITEMS; ++it) {
+    for (int it = 0; it < kHistItems; ++it) {
         const long i = base + (long)it * kHistThreads + threadIdx.x;
         v[it] = i < n ? (int)inv[i] : 0x7fffffff;
         if (sizeof(K) == 8 && i < n) ids32[i] = v[it];
     }
     bool bad_range = false, bad_order = false;
 #pragma unroll
-    for (int it = 0; it < ITEMS; ++it) {
+    for (int it = 0; it < kHistItems; ++it) {
         const long i = base + (long)it * kHistThreads + threadIdx.x;
         if (i >= n) continue;
         if ((unsigned)v[it] >= (unsigned)U) {
@@ -530,25 +830,18 @@ __global__ void narrow_ids_kernel(const long long *__restrict__ ids64, long n, i
     if (i < n) ids32[i] = (int)ids64[i];
 }
 
-// id at position i: of unq_inv itself (rows in order) or of the (id, row) pairs the bucket scatter wrote
-__device__ __forceinline__ int kread(const int *keys, long i, bool packed) {
-    return packed ? keys[2 * i] : keys[i];
-}
-
 // Stable scatter by the high digit.  hist: the exclusive scan of the digit-major tile histograms.
 //   bucket_start [high_bins + 1] (from the scan): first position of every bucket.
 //   stats: zero-filled here (workgroup 0), then UNSORTED / OUT_OF_RANGE of the whole input
 //   and NEED_GENERAL (a bucket above kBktGiant rows: the bucket kernels step aside; not where so few
 //   voxels have so many rows that the low digit has next to nothing left).
-// Rows already in order are not moved: out_keys (if given) receives a copy of the ids, and
-// the next kernel reads unq_inv itself.  out_pairs: (id, row) per position, one 8-byte
-// store; or out_keys / out_rows as two arrays when the order is already final.
-template <int ITEMS>
+// Rows already in order are not moved: the next kernel reads unq_inv itself.  out_pairs: (id, row) per
+// position, one 8-byte store.
 __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
     const int *__restrict__ inv, long n, int U_arg, int high_bits,
     const int *__restrict__ hist, const int *__restrict__ tile_flags, int n_tiles,
-    const int *__restrict__ bucket_start, int *__restrict__ stats, int *__restrict__ out_keys,
-    int *__restrict__ out_rows, int2 *__restrict__ out_pairs, const int *__restrict__ num_unq_dev) {
+    const int *__restrict__ bucket_start, int *__restrict__ stats, int2 *__restrict__ out_pairs,
+    const int *__restrict__ num_unq_dev) {
     // [bins] base_s: first destination of this tile's rows, per digit; then the larger of
     // [kHistWaves][bins] wave counts and the tile's staged (id, row) pairs
     extern __shared__ __align__(8) int lds_base[];
@@ -587,35 +880,28 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
         }
     }
     if (flags & 4) return;  // the caller re-plans with the general sequence
-    const long tile0 = (long)blockIdx.x * (kHistThreads * ITEMS);
-    if (!(flags & kFlagUnsorted)) {
-        if (out_keys)
-            for (int it = 0; it < ITEMS; ++it) {
-                const long i = tile0 + (long)it * kHistThreads + threadIdx.x;
-                if (i < n) out_keys[i] = inv[i];
-            }
-        return;
-    }
+    const long tile0 = (long)blockIdx.x * (kHistThreads * kHistItems);
+    if (!(flags & kFlagUnsorted)) return;
 
     // ---- stable ranking inside the tile
-    const long wbase = tile0 + (long)w * (64 * ITEMS);
-    int key[ITEMS], lrank[ITEMS];
+    const long wbase = tile0 + (long)w * (64 * kHistItems);
+    int key[kHistItems], lrank[kHistItems];
 #pragma unroll
-    for (int it = 0; it < ITEMS; ++it) {
+    for (int it = 0; it < kHistItems; ++it) {
         const long i = wbase + (long)it * 64 + lane;
         const int v = i < n ? inv[i] : -1;
         key[it] = (unsigned)v < (unsigned)U ? v : -1;  // out-of-range ids are dropped (and flagged)
     }
     volatile int *wc = wcount + w * bins;
 #pragma unroll
-    for (int it = 0; it < ITEMS; ++it) {
+    for (int it = 0; it < kHistItems; ++it) {
         const bool valid = key[it] >= 0;
         const unsigned long long mask = wave_match(valid ? key[it] >> low_bits : 0, high_bits, valid);
         // rows of the same bucket in front of this one among the wave's 64, and the group's size
         lrank[it] = __popcll(mask & lanes_below) | (__popcll(mask) << 8);
     }
 #pragma unroll
-    for (int it = 0; it < ITEMS; ++it) {
+    for (int it = 0; it < kHistItems; ++it) {
         const bool valid = key[it] >= 0;
         const int digit = valid ? (key[it] >> low_bits) : 0;
         const int below = lrank[it] & 255, group = lrank[it] >> 8;
@@ -647,7 +933,7 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
     }
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < ITEMS; ++it)
+    for (int it = 0; it < kHistItems; ++it)
         if (key[it] >= 0) lrank[it] += wcount[w * bins + (key[it] >> low_bits)];
     __syncthreads();
     // ---- through LDS (over the wave counts, which are done with): the tile's rows leave in
@@ -656,375 +942,460 @@ __global__ __launch_bounds__(kHistThreads) void bucket_scatter_kernel(
     // 1024 buckets: 37.6 -> 28.5 us; 1M ids, whose tiles hold four rows per bucket only: 15.2 -> 15.6)
     int2 *stage = reinterpret_cast<int2 *>(lds_scatter);
 #pragma unroll
-    for (int it = 0; it < ITEMS; ++it)
+    for (int it = 0; it < kHistItems; ++it)
         if (key[it] >= 0) stage[lrank[it]] = make_int2(key[it], (int)(wbase + (long)it * 64 + lane));
     __syncthreads();
     for (int p = threadIdx.x; p < total; p += kHistThreads) {
         const int2 kr = stage[p];
         const long dst = (long)base_s[kr.x >> low_bits] + p;
         if (dst < 0 || dst >= n) continue;
-        if (out_pairs) {
-            out_pairs[dst] = kr;
-        } else {
-            out_keys[dst] = kr.x;
-            out_rows[dst] = kr.y;
-        }
+        out_pairs[dst] = kr;
     }
 }
 
-// Rows of bucket b that slice j of it covers.  A bucket is cut into slices of kBktSlice rows.
-struct BucketSlice {
-    long s, e;        // the bucket's rows [s, e) in bucket order
-    long my_s, my_e;  // the slice's rows
-    int nsl;          // slices of the bucket
-};
-__device__ __forceinline__ int slices_of(long cnt_b) {
-    return (int)max(1L, (cnt_b + kBktSlice - 1) / kBktSlice);
-}
-__device__ __forceinline__ BucketSlice bucket_slice(long s, long e, int j) {
-    BucketSlice r;
-    r.s = s;
-    r.e = e;
-    r.nsl = slices_of(e - s);
-    r.my_s = s + (long)j * kBktSlice;
-    r.my_e = min(e, r.my_s + kBktSlice);
-    return r;
+// A bucket is cut into slices of slice_rows rows.  The first `more` workgroups (an upper bound) serve the
+// further slices of all buckets, bucket by bucket, and start first, because theirs are the full buckets;
+// those behind them serve the first slice of a bucket each.
+__device__ __forceinline__ int slices_of(int rows, int slice_rows) { return max(1, (rows + slice_rows - 1) / slice_rows); }
+
+// Where the counts of a bucket's slices lie, one row each: no two slices share a row, and there are as
+// many rows as buckets and slice_rows rows.
+__device__ __forceinline__ int count_row(int bucket, int start, int slice_rows) { return bucket + start / slice_rows; }
+
+// (bucket, slice) of further slice number `extra` into s_pick, or (-1, .) if there are no more; the whole
+// workgroup.
+template <int THREADS>
+__device__ __forceinline__ void find_slice(const int *__restrict__ bucket_start, int bins, int slice_rows, int extra,
+                                           int *s_pick) {
+    constexpr int kMost = (1 << kBucketLowBitsMax) / THREADS;
+    const int per = (bins + THREADS - 1) / THREADS;
+    const int d0 = (int)threadIdx.x * per;
+    int start[kMost + 1];
+#pragma unroll
+    for (int k = 0; k <= kMost; ++k) start[k] = bucket_start[min(d0 + min(k, per), bins)];
+    if (threadIdx.x == 0) s_pick[0] = -1;
+    int more = 0;
+#pragma unroll
+    for (int k = 0; k < kMost; ++k) more += slices_of(start[k + 1] - start[k], slice_rows) - 1;
+    int total;
+    int first = wide_exclusive_scan<THREADS / 64>(more, &total);  // (synchronises the workgroup)
+#pragma unroll
+    for (int k = 0; k < kMost; ++k) {
+        const int m = slices_of(start[k + 1] - start[k], slice_rows) - 1;
+        if (extra >= first && extra < first + m) {
+            s_pick[0] = d0 + k;
+            s_pick[1] = 1 + extra - first;
+        }
+        first += m;
+    }
+    __syncthreads();
 }
 
-// Workgroup g serves slice j of bucket b; (b, j) follows from the bucket sizes and is kept with
-// the bucket's bounds in wg_pick[g] = (b, j, start, end) (b = -1: no work) for the kernel that
-// follows, which so learns its work from one load.  Where a bucket has several slices, each
-// workgroup counts the rows of ITS slice per voxel (low digit) and writes the counts to
-// part_hist[g][*]: the slices of a bucket sit in consecutive workgroups, so the next kernel gets a
-// voxel's count in the whole bucket, and in the slices in front of its own, from one short
-// read per slice instead of every workgroup of a crowded bucket counting all of its rows.
-__global__ __launch_bounds__(kBktThreads) void bucket_count_kernel(
-    const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U_arg, int high_bits,
-    const int *__restrict__ bucket_start, const int *__restrict__ stats, int4 *__restrict__ wg_pick,
-    int *__restrict__ part_hist, const int *__restrict__ num_unq_dev) {
-    const int U = voxel_count(U_arg, num_unq_dev), low_bits = low_bits_of(U, high_bits), high_bins = 1 << high_bits;
-    extern __shared__ int cnt_s[];  // [low_bins]
-    __shared__ int s_pick[2];
-    const int low_bins = 1 << low_bits;
-    if (stats[TXS_STAT_NEED_GENERAL] != 0) return;
-    {
-        if (threadIdx.x == 0) s_pick[0] = -1;
-        int carried = 0;
-        for (int bb0 = 0; bb0 < high_bins; bb0 += kBktThreads) {
-            const int bb = bb0 + (int)threadIdx.x;
-            int nsl = 0;
-            if (bb < high_bins && ((long)bb << low_bits) < (long)U)
-                nsl = slices_of((long)bucket_start[bb + 1] - bucket_start[bb]);
-            int total;
-            const int first = carried + wide_exclusive_scan<kBktWaves>(nsl, &total);  // (synchronises the workgroup)
-            if ((int)blockIdx.x >= first && (int)blockIdx.x < first + nsl) {
-                s_pick[0] = bb;
-                s_pick[1] = (int)blockIdx.x - first;
+// Where a bucket's rows come from: the tiles (TILED), a short run of each, or (id, row) pairs in
+// bucket order / the ids themselves where the rows are in order.
+// seen_s[t] rows of the bucket lie in tiles in front of tile t (none lies in the padding, up to a power of
+// two, behind the last tile), and rows[from_s[t] + p] is the row at position p of the bucket if that
+// lies in tile t.
+template <bool TILED>
+struct BucketRows {
+    const unsigned *rows;  // TILED
+    const int *keys;       // pairs (packed) or ids
+    bool packed;
+    const int *seen_s, *from_s;
+    int top, tile_bits;    // top: half the padded number of tiles
+    int u_lo, start;
+    // Low digits and rows at COUNT positions inside the bucket.  Nothing here is under a branch, so that
+    // the searches advance side by side and all loads are in flight before the first is used (each under
+    // its own condition, one after the other: ranks of 1M ids 77 us in bucket_plan_kernel, 46 so).
+    template <int COUNT>
+    __device__ __forceinline__ void get(const int (&p)[COUNT], int (&dig)[COUNT], int (&row)[COUNT]) const {
+        if (TILED) {
+            int t[COUNT];
+            unsigned r[COUNT];
+#pragma unroll
+            for (int k = 0; k < COUNT; ++k) t[k] = 0;
+#pragma unroll 1
+            for (int step = top; step > 0; step >>= 1) {
+#pragma unroll
+                for (int k = 0; k < COUNT; ++k) t[k] += seen_s[t[k] + step] <= p[k] ? step : 0;
             }
-            carried += total;
+#pragma unroll
+            for (int k = 0; k < COUNT; ++k) r[k] = rows[from_s[t[k]] + p[k]];
+#pragma unroll
+            for (int k = 0; k < COUNT; ++k) {
+                dig[k] = (int)(r[k] >> tile_bits);
+                row[k] = (t[k] << tile_bits) + (int)(r[k] & ((1u << tile_bits) - 1u));
+            }
+        } else if (packed) {
+            int2 kr[COUNT];
+#pragma unroll
+            for (int k = 0; k < COUNT; ++k) kr[k] = reinterpret_cast<const int2 *>(keys)[(long)start + p[k]];
+#pragma unroll
+            for (int k = 0; k < COUNT; ++k) {
+                dig[k] = kr[k].x - u_lo;
+                row[k] = kr[k].y;
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < COUNT; ++k) {
+                dig[k] = keys[(long)start + p[k]] - u_lo;
+                row[k] = start + p[k];
+            }
         }
-        __syncthreads();
     }
-    const int b = s_pick[0], j = s_pick[1];
+};
+__host__ __device__ __forceinline__ int padded_tiles(int n_tiles) {
+    return n_tiles > 1 ? 2 << (31 - __builtin_clz((unsigned)(n_tiles - 1))) : 1;
+}
+// Fills seen_s / from_s (padded_tiles entries each) for bucket b; the whole workgroup.  All loads are
+// requested before the first is used.
+template <int THREADS>
+__device__ __forceinline__ void find_rows(const unsigned short *__restrict__ offs, int pitch, int n_tiles, int padded,
+                                          int tile_bits, int b, int *seen_s, int *from_s) {
+    constexpr int kMost = (THREADS == 512 ? kTilesMax : 256) / THREADS;  // (256 threads serve up to 2^19 rows)
+    const int per = (padded + THREADS - 1) / THREADS;
+    const int t0 = (int)threadIdx.x * per;
+    int a[kMost], c[kMost], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kMost; ++k) {
+        const bool in = k < per && t0 + k < n_tiles;
+        // both ends of the tile's run in one load (at a short's alignment)
+        typedef unsigned word __attribute__((aligned(2)));
+        const unsigned o = *reinterpret_cast<const word *>(offs + (long)(in ? t0 + k : 0) * pitch + b);
+        a[k] = in ? (int)(o & 0xffffu) : 0;
+        c[k] = in ? (int)(o >> 16) - (int)(o & 0xffffu) : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < kMost; ++k) sum += c[k];
+    int total;
+    int seen = wide_exclusive_scan<THREADS / 64>(sum, &total);
+#pragma unroll
+    for (int k = 0; k < kMost; ++k) {
+        if (k < per && t0 + k < padded) {
+            seen_s[t0 + k] = t0 + k < n_tiles ? seen : 0x7fffffff;
+            from_s[t0 + k] = ((t0 + k) << tile_bits) + a[k] - seen;
+        }
+        seen += c[k];
+    }
+}
+// Arguments the count and the plan kernel share.
+struct BucketArgs {
+    const int *inv;               // ids, in row order
+    const unsigned *rows;         // TILED: the tiles' rows and
+    const unsigned short *offs;   // first rows per bucket
+    const int *pairs;             // otherwise: (id, row) in bucket order
+    const int *bucket_start, *ctl, *num_unq_dev;
+    int *part_hist;
+    int n, U, high_bits, pitch, n_tiles, padded, tile_bits;
+    int more;                     // workgroups for further slices
+    int self_slices;              // buckets of more slices than this are counted by bucket_count_kernel
+};
+
+// Counts, per voxel (low digit) of its bucket, the rows of one slice of a bucket of more than
+// self_slices slices: part_hist[workgroup][*].
+template <int THREADS, bool TILED>
+__global__ __launch_bounds__(THREADS) void bucket_count_kernel(BucketArgs g, const int *__restrict__ stats) {
+    constexpr int kSlice = THREADS * kBktItems;
+    extern __shared__ int lds_count[];  // [padded] seen, [padded] from (TILED), [low_bins] counts
+    __shared__ int s_pick[2];
+    if (TILED && g.ctl[0] == 0) return;
+    if (stats[TXS_STAT_NEED_GENERAL] != 0) return;
+    const int U = voxel_count(g.U, g.num_unq_dev), low_bits = low_bits_of(U, g.high_bits);
+    const int bins = 1 << g.high_bits, low_bins = 1 << low_bits;
+    int b = (int)blockIdx.x - g.more, j = 0;
     if (b < 0) {
-        if (threadIdx.x == 0) wg_pick[blockIdx.x] = make_int4(-1, 0, 0, 0);
-        return;
+        find_slice<THREADS>(g.bucket_start, bins, kSlice, (int)blockIdx.x, s_pick);
+        b = s_pick[0];
+        j = s_pick[1];
+        if (b < 0) return;
     }
-    const int u_lo = b << low_bits;
+    const int s = g.bucket_start[b], cnt_b = g.bucket_start[b + 1] - s;
+    if (low_bits == 0 || slices_of(cnt_b, kSlice) <= g.self_slices) return;  // (uniform)
+    int *seen_s = lds_count, *from_s = lds_count + (TILED ? g.padded : 0), *cnt_s = from_s + (TILED ? g.padded : 0);
+    if (TILED) find_rows<THREADS>(g.offs, g.pitch, g.n_tiles, g.padded, g.tile_bits, b, seen_s, from_s);
+    for (int k = threadIdx.x; k < low_bins; k += THREADS) cnt_s[k] = 0;
+    __syncthreads();
     const bool packed = stats[TXS_STAT_UNSORTED] != 0;
-    const int *keys = packed ? pairs1 : inv;
-    const BucketSlice sl = bucket_slice(bucket_start[b], bucket_start[b + 1], j);
-    if (threadIdx.x == 0) wg_pick[blockIdx.x] = make_int4(b, j, (int)sl.s, (int)sl.e);
-    if (sl.nsl == 1) return;  // (uniform) the next kernel counts the bucket itself
-    for (int k = threadIdx.x; k < low_bins; k += kBktThreads) cnt_s[k] = 0;
-    __syncthreads();
-    int v[kBktItems];
+    const BucketRows<TILED> src{g.rows, packed ? g.pairs : g.inv, packed, seen_s, from_s, g.padded >> 1, g.tile_bits,
+                                b << low_bits, s};
+    const int p0 = j * kSlice + (int)threadIdx.x;
+    int at[kBktItems], dig[kBktItems], row[kBktItems];
 #pragma unroll
-    for (int it = 0; it < kBktItems; ++it) {
-        const long i = sl.my_s + (long)it * kBktThreads + threadIdx.x;
-        v[it] = i < sl.my_e ? kread(keys, i, packed) : -1;
-    }
+    for (int it = 0; it < kBktItems; ++it) at[it] = min(p0 + it * THREADS, cnt_b - 1);
+    src.get(at, dig, row);
 #pragma unroll
-    for (int it = 0; it < kBktItems; ++it) {
-        const int d = v[it] - u_lo;
-        if (v[it] >= 0 && (unsigned)d < (unsigned)low_bins) atomicAdd(&cnt_s[d], 1);
-    }
+    for (int it = 0; it < kBktItems; ++it)
+        if (p0 + it * THREADS < cnt_b && (unsigned)dig[it] < (unsigned)low_bins) atomicAdd(&cnt_s[dig[it]], 1);
     __syncthreads();
-    int *mine = part_hist + (long)blockIdx.x * low_bins;
-    for (int k = threadIdx.x; k < low_bins; k += kBktThreads) mine[k] = cnt_s[k];
+    int *mine = g.part_hist + ((long)(count_row(b, s, kSlice) + j) << low_bits);
+    for (int k = threadIdx.x; k < low_bins; k += THREADS) mine[k] = cnt_s[k];
 }
 
-// One slice: its rows are counted per voxel by LDS atomics, whose returned values put them, voxel
-// by voxel, into LDS in whatever order the atomics ran; each row then finds its place among its
-// voxel's rows of the slice by counting the smaller row numbers there (rows ascend along a bucket,
-// so that is the stable order).  That costs as many reads, four in flight, as the voxel has rows in
-// the slice: runs above kLongRun rows (at most kMaxLongRuns of them in a slice) are ranked by wave
-// ballots on their number instead, with a count per run and 64 rows in input order.  Rows leave in
-// voxel order, neighbouring lanes to neighbouring addresses.
-// What bounds it is the chain of dependent steps inside a workgroup, far more than bytes: 45 KB of
-// LDS keep 24 waves on a compute unit (the ballots on all 11 bits that this replaces needed a count
-// per wave and voxel as well, left 12, and wrote every row as a request of its own).  Then -> now, us:
-// 4M ids of four sweeps (1.3M voxels, 64 MB moved) 131 -> 47, 1M of one 26.2 -> 21.8, of pillars 21.9 ->
-// 22.8, 1M ids of 50 / 25 / 10 rows per voxel 27.5 -> 29.7, 23.7 -> 27.7, 28.2 -> 20.9.
-__global__ __launch_bounds__(kBktThreads) void bucket_plan_kernel(
-    const int *__restrict__ inv, const int *__restrict__ pairs1, long n, int U_arg,
-    int high_bits, int heavy_threshold,
-    const long long *__restrict__ unq_cnts, int *__restrict__ perm, int *__restrict__ seg,
-    int *__restrict__ preSum, int *__restrict__ slot_of, int *__restrict__ heavy_ids,
-    int *__restrict__ stats, const int4 *__restrict__ wg_pick, const int *__restrict__ part_hist,
-    long long *__restrict__ ranks, const int *__restrict__ num_unq_dev, long long *__restrict__ cnts_out) {
-    const int U = voxel_count(U_arg, num_unq_dev), low_bits = low_bits_of(U, high_bits);
+// One slice.  Its rows, in input order (a wave owns neighbouring positions), are ranked among those of
+// their voxel by wave ballots on the low digit and a 16-bit count per wave and voxel; a scan over
+// the counts then gives every voxel's place in the slice, and a bucket of several slices adds what
+// the other slices hold.  The rows pass through LDS so that they leave in voxel order, neighbouring
+// lanes to neighbouring addresses; ranks leave at once.
+// What bounds it is the chain of dependent steps inside a workgroup, about 10 us for a slice (bounds 0.5,
+// runs in the tiles 1.5, rows 2-3, ranking 2-3, scans 1.5, slots 1, places and stores 1.5), far more
+// than bytes: 64 vector registers and 37 KB of LDS keep three or four workgroups of 512 threads on a compute unit.
+// Index preparation in all, us a call with its host read, against rows moved to bucket order first and a
+// voxel's rows ranked by counting the smaller ones: sweeps 200k 72 -> 52, 1M 93 -> 74, 4M 138 -> 123,
+// pillars 1M 95 -> 68, 1M ids of 4 / 50 / 400 rows per voxel 80 -> 62, 93 -> 66, 91 -> 67, 2M of 20,000 Zipf
+// voxels (through the general sequence) 201 -> 186, 2000 ids 78 -> 45; ranks of 1M 80 -> 69.
+template <int THREADS>
+constexpr int plan_stage_ints() { return THREADS * kBktItems + THREADS * kBktItems / 2; }
+struct PlanLds {
+    int counts, first, step, seen, from, tot, front, ints;  // offsets in ints; counts: shared with the staged rows
+};
+template <int THREADS>
+__host__ __device__ __forceinline__ PlanLds plan_lds(int low_bins, int padded) {
+    const int bins = low_bins > 4 ? low_bins : 4, counts = bins / 2 * (THREADS / 64);
+    PlanLds l;
+    l.counts = 0;
+    l.first = counts > plan_stage_ints<THREADS>() ? counts : plan_stage_ints<THREADS>();  // [bins] shorts
+    l.tot = l.first + bins / 2;                                                           // [bins] rows in the other slices
+    l.front = l.tot + bins;                                                               // [bins] ... and of those in front
+    l.step = l.tot;                                                                       // [bins] (in their place, by the thread that read them)
+    l.seen = l.front + bins;
+    l.from = l.seen + padded;
+    l.ints = l.from + padded;
+    return l;
+}
+template <int THREADS, bool TILED>
+__global__ __launch_bounds__(THREADS) void bucket_plan_kernel(
+    BucketArgs g, VoxelArgs v, int *__restrict__ perm, int *__restrict__ seg, int *__restrict__ stats,
+    long long *__restrict__ ranks) {
+    constexpr int kWaves = THREADS / 64, kSlice = THREADS * kBktItems, kWaveRows = 64 * kBktItems;
+    constexpr unsigned kHeavyMark = 0x8000u;  // in a first place (at most kSlice) and a staged digit (11 bits)
+    static_assert(kSlice < (int)kHeavyMark, "first places leave the mark's bit free");
+    extern __shared__ __align__(16) int lds_plan[];
+    __shared__ int s_red[kWaves], s_bad[kWaves], s_pick[2];
     // ranks != NULL: the caller wants the rank of every row inside its voxel and nothing else
     // (ingroup_inds): the placement writes ranks[row] in place of the permutation and the ids
     const bool rank_mode = ranks != nullptr;
-    constexpr int kBins = 1 << kBucketLowBitsMax;
-    // one after the other: the bucket's counts; a long run's rows per 64 rows of the slice; the slice's
-    // rows in voxel order and their voxels (low digits)
-    __shared__ int pool_s[kBktSlice + kBktSlice / 2];
-    __shared__ int first_s[kBins + 1];            // the slice's counts, then the first place of every voxel in row_s
-    __shared__ int step_s[kBins];                 // rows of the voxel in front of this slice, then place -> destination
-    __shared__ unsigned short mark_s[kBins];      // bits 0-7: number of a long run + 1 (0: short); bit 15: heavy voxel
-    __shared__ int s_red[kBktWaves], s_bad[kBktWaves], s_long;
-    static_assert(kBins <= kBktSlice && kMaxLongRuns * 64 * sizeof(short) <= sizeof(pool_s), "what shares a space fits");
-    int *tot = pool_s, *row_s = pool_s;
-    unsigned short *dig_s = reinterpret_cast<unsigned short *>(pool_s + kBktSlice);
-    auto chunk_s = reinterpret_cast<unsigned short(*)[64]>(pool_s);
+    const int bins = 1 << g.high_bits;
+    // (asked for together: each is a trip to memory)
+    int b = (int)blockIdx.x - g.more, j = 0, s = g.bucket_start[max(b, 0)], e = g.bucket_start[max(b, 0) + 1];
+    const bool step_aside = stats[TXS_STAT_NEED_GENERAL] != 0, unsorted = stats[TXS_STAT_UNSORTED] != 0;
+    const int U = voxel_count(g.U, g.num_unq_dev), low_bits = low_bits_of(U, g.high_bits);
+    if (step_aside) return;
     const int low_bins = 1 << low_bits;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const unsigned long long lanes_below = (1ull << lane) - 1ull;
-    if (stats[TXS_STAT_NEED_GENERAL] != 0) return;
-    const int4 pick = wg_pick[blockIdx.x];
-    const int b = pick.x, j = pick.y;
-    if (b < 0) return;
-    const int u_lo = b << low_bits;
-    const int u_hi = min(U, u_lo + low_bins);
-    const bool unsorted = stats[TXS_STAT_UNSORTED] != 0;
-    const BucketSlice sl = bucket_slice(pick.z, pick.w, j);
-    const long s = sl.s, e = sl.e, my_s = sl.my_s, my_e = sl.my_e;
+    if (b < 0) {
+        find_slice<THREADS>(g.bucket_start, bins, kSlice, (int)blockIdx.x, s_pick);
+        b = s_pick[0];
+        j = s_pick[1];
+        if (b < 0) return;
+        s = g.bucket_start[b];
+        e = g.bucket_start[b + 1];
+    }
+    const int u_lo = b << low_bits, u_hi = min(U, u_lo + low_bins);
+    if (u_lo >= U) return;  // (uniform; such a bucket has no rows)
+    const int cnt_b = e - s, nsl = slices_of(cnt_b, kSlice);
+    // what is left per voxel comes from the bucket's first slice (or has been left, where a bucket is a voxel)
+    const bool voxels = j == 0 && low_bits > 0;
+    if (cnt_b == 0 && !voxels) return;
 
-    // Everything the workgroup reads from memory is requested here, in one go: the slice's rows
-    // and the caller's counts of this bucket's voxels (first slice only; compared once the
-    // kernel's own counts are complete).
-    int dig[kBktItems], row[kBktItems];
-#pragma unroll
-    for (int it = 0; it < kBktItems; ++it) {
-        const long i = my_s + (long)it * kBktThreads + threadIdx.x;
-        int v = -1;
-        row[it] = (int)i;
-        if (i < my_e) {
-            if (unsorted) {
-                const int2 kr = reinterpret_cast<const int2 *>(pairs1)[i];
-                v = kr.x;
-                row[it] = kr.y;
-            } else {
-                v = inv[i];
-            }
-        }
-        dig[it] = (i < my_e && (unsigned)(v - u_lo) < (unsigned)low_bins) ? v - u_lo : -1;
+    const PlanLds l = plan_lds<THREADS>(low_bins, TILED ? g.padded : 0);
+    const int quads = max(low_bins, 4) >> 2;
+    uint2 *cnt4 = reinterpret_cast<uint2 *>(lds_plan + l.counts), *first4 = reinterpret_cast<uint2 *>(lds_plan + l.first);
+    int4 *step4 = reinterpret_cast<int4 *>(lds_plan + l.step), *tot4 = reinterpret_cast<int4 *>(lds_plan + l.tot),
+         *front4 = reinterpret_cast<int4 *>(lds_plan + l.front);
+    const unsigned short *first_s = reinterpret_cast<const unsigned short *>(first4);
+    const int *step_s = lds_plan + l.step;
+    int *tot_s = lds_plan + l.tot, *front_s = lds_plan + l.front;
+    int *seen_s = lds_plan + l.seen, *from_s = lds_plan + l.from;
+
+    const int q = threadIdx.x;  // this thread's four voxels: low digits 4 q .. 4 q + 3
+    for (int k = threadIdx.x; k < kWaves * quads; k += THREADS) cnt4[k] = make_uint2(0u, 0u);
+    if (nsl > 1 && q < quads) {
+        tot4[q] = make_int4(0, 0, 0, 0);
+        front4[q] = make_int4(0, 0, 0, 0);
     }
-    constexpr int kCntPer = kBins / kBktThreads;
-    long long given[kCntPer];
-    const bool check_counts = j == 0 && unq_cnts != nullptr;
-    if (check_counts) {
-#pragma unroll
-        for (int k = 0; k < kCntPer; ++k) {
-            const int d = k * kBktThreads + (int)threadIdx.x;
-            given[k] = (d < low_bins && u_lo + d < u_hi) ? unq_cnts[u_lo + d] : -1;
-        }
-    }
-    for (int k = threadIdx.x; k < low_bins; k += kBktThreads) {
-        tot[k] = 0;
-        first_s[k] = 0;
-        step_s[k] = 0;
-    }
-    if (threadIdx.x == 0) s_long = 0;
+    if (TILED && cnt_b > 0) find_rows<THREADS>(g.offs, g.pitch, g.n_tiles, g.padded, g.tile_bits, b, seen_s, from_s);
     __syncthreads();
-    // ---- the slice's rows per voxel; a row's turn among them, for now in any order
-    int turn[kBktItems];
+    const BucketRows<TILED> src{g.rows, unsorted ? g.pairs : g.inv, unsorted, seen_s, from_s, g.padded >> 1, g.tile_bits,
+                                u_lo, s};
+    const int my_s = j * kSlice, my_e = min(cnt_b, my_s + kSlice);  // the slice's positions in the bucket
+    const int w_s = my_s + w * kWaveRows;
+    const unsigned short *wc = reinterpret_cast<const unsigned short *>(cnt4 + w * quads);
+    int dig[kBktItems], row[kBktItems], turn[kBktItems];
+    if (cnt_b > 0) {  // (uniform)
+        int at[kBktItems];
 #pragma unroll
-    for (int it = 0; it < kBktItems; ++it) turn[it] = dig[it] >= 0 ? atomicAdd(&first_s[dig[it]], 1) : 0;
-    // ---- several slices: counts of the bucket's voxels, and of the rows in front of this slice, as
-    // sums over the per-slice counts of the bucket's workgroups (blockIdx.x - j is the bucket's
-    // first), eight loads in flight per thread
-    if (sl.nsl > 1) {
-        const int *first = part_hist + ((long)blockIdx.x - j) * low_bins;
-        const int total = sl.nsl << low_bits;
-        constexpr int kGather = 8;
-        for (int i0 = threadIdx.x; i0 < total; i0 += kBktThreads * kGather) {
+        for (int it = 0; it < kBktItems; ++it) at[it] = min(w_s + it * 64 + lane, cnt_b - 1);
+        src.get(at, dig, row);
+        // ---- rank inside the wave
+#pragma unroll
+        for (int it = 0; it < kBktItems; ++it)
+            if (w_s + it * 64 + lane >= my_e || (unsigned)dig[it] >= (unsigned)low_bins) dig[it] = -1;
+        if (w_s < my_e) wave_rank<kBktItems>(dig, 0, low_bits, reinterpret_cast<unsigned *>(cnt4 + w * quads), turn);  // (uniform in a wave)
+    }
+    // ---- several slices: counts of the bucket's voxels in the other slices, and in those in front
+    if (nsl > 1 && low_bits == 0) {
+        if (threadIdx.x == 0) {
+            tot_s[0] = cnt_b - (my_e - my_s);
+            front_s[0] = my_s;
+        }
+    } else if (nsl > g.self_slices) {
+        // sums over the per-slice counts of the bucket's workgroups, four loads in flight per thread
+        const int total = nsl << low_bits;
+        constexpr int kGather = 4;
+        for (int i0 = threadIdx.x; i0 < total; i0 += THREADS * kGather) {
             int c[kGather];
 #pragma unroll
-            for (int q = 0; q < kGather; ++q) {
-                const int i = i0 + q * kBktThreads;
-                c[q] = i < total ? first[i] : 0;
+            for (int r = 0; r < kGather; ++r) {
+                const int i = min(i0 + r * THREADS, total - 1), k = i >> low_bits;
+                c[r] = g.part_hist[((long)(count_row(b, s, kSlice) + k) << low_bits) + (i & (low_bins - 1))];
             }
 #pragma unroll
-            for (int q = 0; q < kGather; ++q) {
-                const int i = i0 + q * kBktThreads;
-                if (c[q] == 0) continue;
-                const int d = i & (low_bins - 1), k = i >> low_bits;
-                atomicAdd(&tot[d], c[q]);
-                if (k < j) atomicAdd(&step_s[d], c[q]);
+            for (int r = 0; r < kGather; ++r) {
+                const int i = i0 + r * THREADS, d = i & (low_bins - 1), k = i >> low_bits;
+                if (i >= total || c[r] == 0 || k == j) continue;
+                atomicAdd(&tot_s[d], c[r]);
+                if (k < j) atomicAdd(&front_s[d], c[r]);
+            }
+        }
+    } else if (nsl > 1) {
+        // the bucket's other rows once more, four in flight per thread
+        constexpr int kAgain = 4;
+        const int others = cnt_b - (my_e - my_s);
+        for (int i0 = threadIdx.x; i0 < others; i0 += THREADS * kAgain) {
+            int at[kAgain], d[kAgain], ignored_rows[kAgain];
+#pragma unroll
+            for (int r = 0; r < kAgain; ++r) {
+                const int i = min(i0 + r * THREADS, others - 1);
+                at[r] = i < my_s ? i : i + kSlice;
+            }
+            src.get(at, d, ignored_rows);
+#pragma unroll
+            for (int r = 0; r < kAgain; ++r) {
+                if (i0 + r * THREADS >= others || (unsigned)d[r] >= (unsigned)low_bins) continue;
+                atomicAdd(&tot_s[d[r]], 1);
+                if (i0 + r * THREADS < my_s) atomicAdd(&front_s[d[r]], 1);
             }
         }
     }
     __syncthreads();
-    // ---- exclusive scans over the voxels of the bucket, a run of consecutive voxels per thread:
-    // of the slice's counts and (the same where there is one slice) of the bucket's
-    const int per = (low_bins + kBktThreads - 1) / kBktThreads;
-    const int d0 = (int)threadIdx.x * per, d1 = min(d0 + per, low_bins);
-    int mine = 0, mine_all = 0;
-    for (int d = d0; d < d1; ++d) {
-        mine += first_s[d];
-        if (sl.nsl > 1) mine_all += tot[d];
+    // ---- counts per wave -> rows of the waves in front; scans over the voxels of the slice's counts
+    // and (the same where there is one slice) of the bucket's
+    uint2 run = make_uint2(0u, 0u);
+    int4 more = make_int4(0, 0, 0, 0);
+    if (q < quads) {
+#pragma unroll
+        for (int k = 0; k < kWaves; ++k) {
+            const uint2 c = cnt4[k * quads + q];
+            cnt4[k * quads + q] = run;
+            run.x += c.x;
+            run.y += c.y;
+        }
+        if (nsl > 1) more = tot4[q];
     }
+    const int c[4] = {(int)(run.x & 0xffff), (int)(run.x >> 16), (int)(run.y & 0xffff), (int)(run.y >> 16)};
+    const int all[4] = {c[0] + more.x, c[1] + more.y, c[2] + more.z, c[3] + more.w};
     int placed, ignored;
-    int run = wide_exclusive_scan<kBktWaves>(mine, &placed);
-    int run_all = sl.nsl > 1 ? wide_exclusive_scan<kBktWaves>(mine_all, &ignored) : run;
-    for (int d = d0; d < d1; ++d) {
-        const int c = first_s[d];
-        const int c_all = sl.nsl > 1 ? tot[d] : c;
-        if (sl.nsl == 1) tot[d] = c;
-        int mark = c_all > heavy_threshold ? 0x8000 : 0;
-        if (c > kLongRun) mark |= 1 + atomicAdd(&s_long, 1);
-        mark_s[d] = (unsigned short)mark;
-        first_s[d] = run;
-        // ranks count from the voxel's first row, positions from the bucket's start
-        step_s[d] += (rank_mode ? 0 : (int)s + run_all) - run;
-        if (j == 0 && u_lo + d < u_hi) {
-            preSum[u_lo + d] = (int)s + run_all;
-            if (cnts_out) cnts_out[u_lo + d] = (long long)c_all;
-            if (u_lo + d == U - 1) preSum[U] = (int)n;
-        }
-        run += c;
-        run_all += c_all;
-    }
-    if (threadIdx.x == 0) first_s[low_bins] = placed;
-    __syncthreads();
-    // ---- statistics, special voxels and their slots (first slice only; as plan_special_kernel)
-    if (j == 0 && slot_of != nullptr) {
-        int vmax = 0;
-        bool mismatch = false;
-        if (check_counts) {
+    int at = wide_exclusive_scan<kWaves>(c[0] + c[1] + c[2] + c[3], &placed);
+    int at_all = nsl > 1 ? wide_exclusive_scan<kWaves>(all[0] + all[1] + all[2] + all[3], &ignored) : at;
+    {
+        int4 front = make_int4(0, 0, 0, 0);
+        if (nsl > 1 && q < quads) front = front4[q];
+        const int in_front[4] = {front.x, front.y, front.z, front.w};
+        int first[4], step[4];
 #pragma unroll
-            for (int k = 0; k < kCntPer; ++k) {
-                const int d = k * kBktThreads + (int)threadIdx.x;
-                if (d < low_bins && u_lo + d < u_hi) mismatch |= given[k] != (long long)tot[d];
+        for (int k = 0; k < 4; ++k) {
+            const int u = u_lo + 4 * q + k;
+            first[k] = at | (all[k] > v.heavy_threshold ? (int)kHeavyMark : 0);
+            // ranks count from the voxel's first row, positions from the bucket's start
+            step[k] = (rank_mode ? 0 : s + at_all) + in_front[k] - at;
+            if (voxels && 4 * q + k < low_bins && u < u_hi) {
+                v.preSum[u] = s + at_all;
+                if (v.cnts_out) v.cnts_out[u] = (long long)all[k];
+                if (u == U - 1) v.preSum[U] = g.n;
+            }
+            at += c[k];
+            at_all += all[k];
+        }
+        if (q < quads) {
+            first4[q] = make_uint2((unsigned)first[0] | (unsigned)first[1] << 16, (unsigned)first[2] | (unsigned)first[3] << 16);
+            step4[q] = make_int4(step[0], step[1], step[2], step[3]);
+        }
+    }
+    // ---- statistics, special voxels and their slots (first slice only; as plan_special_kernel)
+    const bool slots = voxels && v.slot_of != nullptr;
+    if (slots) {
+        int most = 0;
+        bool mismatch = false;
+        if (w * 256 < low_bins) {  // (uniform in a wave)
+            const int u = u_lo + 4 * q;
+            const bool in = 4 * q < low_bins;
+            long long given[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) given[k] = v.unq_cnts && in && u + k < u_hi ? v.unq_cnts[u + k] : 0;
+            voxel_slots<4>(v, U, u, in ? u_hi : 0, all, stats);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int cnt = in && u + k < u_hi ? all[k] : 0;
+                if (v.unq_cnts) mismatch |= given[k] != (long long)cnt;
+                most = max(most, cnt);
             }
         }
-        for (int dd = 0; dd < low_bins; dd += kBktThreads) {
-            const int d = dd + (int)threadIdx.x;
-            const int u = u_lo + d;
-            const bool in = d < low_bins && u < u_hi;
-            const int cnt = in ? tot[d] : 0;
-            vmax = max(vmax, cnt);
-            const bool heavy = in && cnt > heavy_threshold;
-            const bool empty = in && cnt == 0;
-            const unsigned long long mh = __ballot(heavy), me = __ballot(empty);
-            int base_h = 0, base_e = 0;
-            if (lane == 0) {
-                if (mh) base_h = atomicAdd(&stats[TXS_STAT_NUM_HEAVY], __popcll(mh));
-                if (me) base_e = atomicAdd(&stats[TXS_STAT_NUM_EMPTY], __popcll(me));
-                if (mh | me) atomicAdd(&stats[TXS_STAT_NUM_SPECIAL], __popcll(mh) + __popcll(me));
-            }
-            base_h = __shfl(base_h, 0, 64);
-            base_e = __shfl(base_e, 0, 64);
-            if (in) {
-                int slot = -1;
-                if (heavy) {
-                    slot = base_h + __popcll(mh & lanes_below);
-                    if (slot < U) heavy_ids[slot] = u;
-                } else if (empty) {
-                    slot = U - 1 - (base_e + __popcll(me & lanes_below));
-                    if (slot >= 0) heavy_ids[slot] = u;
-                }
-                slot_of[u] = slot;
-            }
-        }
-        const int wmax = wave_max_i32(vmax);
+        most = wave_max_i32(most);
         const bool any_mismatch = __ballot(mismatch) != 0ull;
         if (lane == 0) {
-            s_red[w] = wmax;
+            s_red[w] = most;
             s_bad[w] = any_mismatch;
         }
-        __syncthreads();  // (also: the last read of tot, whose space the rows take next)
-        if (threadIdx.x == 0) {
-            int m = 0, bad = 0;
-            for (int k = 0; k < kBktWaves; ++k) {
-                m = max(m, s_red[k]);
-                bad |= s_bad[k];
-            }
-            if (m > 0) atomicMax(&stats[TXS_STAT_MAX_CNT], m);
-            if (bad) stats[TXS_STAT_COUNT_MISMATCH] = 1;
-        }
     }
-
-    // what is known of a row once its place p in voxel order is: p's destination
-    auto put = [&](int d, int p, int row_i) {
-        const long dst = (long)step_s[d] + p;
-        if (rank_mode) {
-            if ((unsigned)row_i < (unsigned)n) ranks[row_i] = dst;
-        } else if (unsorted && dst >= s && dst < e) {
-            perm[dst] = row_i;
+    __syncthreads();
+    if (slots && threadIdx.x == 0) {
+        int m = 0, bad = 0;
+        for (int k = 0; k < kWaves; ++k) {
+            m = max(m, s_red[k]);
+            bad |= s_bad[k];
         }
-    };
-    // ---- long runs: straight from the registers, ranked by 64 rows in input order at a time
-    const int n_long = s_long;  // (uniform)
-    if (n_long > 0) {
-        const int id_bits = 32 - __builtin_clz((unsigned)n_long);
-        for (int k = threadIdx.x; k < n_long * 64; k += kBktThreads) (&chunk_s[0][0])[k] = 0;
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < kBktItems; ++it) {
-            const int id = dig[it] >= 0 ? (mark_s[dig[it]] & 255) : 0;
-            const unsigned long long mask = wave_match(id, id_bits, id > 0);
-            const int below = __popcll(mask & lanes_below);
-            if (id > 0) {
-                turn[it] = below;
-                if (below == 0) chunk_s[id - 1][it * kBktWaves + w] = (unsigned short)__popcll(mask);
-            }
-        }
-        __syncthreads();
-        for (int k = w; k < n_long; k += kBktWaves) {
-            const int c = chunk_s[k][lane];
-            chunk_s[k][lane] = (unsigned short)(wave_inclusive_scan(c) - c);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < kBktItems; ++it) {
-            const int id = dig[it] >= 0 ? (mark_s[dig[it]] & 255) : 0;
-            if (id == 0) continue;
-            turn[it] += chunk_s[id - 1][it * kBktWaves + w];
-            put(dig[it], first_s[dig[it]] + turn[it], row[it]);
-        }
-        __syncthreads();  // (the rows take the chunk counts' space)
+        if (m > 0) atomicMax(&stats[TXS_STAT_MAX_CNT], m);
+        if (bad) stats[TXS_STAT_COUNT_MISMATCH] = 1;
     }
-    // ---- short runs: into voxel order, then by the number of smaller rows in the run
+    if (cnt_b == 0) return;  // (uniform)
+    // ---- places
+    int step[kBktItems];
+#pragma unroll
+    for (int it = 0; it < kBktItems; ++it) {
+        const int d = max(dig[it], 0);
+        const unsigned f = first_s[d];
+        step[it] = rank_mode ? step_s[d] : (int)(f & kHeavyMark);
+        turn[it] += (int)(f & (kHeavyMark - 1u)) + (int)wc[d];
+    }
+    if (rank_mode) {
+#pragma unroll
+        for (int it = 0; it < kBktItems; ++it)
+            if (dig[it] >= 0 && (unsigned)row[it] < (unsigned)g.n) ranks[row[it]] = (long long)(step[it] + turn[it]);
+        return;
+    }
+    __syncthreads();  // (the rows take the counts' space)
+    int *row_s = lds_plan + l.counts;
+    unsigned short *dig_s = reinterpret_cast<unsigned short *>(row_s + kSlice);
 #pragma unroll
     for (int it = 0; it < kBktItems; ++it) {
         if (dig[it] < 0) continue;
-        const int p = first_s[dig[it]] + turn[it];
-        row_s[p] = row[it];
-        dig_s[p] = (unsigned short)dig[it];
+        row_s[turn[it]] = row[it];
+        dig_s[turn[it]] = (unsigned short)(dig[it] | step[it]);
     }
     __syncthreads();
-    for (int p = threadIdx.x; p < placed; p += kBktThreads) {
-        const int d = dig_s[p];
-        const int mark = mark_s[d];
-        if (!rank_mode) {
-            const long dst = (long)step_s[d] + p;
-            if (dst >= s && dst < e) seg[dst] = (u_lo + d) | ((mark & 0x8000) ? kSpecialBit : 0);
-        }
-        if ((mark & 255) != 0 || (!rank_mode && !unsorted)) continue;
-        const int a = first_s[d], z = first_s[d + 1], row_i = row_s[p];
-        int smaller = 0;
-        for (int q = a; q < z; q += 4) {
-            int other[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) other[e] = row_s[min(q + e, kBktSlice - 1)];
+    for (int it = 0; it < kBktItems; ++it) {
+        dig[it] = dig_s[it * THREADS + (int)threadIdx.x];  // (what lies behind the last row is not used)
+        row[it] = row_s[it * THREADS + (int)threadIdx.x];
+    }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) smaller += (q + e < z && other[e] < row_i) ? 1 : 0;
-        }
-        put(d, a + smaller, row_i);
+    for (int it = 0; it < kBktItems; ++it) turn[it] = step_s[min(dig[it] & (int)(kHeavyMark - 1u), max(low_bins, 4) - 1)];
+#pragma unroll
+    for (int it = 0; it < kBktItems; ++it) {
+        const int p = it * THREADS + (int)threadIdx.x, dst = turn[it] + p;
+        if (p >= placed || dst < s || dst >= e) continue;
+        seg[dst] = (u_lo + (dig[it] & (int)(kHeavyMark - 1u))) | ((dig[it] & (int)kHeavyMark) ? kSpecialBit : 0);
+        if (unsorted) perm[dst] = row[it];
     }
 }
 
@@ -1052,6 +1423,55 @@ int plan_general(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int
                  const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum,
                  int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, const int *num_unq_dev, long long *cnts_out,
                  void *stream);
+
+// Workspace of the bucket sort, in int32 entries from the (8-byte aligned) start.
+struct PlanLayout {
+    bool tiled;
+    TileSplit split;                     // tiled
+    int high_bits, hist_tiles, slice_threads;
+    int64_t slices_more;                 // an upper bound of the further slices of all buckets
+    int64_t rows, offs;                  // tiled; the (id, row) pairs of the other route start the workspace
+    int64_t hist, scan_ws;               // otherwise
+    int64_t tile_flags, bucket_start, ctl, part_hist, len;
+};
+PlanLayout plan_layout(int64_t n, int bits) {
+    PlanLayout l = {};
+    l.tiled = n <= kTiledRows;
+    // The rows in tile order do not take the place of the pairs: a call that steps aside for an
+    // overfull bucket leaves that untouched.
+    int64_t at = 2 * n;
+    auto take = [&at](int64_t entries) {
+        const int64_t here = at;
+        at += entries;
+        return here;
+    };
+    if (l.tiled) {
+        l.split = tile_split((long)n, bits);
+        l.high_bits = l.split.high_bits;
+        l.rows = take(n);
+        at = (at + 1) & ~(int64_t)1;
+        l.offs = take((int64_t)l.split.tiles * l.split.pitch / 2);
+        l.tile_flags = take(l.split.tiles);
+    } else {
+        // the bucket digit has 9 bits (narrower, and the buckets of a spatially sorted id space get too
+        // uneven; wider, and a tile sends too few rows to a bucket for the scatter to write whole cache
+        // lines) and the low digit takes the rest, at most 11
+        l.high_bits = bits <= kBucketLowBitsMax ? bits : max(kBucketHighBits, bits - kBucketLowBitsMax);
+        l.hist_tiles = (int)((n + kHistThreads * kHistItems - 1) / (kHistThreads * kHistItems));
+        const int64_t hist = ((int64_t)1 << l.high_bits) * l.hist_tiles + 1;
+        l.hist = take(hist);
+        l.scan_ws = take(scan_tiles((long)hist) + 17);
+        l.tile_flags = take(l.hist_tiles);
+    }
+    l.bucket_start = take(((int64_t)1 << l.high_bits) + 1);
+    l.ctl = take(1);
+    const int low_bits = bits - l.high_bits;
+    l.slice_threads = slice_threads_for((long)n, low_bits);
+    l.slices_more = n / (l.slice_threads * kBktItems);
+    l.part_hist = take(low_bits > 0 ? (((int64_t)1 << l.high_bits) + l.slices_more) << low_bits : 0);
+    l.len = at;
+    return l;
+}
 
 }  // namespace
 
@@ -1182,24 +1602,10 @@ int txs_plan_seg_from_presum(const int32_t *preSum, int64_t num_total, int64_t n
 int64_t txs_plan_workspace_len(int64_t num_total, int64_t num_unq) {
     if (!fits_i32(num_total) || !fits_i32(num_unq)) return -1;
     const int64_t general = txs_sort_workspace_len(num_total, num_unq);
-    const int64_t tile = (int64_t)kHistThreads * hist_items_for(num_total);
-    const int64_t tiles = (num_total + tile - 1) / tile;
-    const int64_t bins = (int64_t)1 << kBucketLowBitsMax;
-    // (id, row) pairs after the bucket scatter, the digit-major histogram, tile flags, bucket
-    // boundaries, the scan workspace
-    const int64_t hist = bins * (tiles > 0 ? tiles : 1) + 1;
-    // per-slice voxel counts of the bucket kernels: (slices + buckets) * voxels per bucket, for
-    // the digit split txs_plan_build uses
-    const int ubits = radix_bits(num_unq > 1 ? num_unq : 1);
-    int low_bits = ubits <= kBucketLowBitsMax ? 0 : ubits - kBucketHighBits;
-    if (low_bits > kBucketLowBitsMax) low_bits = kBucketLowBitsMax;
-    int64_t counts = 0;
-    if (low_bits > 0 && ubits <= kBucketBitsMax) {
-        const int64_t groups = num_total / kBktSlice + ((int64_t)1 << (ubits - low_bits));
-        counts = 4 + 4 * groups + groups * ((int64_t)1 << low_bits);
-    }
-    const int64_t bucket = 2 * num_total + hist + tiles + bins + 1 + scan_tiles(hist + 1) + 17 + counts;
-    return general > bucket ? general : bucket;
+    const int bits = radix_bits((int)(num_unq > 1 ? num_unq : 1));
+    if (bits > kBucketBitsMax) return general;
+    const PlanLayout l = plan_layout(num_total, bits);
+    return general > l.len ? general : l.len;
 }
 
 int txs_plan_build_general(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
@@ -1258,7 +1664,7 @@ int plan_general(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int
 // whether they apply to the extents (otherwise it ranks from the plan this call leaves).
 bool txs_detail::plan_writes_ranks(long num_total, long num_unq) {
     const int bits = radix_bits(num_unq > 1 ? num_unq : 1);
-    return num_total > 0 && num_unq > 0 && bits <= kBucketBitsMax && bits > kBucketLowBitsMax;
+    return num_total > 0 && num_unq > 0 && bits <= kBucketBitsMax;
 }
 
 int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
@@ -1288,81 +1694,101 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
         return plan_general(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum, slot_of,
                             heavy_ids, stats, num_unq_dev, cnts_out, stream);
     }
-    // ids of up to 11 bits are sorted by the bucket pass alone; beyond that the bucket digit has
-    // 9 bits (narrower, and the buckets of a spatially sorted id space get too uneven: every
-    // workgroup of a crowded bucket adds up the counts of all its slices, and above kBktGiant rows the
-    // plan is left to the general sequence; wider, and a tile sends too few rows to a bucket for
-    // the scatter to write whole cache lines) and the low digit takes the rest, at most 11
-    const int low_bits = bits <= kBucketLowBitsMax ? 0 : min(bits - kBucketHighBits, kBucketLowBitsMax);
-    const int high_bits = bits - low_bits;
-    const int high_bins = 1 << high_bits;
-    const int items = hist_items_for(n);
-    const long tile = (long)kHistThreads * items;
-    const int n_tiles = (int)((n + tile - 1) / tile);
-    int *pairs1 = plan_ws;  // (id, row) after the bucket scatter, 8-byte aligned
-    int *hist = plan_ws + 2 * n;
-    const long used = (long)high_bins * n_tiles;
-    int *tile_flags = hist + used + 1;
-    int *bucket_start = tile_flags + n_tiles;
-    int *scan_ws = bucket_start + high_bins + 1;
-    // an upper bound of the (bucket, slice) pairs; workgroups beyond the last pair return at once
-    const long groups = n / kBktSlice + high_bins;
-    int *wg_pick = reinterpret_cast<int *>(  // 16-byte records
-        ((uintptr_t)(scan_ws + scan_tiles(used + 1) + 17) + 15u) & ~(uintptr_t)15u);
-    int *part_hist = wg_pick + 4 * groups;
     // (the attribute belongs to the current device's copy of a kernel: once per device)
     constexpr int kMaxDevices = 64;
     static std::atomic<bool> lds_allowed[kMaxDevices];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return TXS_ERR_LAUNCH;
     if (!lds_allowed[dev].load(std::memory_order_acquire)) {
-        for (const void *k : {reinterpret_cast<const void *>(bucket_scatter_kernel<4>),
-                              reinterpret_cast<const void *>(bucket_scatter_kernel<8>),
-                              reinterpret_cast<const void *>(bucket_scatter_kernel<16>)})
+        for (const void *k : {reinterpret_cast<const void *>(bucket_scatter_kernel),
+                              reinterpret_cast<const void *>(bucket_plan_kernel<512, true>)})
             if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024) != hipSuccess)
                 return TXS_ERR_LAUNCH;
         lds_allowed[dev].store(true, std::memory_order_release);
     }
-    auto hist32 = items == 16 ? bucket_hist_kernel<16, int>
-                              : (items == 8 ? bucket_hist_kernel<8, int> : bucket_hist_kernel<4, int>);
-    auto hist64 = items == 16 ? bucket_hist_kernel<16, long long>
-                              : (items == 8 ? bucket_hist_kernel<8, long long> : bucket_hist_kernel<4, long long>);
-    auto scatter_kernel =
-        items == 16 ? bucket_scatter_kernel<16> : (items == 8 ? bucket_scatter_kernel<8> : bucket_scatter_kernel<4>);
-    if (ids64)
-        hist64<<<dim3(n_tiles), dim3(kHistThreads), 0, st>>>(ids64, n, U, high_bits, hist, tile_flags, n_tiles, ids32,
-                                                             num_unq_dev);
-    else
-        hist32<<<dim3(n_tiles), dim3(kHistThreads), 0, st>>>(unq_inv, n, U, high_bits, hist, tile_flags, n_tiles, nullptr,
-                                                             num_unq_dev);
-    // one entry more than the histogram: it receives the total, the end of the last bucket.  A
-    // bucket's first entry (that of tile 0) is where it starts.
-    if (exclusive_scan(hist, used, hist, used + 1, scan_ws, st, bucket_start, n_tiles) != hipSuccess) return TXS_ERR_LAUNCH;
-    const size_t lds_scatter = (size_t)high_bins * sizeof(int) +
-                               max((size_t)kHistWaves * high_bins * sizeof(int), (size_t)tile * sizeof(int2));
-    if (low_bits == 0) {
-        // a bucket is a voxel: the scatter already gives the final order
-        scatter_kernel<<<dim3(n_tiles), dim3(kHistThreads), lds_scatter, st>>>(
-            unq_inv, n, U, high_bits, hist, tile_flags, n_tiles, bucket_start, stats, seg, perm, nullptr, num_unq_dev);
-        int rc = txs_plan_presum(seg, n, U, preSum, stream);
-        if (slot_of == nullptr) return rc;
-        if (rc == TXS_OK)
-            rc = txs_plan_special(preSum, U, heavy_threshold, unq_cnts, slot_of, heavy_ids, stats, num_unq_dev,
-                                  (int64_t *)cnts_out, stream);
-        if (rc == TXS_OK) rc = txs_plan_seg_flag(seg, n, U, slot_of, stream);
-        return rc;
+    const PlanLayout l = plan_layout(n, bits);
+    const int low_most = bits - l.high_bits;  // (of the voxels there are at most; the kernels know their number)
+    int *bucket_start = plan_ws + l.bucket_start;
+    const int threads = l.slice_threads;
+    BucketArgs g = {};
+    g.inv = unq_inv;
+    g.bucket_start = bucket_start;
+    g.ctl = plan_ws + l.ctl;
+    g.num_unq_dev = num_unq_dev;
+    g.part_hist = plan_ws + l.part_hist;
+    g.n = (int)n;
+    g.U = U;
+    g.high_bits = l.high_bits;
+    g.more = (int)l.slices_more;
+    const VoxelArgs voxels = {heavy_threshold, (const long long *)unq_cnts, preSum, slot_of, heavy_ids, cnts_out};
+    if (l.tiled) {
+        auto rows = reinterpret_cast<unsigned *>(plan_ws + l.rows);
+        auto offs = reinterpret_cast<unsigned short *>(plan_ws + l.offs);
+        int *tile_flags = plan_ws + l.tile_flags, *ctl = plan_ws + l.ctl;
+        const TileSplit &t = l.split;
+        const int tile_threads = t.tile_bits == 10 ? 256 : 512;
+        const size_t bins = (size_t)t.pitch - 4;
+        const size_t lds = 2 * bins + max(2 * bins * (tile_threads / 64), sizeof(int) << t.tile_bits);
+        auto sort_tiles = [&](auto ids) {
+            using K = std::remove_const_t<std::remove_pointer_t<decltype(ids)>>;
+            auto kernel = t.tile_bits == 10   ? tile_sort_kernel<256, 4, K>
+                          : t.tile_bits == 11 ? tile_sort_kernel<512, 4, K>
+                          : t.tile_bits == 12 ? tile_sort_kernel<512, 8, K>
+                                              : tile_sort_kernel<512, 16, K>;
+            kernel<<<dim3(t.tiles), dim3(tile_threads), lds, st>>>(ids, n, U, t.high_bits, rows, offs, t.pitch, tile_flags,
+                                                                   ids32, stats, ctl, num_unq_dev);
+        };
+        if (ids64) sort_tiles(ids64); else sort_tiles(unq_inv);
+        bucket_start_kernel<<<dim3(((1 << t.high_bits) + kStartOwned) / kStartOwned), dim3(kStartThreads), 0, st>>>(
+            offs, t.pitch, t.tiles, (int)n, U, t.high_bits, (threads == 512 ? 1 : kSelfSlices) * threads * kBktItems, tile_flags, bucket_start, stats, ctl, num_unq_dev,
+            voxels);
+        g.rows = rows;
+        g.offs = offs;
+        g.pitch = t.pitch;
+        g.n_tiles = t.tiles;
+        g.padded = padded_tiles(t.tiles);
+        g.tile_bits = t.tile_bits;
+        g.self_slices = threads == 512 ? 1 : kSelfSlices;
+    } else {
+        const int high_bins = 1 << l.high_bits;
+        int *hist = plan_ws + l.hist, *tile_flags = plan_ws + l.tile_flags, *scan_ws = plan_ws + l.scan_ws;
+        const long used = (long)high_bins * l.hist_tiles;
+        if (ids64)
+            bucket_hist_kernel<long long><<<dim3(l.hist_tiles), dim3(kHistThreads), 0, st>>>(
+                ids64, n, U, l.high_bits, hist, tile_flags, l.hist_tiles, ids32, num_unq_dev);
+        else
+            bucket_hist_kernel<int><<<dim3(l.hist_tiles), dim3(kHistThreads), 0, st>>>(
+                unq_inv, n, U, l.high_bits, hist, tile_flags, l.hist_tiles, nullptr, num_unq_dev);
+        // one entry more than the histogram: it receives the total, the end of the last bucket.  A
+        // bucket's first entry (that of tile 0) is where it starts.
+        if (exclusive_scan(hist, used, hist, used + 1, scan_ws, st, bucket_start, l.hist_tiles) != hipSuccess)
+            return TXS_ERR_LAUNCH;
+        const size_t lds = (size_t)high_bins * sizeof(int) + max((size_t)kHistWaves * high_bins * sizeof(int),
+                                                                 (size_t)kHistThreads * kHistItems * sizeof(int2));
+        bucket_scatter_kernel<<<dim3(l.hist_tiles), dim3(kHistThreads), lds, st>>>(
+            unq_inv, n, U, l.high_bits, hist, tile_flags, l.hist_tiles, bucket_start, stats,
+            reinterpret_cast<int2 *>(plan_ws), num_unq_dev);
+        // (a bucket is a voxel where there are at most 2^11 of them, which the host may not know)
+        if (bits <= kBucketLowBitsMax || num_unq_dev)
+            bucket_voxels_kernel<<<dim3((high_bins + 63) / 64), dim3(64), 0, st>>>(bucket_start, (int)n, U, l.high_bits,
+                                                                                  stats, num_unq_dev, voxels);
+        g.pairs = plan_ws;
+        g.self_slices = 1;
     }
-    // a bucket so full that its workgroups would run long after all others have finished
-    // (only a few voxels holding most of the rows do that) sends the call to the general sequence
-    scatter_kernel<<<dim3(n_tiles), dim3(kHistThreads), lds_scatter, st>>>(
-        unq_inv, n, U, high_bits, hist, tile_flags, n_tiles, bucket_start, stats, nullptr, nullptr,
-        reinterpret_cast<int2 *>(pairs1), num_unq_dev);
-    const int low_bins = 1 << low_bits;
-    bucket_count_kernel<<<dim3((unsigned)groups), dim3(kBktThreads), (size_t)low_bins * sizeof(int), st>>>(
-        unq_inv, pairs1, n, U, high_bits, bucket_start, stats, reinterpret_cast<int4 *>(wg_pick), part_hist, num_unq_dev);
-    bucket_plan_kernel<<<dim3((unsigned)groups), dim3(kBktThreads), 0, st>>>(
-        unq_inv, pairs1, n, U, high_bits, heavy_threshold,
-        (const long long *)unq_cnts, perm, seg, preSum, slot_of, heavy_ids, stats,
-        reinterpret_cast<const int4 *>(wg_pick), part_hist, ranks, num_unq_dev, cnts_out);
+    // A bucket so full that its workgroups would run long after all others have finished (only a few
+    // voxels holding most of the rows do that) sends the call to the general sequence.
+    const int low_bins = 1 << low_most, tiles = l.tiled ? g.padded : 0;
+    const dim3 grid((unsigned)(((int64_t)1 << l.high_bits) + l.slices_more));
+    const size_t lds_count = sizeof(int) * (size_t)(low_bins + 2 * tiles);
+    auto place = [&](auto count_kernel, auto plan_kernel, size_t lds) {
+        if (low_most > 0) count_kernel<<<grid, dim3(threads), lds_count, st>>>(g, stats);
+        plan_kernel<<<grid, dim3(threads), lds, st>>>(g, voxels, perm, seg, stats, ranks);
+    };
+    if (!l.tiled)
+        place(bucket_count_kernel<512, false>, bucket_plan_kernel<512, false>, sizeof(int) * plan_lds<512>(low_bins, 0).ints);
+    else if (threads == 512)
+        place(bucket_count_kernel<512, true>, bucket_plan_kernel<512, true>, sizeof(int) * plan_lds<512>(low_bins, tiles).ints);
+    else
+        place(bucket_count_kernel<256, true>, bucket_plan_kernel<256, true>, sizeof(int) * plan_lds<256>(low_bins, tiles).ints);
     return status_of(hipGetLastError());
 }
