@@ -12,10 +12,12 @@
 // torchex/src/utils/functions.cuh:30-64).
 
 #include "txs_common.h"
+#include "txs_internal.h"
 
 namespace {
 
 using txs_detail::exclusive_scan;
+using txs_detail::KeyMap;
 using txs_detail::scan_tiles;
 
 __global__ void fill_i32_kernel(int *p, long n, int value) {
@@ -44,10 +46,11 @@ __device__ __forceinline__ float div_floor_f32(float a, float b) {
 
 // coors = floor((p - lo) / voxel) per axis, key = (x * Y + y) * Z + z
 // (test/test_incremental_mask.py:20-26, operator_py/incremental_points.py:18-19)
+// flag: set to 1 if a point lies outside the grid; map (may be NULL): the keys' occupancy map, marked
 __global__ void voxel_keys_kernel(const float *__restrict__ pts, long n, int stride, float lo0,
                                   float lo1, float lo2, float v0, float v1, float v2, int d0, int d1,
                                   int d2, int *__restrict__ coors, int *__restrict__ keys,
-                                  int *__restrict__ stats) {
+                                  int *__restrict__ flag, unsigned char *__restrict__ map) {
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float *p = pts + i * stride;
@@ -60,8 +63,10 @@ __global__ void voxel_keys_kernel(const float *__restrict__ pts, long n, int str
         coors[i * 3 + 2] = z;
     }
     const bool ok = (unsigned)x < (unsigned)d0 && (unsigned)y < (unsigned)d1 && (unsigned)z < (unsigned)d2;
-    if (!ok) stats[TXS_STAT_OUT_OF_RANGE] = 1;
-    keys[i] = ok ? (x * d1 + y) * d2 + z : 0;
+    const int key = ok ? (x * d1 + y) * d2 + z : 0;
+    if (!ok) flag[0] = 1;
+    keys[i] = key;
+    if (map) map[key] = 1;
 }
 
 // 1 where a new run of equal keys starts
@@ -142,70 +147,78 @@ __global__ void bytemap_mark_kernel(Keys keys, long n, long key_bound, unsigned 
     map[k] = 1;
 }
 
-// 32 map bytes (each 0 or 1) -> one bitmap word and its population count, and the sums of the
-// counts over the tiles of the scan that follows (a workgroup per tile)
+// 32 map bytes (each 0 or 1) -> one cell of the map: their bits, and how many keys occur in the cells in
+// front of it in its tile of kScanTileItems; the number of keys per tile (a workgroup each).  What is in
+// front of a tile is added up by those who read the cells: a few hundred numbers, against a scan over
+// all cells (5 us of a frame's 16.9M keys, in a launch of its own).
 constexpr int kPackThreads = 1024;
 __global__ __launch_bounds__(kPackThreads) void bytemap_pack_kernel(const uint4 *__restrict__ map16, long words,
-                                                                    unsigned *__restrict__ bm, int *__restrict__ cnt,
-                                                                    int *__restrict__ tile_sums) {
+                                                                    uint2 *__restrict__ cells, int *__restrict__ tiles) {
     constexpr int kItems = txs_detail::kScanTileItems / kPackThreads;
     __shared__ int s_sum[kPackThreads / 64];
     // bytes b0..b3 of a word, each 0 or 1 -> bits 0..3: (x * 0x10204080) >> 28 leaves b0 + 2 b1 + 4 b2 + 8 b3
     auto nib = [](unsigned x) -> unsigned { return ((x * 0x10204080u) >> 28) & 15u; };
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const long w0 = (long)blockIdx.x * txs_detail::kScanTileItems + (long)threadIdx.x * kItems;
+    uint4 lo[kItems], hi[kItems];
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+        const bool in = w0 + it < words;
+        lo[it] = in ? map16[2 * (w0 + it)] : make_uint4(0u, 0u, 0u, 0u);
+        hi[it] = in ? map16[2 * (w0 + it) + 1] : make_uint4(0u, 0u, 0u, 0u);
+    }
+    unsigned word[kItems];
     int sum = 0;
 #pragma unroll
     for (int it = 0; it < kItems; ++it) {
-        const long w = (long)blockIdx.x * txs_detail::kScanTileItems + it * kPackThreads + threadIdx.x;
-        if (w >= words) continue;
-        const uint4 lo = map16[2 * w], hi = map16[2 * w + 1];
-        const unsigned word = nib(lo.x) | (nib(lo.y) << 4) | (nib(lo.z) << 8) | (nib(lo.w) << 12) | (nib(hi.x) << 16) |
-                              (nib(hi.y) << 20) | (nib(hi.z) << 24) | (nib(hi.w) << 28);
-        bm[w] = word;
-        const int c = __popc(word);
-        cnt[w] = c;
-        sum += c;
+        word[it] = nib(lo[it].x) | (nib(lo[it].y) << 4) | (nib(lo[it].z) << 8) | (nib(lo[it].w) << 12) |
+                   (nib(hi[it].x) << 16) | (nib(hi[it].y) << 20) | (nib(hi[it].z) << 24) | (nib(hi[it].w) << 28);
+        sum += __popc(word[it]);
     }
-    sum = wave_inclusive_scan(sum);
-    if ((threadIdx.x & 63) == 63) s_sum[threadIdx.x >> 6] = sum;
+    const int inc = wave_inclusive_scan(sum);
+    if (lane == 63) s_sum[wave] = inc;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
-        for (int k = 0; k < kPackThreads / 64; ++k) t += s_sum[k];
-        tile_sums[blockIdx.x] = t;
+    int at = inc - sum, total = 0;
+#pragma unroll
+    for (int k = 0; k < kPackThreads / 64; ++k) {
+        if (k < wave) at += s_sum[k];
+        total += s_sum[k];
     }
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+        if (w0 + it < words) cells[w0 + it] = make_uint2(word[it], (unsigned)at);
+        at += __popc(word[it]);
+    }
+    if (threadIdx.x == 0) tiles[blockIdx.x] = total;
 }
 
-// base: exclusive scan of the population counts, words + 1 entries (the last is the total)
-__global__ void bitmap_total_kernel(const int *__restrict__ base, long words, int *__restrict__ stats) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) stats[TXS_STAT_NUM_UNQ] = base[words];
+// the number of distinct keys, by one workgroup
+__global__ __launch_bounds__(kThreads) void map_total_kernel(KeyMap m) {
+    __shared__ int base_s[txs_detail::kMapTilesSummed];
+    const int total = map_tile_bases<kThreads>(m, base_s);
+    if (threadIdx.x == 0) m.num_unq[0] = total;
 }
 
-template <typename K>
-__global__ void bitmap_assign_kernel(const K *__restrict__ keys, long n, long key_bound,
-                                     const unsigned *__restrict__ bm, const int *__restrict__ base,
-                                     long words, int *__restrict__ inv, int *__restrict__ unq_keys,
-                                     const int *__restrict__ bad, int *__restrict__ found) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (found && i == 0) {  // the number of distinct keys, and whether one lies outside the bound
-        found[0] = base[words];
-        found[1] = bad[0];
-    }
-    if (i < n) {
-        const long k = (long)keys[i];
-        int id = 0;
-        if (k >= 0 && k < key_bound) id = base[k >> 5] + __popc(bm[k >> 5] & ((1u << (k & 31)) - 1u));
-        inv[i] = id;
-    }
-    if (i < words) {
-        unsigned m = bm[i];
-        int r = base[i];
-        while (m) {
-            const int b = __builtin_ctz(m);
-            if (r < n) unq_keys[r] = (int)(i * 32 + b);
-            ++r;
-            m &= m - 1u;
+// Ids of all keys, and the distinct keys: workgroups behind those of the rows list a part of the cells each.
+__global__ __launch_bounds__(kThreads) void map_assign_kernel(KeyMap m, long n, int *__restrict__ inv) {
+    __shared__ int base_s[txs_detail::kMapTilesSummed];
+    const int total = map_tile_bases<kThreads>(m, base_s);
+    if (m.num_unq && blockIdx.x == 0 && threadIdx.x == 0) {
+        m.num_unq[0] = total;
+        if (m.found) {
+            m.found[0] = total;
+            m.found[1] = m.bad[0];
         }
     }
+    const long row_groups = (n + kThreads - 1) / kThreads;
+    if ((long)blockIdx.x >= row_groups) {
+        map_list_part<kThreads>(m, base_s, (long)blockIdx.x - row_groups);
+        return;
+    }
+    const long i = (long)blockIdx.x * kThreads + threadIdx.x;
+    if (i >= n) return;
+    const int key = map_key(m, i);
+    inv[i] = map_id(m, base_s, m.cells[key >> 5], key);
 }
 
 // counts of the voxels from their CSR offsets, as int64 (what torch.unique returns)
@@ -569,18 +582,14 @@ __global__ __launch_bounds__(kThreads) void coor_max_kernel(const K *__restrict_
     }
 }
 
-// the distinct keys in ascending order (from the bitmap), and the table's slots emptied
-__global__ void grid_hash_prepare_kernel(const unsigned *__restrict__ bm, const int *__restrict__ base, long words,
-                                         int num_unq, int *__restrict__ unq_keys,
-                                         unsigned long long *__restrict__ table, long table_size) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < table_size) table[i] = ~0ull;
-    if (i >= words) return;
-    unsigned m = bm[i];
-    for (int r = base[i]; m && r < num_unq; ++r) {
-        unq_keys[r] = (int)(i * 32 + __builtin_ctz(m));
-        m &= m - 1u;
-    }
+// the distinct keys in ascending order (a workgroup per part of the cells), and the table's slots emptied
+__global__ __launch_bounds__(kThreads) void grid_hash_prepare_kernel(KeyMap m, unsigned long long *__restrict__ table,
+                                                                     long table_size) {
+    __shared__ int base_s[txs_detail::kMapTilesSummed];
+    map_tile_bases<kThreads>(m, base_s);
+    for (long i = (long)blockIdx.x * kThreads + threadIdx.x; i < table_size; i += (long)gridDim.x * kThreads)
+        table[i] = ~0ull;
+    map_list_part<kThreads>(m, base_s, (long)blockIdx.x);
 }
 
 // Occupied slots: a byte per slot, and the occupied ones' (key, value) words in slot order.  Two
@@ -635,39 +644,118 @@ __global__ __launch_bounds__(kThreads) void grid_hash_compact_kernel(const unsig
         }
 }
 
-// byte map -> bitmap -> scanned population counts of one set of keys.  Layout of the workspace:
-// byte map (8 ints per word), bitmap, scanned counts (words + 1: the last is the number of distinct
-// keys), a flag for a key outside the bound (used where the caller has no other), scan workspace.
+// byte map -> cells of one set of keys.  Layout of the workspace: byte map (8 ints per cell), cells (2),
+// the number of distinct keys, a flag for a key outside the bound (used where the caller has no other),
+// keys per tile and their scan.
 struct BitmapWs {
     long words;
     uint4 *map16;
-    unsigned *bm;
-    int *base, *bad, *scan_ws;
+    uint2 *cells;
+    int *total, *bad, *tiles;
 };
 BitmapWs bitmap_ws_of(const int32_t *ws_in, int64_t key_bound) {
     int32_t *ws = const_cast<int32_t *>(ws_in);
     BitmapWs r;
     r.words = (long)((key_bound + 31) / 32);
     r.map16 = reinterpret_cast<uint4 *>(ws);
-    r.bm = reinterpret_cast<unsigned *>(ws + 8 * r.words);
-    r.base = ws + 9 * r.words;
-    r.bad = r.base + r.words + 1;
-    r.scan_ws = r.bad + 1;
+    r.cells = reinterpret_cast<uint2 *>(ws + 8 * r.words);
+    r.total = ws + 10 * r.words;
+    r.bad = r.total + 1;
+    r.tiles = r.bad + 1;
     return r;
 }
-template <class Keys>
-int bitmap_count(Keys keys, long n, int64_t key_bound, const BitmapWs &b, int *clear_flag, int *bad, hipStream_t st) {
+// how the kernels above read a finished map
+KeyMap key_map(const BitmapWs &b, const void *keys, int keys64, int64_t key_bound, const int *bad, int *unq_keys, int64_t most) {
+    KeyMap m = {};
+    m.keys = keys;
+    m.keys64 = keys64;
+    m.key_bound = (long)key_bound;
+    m.cells = b.cells;
+    m.tiles = b.tiles;
+    m.n_tiles = (int)scan_tiles(b.words);
+    m.scanned = m.n_tiles > txs_detail::kMapTilesSummed;
+    m.words = b.words;
+    m.bad = bad;
+    m.unq_keys = unq_keys;
+    m.most = (long)most;
+    m.num_unq = b.total;
+    return m;
+}
+int64_t most_keys(int64_t n, int64_t key_bound) { return n < key_bound ? n : key_bound; }
+// the map, cleared; marked by `mark()`; packed
+template <class Mark>
+int bitmap_make(const BitmapWs &b, int *clear_flag, hipStream_t st, Mark mark) {
     bytemap_clear_kernel<<<dim3(blocks_for(2 * b.words)), dim3(kThreads), 0, st>>>(b.map16, 2 * b.words, clear_flag);
-    bytemap_mark_kernel<Keys><<<dim3(blocks_for(n)), dim3(kThreads), 0, st>>>(
-        keys, n, (long)key_bound, reinterpret_cast<unsigned char *>(b.map16), bad);
-    bytemap_pack_kernel<<<dim3((unsigned)scan_tiles(b.words + 1)), dim3(kPackThreads), 0, st>>>(b.map16, b.words, b.bm,
-                                                                                               b.base, b.scan_ws);
-    if (txs_detail::scan_from_tile_sums(b.base, b.words, b.base, b.words + 1, b.scan_ws, st) != hipSuccess)
+    mark();
+    const long tiles = scan_tiles(b.words);
+    bytemap_pack_kernel<<<dim3((unsigned)tiles), dim3(kPackThreads), 0, st>>>(b.map16, b.words, b.cells, b.tiles);
+    if (tiles > txs_detail::kMapTilesSummed &&
+        exclusive_scan(b.tiles, tiles, b.tiles, tiles + 1, b.tiles + tiles + 1, st) != hipSuccess)
         return TXS_ERR_LAUNCH;
     return status_of(hipGetLastError());
 }
+template <class Keys>
+int bitmap_count(Keys keys, long n, int64_t key_bound, const BitmapWs &b, int *clear_flag, int *bad, hipStream_t st) {
+    return bitmap_make(b, clear_flag, st, [&]() {
+        bytemap_mark_kernel<Keys><<<dim3(blocks_for(n)), dim3(kThreads), 0, st>>>(
+            keys, n, (long)key_bound, reinterpret_cast<unsigned char *>(b.map16), bad);
+    });
+}
 
 }  // namespace
+
+int txs_detail::unique_map_keys(const void *keys, int key_is_int64, int64_t num_total, int64_t key_bound,
+                                int32_t *key_flag, int32_t *bitmap_ws, void *stream) {
+    if (!fits_i32(num_total) || num_total == 0 || key_bound <= 0 || key_bound > (1LL << 31)) return TXS_ERR_INVALID_ARG;
+    if (!keys || !bitmap_ws || ((uintptr_t)bitmap_ws & 15u) != 0) return TXS_ERR_INVALID_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
+    int *bad = key_flag ? key_flag : b.bad, *clear_flag = key_flag ? nullptr : b.bad;
+    return key_is_int64 ? bitmap_count(FlatKeys<long long>{static_cast<const long long *>(keys)}, num_total, key_bound, b,
+                                       clear_flag, bad, st)
+                        : bitmap_count(FlatKeys<int>{static_cast<const int *>(keys)}, num_total, key_bound, b, clear_flag,
+                                       bad, st);
+}
+
+int txs_detail::unique_map_points(const float *points, int64_t num_total, int64_t point_stride, const float *range_lo,
+                                  const float *voxel_size, const int32_t *dims, int32_t *coors, int32_t *keys,
+                                  int32_t *bitmap_ws, void *stream) {
+    if (!fits_i32(num_total) || num_total == 0 || point_stride < 3 || !points || !range_lo || !voxel_size || !dims ||
+        !coors || !keys || !bitmap_ws || ((uintptr_t)bitmap_ws & 15u) != 0)
+        return TXS_ERR_INVALID_ARG;
+    int64_t key_bound = 1;
+    for (int a = 0; a < 3; ++a) {
+        if (dims[a] <= 0 || dims[a] > 2147483647LL / key_bound) return TXS_ERR_INVALID_ARG;
+        key_bound *= dims[a];
+    }
+    hipStream_t st = (hipStream_t)stream;
+    const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
+    return bitmap_make(b, b.bad, st, [&]() {
+        voxel_keys_kernel<<<dim3(blocks_for(num_total)), dim3(kThreads), 0, st>>>(
+            points, num_total, (int)point_stride, range_lo[0], range_lo[1], range_lo[2], voxel_size[0], voxel_size[1],
+            voxel_size[2], dims[0], dims[1], dims[2], coors, keys, b.bad, reinterpret_cast<unsigned char *>(b.map16));
+    });
+}
+
+int txs_detail::unique_plan_of_map(const void *keys, int key_is_int64, int64_t num_total, int64_t key_bound,
+                                   const int32_t *key_flag, int32_t *bitmap_ws, int32_t heavy_threshold,
+                                   int32_t *plan_ws, int32_t *unq_inv, int32_t *unq_keys, int64_t *unq_cnts,
+                                   int32_t *perm, int32_t *seg, int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids,
+                                   int32_t *stats, void *stream) {
+    if (!unq_inv || !unq_keys || !unq_cnts || !slot_of || !heavy_ids || !stats) return TXS_ERR_INVALID_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
+    const int64_t most = most_keys(num_total, key_bound);
+    KeyMap m = key_map(b, keys, key_is_int64, key_bound, key_flag ? key_flag : b.bad, unq_keys, most);
+    m.found = stats + TXS_STATS_LEN;
+    const bool fused = txs_detail::plan_takes_map(num_total, most);
+    if (!fused)
+        map_assign_kernel<<<dim3(blocks_for(num_total) + (unsigned)map_parts(m)), dim3(kThreads), 0, st>>>(m, num_total,
+                                                                                                       unq_inv);
+    return txs_detail::plan_build(unq_inv, num_total, most, heavy_threshold, nullptr, plan_ws, perm, seg, preSum,
+                                  slot_of, heavy_ids, stats, nullptr, m.num_unq, (long long *)unq_cnts, nullptr,
+                                  fused ? &m : nullptr, stream);
+}
 
 extern "C" {
 
@@ -682,15 +770,16 @@ int txs_voxel_keys(const float *points, int64_t num_total, int64_t point_stride,
     if (!points || !keys) return TXS_ERR_INVALID_ARG;
     voxel_keys_kernel<<<dim3(blocks_for(num_total)), dim3(kThreads), 0, (hipStream_t)stream>>>(
         points, num_total, (int)point_stride, range_lo[0], range_lo[1], range_lo[2], voxel_size[0],
-        voxel_size[1], voxel_size[2], dims[0], dims[1], dims[2], coors, keys, stats);
+        voxel_size[1], voxel_size[2], dims[0], dims[1], dims[2], coors, keys, stats + TXS_STAT_OUT_OF_RANGE, nullptr);
     return status_of(hipGetLastError());
 }
 
 int64_t txs_unique_bitmap_workspace_len(int64_t key_bound) {
     if (key_bound <= 0 || key_bound > (1LL << 31)) return -1;
     const int64_t words = (key_bound + 31) / 32;
-    // byte map (32 bytes per word), bitmap, scanned counts, range flag, scan workspace
-    return 8 * words + words + (words + 1) + 1 + scan_tiles(words + 1) + 17;
+    // byte map (32 bytes per cell), cells, their number, range flag, keys per tile, scan workspace
+    const int64_t tiles = scan_tiles(words);
+    return 8 * words + 2 * words + 2 + tiles + 1 + scan_tiles(tiles + 1);
 }
 
 int txs_unique_bitmap_count(const void *keys, int key_is_int64, int64_t num_total, int64_t key_bound,
@@ -707,7 +796,9 @@ int txs_unique_bitmap_count(const void *keys, int key_is_int64, int64_t num_tota
                        : bitmap_count(FlatKeys<int>{static_cast<const int *>(keys)}, num_total, key_bound, b, nullptr,
                                       bad, st);
     if (rc != TXS_OK) return rc;
-    bitmap_total_kernel<<<dim3(1), dim3(64), 0, st>>>(b.base, b.words, stats);
+    KeyMap m = key_map(b, keys, key_is_int64, key_bound, nullptr, nullptr, 0);
+    m.num_unq = stats + TXS_STAT_NUM_UNQ;
+    map_total_kernel<<<dim3(1), dim3(kThreads), 0, st>>>(m);
     return status_of(hipGetLastError());
 }
 
@@ -741,10 +832,13 @@ int txs_coor_bitmap_count(const void *coors, int coor_is_int64, int64_t num_tota
     hipStream_t st = (hipStream_t)stream;
     const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
     const long s0 = (long)(dims[1] * dims[2]), s1 = (long)dims[2];
-    if (coor_is_int64)
-        return bitmap_count(CoorKeys<long long>{static_cast<const long long *>(coors), s0, s1}, num_total, key_bound, b,
-                            b.bad, b.bad, st);
-    return bitmap_count(CoorKeys<int>{static_cast<const int *>(coors), s0, s1}, num_total, key_bound, b, b.bad, b.bad, st);
+    const int rc = coor_is_int64 ? bitmap_count(CoorKeys<long long>{static_cast<const long long *>(coors), s0, s1},
+                                                num_total, key_bound, b, b.bad, b.bad, st)
+                                 : bitmap_count(CoorKeys<int>{static_cast<const int *>(coors), s0, s1}, num_total,
+                                                key_bound, b, b.bad, b.bad, st);
+    if (rc != TXS_OK) return rc;
+    map_total_kernel<<<dim3(1), dim3(kThreads), 0, st>>>(key_map(b, nullptr, 0, key_bound, nullptr, nullptr, 0));
+    return status_of(hipGetLastError());
 }
 
 int64_t txs_grid_hash_index_workspace_len(int64_t num_unq, int64_t table_size) {
@@ -765,9 +859,8 @@ int txs_grid_hash_index(const int32_t *bitmap_ws, int64_t key_bound, int64_t num
     const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
     auto slots = reinterpret_cast<unsigned long long *>(table);
     int *unq_keys = index_ws, *tile_sums = index_ws + num_unq;
-    const long span = b.words > table_size ? b.words : (long)table_size;
-    grid_hash_prepare_kernel<<<dim3(blocks_for(span)), dim3(kThreads), 0, st>>>(b.bm, b.base, b.words, (int)num_unq,
-                                                                               unq_keys, slots, table_size);
+    const KeyMap m = key_map(b, nullptr, 0, key_bound, nullptr, unq_keys, num_unq);
+    grid_hash_prepare_kernel<<<dim3((unsigned)map_parts(m)), dim3(kThreads), 0, st>>>(m, slots, table_size);
     grid_hash_build_kernel<<<dim3(blocks_for(num_unq)), dim3(kThreads), 0, st>>>(unq_keys, nullptr, slots,
                                                                                 (int)table_size, num_unq, nullptr);
     const long tiles = (table_size + kValidTile - 1) / kValidTile;
@@ -786,18 +879,10 @@ int txs_unique_bitmap_assign(const void *keys, int key_is_int64, int64_t num_tot
     if (num_total == 0) return TXS_OK;
     if (!keys || !bitmap_ws || !unq_inv || !unq_keys) return TXS_ERR_INVALID_ARG;
     hipStream_t st = (hipStream_t)stream;
-    const long n = num_total;
     const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
-    const long words = b.words;
-    const unsigned *bm = b.bm;
-    const int *base = b.base;
-    const long span = n > words ? n : words;
-    if (key_is_int64)
-        bitmap_assign_kernel<long long><<<dim3(blocks_for(span)), dim3(kThreads), 0, st>>>(
-            static_cast<const long long *>(keys), n, (long)key_bound, bm, base, words, unq_inv, unq_keys, nullptr, nullptr);
-    else
-        bitmap_assign_kernel<int><<<dim3(blocks_for(span)), dim3(kThreads), 0, st>>>(
-            static_cast<const int *>(keys), n, (long)key_bound, bm, base, words, unq_inv, unq_keys, nullptr, nullptr);
+    KeyMap m = key_map(b, keys, key_is_int64, key_bound, nullptr, unq_keys, most_keys(num_total, key_bound));
+    m.num_unq = nullptr;  // (txs_unique_bitmap_count has left it where the caller asked for it)
+    map_assign_kernel<<<dim3(blocks_for(num_total) + (unsigned)map_parts(m)), dim3(kThreads), 0, st>>>(m, num_total, unq_inv);
     return status_of(hipGetLastError());
 }
 
@@ -805,33 +890,12 @@ int txs_unique_plan(const void *keys, int key_is_int64, int64_t num_total, int64
                     int32_t *bitmap_ws, int32_t heavy_threshold, int32_t *plan_ws, int32_t *unq_inv,
                     int32_t *unq_keys, int64_t *unq_cnts, int32_t *perm, int32_t *seg, int32_t *preSum,
                     int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream) {
-    if (!fits_i32(num_total) || num_total == 0 || key_bound <= 0 || key_bound > (1LL << 31)) return TXS_ERR_INVALID_ARG;
-    if (!keys || !bitmap_ws || ((uintptr_t)bitmap_ws & 15u) != 0 || !unq_inv || !unq_keys || !unq_cnts || !slot_of ||
-        !heavy_ids || !stats)
-        return TXS_ERR_INVALID_ARG;
-    hipStream_t st = (hipStream_t)stream;
-    const long n = num_total;
-    const BitmapWs b = bitmap_ws_of(bitmap_ws, key_bound);
-    int *bad = key_flag ? key_flag : b.bad, *clear_flag = key_flag ? nullptr : b.bad;
-    int *found = stats + TXS_STATS_LEN;
-    const dim3 grid(blocks_for(n > b.words ? n : b.words)), blk(kThreads);
-    int rc;
-    if (key_is_int64) {
-        auto k = static_cast<const long long *>(keys);
-        rc = bitmap_count(FlatKeys<long long>{k}, n, key_bound, b, clear_flag, bad, st);
-        bitmap_assign_kernel<long long><<<grid, blk, 0, st>>>(k, n, (long)key_bound, b.bm, b.base, b.words, unq_inv,
-                                                              unq_keys, bad, found);
-    } else {
-        auto k = static_cast<const int *>(keys);
-        rc = bitmap_count(FlatKeys<int>{k}, n, key_bound, b, clear_flag, bad, st);
-        bitmap_assign_kernel<int><<<grid, blk, 0, st>>>(k, n, (long)key_bound, b.bm, b.base, b.words, unq_inv, unq_keys,
-                                                        bad, found);
-    }
-    if (rc != TXS_OK || hipGetLastError() != hipSuccess) return TXS_ERR_LAUNCH;
-    const int64_t most = num_total < key_bound ? num_total : key_bound;
-    return txs_detail::plan_build(unq_inv, num_total, most, heavy_threshold, nullptr, plan_ws, perm, seg, preSum,
-                                  slot_of, heavy_ids, stats, nullptr, b.base + b.words, (long long *)unq_cnts, nullptr,
-                                  stream);
+    if (!unq_inv || !unq_keys || !unq_cnts || !slot_of || !heavy_ids || !stats) return TXS_ERR_INVALID_ARG;
+    const int rc = txs_detail::unique_map_keys(keys, key_is_int64, num_total, key_bound, key_flag, bitmap_ws, stream);
+    if (rc != TXS_OK) return rc;
+    return txs_detail::unique_plan_of_map(keys, key_is_int64, num_total, key_bound, key_flag, bitmap_ws, heavy_threshold,
+                                          plan_ws, unq_inv, unq_keys, unq_cnts, perm, seg, preSum, slot_of, heavy_ids,
+                                          stats, stream);
 }
 
 int txs_counts_from_presum(const int32_t *preSum, int64_t num_unq, int64_t *unq_cnts, void *stream) {
@@ -876,7 +940,7 @@ static int group_ranks(const long long *ids64, const int32_t *group_ids, int64_t
     const bool fused = txs_detail::plan_writes_ranks(num_total, num_groups);
     const int rc = txs_detail::plan_build(group_ids, num_total, num_groups, heavy, nullptr, plan_ws, perm, seg, preSum,
                                           nullptr, nullptr, stats, fused ? (long long *)out : nullptr, nullptr, nullptr,
-                                          ids64, stream);
+                                          ids64, nullptr, stream);
     if (rc != TXS_OK || fused) return rc;
     ingroup_inds_auto_kernel<<<dim3(blocks_for(num_total)), dim3(kThreads), 0, (hipStream_t)stream>>>(
         seg, perm, preSum, stats, num_total, (int)num_groups, (long long *)out);

@@ -202,6 +202,7 @@ hipError_t scan_from_tile_sums(const int *in, long n_in, int *out, long n_out, i
 namespace {
 
 using txs_detail::exclusive_scan;
+using txs_detail::KeyMap;
 using txs_detail::scan_tiles;
 
 __device__ __forceinline__ int wave_max_i32(int x) {
@@ -547,19 +548,41 @@ __device__ __forceinline__ void wave_rank(const int (&key)[COUNT], int shift, in
 // A tile's rows in bucket order: rows_out[tile's first row + k] = low digit << tile bits | row inside
 // the tile; offs[tile][d] = the tile's rows in buckets below d (d up to the number of buckets).
 // K = long long: ids as torch.unique returns them, cut to 32 bits and left in `ids32` for later readers.
+// K = KeyMap: the ids are looked up by key and left in `ids32` (a kernel of its own for that, which this one
+// then read again, took 6 us of 200k rows in 16.9M cells); the workgroups behind those of the tiles list
+// the occurring keys.
 // stats and ctl are cleared for the kernels that follow.
 // Ranking is by wave ballots on the digit's bits and a 16-bit count per wave and bucket; the rows pass
 // through LDS so that they leave as one stream.
 template <int THREADS, int ITEMS, typename K>
 __global__ __launch_bounds__(THREADS) void tile_sort_kernel(
-    const K *__restrict__ ids, long n, int U_arg, int high_bits, unsigned *__restrict__ rows_out,
-    unsigned short *__restrict__ offs, int pitch, int *__restrict__ tile_flags, int *__restrict__ ids32,
-    int *__restrict__ stats, int *__restrict__ ctl, const int *__restrict__ num_unq_dev) {
+    std::conditional_t<std::is_same_v<K, KeyMap>, KeyMap, const K *> ids, long n, int n_tiles, int U_arg, int high_bits,
+    unsigned *__restrict__ rows_out, unsigned short *__restrict__ offs, int pitch, int *__restrict__ tile_flags,
+    int *__restrict__ ids32, int *__restrict__ stats, int *__restrict__ ctl, const int *__restrict__ num_unq_dev) {
     constexpr int WAVES = THREADS / 64, kRows = THREADS * ITEMS, kTileBits = __builtin_ctz(kRows);
     // [bins] first place of every bucket, then the larger of [WAVES][bins] counts and the staged rows
     extern __shared__ __align__(16) uint2 lds_tile[];
+    constexpr bool kMap = std::is_same_v<K, KeyMap>;
     __shared__ int s_flags;
-    const int U = voxel_count(U_arg, num_unq_dev), low_bits = low_bits_of(U, high_bits);
+    __shared__ int base_s[kMap ? txs_detail::kMapTilesSummed : 1];
+    int U;
+    if constexpr (kMap) {
+        U = min(U_arg, map_tile_bases<THREADS>(ids, base_s));
+        if ((int)blockIdx.x >= n_tiles) {
+            map_list_part<THREADS>(ids, base_s, (int)blockIdx.x - n_tiles);
+            return;
+        }
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            ids.num_unq[0] = U;
+            if (ids.found) {
+                ids.found[0] = U;
+                ids.found[1] = ids.bad[0];
+            }
+        }
+    } else {
+        U = voxel_count(U_arg, num_unq_dev);
+    }
+    const int low_bits = low_bits_of(U, high_bits);
     const int quads = max(1 << high_bits, 4) >> 2;  // bins / 4
     uint2 *first4 = lds_tile, *cnt4 = lds_tile + quads;
     const unsigned short *first = reinterpret_cast<const unsigned short *>(first4);
@@ -574,11 +597,20 @@ __global__ __launch_bounds__(THREADS) void tile_sort_kernel(
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
         const long i = wbase + (long)it * 64 + lane;
-        key[it] = i < n ? (int)ids[i] : 0x7fffffff;
+        if constexpr (kMap) key[it] = i < n ? map_key(ids, i) : 0x7fffffff;
+        else key[it] = i < n ? (int)ids[i] : 0x7fffffff;
     }
-    // the id behind the wave's rows
+    // the id (or key: they ascend together) behind the wave's rows
     int behind = 0x7fffffff;
-    if (lane == 63 && wbase + 64 * ITEMS < n) behind = (int)ids[wbase + 64 * ITEMS];
+    if (lane == 63 && wbase + 64 * ITEMS < n) {
+        if constexpr (kMap) behind = map_key(ids, wbase + 64 * ITEMS);
+        else behind = (int)ids[wbase + 64 * ITEMS];
+    }
+    uint2 cell[kMap ? ITEMS : 1];
+    if constexpr (kMap) {
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it) cell[it] = ids.cells[wbase + (long)it * 64 + lane < n ? key[it] >> 5 : 0];
+    }
     if (threadIdx.x == 0) s_flags = 0;
     for (int k = threadIdx.x; k < WAVES * quads; k += THREADS) cnt4[k] = make_uint2(0u, 0u);
     __syncthreads();
@@ -586,11 +618,14 @@ __global__ __launch_bounds__(THREADS) void tile_sort_kernel(
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
         const long i = wbase + (long)it * 64 + lane;
-        if (sizeof(K) == 8 && i < n) ids32[i] = key[it];
+        if (std::is_same_v<K, long long> && i < n) ids32[i] = key[it];
         int next = __shfl_down(key[it], 1, 64);
         const int wrap = it + 1 < ITEMS ? __builtin_amdgcn_readfirstlane(key[it + 1 < ITEMS ? it + 1 : 0]) : behind;
         if (lane == 63) next = wrap;
         bad_order |= next < key[it];  // (rows behind the last one compare as the largest id)
+        if constexpr (kMap) {
+            if (i < n) ids32[i] = key[it] = map_id(ids, base_s, cell[it], key[it]);
+        }
         if ((unsigned)key[it] >= (unsigned)U) {
             bad_range |= i < n;
             key[it] = -1;  // out-of-range ids are dropped (and flagged)
@@ -1619,7 +1654,7 @@ int txs_plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, i
                    const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum,
                    int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream) {
     return txs_detail::plan_build(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum,
-                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, nullptr, stream);
+                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, nullptr, nullptr, stream);
 }
 
 int txs_plan_build_i64(const int64_t *ids, int32_t *unq_inv, int64_t num_total, int64_t num_unq,
@@ -1627,7 +1662,7 @@ int txs_plan_build_i64(const int64_t *ids, int32_t *unq_inv, int64_t num_total, 
                        int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream) {
     if (num_total > 0 && !ids) return TXS_ERR_INVALID_ARG;
     return txs_detail::plan_build(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum,
-                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, (const long long *)ids, stream);
+                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, (const long long *)ids, nullptr, stream);
 }
 
 }  // extern "C"
@@ -1667,11 +1702,15 @@ bool txs_detail::plan_writes_ranks(long num_total, long num_unq) {
     return num_total > 0 && num_unq > 0 && bits <= kBucketBitsMax;
 }
 
+bool txs_detail::plan_takes_map(long num_total, long num_unq) {
+    return num_total > 0 && num_total <= kTiledRows && num_unq > 0 && radix_bits((int)(num_unq > 1 ? num_unq : 1)) <= kBucketBitsMax;
+}
+
 int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
                            const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg,
                            int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids, int32_t *stats,
                            long long *ranks, const int *num_unq_dev, long long *cnts_out,
-                           const long long *ids64, void *stream) {
+                           const long long *ids64, const KeyMap *map, void *stream) {
     if (!fits_i32(num_total) || !fits_i32(num_unq) || !stats || !preSum || heavy_threshold < kChunk)
         return TXS_ERR_INVALID_ARG;
     hipStream_t st = (hipStream_t)stream;
@@ -1729,16 +1768,18 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
         const int tile_threads = t.tile_bits == 10 ? 256 : 512;
         const size_t bins = (size_t)t.pitch - 4;
         const size_t lds = 2 * bins + max(2 * bins * (tile_threads / 64), sizeof(int) << t.tile_bits);
-        auto sort_tiles = [&](auto ids) {
+        auto sort_tiles = [&](auto ids, int more) {
             using K = std::remove_const_t<std::remove_pointer_t<decltype(ids)>>;
             auto kernel = t.tile_bits == 10   ? tile_sort_kernel<256, 4, K>
                           : t.tile_bits == 11 ? tile_sort_kernel<512, 4, K>
                           : t.tile_bits == 12 ? tile_sort_kernel<512, 8, K>
                                               : tile_sort_kernel<512, 16, K>;
-            kernel<<<dim3(t.tiles), dim3(tile_threads), lds, st>>>(ids, n, U, t.high_bits, rows, offs, t.pitch, tile_flags,
-                                                                   ids32, stats, ctl, num_unq_dev);
+            kernel<<<dim3(t.tiles + more), dim3(tile_threads), lds, st>>>(ids, n, t.tiles, U, t.high_bits, rows, offs, t.pitch,
+                                                                          tile_flags, ids32, stats, ctl, num_unq_dev);
         };
-        if (ids64) sort_tiles(ids64); else sort_tiles(unq_inv);
+        if (map) sort_tiles(*map, map_parts(*map));
+        else if (ids64) sort_tiles(ids64, 0);
+        else sort_tiles(unq_inv, 0);
         bucket_start_kernel<<<dim3(((1 << t.high_bits) + kStartOwned) / kStartOwned), dim3(kStartThreads), 0, st>>>(
             offs, t.pitch, t.tiles, (int)n, U, t.high_bits, (threads == 512 ? 1 : kSelfSlices) * threads * kBktItems, tile_flags, bucket_start, stats, ctl, num_unq_dev,
             voxels);

@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "torchex_scatter.h"
+#include "txs_internal.h"
 
 namespace {
 
@@ -68,16 +69,20 @@ Tensor empty_i32(int64_t n, const Tensor &like) {
     return at::empty({n}, like.options().dtype(at::kInt));
 }
 
+// A few numbers from the device: an asynchronous copy into pinned host memory (from the caching host
+// allocator), then a wait on the stream.
+Tensor read_back(const Tensor &x) {
+    Tensor h = at::empty(x.sizes(), x.options().device(at::kCPU).pinned_memory(true));
+    h.copy_(x, /*non_blocking=*/true);
+    c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.device().index()).synchronize();
+    return h;
+}
+
+// the one host synchronisation of index preparation
 std::vector<int64_t> read_stats(const Tensor &stats) {
-    const int64_t len = stats.numel();
-    // the one host synchronisation of index preparation: an asynchronous copy into pinned
-    // host memory (from the caching host allocator), then a wait on the stream
-    Tensor h = at::empty({len}, stats.options().device(at::kCPU).pinned_memory(true));
-    h.copy_(stats, /*non_blocking=*/true);
-    c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(stats.device().index()).synchronize();
-    std::vector<int64_t> v(len);
-    for (int64_t i = 0; i < len; ++i) v[i] = h.data_ptr<int32_t>()[i];
-    return v;
+    const Tensor h = read_back(stats);
+    const int32_t *p = h.data_ptr<int32_t>();
+    return std::vector<int64_t>(p, p + h.numel());
 }
 
 // The special-voxel list the forward call takes: txs_plan_special leaves the heavy
@@ -225,17 +230,22 @@ std::tuple<Tensor, Tensor, Tensor, std::vector<int64_t>> plan_from_presum(
     return {seg, slot_of, heavy_ids, hs};
 }
 
+void check_points(const Tensor &points, const std::vector<double> &range_lo, const std::vector<double> &voxel_size,
+                  const std::vector<int64_t> &dims) {
+    check_dev(points, "points");
+    TORCH_CHECK(points.dim() == 2 && points.size(1) >= 3, "points must be [N, >=3]");
+    TORCH_CHECK(points.scalar_type() == at::kFloat, "points must be float32");
+    TORCH_CHECK(range_lo.size() == 3 && voxel_size.size() == 3 && dims.size() == 3,
+                "range_lo, voxel_size and dims need 3 entries");
+}
+
 // Dynamic voxelization front-end: coors and linear keys of every point; no host
 // synchronisation (range violations are flagged in the returned stats tensor).
 // returns (coors [N,3] int32, keys [N] int32, stats [TXS_STATS_LEN] int32)
 std::tuple<Tensor, Tensor, Tensor> voxel_keys(const Tensor &points, std::vector<double> range_lo,
                                               std::vector<double> voxel_size,
                                               std::vector<int64_t> dims) {
-    check_dev(points, "points");
-    TORCH_CHECK(points.dim() == 2 && points.size(1) >= 3, "points must be [N, >=3]");
-    TORCH_CHECK(points.scalar_type() == at::kFloat, "points must be float32");
-    TORCH_CHECK(range_lo.size() == 3 && voxel_size.size() == 3 && dims.size() == 3,
-                "range_lo, voxel_size and dims need 3 entries");
+    check_points(points, range_lo, voxel_size, dims);
     c10::hip::HIPGuardMasqueradingAsCUDA guard(points.device());
     const int64_t N = points.size(0);
     const float lo[3] = {(float)range_lo[0], (float)range_lo[1], (float)range_lo[2]};
@@ -302,6 +312,53 @@ UniquePlan unique_plan_counted(const Tensor &keys, int64_t key_bound, int64_t he
 // 109 / 112, 2M 138 / 122, 4M 216 / 172; in 1024 of Zipf occupancy 800k 127 / 123, 2M 174 / 138.
 constexpr int64_t kUncountedVoxels = int64_t(1) << 20;
 
+// Whether the number of voxels is left on the device: an occupancy map, and few enough of them.
+bool leaves_count(int64_t N, int64_t key_bound) {
+    return N > 0 && bitmap_is_cheaper(N, key_bound) && std::min(N, key_bound) <= kUncountedVoxels;
+}
+
+// unique_plan from the map of the keys in `bws`: everything is sized for as many voxels as there can be
+// and allocated while the map is being made.  flag: where a key outside the bound has been told of (NULL:
+// in the map's own).
+UniquePlan unique_plan_uncounted(const Tensor &keys, int64_t key_bound, int64_t heavy_threshold, const int32_t *flag,
+                                 Tensor &bws) {
+    const int64_t N = keys.numel(), most = std::min(N, key_bound);
+    void *st = cur_stream(keys);
+    const auto i32 = keys.options().dtype(at::kInt);
+    Tensor inv = at::empty({N}, i32), unq = at::empty({most}, i32), seg = at::empty({N}, i32);
+    Tensor perm = at::empty({N}, i32), preSum = at::empty({most + 1}, i32);
+    Tensor slot_of = at::empty({most}, i32), heavy_all = at::empty({most}, i32);
+    Tensor cnts = at::empty({most}, keys.options().dtype(at::kLong));
+    Tensor ws = at::empty({txs_plan_workspace_len(N, most)}, i32);
+    Tensor stats = at::empty({TXS_STATS_LEN + 2}, i32);
+    check_status(txs_detail::unique_plan_of_map(keys.data_ptr(), keys.scalar_type() == at::kLong, N, key_bound, flag,
+                                                i32w(bws), (int32_t)heavy_threshold, i32w(ws), i32w(inv), i32w(unq),
+                                                cnts.data_ptr<int64_t>(), i32w(perm), i32w(seg), i32w(preSum),
+                                                i32w(slot_of), i32w(heavy_all), i32w(stats), st),
+                 "unique_plan");
+    std::vector<int64_t> hs = read_stats(stats);
+    const int64_t U = hs[TXS_STATS_LEN];
+    TORCH_CHECK(hs[TXS_STATS_LEN + 1] == 0, "keys (or points) outside the grid: keys must be in [0, ", key_bound, ")");
+    if (hs[TXS_STAT_NEED_GENERAL]) {
+        // a few voxels own most of the rows: the bucket kernels stepped aside
+        stats.zero_();
+        check_status(txs_plan_build_general(i32p(inv), N, U, (int32_t)heavy_threshold, nullptr, i32w(ws),
+                                            i32w(perm), i32w(seg), i32w(preSum), i32w(slot_of),
+                                            i32w(heavy_all), i32w(stats), st),
+                     "plan_build_general");
+        check_status(txs_counts_from_presum(i32p(preSum), U, cnts.data_ptr<int64_t>(), st), "counts_from_presum");
+        hs = read_stats(stats);
+    }
+    hs.resize(TXS_STATS_LEN);
+    hs[TXS_STAT_NUM_UNQ] = U;
+    demote_few_heavy(hs, heavy_threshold, preSum, seg, slot_of, heavy_all, stats, N, U, st);
+    OptTensor perm_out;
+    if (hs[TXS_STAT_UNSORTED]) perm_out = perm;
+    // (every voxel owns rows: heavy ones are the only special ones, at the front of the list)
+    return {unq.narrow(0, 0, U), inv, cnts.narrow(0, 0, U), preSum.narrow(0, 0, U + 1), perm_out, seg,
+            slot_of.narrow(0, 0, U), special_list(heavy_all, most, hs), hs};
+}
+
 // torch.unique(keys, return_inverse=True, return_counts=True) fused with the
 // scatter plan.
 // returns (unq_keys, unq_inv, unq_cnts, preSum, perm | None, seg, slot_of, heavy_ids, stats)
@@ -323,45 +380,15 @@ UniquePlan unique_plan(const Tensor &keys_in, int64_t key_bound, int64_t heavy_t
     // index preparation of those ids.  The number of distinct keys is read back with the plan's own
     // figures: until then everything is sized for as many as there can be.
     if (N > 0 && bitmap_is_cheaper(N, key_bound)) {
-        const int64_t most = std::min(N, key_bound);
-        if (most > kUncountedVoxels)
+        if (!leaves_count(N, key_bound))
             return unique_plan_counted(keys_in, key_bound, heavy_threshold,
                                        stats_in.has_value() ? *stats_in : at::zeros({TXS_STATS_LEN}, i32));
-        Tensor inv = at::empty({N}, i32), unq = at::empty({most}, i32), seg = at::empty({N}, i32);
-        Tensor perm = at::empty({N}, i32), preSum = at::empty({most + 1}, i32);
-        Tensor slot_of = at::empty({most}, i32), heavy_all = at::empty({most}, i32);
-        Tensor cnts = at::empty({most}, keys_in.options().dtype(at::kLong));
         Tensor bws = at::empty({txs_unique_bitmap_workspace_len(key_bound)}, i32);
-        Tensor ws = at::empty({txs_plan_workspace_len(N, most)}, i32);
-        Tensor stats = at::empty({TXS_STATS_LEN + 2}, i32);
-        check_status(txs_unique_plan(keys_in.data_ptr(), keys_in.scalar_type() == at::kLong, N, key_bound,
-                                     stats_in.has_value() ? stats_in->data_ptr<int32_t>() + TXS_STAT_OUT_OF_RANGE
-                                                          : nullptr,
-                                     i32w(bws), (int32_t)heavy_threshold, i32w(ws), i32w(inv), i32w(unq),
-                                     cnts.data_ptr<int64_t>(), i32w(perm), i32w(seg), i32w(preSum), i32w(slot_of),
-                                     i32w(heavy_all), i32w(stats), st),
+        int32_t *flag = stats_in.has_value() ? stats_in->data_ptr<int32_t>() + TXS_STAT_OUT_OF_RANGE : nullptr;
+        check_status(txs_detail::unique_map_keys(keys_in.data_ptr(), keys_in.scalar_type() == at::kLong, N, key_bound,
+                                                 flag, i32w(bws), st),
                      "unique_plan");
-        std::vector<int64_t> hs = read_stats(stats);
-        const int64_t U = hs[TXS_STATS_LEN];
-        TORCH_CHECK(hs[TXS_STATS_LEN + 1] == 0, "keys (or points) outside the grid: keys must be in [0, ", key_bound, ")");
-        if (hs[TXS_STAT_NEED_GENERAL]) {
-            // a few voxels own most of the rows: the bucket kernels stepped aside
-            stats.zero_();
-            check_status(txs_plan_build_general(i32p(inv), N, U, (int32_t)heavy_threshold, nullptr, i32w(ws),
-                                                i32w(perm), i32w(seg), i32w(preSum), i32w(slot_of),
-                                                i32w(heavy_all), i32w(stats), st),
-                         "plan_build_general");
-            check_status(txs_counts_from_presum(i32p(preSum), U, cnts.data_ptr<int64_t>(), st), "counts_from_presum");
-            hs = read_stats(stats);
-        }
-        hs.resize(TXS_STATS_LEN);
-        hs[TXS_STAT_NUM_UNQ] = U;
-        demote_few_heavy(hs, heavy_threshold, preSum, seg, slot_of, heavy_all, stats, N, U, st);
-        OptTensor perm_out;
-        if (hs[TXS_STAT_UNSORTED]) perm_out = perm;
-        // (every voxel owns rows: heavy ones are the only special ones, at the front of the list)
-        return {unq.narrow(0, 0, U), inv, cnts.narrow(0, 0, U), preSum.narrow(0, 0, U + 1), perm_out, seg,
-                slot_of.narrow(0, 0, U), special_list(heavy_all, most, hs), hs};
+        return unique_plan_uncounted(keys_in, key_bound, heavy_threshold, flag, bws);
     }
     Tensor stats = stats_in.has_value() ? *stats_in : at::zeros({TXS_STATS_LEN}, i32);
     // int64 keys are narrowed for the sort; one outside int32 is first pinned to a value that
@@ -399,6 +426,33 @@ UniquePlan unique_plan(const Tensor &keys_in, int64_t key_bound, int64_t heavy_t
     if (hs[TXS_STAT_UNSORTED]) perm_out = perm;
     return {unq.narrow(0, 0, U), inv, cnts.narrow(0, 0, U), preSum.narrow(0, 0, U + 1), perm_out, seg,
             slot_of.narrow(0, 0, U), special_list(heavy_all, N, hs), hs};
+}
+
+// voxel_keys and unique_plan of its keys in one: (coors, unique_plan(...)).  Where the map is used and the
+// number of voxels stays on the device, the points' kernel marks the map itself, and nothing but the
+// coordinates, the keys and the map is allocated in front of the first launch.
+std::tuple<Tensor, UniquePlan> points_plan(const Tensor &points, std::vector<double> range_lo,
+                                           std::vector<double> voxel_size, std::vector<int64_t> dims,
+                                           int64_t heavy_threshold) {
+    int64_t bound = 1;
+    for (int64_t d : dims) bound = bound > 0 && d > 0 && d <= (int64_t(1) << 28) / bound ? bound * d : 0;
+    if (bound == 0 || dims.size() != 3 || points.dim() != 2 || !leaves_count(points.size(0), bound)) {
+        auto [coors, keys, stats] = voxel_keys(points, range_lo, voxel_size, dims);
+        return {coors, unique_plan(keys, dims[0] * dims[1] * dims[2], heavy_threshold, stats)};
+    }
+    check_points(points, range_lo, voxel_size, dims);
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(points.device());
+    const int64_t N = points.size(0);
+    const auto i32 = points.options().dtype(at::kInt);
+    const float lo[3] = {(float)range_lo[0], (float)range_lo[1], (float)range_lo[2]};
+    const float vs[3] = {(float)voxel_size[0], (float)voxel_size[1], (float)voxel_size[2]};
+    const int32_t dm[3] = {(int32_t)dims[0], (int32_t)dims[1], (int32_t)dims[2]};
+    Tensor coors = at::empty({N, 3}, i32), keys = at::empty({N}, i32);
+    Tensor bws = at::empty({txs_unique_bitmap_workspace_len(bound)}, i32);
+    check_status(txs_detail::unique_map_points(points.data_ptr<float>(), N, points.size(1), lo, vs, dm, i32w(coors),
+                                               i32w(keys), i32w(bws), cur_stream(points)),
+                 "points_plan");
+    return {coors, unique_plan_uncounted(keys, bound, heavy_threshold, nullptr, bws)};
 }
 
 // ingroup_inds(seg, perm | None, preSum, num_unq) -> int64 [N]
@@ -531,7 +585,7 @@ std::tuple<Tensor, Tensor, Tensor> dynamic_point_pool(const Tensor &rois, const 
                                         max_all_pts ? feats.data_ptr<float>() : nullptr, i32w(num),
                                         cur_stream(pts)),
                  "dynamic_point_pool");
-    const int64_t M = num.cpu().data_ptr<int32_t>()[0];
+    const int64_t M = read_back(num).data_ptr<int32_t>()[0];
     return {idx.narrow(0, 0, M), roi.narrow(0, 0, M), feats.narrow(0, 0, M)};
 }
 
@@ -654,7 +708,7 @@ std::tuple<std::vector<int64_t>, OptTensor, OptTensor, OptTensor> grid_hash_inde
     const int64_t num_parts = txs_coor_max_parts();
     Tensor parts = at::empty({num_parts, 3}, coors.options().dtype(at::kLong));
     check_status(txs_coor_max(coors.data_ptr(), is64, N, parts.data_ptr<int64_t>(), st), "coor_max");
-    const Tensor parts_host = parts.cpu();
+    const Tensor parts_host = read_back(parts);
     const int64_t *ph = parts_host.data_ptr<int64_t>();
     std::vector<int64_t> dims(ph, ph + 3);
     for (int64_t k = 1; k < num_parts; ++k)
@@ -669,7 +723,7 @@ std::tuple<std::vector<int64_t>, OptTensor, OptTensor, OptTensor> grid_hash_inde
     if (!grid || !bitmap_is_cheaper(N, bound)) return {dims, std::nullopt, std::nullopt, std::nullopt};
     Tensor bws = at::empty({txs_unique_bitmap_workspace_len(bound)}, i32);
     check_status(txs_coor_bitmap_count(coors.data_ptr(), is64, N, dims.data(), i32w(bws), st), "coor_bitmap_count");
-    const Tensor found = bws.narrow(0, txs_coor_bitmap_count_offset(bound), 2).cpu();
+    const Tensor found = read_back(bws.narrow(0, txs_coor_bitmap_count_offset(bound), 2));
     const int64_t U = found.data_ptr<int32_t>()[0];
     TORCH_CHECK(found.data_ptr<int32_t>()[1] == 0, "keys (or points) outside the grid: keys must be in [0, ", bound, ")");
     const int64_t size = up_2n_host(U);
@@ -1041,6 +1095,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           pybind11::arg("unq_cnts"), pybind11::arg("assume_sorted") = false);
     m.def("plan_from_presum", &plan_from_presum, "index preparation from CSR offsets");
     m.def("voxel_keys", &voxel_keys, "voxel_keys(points, range_lo, voxel_size, dims) -> (coors, keys, stats)");
+    m.def("points_plan", &points_plan, "points_plan(points, range_lo, voxel_size, dims, heavy_threshold) -> (coors, unique_plan(...))");
     m.def("unique_plan", &unique_plan, "unique_plan(keys, key_bound, heavy_threshold, stats|None)");
     m.def("ingroup_inds", &ingroup_inds, "ingroup_inds(seg, perm|None, preSum, num_unq)");
     m.def("group_ranks", &group_ranks, "group_ranks(group_inds) -> int64 rank of every element inside its group");

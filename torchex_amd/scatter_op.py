@@ -21,6 +21,8 @@ reference is undefined, the smallest row index.  ``max_tie_rule`` forces either.
 There is no PyTorch fallback: everything runs in the HIP kernels behind
 ``scatter_ext``.
 """
+import math
+
 import torch
 from torch.autograd import Function
 
@@ -42,6 +44,10 @@ def _resolve_tie_rule(rule, grouped):
     if rule is None:
         return "reference" if grouped else "first"
     return rule
+
+
+def _heavy_threshold(given):
+    return int(scatter_ext.default_heavy_threshold() if given is None else given)
 
 
 _SCRATCH_KEPT = 4   # forward workspaces a ScatterData keeps (most recently used)
@@ -88,9 +94,7 @@ class ScatterData:
         else:
             self.unq_cnts = unq_cnts
         _check_tie_rule(max_tie_rule)
-        if heavy_threshold is None:
-            heavy_threshold = scatter_ext.default_heavy_threshold()
-        self.heavy_threshold = int(heavy_threshold)
+        self.heavy_threshold = _heavy_threshold(heavy_threshold)
         num_unq = self.unq_cnts.shape[0]
         cnts64 = self.unq_cnts.reshape(-1).long().contiguous()
         if unq_inv.dtype == torch.int64 and unq_inv.is_cuda and not assume_sorted:
@@ -130,18 +134,22 @@ class ScatterData:
         back once, or twice where both the rows and the bound exceed 2^20 or a few neighbouring voxels own
         most of the rows."""
         _check_tie_rule(max_tie_rule)
-        self = cls.__new__(cls)
-        if heavy_threshold is None:
-            heavy_threshold = scatter_ext.default_heavy_threshold()
-        self.heavy_threshold = int(heavy_threshold)
+        heavy_threshold = _heavy_threshold(heavy_threshold)
         flat = keys.reshape(-1)
         if flat.dtype not in (torch.int32, torch.int64):
             flat = flat.int()
         flat = flat.contiguous()
+        plan = scatter_ext.unique_plan(flat, int(key_bound), heavy_threshold, _stats)
+        return cls._from_unique(plan, heavy_threshold, max_tie_rule)
+
+    @classmethod
+    def _from_unique(cls, plan, heavy_threshold, max_tie_rule):
+        self = cls.__new__(cls)
+        self.heavy_threshold = heavy_threshold
         (self.unq_keys, self.unq_inv, cnts, self.preSum, self.perm, self.seg, self.slot_of,
-         self.heavy_ids, stats) = scatter_ext.unique_plan(flat, int(key_bound), self.heavy_threshold, _stats)
+         self.heavy_ids, stats) = plan
         self.unq_cnts = cnts.unsqueeze(-1)
-        self.num_total = flat.shape[0]
+        self.num_total = self.unq_inv.shape[0]
         self.is_sorted = self.perm is None
         self.row_ids = None if self.is_sorted else self.unq_inv
         self.path = scatter_ext.PATH_AUTO
@@ -160,8 +168,11 @@ class ScatterData:
         x-major linear keys (``operator_py/incremental_points.py:18-19``), unique and
         scatter plan.  Points outside ``pc_range`` raise.  Extra attributes:
         ``coors`` (int32 ``[N, 3]``), ``spatial_size``."""
-        coors, keys, stats, dims = _voxel_keys(points, voxel_size, pc_range)
-        self = cls.from_keys(keys, dims[0] * dims[1] * dims[2], heavy_threshold, max_tie_rule, _stats=stats)
+        _check_tie_rule(max_tie_rule)
+        heavy_threshold = _heavy_threshold(heavy_threshold)
+        lo, vs, dims = _grid(voxel_size, pc_range)
+        coors, plan = scatter_ext.points_plan(points, lo, vs, dims, heavy_threshold)
+        self = cls._from_unique(plan, heavy_threshold, max_tie_rule)
         self.coors = coors
         self.spatial_size = dims
         return self
@@ -295,12 +306,16 @@ class GetPreSumFunction(Function):
         return None
 
 
-def _voxel_keys(points, voxel_size, pc_range):
-    import math
+def _grid(voxel_size, pc_range):
+    """(lower corner, voxel edges, cells per axis) of a range."""
     lo = [float(v) for v in pc_range[:3]]
     hi = [float(v) for v in pc_range[3:6]]
     vs = [float(v) for v in voxel_size]
-    dims = [max(1, int(math.ceil((h - l) / v - 1e-6))) for l, h, v in zip(lo, hi, vs)]
+    return lo, vs, [max(1, int(math.ceil((h - l) / v - 1e-6))) for l, h, v in zip(lo, hi, vs)]
+
+
+def _voxel_keys(points, voxel_size, pc_range):
+    lo, vs, dims = _grid(voxel_size, pc_range)
     coors, keys, stats = scatter_ext.voxel_keys(points, lo, vs, dims)
     return coors, keys, stats, dims
 
