@@ -513,41 +513,109 @@ __device__ __forceinline__ int grid_hash_slot(int key, int probe_i, int table_si
     return (int)(((k & mask) + (unsigned long long)probe_i * (k * 2ull + 1ull)) & mask);
 }
 
-// values == NULL: key number i gets the value i
-__global__ void grid_hash_build_kernel(const int *__restrict__ keys, const int *__restrict__ values,
-                                       unsigned long long *__restrict__ table, int table_size, long n,
-                                       int *__restrict__ fail) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int key = keys[i];
-    const unsigned long long word =
-        ((unsigned long long)(unsigned)(values ? values[i] : (int)i) << 32) | (unsigned long long)(unsigned)key;
-    const unsigned long long empty = ~0ull;  // (-1, -1)
-    for (int t = 0; key >= 0 && t < table_size; ++t) {
-        const int s = grid_hash_slot(key, t, table_size);
-        if (atomicCAS(table + s, empty, word) == empty) return;
-    }
-    if (fail) fail[0] = 1;  // table full or key negative (the reference asserts)
+// A key's probe sequence is followed by its own lane for kHashOwn slots (the first one by itself, then
+// kHashStep at a time); what is left of it is looked at by the whole wave, 64 slots at a time.  The mean key needs 1.3 - 2.2 slots, but where the grid's strides fall
+// badly on the table's size (a frame's 748 x 30 cells a column, 2^18 slots) a few need hundreds, and the
+// kernels waited for those alone, a trip to memory per slot: 146k keys built in 13 / 48 / 226 us and 300k
+// probed in 11 / 47 / 111, by the frame; now 16 / 20 / 28 and 7 / 8 / 10.
+constexpr int kHashStep = 4, kHashOwn = 1 + 4 * kHashStep;
+
+// A slot as it is now or was a moment ago.  A slot only ever goes from empty to taken, so that one seen taken
+// is, and one seen empty may be (the compare-and-swap decides).
+__device__ __forceinline__ unsigned long long grid_hash_peek(const unsigned long long *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-__device__ __forceinline__ int grid_hash_find(int key, const unsigned long long *__restrict__ table, int table_size) {
-    for (int t = 0; key >= 0 && t < table_size; ++t) {
-        const unsigned long long word = table[grid_hash_slot(key, t, table_size)];
-        const int slot_key = (int)(unsigned)(word & 0xffffffffull);
-        if (slot_key == key) return (int)(unsigned)(word >> 32);
-        // An empty slot on the probe sequence proves the key was never inserted
-        // (no deletions).  The reference keeps scanning all table_size slots
-        // before giving up (functions.cuh:54-63), with the same answer.
-        if (slot_key == -1) break;
+// values == NULL: key number i gets the value i
+__global__ __launch_bounds__(kThreads) void grid_hash_build_kernel(const int *__restrict__ keys,
+                                                                   const int *__restrict__ values,
+                                                                   unsigned long long *__restrict__ table,
+                                                                   int table_size, long n, int *__restrict__ fail) {
+    // neighbouring keys (those with long sequences are, where the keys are in order) go to different waves
+    const int lane = threadIdx.x & 63;
+    const long i = (long)lane * gridDim.x * (kThreads / 64) + (long)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+    const int key = i < n ? keys[i] : -1;
+    const unsigned value = i < n ? (unsigned)(values ? values[i] : (int)i) : 0u;
+    const unsigned long long word = ((unsigned long long)value << 32) | (unsigned long long)(unsigned)key;
+    const unsigned long long empty = ~0ull;  // (-1, -1)
+    bool pending = i < n && key >= 0, failed = i < n && key < 0;
+    if (pending) pending = atomicCAS(table + grid_hash_slot(key, 0, table_size), empty, word) != empty;
+    for (int t = 1; t < kHashOwn && pending; t += kHashStep) {
+        unsigned long long *slot[kHashStep], seen[kHashStep];
+#pragma unroll
+        for (int k = 0; k < kHashStep; ++k) {
+            slot[k] = table + grid_hash_slot(key, min(t + k, table_size - 1), table_size);
+            seen[k] = grid_hash_peek(slot[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < kHashStep; ++k)
+            if (pending && t + k < table_size && seen[k] == empty) pending = atomicCAS(slot[k], empty, word) != empty;
     }
-    return -1;
+    for (unsigned long long left = __ballot(pending); left != 0ull; left &= left - 1ull) {
+        const int owner = __builtin_ctzll(left);
+        const int k = __shfl(key, owner, 64);
+        const unsigned long long w = ((unsigned long long)(unsigned)__shfl((int)value, owner, 64) << 32) | (unsigned)k;
+        bool placed = false;  // (uniform)
+        for (int t0 = kHashOwn; t0 < table_size && !placed; t0 += 64) {
+            const int t = t0 + lane;
+            unsigned long long *slot = table + grid_hash_slot(k, min(t, table_size - 1), table_size);
+            unsigned long long free = __ballot(t < table_size && grid_hash_peek(slot) == empty);
+            // the first empty slot, or the next one if that was taken in between
+            for (; free != 0ull && !placed; free &= free - 1ull) {
+                const int first = __builtin_ctzll(free);
+                placed = __ballot(lane == first && atomicCAS(slot, empty, w) == empty) != 0ull;
+            }
+        }
+        if (!placed && lane == owner) failed = true;
+    }
+    if (failed && fail) fail[0] = 1;  // table full or key negative (the reference asserts)
+}
+
+// Value of the lane's key (-1: absent); a wave at a time, `in`: the lane has a key.
+__device__ __forceinline__ int grid_hash_find(int key, bool in, const unsigned long long *__restrict__ table, int table_size) {
+    const int lane = threadIdx.x & 63;
+    int found = -1;
+    bool pending = in && key >= 0;
+    // An empty slot on the probe sequence proves the key was never inserted (no deletions).  The
+    // reference keeps scanning all table_size slots before giving up (functions.cuh:54-63), with the
+    // same answer.
+    auto look = [&](int t, unsigned long long word) {
+        const int slot_key = (int)(unsigned)(word & 0xffffffffull);
+        if (!pending || t >= table_size) return;
+        if (slot_key == key) found = (int)(unsigned)(word >> 32);
+        pending = slot_key != key && slot_key != -1;
+    };
+    if (pending) look(0, table[grid_hash_slot(key, 0, table_size)]);
+    for (int t = 1; t < kHashOwn && pending; t += kHashStep) {
+        unsigned long long word[kHashStep];
+#pragma unroll
+        for (int k = 0; k < kHashStep; ++k) word[k] = table[grid_hash_slot(key, min(t + k, table_size - 1), table_size)];
+#pragma unroll
+        for (int k = 0; k < kHashStep; ++k) look(t + k, word[k]);
+    }
+    for (unsigned long long left = __ballot(pending); left != 0ull; left &= left - 1ull) {
+        const int owner = __builtin_ctzll(left), k = __shfl(key, owner, 64);
+        for (int t0 = kHashOwn; t0 < table_size; t0 += 64) {
+            const int t = t0 + lane;
+            const unsigned long long word = table[grid_hash_slot(k, min(t, table_size - 1), table_size)];
+            const int slot_key = (int)(unsigned)(word & 0xffffffffull);
+            const unsigned long long ends = __ballot(t < table_size && (slot_key == k || slot_key == -1));
+            if (ends == 0ull) continue;
+            const int first = __builtin_ctzll(ends);
+            const int value = __shfl((int)(unsigned)(word >> 32), first, 64), at = __shfl(slot_key, first, 64);
+            if (lane == owner && at == k) found = value;
+            break;
+        }
+    }
+    return found;
 }
 
 template <class Keys>
 __global__ void grid_hash_probe_kernel(Keys keys, const unsigned long long *__restrict__ table, int table_size,
                                        long n, int *__restrict__ out) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = grid_hash_find((int)keys(i), table, table_size);
+    const int value = grid_hash_find(i < n ? (int)keys(i) : -1, i < n, table, table_size);
+    if (i < n) out[i] = value;
 }
 
 // ---- a hash of the distinct voxel coordinates -------------------------------------
