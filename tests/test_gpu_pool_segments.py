@@ -34,3 +34,42 @@ def test_pool_segments(B, P, cap, max_all):
         return
     assert np.array_equal(idx.cpu().numpy(), wi) and np.array_equal(roi.cpu().numpy(), wr)
     assert np.array_equal(feats.cpu().numpy().view(np.uint32), wf.view(np.uint32))
+
+
+def test_boxes_of_every_reach():
+    """The grid that a group of boxes is laid on: boxes of one point, one that covers the rest, boxes far out, not
+    finite or larger than the grid takes, groups of nothing but those, points on the grid's outermost sides,
+    far out and not finite, and both with the samples of a batch."""
+    g = torch.Generator().manual_seed(3)
+    B, P = 130, 30_000
+    rois = torch.zeros((B, 7))
+    rois[:, :3] = torch.rand((B, 3), generator=g) * torch.tensor([100.0, 100.0, 1.0]) - torch.tensor([50.0, 50.0, 1.5])
+    rois[:, 3:6] = torch.rand((B, 3), generator=g) * 5.0 + 0.5
+    rois[:, 6] = torch.rand((B,), generator=g) * 6.283
+    rois[3, 3:6] = 0.0
+    rois[5, 3:6] = 300.0
+    rois[7, 0] = 3e7
+    rois[9, :2] = torch.tensor([1e6, -1e6])
+    for b in range(32, 64):        # a group without a single ordinary box
+        rois[b, :2] = 0.0
+        rois[b, 3:6] = [1e16, 3e20, float("inf"), float("nan")][b % 4]
+    rois[64, 0], rois[65, 1], rois[66, 0] = float("inf"), float("-inf"), float("nan")
+    rois[67, 6] = float("nan")
+    rois[96:128, 0] = 12.0         # a group on one line
+    rois[128:, :2] = torch.tensor([[-2e4, 7.0], [3e4, 7.0]])
+    pts = torch.rand((P, 3), generator=g) * torch.tensor([110.0, 110.0, 4.0]) - torch.tensor([55.0, 55.0, 2.0])
+    pts[:130] = rois[:, :3] + torch.tensor([0.0, 0.0, 0.1])
+    pts[130:260] = rois[:, :3] + rois[:, 3:6] * torch.tensor([0.5, 0.5, 0.5])
+    pts[260:264] = torch.tensor([[float("nan"), 0, 0], [float("inf"), 0, 0], [0, float("-inf"), 0], [3e38, -3e38, 0]])
+    pts = pts[torch.randperm(P, generator=g)]
+    rb, pb = torch.randint(0, 3, (B,), generator=g), torch.randint(0, 3, (P,), generator=g)
+    for mixed in (False, True):
+        kw = {"rois_batch": rb.cuda(), "pts_batch": pb.cuda()} if mixed else {}
+        idx, roi, feats = T.dynamic_point_pool(rois.cuda(), pts.cuda(), [0.3, 0.2, 0.1], 5000, 1_000_000, **kw)
+        wi, wr, wf = orc.dynamic_point_pool(rois.numpy(), pts.numpy(), [0.3, 0.2, 0.1], 5000, 1_000_000,
+                                            *((rb.numpy(), pb.numpy()) if mixed else ()))
+        assert wi.shape[0] > 10_000
+        assert np.array_equal(idx.cpu().numpy(), wi) and np.array_equal(roi.cpu().numpy(), wr)
+        got = feats.cpu().numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(wf))
+        assert np.array_equal(np.nan_to_num(got).view(np.uint32), np.nan_to_num(wf).view(np.uint32))

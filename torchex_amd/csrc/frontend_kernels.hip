@@ -265,8 +265,8 @@ __global__ void ingroup_inds_auto_kernel(const int *__restrict__ seg, const int 
 // (box, point) order: the outcome the reference's own comment calls the usual
 // one ("out_roi_idx is automatically sorted"), made deterministic.  The count of
 // hits per tile of 256 points and group of 8 boxes, a scan, and a second pass over all results, which
-// this replaces, took 34 + 10 + 30 us for 200 boxes and 200k points; the first pass takes 27 now,
-// the writing 13.
+// this replaces, took 34 + 10 + 30 us for 200 boxes and 200k points; the first pass takes 11 now,
+// the writing 10.
 
 constexpr int kDppInfo = 13;
 
@@ -333,14 +333,21 @@ __device__ __forceinline__ int dpp_test(const DppBox &bx, float x, float y, floa
     return in_box ? 2 : (in_large ? 1 : 0);
 }
 
-// A workgroup keeps its 1024 points in registers, four per lane, and walks kDppGroup boxes, whose
-// constants come through the scalar path; the words of the bit matrix are collected in LDS and
-// leave as whole lines (16 words of a box).
+// A workgroup takes 1024 points, four per lane, and kDppGroup boxes.  It lays a grid of kDppCells x kDppCells
+// cells over its boxes and marks in every cell the boxes whose circle may reach it; a point looks its
+// cell up and meets those boxes alone.  The pairs are queued by wave and tested 64 at a time, whatever their
+// boxes.  Every point against every box's circle was bound by the vector units, ten instructions for each of
+// 40M pairs of 200 boxes and 200k points, and the exact test behind it ran with few lanes: 27 us, now 11.
+// The words of the bit matrix are collected in LDS and leave as whole lines (16 words of a box).
 constexpr int kDppItems = 4;
 constexpr int kDppTile = kThreads * kDppItems;
 constexpr int kDppWords = kDppTile / 64;   // words of a tile per box
 constexpr int kDppGroup = 32;              // boxes per workgroup
 constexpr int kDppSegTiles = kThreads / kDppWords;  // tiles an emitting workgroup covers: one word per thread
+constexpr int kDppCells = 32;
+constexpr int kDppListed = 8192;
+constexpr int kDppDense = 24;              // points of a wave that may lie in a box from which on they are not queued
+constexpr float kDppFar = 1e15f;           // boxes further out or larger than this are tested against every point
 constexpr int kDppSumBoxes = 2048;         // up to this many boxes the emitting workgroups add up the boxes in front themselves
 
 // (pts_batch / rois_batch, both NULL or both given: a point meets only the boxes of its own
@@ -352,23 +359,109 @@ __global__ __launch_bounds__(kThreads) void dpp_mask_kernel(const float *__restr
                                                             const int *__restrict__ pts_batch,
                                                             const int *__restrict__ rois_batch) {
     __shared__ unsigned long long m_s[kDppGroup][kDppWords];
+    __shared__ float pts_s[3][kDppTile];
+    __shared__ DppBox boxes_s[kDppGroup];
+    __shared__ int box_sample_s[kDppGroup];
+    __shared__ unsigned cells_s[kDppCells * kDppCells];     // a bit per box
+    __shared__ unsigned short queue_s[kThreads / 64][128];  // box << 10 | point, of the workgroup's boxes and points
+    __shared__ float grid_s[4];                             // corner, cells per unit of x and y
+    __shared__ unsigned everywhere_s;
+    static_assert(kDppTile == 1 << 10 && kDppGroup == 32, "a pair fits in 16 bits, a cell's boxes in 32");
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const unsigned long long lanes_below = (1ull << lane) - 1ull;
     const int b0 = blockIdx.y * kDppGroup;
     const int nb = min(kDppGroup, B - b0);
-    float x[kDppItems], y[kDppItems], z[kDppItems];
+    float x[kDppItems], y[kDppItems];
     int sample[kDppItems];
     bool in[kDppItems];
 #pragma unroll
     for (int it = 0; it < kDppItems; ++it) {
-        const long p = (long)blockIdx.x * kDppTile + w * (64 * kDppItems) + it * 64 + lane;
+        const int at = w * (64 * kDppItems) + it * 64 + lane;
+        const long p = (long)blockIdx.x * kDppTile + at;
         in[it] = p < P;
         const size_t q = in[it] ? (size_t)p : 0;
-        x[it] = pts[q * 3];
-        y[it] = pts[q * 3 + 1];
-        z[it] = pts[q * 3 + 2];
+        x[it] = pts_s[0][at] = pts[q * 3];
+        y[it] = pts_s[1][at] = pts[q * 3 + 1];
+        pts_s[2][at] = pts[q * 3 + 2];
         sample[it] = pts_batch ? pts_batch[q] : 0;
     }
-    for (int bb = 0; bb < nb; ++bb) {
+    constexpr int kBoxWords = sizeof(DppBox) / sizeof(int);
+    for (int t = threadIdx.x; t < nb * kBoxWords; t += kThreads)
+        reinterpret_cast<int *>(boxes_s)[t] = reinterpret_cast<const int *>(boxes + b0)[t];
+    if ((int)threadIdx.x < nb) box_sample_s[threadIdx.x] = rois_batch ? rois_batch[b0 + threadIdx.x] : 0;
+    for (int t = threadIdx.x; t < kDppGroup * kDppWords; t += kThreads) (&m_s[0][0])[t] = 0ull;
+    for (int t = threadIdx.x; t < kDppCells * kDppCells; t += kThreads) cells_s[t] = 0u;
+    __syncthreads();
+    // ---- the grid.  Eight threads a box; a box's square holds its circle whatever the rounding of its sides
+    // (a few parts in 10^7 of the coordinates), and a box of no finite or sensible square, or of most of the grid, is everywhere.
+    const int mine = (int)threadIdx.x >> 3, sub = threadIdx.x & 7;
+    float lo[2] = {INFINITY, INFINITY}, hi[2] = {-INFINITY, -INFINITY};
+    bool far = false;
+    if (mine < nb) {
+        const DppBox &bx = boxes_s[mine];
+        const float r = sqrtf(bx.r2) * 1.0001f;
+        const float c[2] = {bx.cx, bx.cy};
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            lo[k] = c[k] - r - fabsf(c[k]) * 4e-7f;
+            hi[k] = c[k] + r + fabsf(c[k]) * 4e-7f;
+            far |= !(lo[k] > -kDppFar && hi[k] < kDppFar);
+        }
+    }
+    if (w == 0) {  // (32 boxes: one wave looks at all of them for the corners)
+        float l[2] = {INFINITY, INFINITY}, h[2] = {-INFINITY, -INFINITY};
+        bool out = false;
+        if (lane < nb) {
+            const DppBox &bx = boxes_s[lane];
+            const float r = sqrtf(bx.r2) * 1.0001f;
+            const float c[2] = {bx.cx, bx.cy};
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                l[k] = c[k] - r - fabsf(c[k]) * 4e-7f;
+                h[k] = c[k] + r + fabsf(c[k]) * 4e-7f;
+                out |= !(l[k] > -kDppFar && h[k] < kDppFar);
+            }
+        }
+        const unsigned long long outs = __ballot(out);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            if (out) {
+                l[k] = INFINITY;
+                h[k] = -INFINITY;
+            }
+#pragma unroll
+            for (int d = 16; d >= 1; d >>= 1) {
+                l[k] = fminf(l[k], __shfl_xor(l[k], d, 64));
+                h[k] = fmaxf(h[k], __shfl_xor(h[k], d, 64));
+            }
+        }
+        if (lane == 0) {
+            everywhere_s = (unsigned)outs;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                grid_s[k] = l[k];
+                grid_s[2 + k] = h[k] > l[k] ? kDppCells / (h[k] - l[k]) : 0.0f;
+            }
+        }
+    }
+    __syncthreads();
+    // a coordinate's place in the grid ascends with it, rounding included, so that a point inside a box's
+    // square lies in one of the cells from the place of its lower to that of its upper side
+    auto place = [&](int axis, float v) { return (v - grid_s[axis]) * grid_s[2 + axis]; };
+    if (mine < nb && !far) {
+        const int x0 = max(0, (int)place(0, lo[0])), x1 = min(kDppCells - 1, (int)place(0, hi[0]));
+        const int y0 = max(0, (int)place(1, lo[1])), y1 = min(kDppCells - 1, (int)place(1, hi[1]));
+        if ((x1 - x0 + 1) * (y1 - y0 + 1) > kDppCells * kDppCells / 2) {  // (most points are to be tested anyway)
+            if (sub == 0) atomicOr(&everywhere_s, 1u << mine);
+        } else {
+            for (int cy = y0 + sub; cy <= y1; cy += 8)
+                for (int cx = x0; cx <= x1; ++cx) atomicOr(&cells_s[cy * kDppCells + cx], 1u << mine);
+        }
+    }
+    __syncthreads();
+    // ---- boxes that are everywhere: every point, one box after the other
+    for (unsigned left = everywhere_s; left != 0u; left &= left - 1u) {
+        const int bb = __builtin_ctz(left);
         const DppBox &bx = boxes[b0 + bb];
         const int box_sample = rois_batch ? rois_batch[b0 + bb] : 0;
         bool near[kDppItems], any = false;
@@ -377,19 +470,66 @@ __global__ __launch_bounds__(kThreads) void dpp_mask_kernel(const float *__restr
             near[it] = in[it] && sample[it] == box_sample && dpp_near(bx, x[it], y[it]);
             any |= near[it];
         }
-        unsigned long long m[kDppItems] = {};
-        if (__ballot(any) != 0ull) {
+        if (__ballot(any) == 0ull) continue;
 #pragma unroll
-            for (int it = 0; it < kDppItems; ++it) {
-                float lx, ly;
-                m[it] = __ballot(near[it] && dpp_test(bx, x[it], y[it], z[it], lx, ly) != 0);
-            }
-        }
-        if (lane == 0) {
-#pragma unroll
-            for (int it = 0; it < kDppItems; ++it) m_s[bb][w * kDppItems + it] = m[it];
+        for (int it = 0; it < kDppItems; ++it) {
+            float lx, ly;
+            const float z = pts_s[2][w * (64 * kDppItems) + it * 64 + lane];
+            const unsigned long long hits = __ballot(near[it] && dpp_test(bx, x[it], y[it], z, lx, ly) != 0);
+            if (lane == 0) m_s[bb][w * kDppItems + it] = hits;
         }
     }
+    // ---- the others: those of a point's cell
+    // the last `count` (at most 64) queued pairs
+    auto test = [&](int queued, int count) {
+        if (lane >= count) return;
+        const int pair = queue_s[w][queued - count + lane], bb = pair >> 10, at = pair & (kDppTile - 1);
+        const DppBox &bx = boxes_s[bb];
+        const float px = pts_s[0][at], py = pts_s[1][at];
+        float lx, ly;
+        if (dpp_near(bx, px, py) && dpp_test(bx, px, py, pts_s[2][at], lx, ly) != 0)
+            atomicOr(reinterpret_cast<unsigned *>(&m_s[bb][0]) + (at >> 5), 1u << (at & 31));
+    };
+    int queued = 0;
+#pragma unroll
+    for (int it = 0; it < kDppItems; ++it) {
+        unsigned boxes_here = 0u;
+        if (in[it]) {
+            const float gx = place(0, x[it]), gy = place(1, y[it]);
+            // (a place at the very end may round up to kDppCells; NaN is nowhere)
+            const bool inside = gx >= 0.0f && gx < kDppCells + 0.5f && gy >= 0.0f && gy < kDppCells + 0.5f;
+            const int cx = inside ? min((int)gx, kDppCells - 1) : 0, cy = inside ? min((int)gy, kDppCells - 1) : 0;
+            boxes_here = inside ? cells_s[cy * kDppCells + cx] : 0u;
+        }
+        for (unsigned long long left = __ballot(boxes_here != 0u); left != 0ull; left = __ballot(boxes_here != 0u)) {
+            // a box that many of the wave's points may lie in is put to the test at once
+            const int wide = __builtin_ctz(__shfl((int)boxes_here, __builtin_ctzll(left), 64));  // (uniform)
+            const bool mine_too = (boxes_here >> wide & 1u) != 0u;
+            if (__popcll(__ballot(mine_too)) >= kDppDense) {
+                float lx, ly;
+                const DppBox &bx = boxes_s[wide];
+                const unsigned long long hits =
+                    __ballot(mine_too && sample[it] == box_sample_s[wide] && dpp_near(bx, x[it], y[it]) &&
+                             dpp_test(bx, x[it], y[it], pts_s[2][w * (64 * kDppItems) + it * 64 + lane], lx, ly) != 0);
+                if (lane == 0 && hits) atomicOr(&m_s[wide][w * kDppItems + it], hits);
+                boxes_here &= ~(1u << wide);
+                continue;
+            }
+            const int bb = boxes_here ? __builtin_ctz(boxes_here) : 0;
+            const bool meet = boxes_here != 0u && sample[it] == box_sample_s[bb];
+            const unsigned long long m = __ballot(meet);
+            if (meet) queue_s[w][queued + __popcll(m & lanes_below)] = (unsigned short)(bb << 10 | (w * (64 * kDppItems) + it * 64 + lane));
+            queued += __popcll(m);
+            boxes_here &= boxes_here - 1u;
+            __builtin_amdgcn_wave_barrier();
+            if (queued >= 64) {
+                test(queued, 64);
+                queued -= 64;
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+    }
+    test(queued, queued);
     __syncthreads();
     for (int t = threadIdx.x; t < nb * kDppWords; t += kThreads) {
         const int bb = t / kDppWords, k = t % kDppWords;  // (kDppWords lanes per box, all of them here or none)
@@ -428,71 +568,85 @@ __global__ __launch_bounds__(kThreads) void dpp_emit_kernel(
     const int *__restrict__ box_base, int cap, int max_all, long long *__restrict__ out_pts_idx,
     long long *__restrict__ out_roi_idx, float *__restrict__ out_feats, int *__restrict__ num_out) {
 #pragma clang fp contract(off)
-    __shared__ unsigned short hit_s[kThreads * 64];  // the segment's hits: point - first point of the segment
+    // up to kDppListed of the segment's hits at a time: point - first point of the segment (room for all 16384 of
+    // them left a compute unit four workgroups, of which nearly all list a handful)
+    __shared__ unsigned short hit_s[kDppListed];
     const int b = blockIdx.y;
     const int tile0 = blockIdx.x * kDppSegTiles, tile1 = min(n_tiles, tile0 + kDppSegTiles);
     const bool reports = b == B - 1 && blockIdx.x == 0;
     const int *mine = counts + (size_t)b * n_tiles;
-    // hits of this box in front of the segment, and in it
-    int front = 0, here = 0;
+    // hits of this box in front of the segment, and in it; entries of the boxes in front, in two halves so
+    // that no sum leaves 32 bits.  Asked for and added up together: one after the other, each was a trip
+    // to memory or two barriers.
+    int sums[4] = {0, 0, 0, 0};
     for (int t = threadIdx.x; t < tile1; t += kThreads) {
         const int c = mine[t];
-        if (t < tile0) front += c; else here += c;
+        if (t < tile0) sums[0] += c; else sums[1] += c;
     }
-    block_exclusive_scan(front, &front);
-    block_exclusive_scan(here, &here);
-    if (!reports && (here == 0 || front >= cap)) return;  // (uniform)
-    long base = 0;
-    if (box_base) {
-        base = box_base[b];
-    } else {
-        // entries of the boxes in front, in two halves so that no sum leaves 32 bits
-        int lo = 0, hi = 0;
+    if (!box_base) {
         for (int k = threadIdx.x; k < b; k += kThreads) {
             const int kept = min(totals[(size_t)k * kDppTotalStep], cap);
-            lo += kept & 0xffff;
-            hi += kept >> 16;
+            sums[2] += kept & 0xffff;
+            sums[3] += kept >> 16;
         }
-        block_exclusive_scan(lo, &lo);
-        block_exclusive_scan(hi, &hi);
-        base = lo + ((long)hi << 16);
     }
+    __shared__ int sums_s[kThreads / 64][4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) sums[k] += __shfl_xor(sums[k], d, 64);
+        if ((threadIdx.x & 63) == 0) sums_s[threadIdx.x >> 6][k] = sums[k];
+    }
+    __syncthreads();
+    int front = 0, here = 0;
+    long base = box_base ? box_base[b] : 0;
+#pragma unroll
+    for (int k = 0; k < kThreads / 64; ++k) {
+        front += sums_s[k][0];
+        here += sums_s[k][1];
+        if (!box_base) base += sums_s[k][2] + ((long)sums_s[k][3] << 16);
+    }
+    if (!reports && (here == 0 || front >= cap)) return;  // (uniform)
     if (reports && threadIdx.x == 0) num_out[0] = (int)min((long)max_all, base + min(totals[(size_t)b * kDppTotalStep], cap));
     if (here == 0 || front >= cap || base + front >= max_all) return;
     const int word = tile0 * kDppWords + (int)threadIdx.x;
     unsigned long long m = word < tile1 * kDppWords ? masks[(size_t)b * n_tiles * kDppWords + word] : 0ull;
     int total;
-    int at = block_exclusive_scan(__popcll(m), &total);
-    while (m) {
-        hit_s[at++] = (unsigned short)((int)threadIdx.x * 64 + __builtin_ctzll(m));
-        m &= m - 1ull;
-    }
-    __syncthreads();
+    const int at = block_exclusive_scan(__popcll(m), &total);
     const DppBox bx = boxes[b];
     const long kept = min(min((long)total, (long)cap - front), max_all - base - front);
-    for (int h = threadIdx.x; h < kept; h += kThreads) {
-        const long pos = base + front + h;
-        const long p = (long)tile0 * kDppTile + hit_s[h];
-        const float x = pts[(size_t)p * 3], y = pts[(size_t)p * 3 + 1], z = pts[(size_t)p * 3 + 2];
-        float lx, ly;
-        const int flag = dpp_test(bx, x, y, z, lx, ly);  // the same arithmetic as in the first pass
-        const float local_z = (float)((double)z - ((double)bx.cz_bottom + (double)bx.h / 2.0));  // (:103)
-        float *f = out_feats + pos * kDppInfo;
-        out_pts_idx[pos] = p;
-        out_roi_idx[pos] = b;
-        f[0] = x;
-        f[1] = y;
-        f[2] = z;
-        f[3] = lx;
-        f[4] = ly;
-        f[5] = local_z;
-        f[6] = lx + bx.l / 2;
-        f[7] = ly + bx.w / 2;
-        f[8] = local_z + bx.h / 2;
-        f[9] = -lx + bx.l / 2;
-        f[10] = -ly + bx.w / 2;
-        f[11] = -local_z + bx.h / 2;
-        f[12] = flag == 1 ? 1.0f : 0.0f;
+    for (long listed = 0; listed < kept; listed += kDppListed) {
+        const int here_now = (int)min((long)kDppListed, kept - listed);
+        int place = at - (int)listed;
+        if (place + 64 > 0)
+            for (unsigned long long left = m; left != 0ull && place < here_now; left &= left - 1ull, ++place)
+                if (place >= 0) hit_s[place] = (unsigned short)((int)threadIdx.x * 64 + __builtin_ctzll(left));
+        __syncthreads();
+        for (int h = threadIdx.x; h < here_now; h += kThreads) {
+            const long pos = base + front + listed + h;
+            const long p = (long)tile0 * kDppTile + hit_s[h];
+            const float x = pts[(size_t)p * 3], y = pts[(size_t)p * 3 + 1], z = pts[(size_t)p * 3 + 2];
+            float lx, ly;
+            const int flag = dpp_test(bx, x, y, z, lx, ly);  // the same arithmetic as in the first pass
+            const float local_z = (float)((double)z - ((double)bx.cz_bottom + (double)bx.h / 2.0));  // (:103)
+            float *f = out_feats + pos * kDppInfo;
+            out_pts_idx[pos] = p;
+            out_roi_idx[pos] = b;
+            f[0] = x;
+            f[1] = y;
+            f[2] = z;
+            f[3] = lx;
+            f[4] = ly;
+            f[5] = local_z;
+            f[6] = lx + bx.l / 2;
+            f[7] = ly + bx.w / 2;
+            f[8] = local_z + bx.h / 2;
+            f[9] = -lx + bx.l / 2;
+            f[10] = -ly + bx.w / 2;
+            f[11] = -local_z + bx.h / 2;
+            f[12] = flag == 1 ? 1.0f : 0.0f;
+        }
+        __syncthreads();
     }
 }
 

@@ -576,7 +576,7 @@ std::tuple<Tensor, Tensor, Tensor> dynamic_point_pool(const Tensor &rois, const 
     Tensor idx = at::empty({max_all_pts}, pts.options().dtype(at::kLong));
     Tensor roi = at::empty({max_all_pts}, pts.options().dtype(at::kLong));
     Tensor feats = at::empty({max_all_pts, 13}, pts.options());
-    Tensor num = at::zeros({1}, iopt);
+    Tensor num = at::empty({1}, iopt);  // (written whatever the sizes)
     check_status(txs_dynamic_point_pool_mixed(B ? rois.data_ptr<float>() : nullptr, opt_i32p(rois_batch),
                                         P ? pts.data_ptr<float>() : nullptr, opt_i32p(pts_batch),
                                         B, P, extra, (int32_t)max_pts_per_box, max_all_pts, i32w(ws),
@@ -626,7 +626,7 @@ void dpp_into(const Tensor &rois, const OptTensor &rois_batch, const Tensor &pts
     const float extra[3] = {(float)extra_wlh[0], (float)extra_wlh[1], (float)extra_wlh[2]};
     auto iopt = pts.options().dtype(at::kInt);
     Tensor ws = at::empty({txs_dpp_workspace_len(P, B) + 2}, iopt);
-    Tensor num = at::zeros({1}, iopt);
+    Tensor num = at::empty({1}, iopt);  // (written whatever the sizes)
     check_status(txs_dynamic_point_pool_mixed(B ? rois.data_ptr<float>() : nullptr, opt_i32p(rois_batch),
                                               P ? pts.data_ptr<float>() : nullptr, opt_i32p(pts_batch), B, P, extra,
                                               (int32_t)max_pts_per_box, M, i32w(ws),
