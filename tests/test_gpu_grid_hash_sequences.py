@@ -43,3 +43,16 @@ def test_a_frames_columns():
     table = T.GridHash(near.cuda())
     assert torch.equal(table.probe(near.cuda()).cpu().long(), inv)
     assert len(table.valid_table) == len(unq)
+
+
+def test_a_grid_of_many_tiles():
+    """So large a grid that its tiles of cells are scanned before they are read."""
+    g = torch.Generator().manual_seed(1)
+    coors = torch.randint(0, 410, (1_200_000, 3), generator=g).int()
+    coors[0] = 409
+    key = (coors[:, 0].long() * 410 + coors[:, 1]) * 410 + coors[:, 2]
+    unq, inv = torch.unique(key, return_inverse=True)
+    table = T.GridHash(coors.cuda())
+    assert torch.equal(table.probe(coors.cuda()).cpu().long(), inv)
+    kept = table.valid_table.cpu().long()
+    assert torch.equal(torch.sort(kept[:, 0])[0], unq) and torch.equal(unq[kept[:, 1]], kept[:, 0])

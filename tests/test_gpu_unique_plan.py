@@ -108,3 +108,63 @@ def test_what_is_kept_per_voxel_is_bounded():
         kept = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes()
                 for t in (d.unq_cnts, d.preSum, d.slot_of, d.heavy_ids)}
         assert d.num_unq == 64 and sum(kept.values()) <= most + 64
+
+
+@pytest.mark.parametrize("n,bound,used", [(1 << 20, 1 << 26, 1 << 20), (4_300_000, 1 << 28, 50_000)])
+def test_maps_of_many_tiles(n, bound, used):
+    """The most tiles of cells whose keys are added up where the cells are read, and four times as many,
+    which are scanned first."""
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, used, n) * (bound // used)
+    keys[0], keys[1] = bound - 1, 0
+    _check(keys, bound, torch.int64)
+
+
+@pytest.mark.parametrize("is64", [0, 1])
+def test_few_keys_of_a_map_of_scanned_tiles(is64):
+    lib = _native.cabi()
+    vp, i64, bound, n = ctypes.c_void_p, ctypes.c_int64, (1 << 26) + 33, 5000
+    rng = np.random.default_rng(is64)
+    keys = rng.integers(0, bound, n)
+    keys[:2] = bound - 1, 0
+    keys[100:300] = keys[0]
+    unq, inv, cnt = np.unique(keys, return_inverse=True, return_counts=True)
+    lib.txs_unique_bitmap_workspace_len.restype = lib.txs_plan_workspace_len.restype = i64
+
+    def i32(m):
+        return torch.full((m,), -7, dtype=torch.int32, device="cuda")
+    k = torch.from_numpy(keys).to(torch.int64 if is64 else torch.int32).cuda()
+    bws, ws = i32(lib.txs_unique_bitmap_workspace_len(i64(bound))), i32(lib.txs_plan_workspace_len(i64(n), i64(n)))
+    o_inv, o_unq, perm, seg, pre, slot, heavy, stats = (i32(m) for m in (n, n, n, n, n + 1, n, n, 18))
+    o_cnt = torch.empty((n,), dtype=torch.int64, device="cuda")
+    rc = lib.txs_unique_plan(vp(k.data_ptr()), ctypes.c_int(is64), i64(n), i64(bound), vp(0), vp(bws.data_ptr()),
+                             ctypes.c_int32(64), vp(ws.data_ptr()), vp(o_inv.data_ptr()), vp(o_unq.data_ptr()),
+                             vp(o_cnt.data_ptr()), vp(perm.data_ptr()), vp(seg.data_ptr()), vp(pre.data_ptr()),
+                             vp(slot.data_ptr()), vp(heavy.data_ptr()), vp(stats.data_ptr()),
+                             vp(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    st, U = stats.cpu().numpy(), unq.size
+    assert st[16] == U and st[17] == 0 and st[8] == 0 and st[2] == cnt.max() and st[7] == (cnt > 64).sum()
+    assert np.array_equal(o_inv.cpu().numpy(), inv) and np.array_equal(o_unq.cpu().numpy()[:U], unq)
+    assert np.array_equal(o_cnt.cpu().numpy()[:U], cnt)
+    assert np.array_equal(perm.cpu().numpy(), np.argsort(inv, kind="stable"))
+    assert (o_unq.cpu().numpy()[U:] == -7).all()      # nothing behind the last key
+
+
+def test_points_and_their_keys_make_the_same_plan():
+    g = torch.Generator().manual_seed(2)
+    size, rng = [0.5, 0.4, 0.3], [-10.0, -8.0, -2.0, 10.0, 8.0, 2.0]
+    for n in (1, 1000, 50_001):
+        pts = torch.rand((n, 4), generator=g) * torch.tensor([19.9, 15.9, 3.9, 1.0]) + torch.tensor([-9.95, -7.95, -1.95, 0.0])
+        a = T.ScatterData.from_points(pts.cuda(), size, rng)
+        c = T.voxelize(pts.cuda(), size, rng)
+        assert torch.equal(a.coors, c) and a.spatial_size == [40, 40, 14]
+        b = T.ScatterData.from_keys((c[:, 0] * 40 + c[:, 1]) * 14 + c[:, 2], 40 * 40 * 14)
+        for x, y in ((a.unq_keys, b.unq_keys), (a.unq_inv, b.unq_inv), (a.unq_cnts, b.unq_cnts), (a.preSum, b.preSum),
+                     (a.seg, b.seg), (a.perm, b.perm)):
+            assert (x is None and y is None) or torch.equal(x, y)
+        for outside in (torch.tensor([30.0, 0, 0, 0]), torch.tensor([0, 0, -2.5, 0])):
+            bad = pts.clone()
+            bad[n // 2] = outside
+            with pytest.raises(RuntimeError):
+                T.ScatterData.from_points(bad.cuda(), size, rng)

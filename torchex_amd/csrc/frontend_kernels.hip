@@ -11,7 +11,7 @@
 // grid_hash (torchex/src/grid_hash/grid_hash_kernel.cu:19-49,
 // torchex/src/utils/functions.cuh:30-64).
 
-#include "txs_common.h"
+#include "key_map.h"
 #include "txs_internal.h"
 
 namespace {
@@ -970,13 +970,13 @@ int txs_detail::unique_plan_of_map(const void *keys, int key_is_int64, int64_t n
     const int64_t most = most_keys(num_total, key_bound);
     KeyMap m = key_map(b, keys, key_is_int64, key_bound, key_flag ? key_flag : b.bad, unq_keys, most);
     m.found = stats + TXS_STATS_LEN;
-    const bool fused = txs_detail::plan_takes_map(num_total, most);
-    if (!fused)
-        map_assign_kernel<<<dim3(blocks_for(num_total) + (unsigned)map_parts(m)), dim3(kThreads), 0, st>>>(m, num_total,
-                                                                                                       unq_inv);
+    if (txs_detail::plan_takes_map(num_total, most))
+        return txs_detail::plan_build_mapped(m, unq_inv, num_total, most, heavy_threshold, plan_ws, perm, seg, preSum,
+                                             slot_of, heavy_ids, stats, (long long *)unq_cnts, stream);
+    map_assign_kernel<<<dim3(blocks_for(num_total) + (unsigned)map_parts(m)), dim3(kThreads), 0, st>>>(m, num_total,
+                                                                                                   unq_inv);
     return txs_detail::plan_build(unq_inv, num_total, most, heavy_threshold, nullptr, plan_ws, perm, seg, preSum,
-                                  slot_of, heavy_ids, stats, nullptr, m.num_unq, (long long *)unq_cnts, nullptr,
-                                  fused ? &m : nullptr, stream);
+                                  slot_of, heavy_ids, stats, nullptr, m.num_unq, (long long *)unq_cnts, nullptr, stream);
 }
 
 extern "C" {
@@ -1162,7 +1162,7 @@ static int group_ranks(const long long *ids64, const int32_t *group_ids, int64_t
     const bool fused = txs_detail::plan_writes_ranks(num_total, num_groups);
     const int rc = txs_detail::plan_build(group_ids, num_total, num_groups, heavy, nullptr, plan_ws, perm, seg, preSum,
                                           nullptr, nullptr, stats, fused ? (long long *)out : nullptr, nullptr, nullptr,
-                                          ids64, nullptr, stream);
+                                          ids64, stream);
     if (rc != TXS_OK || fused) return rc;
     ingroup_inds_auto_kernel<<<dim3(blocks_for(num_total)), dim3(kThreads), 0, (hipStream_t)stream>>>(
         seg, perm, preSum, stats, num_total, (int)num_groups, (long long *)out);

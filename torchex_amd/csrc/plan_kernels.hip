@@ -9,7 +9,7 @@
 // (torchex/operator_py/scatter_op.py:7-21) and getPreSum
 // (torchex/src/scatter/scatter_kernel.cu:85-100).
 
-#include "txs_common.h"
+#include "key_map.h"
 
 #include <atomic>
 
@@ -1654,7 +1654,7 @@ int txs_plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, i
                    const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum,
                    int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream) {
     return txs_detail::plan_build(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum,
-                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, nullptr, nullptr, stream);
+                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, nullptr, stream);
 }
 
 int txs_plan_build_i64(const int64_t *ids, int32_t *unq_inv, int64_t num_total, int64_t num_unq,
@@ -1662,7 +1662,7 @@ int txs_plan_build_i64(const int64_t *ids, int32_t *unq_inv, int64_t num_total, 
                        int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids, int32_t *stats, void *stream) {
     if (num_total > 0 && !ids) return TXS_ERR_INVALID_ARG;
     return txs_detail::plan_build(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum,
-                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, (const long long *)ids, nullptr, stream);
+                                  slot_of, heavy_ids, stats, nullptr, nullptr, nullptr, (const long long *)ids, stream);
 }
 
 }  // extern "C"
@@ -1706,11 +1706,13 @@ bool txs_detail::plan_takes_map(long num_total, long num_unq) {
     return num_total > 0 && num_total <= kTiledRows && num_unq > 0 && radix_bits((int)(num_unq > 1 ? num_unq : 1)) <= kBucketBitsMax;
 }
 
-int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
-                           const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg,
-                           int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids, int32_t *stats,
-                           long long *ranks, const int *num_unq_dev, long long *cnts_out,
-                           const long long *ids64, const KeyMap *map, void *stream) {
+namespace {
+
+// map (may be NULL): see plan_build_mapped
+int build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold, const int64_t *unq_cnts,
+          int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids,
+          int32_t *stats, long long *ranks, const int *num_unq_dev, long long *cnts_out, const long long *ids64,
+          const KeyMap *map, void *stream) {
     if (!fits_i32(num_total) || !fits_i32(num_unq) || !stats || !preSum || heavy_threshold < kChunk)
         return TXS_ERR_INVALID_ARG;
     hipStream_t st = (hipStream_t)stream;
@@ -1832,4 +1834,23 @@ int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t nu
     else
         place(bucket_count_kernel<256, true>, bucket_plan_kernel<256, true>, sizeof(int) * plan_lds<256>(low_bins, tiles).ints);
     return status_of(hipGetLastError());
+}
+
+}  // namespace
+
+int txs_detail::plan_build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t heavy_threshold,
+                           const int64_t *unq_cnts, int32_t *plan_ws, int32_t *perm, int32_t *seg,
+                           int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids, int32_t *stats,
+                           long long *ranks, const int *num_unq_dev, long long *cnts_out,
+                           const long long *ids64, void *stream) {
+    return build(unq_inv, num_total, num_unq, heavy_threshold, unq_cnts, plan_ws, perm, seg, preSum, slot_of, heavy_ids,
+                 stats, ranks, num_unq_dev, cnts_out, ids64, nullptr, stream);
+}
+
+int txs_detail::plan_build_mapped(const KeyMap &map, int32_t *unq_inv, int64_t num_total, int64_t num_unq,
+                                  int32_t heavy_threshold, int32_t *plan_ws, int32_t *perm, int32_t *seg,
+                                  int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids, int32_t *stats,
+                                  long long *cnts_out, void *stream) {
+    return build(unq_inv, num_total, num_unq, heavy_threshold, nullptr, plan_ws, perm, seg, preSum, slot_of, heavy_ids,
+                 stats, nullptr, map.num_unq, cnts_out, nullptr, &map, stream);
 }
