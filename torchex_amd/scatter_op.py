@@ -184,7 +184,7 @@ class ScatterData:
         channel count and per stream (calls queued on one stream are ordered, and forwards
         that run concurrently on different streams each get a workspace of their own), the
         ``_SCRATCH_KEPT`` most recently used at most."""
-        key = (channel, torch.cuda.current_stream(self.seg.device).stream_id)
+        key = (channel, scatter_ext.stream_id(self.seg))
         buf = self._scratch.pop(key, None)
         if buf is None:
             buf = scatter_ext.make_scratch(self.num_total, channel, self.num_unq, self.num_heavy, self.seg)
