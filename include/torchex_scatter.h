@@ -178,9 +178,9 @@ int txs_plan_special(const int32_t *preSum, int64_t num_unq, int32_t heavy_thres
  * permutation, CSR offsets, special-voxel table, statistics and the flagged per-position
  * ids (what txs_plan_check, txs_plan_sort, txs_plan_presum, txs_plan_special and
  * txs_plan_seg_flag produce one after the other).  Up to 2^22 voxels this runs as a
- * bucket sort -- tile histograms of the high digit of the ids; scan; stable scatter by
- * bucket; then workgroups that sort a bucket's low digit in LDS and write the bucket's
- * slice of all outputs -- beyond that it runs the calls named above.
+ * bucket sort -- tiles of rows sorted by the high digit of the ids (above 2^24 rows: all rows
+ * moved to bucket order); then workgroups that sort a bucket's low digit in LDS and write the
+ * bucket's slice of all outputs -- beyond that it runs the calls named above.
  * stats [TXS_STATS_LEN] needs no initialisation for up to 2^22 voxels (also with no rows or
  * no voxels at all: the call clears it) and must be zero-filled by the caller beyond
  * (zero-filling always is fine); perm is left unwritten when
@@ -376,7 +376,7 @@ int txs_grid_hash_probe(const int32_t *keys, int64_t num_keys, const int32_t *ta
  *   txs_coor_max: the largest coordinate per axis, as txs_coor_max_parts() partial triples
  *     (int64 [parts, 3]) for the host to fold; dims = largest + 1.
  *   txs_coor_bitmap_count: occupancy bitmap of the linear keys (x * dims[1] + y) * dims[2] + z
- *     (cut to 32 bits) and its scanned population counts.  bitmap_ws: int32 array of
+ *     (cut to 32 bits), packed into cells.  bitmap_ws: int32 array of
  *     txs_unique_bitmap_workspace_len(dims[0] * dims[1] * dims[2]) entries, 16-byte aligned; its
  *     entries [off, off + 2), off = txs_coor_bitmap_count_offset(key bound), then hold the number
  *     of distinct keys and a flag, nonzero if a key lies outside [0, key bound).

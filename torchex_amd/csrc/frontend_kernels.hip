@@ -103,10 +103,10 @@ __global__ void unique_finish_kernel(const int *__restrict__ ks, const int *__re
 // ---- unique by occupancy map (keys from a bounded grid) ----------------------
 // One byte per possible key, set by plain stores (every writer stores the same 1, so no
 // atomic is needed; device-scope atomics on a bitmap were measured at 220 us for 1M keys),
-// then packed into one bit per key.  The dense id of a key is the number of occupied keys
-// below it: the exclusive scan of the words' population counts plus the bits below the key
-// inside its word.  That is the inverse torch.unique returns (ids ascend with the keys),
-// found without sorting the keys.
+// then packed into a cell per 32 keys.  The dense id of a key is the number of occupied keys
+// below it: those of the tiles of cells in front, of the cells in front in its tile, and the bits
+// below the key inside its cell.  That is the inverse torch.unique returns (ids ascend with the
+// keys), found without sorting the keys.
 
 // Where the keys come from: an array of them, or voxel coordinates [n, 3], linearised here
 // (x-major, and cut to 32 bits before the range check, as a caller who stores int32 keys would).

@@ -304,9 +304,9 @@ UniquePlan unique_plan_counted(const Tensor &keys, int64_t key_bound, int64_t he
 // Up to this many possible voxels the plan is queued without waiting for their number; above it
 // the count is read back first.  The one round trip saved is worth about 12 us.  Against that, ids of
 // up to 22 bits, which have to be provided for, mean up to 2048 buckets instead of 512, more bits send
-// the call to the general sequence, ids of at most 11 bits miss the shorter sequence that ends
-// with the bucket scatter, and what is kept per voxel is as long as the input (20 bytes a row).
-// ScatterData.from_points / from_keys, us, without waiting / counted first: 300k points of a sweep,
+// the call to the general sequence, and what is kept per voxel is as long as the input (20 bytes a row).
+// ScatterData.from_points / from_keys, us, without waiting / counted first (measured before rows were
+// sorted in tiles, which takes the same off both sides): 300k points of a sweep,
 // in pillars, in 0.32 m columns 117 / 128, 112 / 124, 101 / 113; 1M 146 / 144, 124 / 138, 117 / 127;
 // 2M 171 / 167, 140 / 153, 149 / 160; 4M 262 / 245, 207 / 212, 198 / 206; keys in 64 voxels 800k
 // 109 / 112, 2M 138 / 122, 4M 216 / 172; in 1024 of Zipf occupancy 800k 127 / 123, 2M 174 / 138.
