@@ -73,3 +73,24 @@ def test_boxes_of_every_reach():
         got = feats.cpu().numpy()
         assert np.array_equal(np.isnan(got), np.isnan(wf))
         assert np.array_equal(np.nan_to_num(got).view(np.uint32), np.nan_to_num(wf).view(np.uint32))
+
+
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("out", [-1e14, -1e10, -3e9, -5e8, -2e8, -1e6, -1e4, 1e4, 5e8, 1e14])
+def test_one_box_far_out_keeps_the_others(out, axis):
+    """One box of every group far out on either side, where the grid's cells are so wide that the sides of
+    all other boxes fall on its end."""
+    g = torch.Generator().manual_seed(5)
+    B, P = 70, 8000
+    rois = torch.zeros((B, 7))
+    rois[:, :2] = torch.rand((B, 2), generator=g) * 100.0 - 50.0
+    rois[:, 3:6] = torch.rand((B, 3), generator=g) * 5.0 + 0.5
+    rois[:, 6] = torch.rand((B,), generator=g) * 6.283
+    rois[[4, 40, 69], axis] = out
+    pts = torch.rand((P, 3), generator=g) * torch.tensor([110.0, 110.0, 4.0]) - torch.tensor([55.0, 55.0, 2.0])
+    pts[:B] = rois[:, :3] + torch.tensor([0.0, 0.0, 0.1])
+    idx, roi, feats = T.dynamic_point_pool(rois.cuda(), pts.cuda(), [0.3, 0.2, 0.1], 5000, 100_000)
+    wi, wr, wf = orc.dynamic_point_pool(rois.numpy(), pts.numpy(), [0.3, 0.2, 0.1], 5000, 100_000)
+    assert set(wr.tolist()) == set(range(B))
+    assert np.array_equal(idx.cpu().numpy(), wi) and np.array_equal(roi.cpu().numpy(), wr)
+    assert np.array_equal(feats.cpu().numpy().view(np.uint32), wf.view(np.uint32))

@@ -445,12 +445,14 @@ __global__ __launch_bounds__(kThreads) void dpp_mask_kernel(const float *__restr
         }
     }
     __syncthreads();
-    // a coordinate's place in the grid ascends with it, rounding included, so that a point inside a box's
-    // square lies in one of the cells from the place of its lower to that of its upper side
+    // a coordinate's place in the grid, and so its cell, ascends with it, rounding included, so that a point inside
+    // a box's square lies in one of the cells from that of its lower to that of its upper side.  Either side
+    // may round to the grid's very end (with one box far out on the negative side, those of all others do).
     auto place = [&](int axis, float v) { return (v - grid_s[axis]) * grid_s[2 + axis]; };
+    auto cell = [](float at) { return min(kDppCells - 1, max(0, (int)at)); };
     if (mine < nb && !far) {
-        const int x0 = max(0, (int)place(0, lo[0])), x1 = min(kDppCells - 1, (int)place(0, hi[0]));
-        const int y0 = max(0, (int)place(1, lo[1])), y1 = min(kDppCells - 1, (int)place(1, hi[1]));
+        const int x0 = cell(place(0, lo[0])), x1 = cell(place(0, hi[0]));
+        const int y0 = cell(place(1, lo[1])), y1 = cell(place(1, hi[1]));
         if ((x1 - x0 + 1) * (y1 - y0 + 1) > kDppCells * kDppCells / 2) {  // (most points are to be tested anyway)
             if (sub == 0) atomicOr(&everywhere_s, 1u << mine);
         } else {
@@ -498,8 +500,7 @@ __global__ __launch_bounds__(kThreads) void dpp_mask_kernel(const float *__restr
             const float gx = place(0, x[it]), gy = place(1, y[it]);
             // (a place at the very end may round up to kDppCells; NaN is nowhere)
             const bool inside = gx >= 0.0f && gx < kDppCells + 0.5f && gy >= 0.0f && gy < kDppCells + 0.5f;
-            const int cx = inside ? min((int)gx, kDppCells - 1) : 0, cy = inside ? min((int)gy, kDppCells - 1) : 0;
-            boxes_here = inside ? cells_s[cy * kDppCells + cx] : 0u;
+            boxes_here = inside ? cells_s[cell(gy) * kDppCells + cell(gx)] : 0u;
         }
         for (unsigned long long left = __ballot(boxes_here != 0u); left != 0ull; left = __ballot(boxes_here != 0u)) {
             // a box that many of the wave's points may lie in is put to the test at once
