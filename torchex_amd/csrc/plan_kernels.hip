@@ -1184,19 +1184,29 @@ struct PlanLds {
     int counts, first, step, seen, from, tot, front, ints;  // offsets in ints; counts: shared with the staged rows
 };
 template <int THREADS>
-__host__ __device__ __forceinline__ PlanLds plan_lds(int low_bins, int padded) {
+__host__ __device__ __forceinline__ constexpr PlanLds plan_lds(int low_bins, int padded) {
     const int bins = low_bins > 4 ? low_bins : 4, counts = bins / 2 * (THREADS / 64);
-    PlanLds l;
-    l.counts = 0;
+    PlanLds l = {};
     l.first = counts > plan_stage_ints<THREADS>() ? counts : plan_stage_ints<THREADS>();  // [bins] shorts
-    l.tot = l.first + bins / 2;                                                           // [bins] rows in the other slices
-    l.front = l.tot + bins;                                                               // [bins] ... and of those in front
-    l.step = l.tot;                                                                       // [bins] (in their place, by the thread that read them)
+    l.tot = (l.first + bins / 2 + 3) & ~3;  // [bins] rows in the other slices
+    l.front = l.tot + bins;                 // [bins] ... and of those in front
+    l.step = l.tot;                         // [bins] (in their place, by the thread that read them)
     l.seen = l.front + bins;
     l.from = l.seen + padded;
     l.ints = l.from + padded;
     return l;
 }
+// counts and first places are read two words at a time, the other three arrays four
+template <int THREADS>
+constexpr bool plan_lds_aligned() {
+    for (int bits = 0; bits <= kBucketLowBitsMax; ++bits)
+        for (int padded = 0; padded <= kTilesMax; padded = padded ? 2 * padded : 1) {
+            const PlanLds l = plan_lds<THREADS>(1 << bits, padded);
+            if (l.counts % 2 || l.first % 2 || l.tot % 4 || l.front % 4 || l.step % 4) return false;
+        }
+    return true;
+}
+static_assert(plan_lds_aligned<256>() && plan_lds_aligned<512>(), "vector accesses lie at their alignment");
 template <int THREADS, bool TILED>
 __global__ __launch_bounds__(THREADS) void bucket_plan_kernel(
     BucketArgs g, VoxelArgs v, int *__restrict__ perm, int *__restrict__ seg, int *__restrict__ stats,
