@@ -94,3 +94,26 @@ def test_one_box_far_out_keeps_the_others(out, axis):
     assert set(wr.tolist()) == set(range(B))
     assert np.array_equal(idx.cpu().numpy(), wi) and np.array_equal(roi.cpu().numpy(), wr)
     assert np.array_equal(feats.cpu().numpy().view(np.uint32), wf.view(np.uint32))
+
+
+def test_sides_at_the_ends_of_the_float_range():
+    """Half a side where a float cannot hold it, sides of no extent, negative ones and the largest, with points as
+    close to the box's centre and as far from it as floats go."""
+    tiny, big = float(np.float32(1e-45)), float(np.finfo(np.float32).max)
+    sides = [0.0, tiny, 2 * tiny, 3 * tiny, 5 * tiny, 1.0, big / 2, big, float("inf"), -1.0, -3 * tiny]
+    rois = torch.zeros((3 * len(sides), 7))
+    for k, s in enumerate(sides):
+        for axis in range(3):
+            rois[3 * k + axis, 3:6] = 2.0
+            rois[3 * k + axis, 3 + axis] = s
+    rois[:, 6] = -np.pi / 2       # no turn
+    near = [0.0, tiny, -tiny, 2 * tiny, -2 * tiny, 3 * tiny, 0.4, -0.4, 1.1, big / 2, -big / 2, big, -big]
+    pts = torch.tensor([[x, y, z] for x in near for y in near for z in near])
+    for extra in ([0.0, 0.0, 0.0], [tiny, 3 * tiny, tiny], [0.5, 0.5, 0.5]):
+        idx, roi, feats = T.dynamic_point_pool(rois.cuda(), pts.cuda(), extra, 3000, 200_000)
+        wi, wr, wf = orc.dynamic_point_pool(rois.numpy(), pts.numpy(), extra, 3000, 200_000)
+        assert wi.shape[0] > 1000
+        assert np.array_equal(idx.cpu().numpy(), wi) and np.array_equal(roi.cpu().numpy(), wr)
+        got = feats.cpu().numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(wf))
+        assert np.array_equal(np.nan_to_num(got).view(np.uint32), np.nan_to_num(wf).view(np.uint32))

@@ -271,7 +271,8 @@ __global__ void ingroup_inds_auto_kernel(const int *__restrict__ seg, const int 
 constexpr int kDppInfo = 13;
 
 struct DppBox {
-    float cx, cy, czc, w, l, h, cosa, sina, large_w, large_l, large_h, cz_bottom;
+    float cx, cy, czc, w, l, h, cosa, sina, cz_bottom;
+    float half_w, half_l, half_h, half_large_w, half_large_l, half_large_h;  // see half_of
     float r2;  // squared radius of a circle around (cx, cy) that contains the box and its margin
 };
 
@@ -279,6 +280,17 @@ struct DppBox {
 // complete one after the other, so every box's count has a line of its own: packed, 200 of
 // them on 7 lines, they held the first pass up (200 boxes, 200k points: 33-36 -> 27 us).
 constexpr int kDppTotalStep = 32;  // ints from one box's count to the next
+
+// The reference compares floats with (double)side / 2.0.  Half a side as a float is the same bound where it is
+// exact; the half of an odd multiple of the smallest float is not, and is then rounded `up` for v < half and
+// v > -half, down for v > half, which no float v can tell from the exact one.  (Tests in 64 bits: the first pass of
+// 32 boxes around all of 100k points 51.5 us, now 47.6.)
+__device__ __forceinline__ float half_of(float side, bool up) {
+    const float half = 0.5f * side;
+    if (up && half + half < side) return nextafterf(half, INFINITY);
+    if (!up && half + half > side) return nextafterf(half, -INFINITY);
+    return half;
+}
 
 // per-box constants, computed once so both passes see identical numbers; the
 // rotation terms are evaluated in double and rounded (within an ulp of any cosf)
@@ -295,17 +307,21 @@ __global__ void dpp_box_kernel(const float *__restrict__ rois, int B, float extr
     bx.w = r[3];
     bx.l = r[4];
     bx.h = r[5];
-    bx.large_w = bx.w + extra_w;
-    bx.large_l = bx.l + extra_l;
-    bx.large_h = bx.h + extra_h;
+    const float large_w = bx.w + extra_w, large_l = bx.l + extra_l, large_h = bx.h + extra_h;
+    bx.half_w = half_of(bx.w, true);
+    bx.half_l = half_of(bx.l, true);
+    bx.half_h = half_of(bx.h, true);
+    bx.half_large_w = half_of(large_w, true);
+    bx.half_large_l = half_of(large_l, true);
+    bx.half_large_h = half_of(large_h, false);
     bx.czc = (float)((double)r[2] + (double)bx.h / 2.0);  // bottom centre -> centre (:46)
     const float rot = (float)((double)r[6] + 3.14159265358979323846 / 2);  // (:24)
     bx.cosa = (float)cos((double)rot);
     bx.sina = (float)sin((double)rot);
     // generous bound (0.1 % + 1 mm^2): a point outside this circle fails the exact
     // test whatever the rounding, so skipping it cannot change the result
-    const float hl = 0.5f * fmaxf(fabsf(bx.l), fabsf(bx.large_l));
-    const float hw = 0.5f * fmaxf(fabsf(bx.w), fabsf(bx.large_w));
+    const float hl = 0.5f * fmaxf(fabsf(bx.l), fabsf(large_l));
+    const float hw = 0.5f * fmaxf(fabsf(bx.w), fabsf(large_w));
     bx.r2 = (hl * hl + hw * hw) * 1.001f + 1e-6f;
     boxes[b] = bx;
 }
@@ -320,16 +336,15 @@ __device__ __forceinline__ bool dpp_near(const DppBox &bx, float x, float y) {
 __device__ __forceinline__ int dpp_test(const DppBox &bx, float x, float y, float z, float &local_x,
                                         float &local_y) {
 #pragma clang fp contract(off)
-    if ((double)fabsf(z - bx.czc) > (double)bx.large_h / 2.0) return 0;
+    const float dz = fabsf(z - bx.czc);
+    if (dz > bx.half_large_h) return 0;
     const float sx = x - bx.cx, sy = y - bx.cy;
     local_x = sx * bx.cosa + sy * (-bx.sina);
     local_y = sx * bx.sina + sy * bx.cosa;
-    const double lx = local_x, ly = local_y;
-    const bool in_box = (lx > -(double)bx.l / 2.0) & (lx < (double)bx.l / 2.0) &
-                        (ly > -(double)bx.w / 2.0) & (ly < (double)bx.w / 2.0) &
-                        ((double)fabsf(z - bx.czc) < (double)bx.h / 2.0);
-    const bool in_large = (lx > -(double)bx.large_l / 2.0) & (lx < (double)bx.large_l / 2.0) &
-                          (ly > -(double)bx.large_w / 2.0) & (ly < (double)bx.large_w / 2.0);
+    const bool in_box = (local_x > -bx.half_l) & (local_x < bx.half_l) & (local_y > -bx.half_w) &
+                        (local_y < bx.half_w) & (dz < bx.half_h);
+    const bool in_large = (local_x > -bx.half_large_l) & (local_x < bx.half_large_l) &
+                          (local_y > -bx.half_large_w) & (local_y < bx.half_large_w);
     return in_box ? 2 : (in_large ? 1 : 0);
 }
 
@@ -461,8 +476,12 @@ __global__ __launch_bounds__(kThreads) void dpp_mask_kernel(const float *__restr
         }
     }
     __syncthreads();
-    // ---- boxes that are everywhere: every point, one box after the other
-    for (unsigned left = everywhere_s; left != 0u; left &= left - 1u) {
+    // ---- boxes that are everywhere: every point, one box after the other (heights in registers: read again for
+    // every box, each step of this chain waited for LDS as well)
+    float z[kDppItems];
+#pragma unroll
+    for (int it = 0; it < kDppItems; ++it) z[it] = pts_s[2][w * (64 * kDppItems) + it * 64 + lane];
+    for (unsigned left = __builtin_amdgcn_readfirstlane(everywhere_s); left != 0u; left &= left - 1u) {
         const int bb = __builtin_ctz(left);
         const DppBox &bx = boxes[b0 + bb];
         const int box_sample = rois_batch ? rois_batch[b0 + bb] : 0;
@@ -476,8 +495,7 @@ __global__ __launch_bounds__(kThreads) void dpp_mask_kernel(const float *__restr
 #pragma unroll
         for (int it = 0; it < kDppItems; ++it) {
             float lx, ly;
-            const float z = pts_s[2][w * (64 * kDppItems) + it * 64 + lane];
-            const unsigned long long hits = __ballot(near[it] && dpp_test(bx, x[it], y[it], z, lx, ly) != 0);
+            const unsigned long long hits = __ballot(near[it] && dpp_test(bx, x[it], y[it], z[it], lx, ly) != 0);
             if (lane == 0) m_s[bb][w * kDppItems + it] = hits;
         }
     }
