@@ -360,6 +360,8 @@ constexpr int kDppWords = kDppTile / 64;   // words of a tile per box
 constexpr int kDppGroup = 32;              // boxes per workgroup
 constexpr int kDppSegTiles = kThreads / kDppWords;  // tiles an emitting workgroup covers: one word per thread
 constexpr int kDppCells = 32;
+// Hits of a segment that are listed: with room for all 16384 points a compute unit took four of the emitting
+// workgroups, of which nearly all list a handful (200 boxes, 200k points, no cap: 56 us, now 53).
 constexpr int kDppListed = 8192;
 constexpr int kDppDense = 24;              // points of a wave that may lie in a box from which on they are not queued
 constexpr float kDppFar = 1e15f;           // boxes further out or larger than this are tested against every point
@@ -587,9 +589,13 @@ __global__ __launch_bounds__(kThreads) void dpp_emit_kernel(
     const int *__restrict__ box_base, int cap, int max_all, long long *__restrict__ out_pts_idx,
     long long *__restrict__ out_roi_idx, float *__restrict__ out_feats, int *__restrict__ num_out) {
 #pragma clang fp contract(off)
-    // up to kDppListed of the segment's hits at a time: point - first point of the segment (room for all 16384 of
-    // them left a compute unit four workgroups, of which nearly all list a handful)
-    __shared__ unsigned short hit_s[kDppListed];
+    // the segment's hits: point - first point of the segment; or, where there are more, its words and how many
+    // hits lie in front of each
+    __shared__ __align__(8) unsigned short hit_s[kDppListed];
+    constexpr int kWords = kDppSegTiles * kDppWords;
+    static_assert(kWords == kThreads && sizeof(hit_s) >= kWords * (sizeof(unsigned long long) + sizeof(int)), "a word a thread");
+    unsigned long long *word_s = reinterpret_cast<unsigned long long *>(hit_s);
+    int *first_s = reinterpret_cast<int *>(word_s + kWords);
     const int b = blockIdx.y;
     const int tile0 = blockIdx.x * kDppSegTiles, tile1 = min(n_tiles, tile0 + kDppSegTiles);
     const bool reports = b == B - 1 && blockIdx.x == 0;
@@ -634,38 +640,60 @@ __global__ __launch_bounds__(kThreads) void dpp_emit_kernel(
     const int at = block_exclusive_scan(__popcll(m), &total);
     const DppBox bx = boxes[b];
     const long kept = min(min((long)total, (long)cap - front), max_all - base - front);
-    for (long listed = 0; listed < kept; listed += kDppListed) {
-        const int here_now = (int)min((long)kDppListed, kept - listed);
-        int place = at - (int)listed;
-        if (place + 64 > 0)
-            for (unsigned long long left = m; left != 0ull && place < here_now; left &= left - 1ull, ++place)
-                if (place >= 0) hit_s[place] = (unsigned short)((int)threadIdx.x * 64 + __builtin_ctzll(left));
+    // point number p as entry number pos
+    auto emit = [&](long pos, long p, float x, float y, float z) {
+        float lx, ly;
+        const int flag = dpp_test(bx, x, y, z, lx, ly);  // the same arithmetic as in the first pass
+        const float local_z = (float)((double)z - ((double)bx.cz_bottom + (double)bx.h / 2.0));  // (:103)
+        float *f = out_feats + pos * kDppInfo;
+        out_pts_idx[pos] = p;
+        out_roi_idx[pos] = b;
+        f[0] = x;
+        f[1] = y;
+        f[2] = z;
+        f[3] = lx;
+        f[4] = ly;
+        f[5] = local_z;
+        f[6] = lx + bx.l / 2;
+        f[7] = ly + bx.w / 2;
+        f[8] = local_z + bx.h / 2;
+        f[9] = -lx + bx.l / 2;
+        f[10] = -ly + bx.w / 2;
+        f[11] = -local_z + bx.h / 2;
+        f[12] = flag == 1 ? 1.0f : 0.0f;
+    };
+    if (kept > kDppListed) {
+        // (uniform) over half of the segment's points: a lane per point, word by word.  (32 boxes around all of
+        // 100k points, the whole call: listed at once, with room for all, 129 us, in two rounds 136, so 123)
+        word_s[threadIdx.x] = m;
+        first_s[threadIdx.x] = at;
         __syncthreads();
-        for (int h = threadIdx.x; h < here_now; h += kThreads) {
-            const long pos = base + front + listed + h;
-            const long p = (long)tile0 * kDppTile + hit_s[h];
-            const float x = pts[(size_t)p * 3], y = pts[(size_t)p * 3 + 1], z = pts[(size_t)p * 3 + 2];
-            float lx, ly;
-            const int flag = dpp_test(bx, x, y, z, lx, ly);  // the same arithmetic as in the first pass
-            const float local_z = (float)((double)z - ((double)bx.cz_bottom + (double)bx.h / 2.0));  // (:103)
-            float *f = out_feats + pos * kDppInfo;
-            out_pts_idx[pos] = p;
-            out_roi_idx[pos] = b;
-            f[0] = x;
-            f[1] = y;
-            f[2] = z;
-            f[3] = lx;
-            f[4] = ly;
-            f[5] = local_z;
-            f[6] = lx + bx.l / 2;
-            f[7] = ly + bx.w / 2;
-            f[8] = local_z + bx.h / 2;
-            f[9] = -lx + bx.l / 2;
-            f[10] = -ly + bx.w / 2;
-            f[11] = -local_z + bx.h / 2;
-            f[12] = flag == 1 ? 1.0f : 0.0f;
+        const int lane = threadIdx.x & 63;
+        constexpr int kAhead = 4;  // words a wave asks for the points of at a time
+        for (int k0 = (threadIdx.x >> 6) * kAhead; k0 < kWords; k0 += kThreads / 64 * kAhead) {
+            float x[kAhead], y[kAhead], z[kAhead];
+            int h[kAhead];
+#pragma unroll
+            for (int r = 0; r < kAhead; ++r) {
+                const unsigned long long word = word_s[k0 + r];
+                h[r] = (word >> lane & 1ull) != 0ull ? first_s[k0 + r] + __popcll(word & ((1ull << lane) - 1ull)) : 0x7fffffff;
+                const long p = (long)tile0 * kDppTile + (h[r] < kept ? (k0 + r) * 64 + lane : 0);
+                x[r] = pts[p * 3];
+                y[r] = pts[p * 3 + 1];
+                z[r] = pts[p * 3 + 2];
+            }
+#pragma unroll
+            for (int r = 0; r < kAhead; ++r)
+                if (h[r] < kept) emit(base + front + h[r], (long)tile0 * kDppTile + (k0 + r) * 64 + lane, x[r], y[r], z[r]);
         }
-        __syncthreads();
+        return;
+    }
+    for (int place = at; m != 0ull && place < kept; m &= m - 1ull, ++place)
+        hit_s[place] = (unsigned short)((int)threadIdx.x * 64 + __builtin_ctzll(m));
+    __syncthreads();
+    for (int h = threadIdx.x; h < kept; h += kThreads) {
+        const long p = (long)tile0 * kDppTile + hit_s[h];
+        emit(base + front + h, p, pts[p * 3], pts[p * 3 + 1], pts[p * 3 + 2]);
     }
 }
 
