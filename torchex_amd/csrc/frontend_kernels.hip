@@ -542,11 +542,11 @@ __global__ __launch_bounds__(kThreads) void dpp_mask_kernel(const float *__restr
             if (meet) queue_s[w][queued + __popcll(m & lanes_below)] = (unsigned short)(bb << 10 | (w * (64 * kDppItems) + it * 64 + lane));
             queued += __popcll(m);
             boxes_here &= boxes_here - 1u;
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_fence();
             if (queued >= 64) {
                 test(queued, 64);
                 queued -= 64;
-                __builtin_amdgcn_wave_barrier();
+                wave_lds_fence();
             }
         }
     }
