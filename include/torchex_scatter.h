@@ -188,7 +188,9 @@ int txs_plan_special(const int32_t *preSum, int64_t num_unq, int32_t heavy_thres
  * for a caller that wants the order and the offsets only (the ranks of ingroup_inds): no
  * special-voxel table is made then, seg carries plain ids, and of the statistics only
  * UNSORTED, OUT_OF_RANGE and NEED_GENERAL are set.  plan_ws: int32 workspace of
- * txs_plan_workspace_len(num_total, num_unq) entries, 8-byte aligned.
+ * txs_plan_workspace_len(num_total, num_unq) entries, 8-byte aligned.  (This and every other
+ * workspace length is to be asked of the library that is loaded: it may change without the ABI
+ * version.)  What a call leaves in it is not for the caller.
  * One bucket holding more than 262,144 rows (a few voxels that own most of the rows)
  * makes the bucket kernels step aside: stats[NEED_GENERAL] is then 1, only
  * stats[UNSORTED] and stats[OUT_OF_RANGE] are valid, and the caller zero-fills stats

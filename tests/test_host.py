@@ -75,6 +75,14 @@ def test_host_only_entry_points():
     assert lib.txs_sort_workspace_len(ctypes.c_int64(n), ctypes.c_int64(120000)) >= 2 * n
 
 
+def test_index_preparation_needs_three_words_a_row_at_most():
+    lib = _lib()
+    lib.txs_plan_workspace_len.restype = ctypes.c_int64
+    for n in (200_000, 1_000_000, 1 << 20, 4_000_000, 1 << 24):
+        for u in (1, 1000, 70_000, n // 4, min(n, 1 << 22)):
+            assert lib.txs_plan_workspace_len(ctypes.c_int64(n), ctypes.c_int64(u)) <= 3 * n, (n, u)
+
+
 def test_argument_validation_needs_no_gpu():
     # these return before any launch
     lib = _lib()

@@ -1475,16 +1475,14 @@ struct PlanLayout {
     TileSplit split;                     // tiled
     int high_bits, hist_tiles, slice_threads;
     int64_t slices_more;                 // an upper bound of the further slices of all buckets
-    int64_t rows, offs;                  // tiled; the (id, row) pairs of the other route start the workspace
+    int64_t rows, offs;                  // tiled; the other route starts with the (id, row) pairs
     int64_t hist, scan_ws;               // otherwise
     int64_t tile_flags, bucket_start, ctl, part_hist, len;
 };
 PlanLayout plan_layout(int64_t n, int bits) {
     PlanLayout l = {};
     l.tiled = n <= kTiledRows;
-    // The rows in tile order do not take the place of the pairs: a call that steps aside for an
-    // overfull bucket leaves that untouched.
-    int64_t at = 2 * n;
+    int64_t at = 0;
     auto take = [&at](int64_t entries) {
         const int64_t here = at;
         at += entries;
@@ -1498,6 +1496,7 @@ PlanLayout plan_layout(int64_t n, int bits) {
         l.offs = take((int64_t)l.split.tiles * l.split.pitch / 2);
         l.tile_flags = take(l.split.tiles);
     } else {
+        take(2 * n);
         // the bucket digit has 9 bits (narrower, and the buckets of a spatially sorted id space get too
         // uneven; wider, and a tile sends too few rows to a bucket for the scatter to write whole cache
         // lines) and the low digit takes the rest, at most 11
