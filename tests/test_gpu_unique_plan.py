@@ -40,6 +40,18 @@ def test_one_voxel_owns_most_rows(n, voxels, rows):
     _check(rng.permutation(keys), 1 << 23, torch.int32)
 
 
+@pytest.mark.parametrize("used,dtype", [(1500, torch.int32), (2048, torch.int64), (2049, torch.int32), (70_000, torch.int64),
+                                        (1 << 20, torch.int32)])
+def test_more_rows_than_are_sorted_in_tiles(used, dtype):
+    """Above 2^24 rows, with the number of voxels on the device only: the host provides for ids of 20 bits,
+    and a bucket is a voxel (at most 2048 of them) or many."""
+    n, bound = (1 << 24) + 1, 1 << 20
+    rng = np.random.default_rng(used)
+    keys = rng.integers(0, used, n) * (bound // used)
+    keys[0] = bound - 1
+    _check(keys, bound, dtype)
+
+
 def _check(keys, bound, dtype):
     unq, inv, cnt = np.unique(keys, return_inverse=True, return_counts=True)
     d = T.ScatterData.from_keys(torch.from_numpy(keys).to(dtype).cuda(), bound)
