@@ -21,6 +21,7 @@ pytestmark = pytest.mark.gpu
     (20_000, (1 << 25) + 1, 20_000), (60_000, 1 << 24, 1 << 24), (400_000, 1 << 20, 3), (400_000, 1 << 20, 5000),
     (4_300_000, 1 << 22, 1 << 22), (1 << 20, 1 << 24, 700), ((1 << 20) + 1, 1 << 24, 700),
     ((1 << 20) + 1, 1 << 24, 1 << 24), (1_000_000, 1 << 23, 2000), (4_300_000, 1 << 23, 90_000),
+    (1 << 21, 1 << 20, 70_000), ((1 << 21) + 1, 1 << 20, 70_000), (2_098_000, 1 << 20, 1500), (2_100_000, 3, 3),
 ])
 def test_unique_plan(n, bound, used, dtype):
     rng = np.random.default_rng(n + bound)

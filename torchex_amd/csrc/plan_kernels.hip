@@ -440,6 +440,7 @@ __device__ __forceinline__ int voxel_count(int U_arg, const int *__restrict__ nu
 constexpr int kTileRowsMax = 8192;
 constexpr int kTilesMax = 2048;
 constexpr long kTiledRows = (long)kTileRowsMax * kTilesMax;
+constexpr long kMappedRows = 1L << 21;  // rows up to which ids are looked up by the kernel that sorts the tiles
 struct TileSplit {
     int tile_bits;   // log2(rows per tile)
     int high_bits;
@@ -448,7 +449,7 @@ struct TileSplit {
 };
 TileSplit tile_split(long n, int bits) {
     TileSplit r;
-    r.tile_bits = n <= (1L << 18) ? 10 : (n <= (5L << 18) ? 11 : (n <= (1L << 21) ? 12 : 13));
+    r.tile_bits = n <= (1L << 18) ? 10 : (n <= (5L << 18) ? 11 : (n <= kMappedRows ? 12 : 13));
     r.high_bits = bits <= kBucketLowBitsMax ? bits : min(max(kBucketHighBits, bits - 10), kBucketLowBitsMax);
     if (r.high_bits > 10 && r.tile_bits < 11) r.tile_bits = 11;  // (256 threads scan at most 1024 buckets)
     r.tiles = (int)((n + (1L << r.tile_bits) - 1) >> r.tile_bits);
@@ -1711,8 +1712,11 @@ bool txs_detail::plan_writes_ranks(long num_total, long num_unq) {
     return num_total > 0 && num_unq > 0 && bits <= kBucketBitsMax;
 }
 
+// Above kMappedRows rows, in tiles of 8192, a thread would hold 16 rows' keys and cells: 199 registers, one workgroup
+// on a compute unit.  A kernel for the ids alone, which the sorting kernel then reads, is faster there: 2.2M keys in
+// 2^20 139 -> 132 us, 8M 295 -> 276, 16M 582 -> 517 (8M of 2048 keys 265 -> 238, 16M 462 -> 405).
 bool txs_detail::plan_takes_map(long num_total, long num_unq) {
-    return num_total > 0 && num_total <= kTiledRows && num_unq > 0 && radix_bits((int)(num_unq > 1 ? num_unq : 1)) <= kBucketBitsMax;
+    return num_total > 0 && num_total <= kMappedRows && num_unq > 0 && radix_bits((int)(num_unq > 1 ? num_unq : 1)) <= kBucketBitsMax;
 }
 
 namespace {
@@ -1722,6 +1726,7 @@ int build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t he
           int32_t *plan_ws, int32_t *perm, int32_t *seg, int32_t *preSum, int32_t *slot_of, int32_t *heavy_ids,
           int32_t *stats, long long *ranks, const int *num_unq_dev, long long *cnts_out, const long long *ids64,
           const KeyMap *map, void *stream) {
+    if (map && !txs_detail::plan_takes_map(num_total, num_unq)) return TXS_ERR_INVALID_ARG;
     if (!fits_i32(num_total) || !fits_i32(num_unq) || !stats || !preSum || heavy_threshold < kChunk)
         return TXS_ERR_INVALID_ARG;
     hipStream_t st = (hipStream_t)stream;
@@ -1783,8 +1788,9 @@ int build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t he
             using K = std::remove_const_t<std::remove_pointer_t<decltype(ids)>>;
             auto kernel = t.tile_bits == 10   ? tile_sort_kernel<256, 4, K>
                           : t.tile_bits == 11 ? tile_sort_kernel<512, 4, K>
-                          : t.tile_bits == 12 ? tile_sort_kernel<512, 8, K>
-                                              : tile_sort_kernel<512, 16, K>;
+                                              : tile_sort_kernel<512, 8, K>;
+            if constexpr (!std::is_same_v<K, KeyMap>)
+                if (t.tile_bits == 13) kernel = tile_sort_kernel<512, 16, K>;
             kernel<<<dim3(t.tiles + more), dim3(tile_threads), lds, st>>>(ids, n, t.tiles, U, t.high_bits, rows, offs, t.pitch,
                                                                           tile_flags, ids32, stats, ctl, num_unq_dev);
         };
