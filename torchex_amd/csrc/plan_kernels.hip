@@ -436,7 +436,15 @@ __device__ __forceinline__ int voxel_count(int U_arg, const int *__restrict__ nu
     return num_unq_dev ? min(U_arg, *num_unq_dev) : U_arg;
 }
 
-// How the rows are cut into tiles and the ids into digits, for ids of `bits` bits.
+// How the rows are cut into tiles and the ids into digits, for ids of `bits` bits.  Short tiles keep workgroups
+// short and many, long ones leave fewer runs of a bucket to find.  Plans of a sweep, of rows in clusters of 4 and of 50, us
+// a call with their host read, on either side of the lines:
+//   2^18 rows (tiles of 1024 / 2048): 60k rows 48 / 48, 49 / 49, 50 / 50; 2^18 53 / 53, 51 / 51, 53 / 52.  256 threads, which
+//     serve a slice best up to here (below), look at 256 tiles at most.
+//   5 * 2^18 rows (2048 / 4096): plans gain 1 - 4 % from the longer tiles from 600k rows on (1M 74 / 72, 62 / 60, 66 / 63; 1.5M
+//     80 / 78, 81 / 77, 74 / 74), plans from keys, whose ids are looked up on the way, lose up to 9 % (1M 116 / 117,
+//     105 / 111, 103 / 107; 1.3M 114 / 116, 103 / 110, 114 / 115).
+//   2^21 rows (4096 / 8192): 2.1M 87 / 88, 89 / 87, 86 / 85; 4M 123 / 118, 138 / 125, 114 / 106.
 constexpr int kTileRowsMax = 8192;
 constexpr int kTilesMax = 2048;
 constexpr long kTiledRows = (long)kTileRowsMax * kTilesMax;
@@ -456,8 +464,10 @@ TileSplit tile_split(long n, int bits) {
     r.pitch = max(1 << r.high_bits, 4) + 4;
     return r;
 }
-// threads of the workgroups that serve a slice of kBktItems rows per thread
-int slice_threads_for(long n, int low_bits) { return n > (1L << 19) || low_bits > 10 ? 512 : 256; }  // (four voxels a thread)
+// Threads of the workgroups that serve a slice of kBktItems rows per thread: 256 while they can look at all tiles
+// (256 of them; 2^19 rows) and at all of a bucket's voxels (four a thread).  256 / 512: 60k rows in 1500 voxels 47 / 56 us a
+// plan, grouped 51 / 61; 262k in 1500 voxels 52 / 60, a sweep 53 / 50; 2^19 rows 62 / 63 and 56 / 63.
+int slice_threads_for(long n, int low_bits) { return n > (1L << 19) || low_bits > 10 ? 512 : 256; }
 
 // exclusive scan of one int per thread across a workgroup of WAVES wavefronts
 template <int WAVES>
@@ -1042,7 +1052,7 @@ struct BucketRows {
     int u_lo, start;
     // Low digits and rows at COUNT positions inside the bucket.  Nothing here is under a branch, so that
     // the searches advance side by side and all loads are in flight before the first is used (each under
-    // its own condition, one after the other: ranks of 1M ids 77 us in bucket_plan_kernel, 46 so).
+    // its own condition, one after the other: ranks of 1M ids 77 us in bucket_plan_kernel as it was then, 46 so; 25 by now).
     template <int COUNT>
     __device__ __forceinline__ void get(const int (&p)[COUNT], int (&dig)[COUNT], int (&row)[COUNT]) const {
         if (TILED) {
@@ -1174,7 +1184,7 @@ __global__ __launch_bounds__(THREADS) void bucket_count_kernel(BucketArgs g, con
 // lanes to neighbouring addresses; ranks leave at once.
 // What bounds it is the chain of dependent steps inside a workgroup, about 10 us for a slice (bounds 0.5,
 // runs in the tiles 1.5, rows 2-3, ranking 2-3, scans 1.5, slots 1, places and stores 1.5), far more
-// than bytes: 64 vector registers and 37 KB of LDS keep three or four workgroups of 512 threads on a compute unit.
+// than bytes: 66 vector registers, seven waves a SIMD, keep three workgroups of 512 threads on a compute unit.
 // Index preparation in all, us a call with its host read, against rows moved to bucket order first and a
 // voxel's rows ranked by counting the smaller ones: sweeps 200k 72 -> 52, 1M 93 -> 74, 4M 138 -> 123,
 // pillars 1M 95 -> 68, 1M ids of 4 / 50 / 400 rows per voxel 80 -> 62, 93 -> 66, 91 -> 67, 2M of 20,000 Zipf
@@ -1712,8 +1722,10 @@ bool txs_detail::plan_writes_ranks(long num_total, long num_unq) {
     return num_total > 0 && num_unq > 0 && bits <= kBucketBitsMax;
 }
 
-// Above kMappedRows rows, in tiles of 8192, a thread would hold 16 rows' keys and cells: 199 registers, one workgroup
-// on a compute unit.  A kernel for the ids alone, which the sorting kernel then reads, is faster there: 2.2M keys in
+// Up to kMappedRows rows the lookup on the way saves a pass and a launch (sweeps, pillars, clusters, grouped rows; looked up
+// on the way / apart: 140k keys 79 - 89 / 84 - 92 us, 1M 91 - 115 / 97 - 118, 2M 105 - 127 / 110 - 131).  Above, in tiles of 8192,
+// a thread would hold 16 rows' keys and cells: 199 registers, one workgroup on a compute unit.  A kernel for the ids
+// alone, which the sorting kernel then reads, is faster there: 2.2M keys in
 // 2^20 139 -> 132 us, 8M 295 -> 276, 16M 582 -> 517 (8M of 2048 keys 265 -> 238, 16M 462 -> 405).
 bool txs_detail::plan_takes_map(long num_total, long num_unq) {
     return num_total > 0 && num_total <= kMappedRows && num_unq > 0 && radix_bits((int)(num_unq > 1 ? num_unq : 1)) <= kBucketBitsMax;

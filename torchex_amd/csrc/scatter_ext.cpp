@@ -302,14 +302,12 @@ UniquePlan unique_plan_counted(const Tensor &keys, int64_t key_bound, int64_t he
 }
 
 // Up to this many possible voxels the plan is queued without waiting for their number; above it
-// the count is read back first.  The one round trip saved is worth about 12 us.  Against that, ids of
-// up to 22 bits, which have to be provided for, mean up to 2048 buckets instead of 512, more bits send
-// the call to the general sequence, and what is kept per voxel is as long as the input (20 bytes a row).
-// ScatterData.from_points / from_keys, us, without waiting / counted first (measured before rows were
-// sorted in tiles, which takes the same off both sides): 300k points of a sweep,
-// in pillars, in 0.32 m columns 117 / 128, 112 / 124, 101 / 113; 1M 146 / 144, 124 / 138, 117 / 127;
-// 2M 171 / 167, 140 / 153, 149 / 160; 4M 262 / 245, 207 / 212, 198 / 206; keys in 64 voxels 800k
-// 109 / 112, 2M 138 / 122, 4M 216 / 172; in 1024 of Zipf occupancy 800k 127 / 123, 2M 174 / 138.
+// the count is read back first.  The line lies where it does for memory: without the count, what is kept
+// per voxel for as long as the ScatterData is as long as the input (20 bytes a row, 20 MB at the line).  In
+// time, ScatterData.from_points / from_keys, us, without waiting / counted first: 300k points of a sweep,
+// in pillars, in 0.32 m columns 94 / 108, 92 / 102, 93 / 103; 1M 119 / 127, 111 / 116, 105 / 115;
+// 2M 146 / 150, 126 / 134, 117 / 130; 4M 201 / 211, 166 / 182, 161 / 174; keys in 64 voxels 1M
+// 90 / 98, 2M 107 / 109, 4M 136 / 135; in 1024 of Zipf occupancy 1M 98 / 107, 2M 113 / 117, 4M 146 / 145.
 constexpr int64_t kUncountedVoxels = int64_t(1) << 20;
 
 // Whether the number of voxels is left on the device: an occupancy map, and few enough of them.
