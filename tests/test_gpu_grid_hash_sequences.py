@@ -1,6 +1,6 @@
 """Grid hash keys that share one probe sequence: keys equal modulo the table's size start in the same slot and
-step alike, so that the n-th one has to pass n - 1 taken slots.  Lengths on either side of what a lane
-looks at by itself (17 slots), of the 64 more a wave looks at at once, and a table that is full."""
+step alike, so that the n-th one has to pass n - 1 taken slots.  Lengths on either side of what a lane looks at by
+itself and of what a wave's lanes look at for a few keys or one, nearly full tables, and a table that is full."""
 import numpy as np
 import pytest
 import torch
@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("shuffled", [False, True])
-@pytest.mark.parametrize("n", [1, 2, 17, 18, 19, 80, 81, 82, 146, 1000, 4096])
+@pytest.mark.parametrize("n", [1, 2, 9, 16, 17, 18, 19, 33, 34, 63, 64, 65, 80, 81, 82, 146, 288, 1000, 4096])
 def test_keys_of_one_sequence(n, shuffled):
     size = 1 << max(0, (n - 1).bit_length())
     rng = np.random.default_rng(n)
@@ -30,6 +30,31 @@ def test_keys_of_one_sequence(n, shuffled):
     known = dict(zip(keys[:n].tolist(), values.tolist()))
     got = T.grid_hash_probe(torch.from_numpy(asked[order]).cuda(), table).cpu().numpy()
     assert np.array_equal(got, [known.get(int(k), -1) for k in asked[order]])
+
+
+@pytest.mark.parametrize("n,probes", [(1000, 5000), (30_000, 70_001), (65_536, 100_000), (3 << 17, 1 << 20),
+                                      ((3 << 17) + 1, (1 << 20) + 1)])
+def test_one_long_sequence_among_many_short_ones(n, probes):
+    """Numbers of keys on either side of where fewer of them get the lanes of others; 300 keys of one sequence, next to
+    each other and then anywhere, among keys that find a slot soon (or, in a table that is nearly full, do not)."""
+    size = 1 << (n - 1).bit_length()
+    rng = np.random.default_rng(n)
+    others = np.setdiff1d(rng.integers(0, 2**31 - 1, 2 * n), 5 + size * np.arange(600))
+    keys = np.concatenate([5 + size * np.arange(300), rng.permutation(others)[: n - 300]]).astype(np.int32)
+    for order in (np.arange(n), rng.permutation(n)):
+        placed, values = keys[order], rng.permutation(n).astype(np.int32)
+        table = T.grid_hash_build(torch.from_numpy(placed).cuda(), torch.from_numpy(values).cuda())
+        asked = np.concatenate([placed[:probes // 2], 5 + size * np.arange(600),
+                                rng.integers(0, 2**31 - 1, probes)])[:probes].astype(np.int32)
+        asked = rng.permutation(asked)
+        by_key = np.argsort(placed, kind="stable")
+        at = np.minimum(np.searchsorted(placed[by_key], asked), n - 1)
+        want = np.where(placed[by_key][at] == asked, values[by_key][at], -1)
+        if n == size:     # (an absent key is looked for in every slot of a full table)
+            asked, want = asked[want >= 0], want[want >= 0]
+        assert np.array_equal(T.grid_hash_probe(torch.from_numpy(asked).cuda(), table).cpu().numpy(), want)
+        host = table.cpu().numpy()
+        assert np.array_equal(np.sort(host[host[:, 0] != -1, 0]), np.sort(placed))
 
 
 def test_a_frames_columns():

@@ -726,12 +726,54 @@ __device__ __forceinline__ int grid_hash_slot(int key, int probe_i, int table_si
     return (int)(((k & mask) + (unsigned long long)probe_i * (k * 2ull + 1ull)) & mask);
 }
 
-// A key's probe sequence is followed by its own lane for kHashOwn slots (the first one by itself, then
-// kHashStep at a time); what is left of it is looked at by the whole wave, 64 slots at a time.  The mean key needs 1.3 - 2.2 slots, but where the grid's strides fall
-// badly on the table's size (a frame's 748 x 30 cells a column, 2^18 slots) a few need hundreds, and the
-// kernels waited for those alone, a trip to memory per slot: 146k keys built in 13 / 48 / 226 us and 300k
-// probed in 11 / 47 / 111, by the frame; now 16 / 20 / 28 and 7 / 8 / 10.
-constexpr int kHashStep = 4, kHashOwn = 1 + 4 * kHashStep;
+// The probe sequences of a wave's keys are followed together.  While many keys are still looking, each looks at its
+// next slot with its own lane; as they become fewer, the wave's lanes are dealt out among them and every key
+// looks at more slots of its sequence at a time, in order.  The mean key needs 1.3 - 2.2 slots, but where the grid's
+// strides fall badly on the table's size (a frame's 748 x 30 cells a column, 2^18 slots) a few need hundreds.  With a
+// lane to a key to the end, the kernels waited for those alone, a trip to memory per slot: 146k keys of a frame built
+// in 13 / 218 us and 300k probed in 7 / 100, by the frame, now 13 / 23 and 6 / 9.  (With a lane to a key for 17 slots and the
+// wave's lanes for one key after the other from there on, and keys in order spread over all waves, which takes
+// a line for each: 16 / 27, and 1M keys in order 50 us against 17 now and with a lane to a key, 3M probes 115 against 86.)
+//
+// How long a key keeps its own lane, us a call with it / with lanes dealt out at once:
+//   placing, up to kHashFewBuilt keys, which wait for trips to memory: while more than 16 keys of the wave look.  A key
+//     tries its slot at once, where a group looks first: a trip more.  In a crowd of long sequences that lasts
+//     kHashCrowd slots, as looking ahead is cheaper than trying: 262k keys in 2^18 slots 3010 / 1210, then 1440;
+//     262k keys 448 apart 404 / 723.
+//   placing, more keys: kHashOwnMany slots while more than 8 keys look.  600k keys 55 / 88, 3M 234 / 361, 1M keys 448 apart
+//     1240 (no end to it) / 668.
+//   looking, up to kHashFewProbes keys: while more than 32 keys look.  1M absent keys in a table 0.95 full 290, 397 as above.
+//   looking, more keys, which wait for the memory itself, so that what is looked at behind a sequence's end costs
+//     time: kHashOwn slots.  3M coordinates 86 / 146, 3M absent keys 194 / 275, 2M in a table 0.95 full 646 / 834.
+// From kHashLong slots on, the sequences left are long ones, and a lane asks for kHashAhead slots at a time.
+constexpr int kHashLong = 32, kHashAhead = 4;
+constexpr long kHashFewBuilt = 3L << 17, kHashFewProbes = 1L << 20;
+constexpr int kHashCrowd = 64, kHashOwnMany = 8, kHashOwn = 128;
+
+// How a wave's lanes are dealt out among the keys that are still looking: a group of 2^log2 lanes each, the first
+// key's first.
+struct HashDeal {
+    int log2, group, rank;       // the group this lane works in, and the one that works for this lane's key
+    unsigned long long members;  // the lanes of a group, shifted to the first one's place
+    int from;                    // the lane whose key the group works for
+    bool works;                  // the group works for a key
+    __device__ __forceinline__ HashDeal(unsigned long long looking) {
+        const int lane = threadIdx.x & 63, keys = __popcll(looking);
+        const unsigned long long below = (1ull << lane) - 1ull;
+        log2 = 6 - (keys > 1 ? 32 - __builtin_clz((unsigned)(keys - 1)) : 0);
+        group = lane >> log2;
+        const bool looks = (looking >> lane & 1ull) != 0ull;
+        rank = looks ? __popcll(looking & below) : 0;
+        members = log2 == 6 ? ~0ull : (1ull << (1 << log2)) - 1ull;
+        works = group < keys;
+        // every lane's number, those that are looking first
+        const int place = looks ? rank : keys + __popcll(~looking & below);
+        from = __shfl(__builtin_amdgcn_ds_permute(place << 2, lane), group, 64);
+    }
+    // of a ballot, what the group that works in this lane / for this lane's key has left there
+    __device__ __forceinline__ unsigned long long here(unsigned long long ballot) const { return (ballot >> (group << log2)) & members; }
+    __device__ __forceinline__ unsigned long long mine(unsigned long long ballot) const { return (ballot >> (rank << log2)) & members; }
+};
 
 // A slot as it is now or was a moment ago.  A slot only ever goes from empty to taken, so that one seen taken
 // is, and one seen empty may be (the compare-and-swap decides).
@@ -739,95 +781,143 @@ __device__ __forceinline__ unsigned long long grid_hash_peek(const unsigned long
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// values == NULL: key number i gets the value i
+// Slots number t0 + k of a group's key, for k < AHEAD << deal.log2: the first empty one is taken, or the next one
+// if that was taken in between, by all groups at a time.  pending: this lane's key has no slot yet.
+template <int AHEAD>
+__device__ __forceinline__ void hash_place(const HashDeal &deal, int t0, int key, unsigned long long word,
+                                           unsigned long long *__restrict__ table, int table_size, bool &pending) {
+    constexpr unsigned long long kEmpty = ~0ull;  // (-1, -1)
+    const int lane = threadIdx.x & 63, step = 1 << deal.log2, part = lane & (step - 1);
+    const int k = __shfl(key, deal.from, 64);
+    const unsigned long long w = ((unsigned long long)(unsigned)__shfl((int)(word >> 32), deal.from, 64) << 32) | (unsigned)k;
+    unsigned empty = 0u;  // of this lane's slots, a bit each
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a) {
+        const int t = t0 + a * step + part;
+        const unsigned long long seen = grid_hash_peek(table + grid_hash_slot(k, min(t, table_size - 1), table_size));
+        if (deal.works && t < table_size && seen == kEmpty) empty |= 1u << a;
+    }
+    unsigned long long placed = 0ull;  // lanes that have placed their group's key
+    while (__ballot(empty != 0u) != 0ull) {  // (every turn takes a bit from every group that has one)
+        // the group's first empty slot
+        int first = -1;
+        bool tries = false;
+#pragma unroll
+        for (int a = 0; a < AHEAD; ++a) {
+            const unsigned long long here = deal.here(__ballot((empty >> a & 1u) != 0u));
+            if (first < 0 && here != 0ull) {
+                first = a;
+                tries = part == __builtin_ctzll(here);
+            }
+        }
+        bool done = false;
+        if (tries) {
+            done = atomicCAS(table + grid_hash_slot(k, t0 + first * step + part, table_size), kEmpty, w) == kEmpty;
+            empty &= ~(1u << first);
+        }
+        placed |= __ballot(done);
+        if (deal.here(placed) != 0ull) empty = 0u;
+    }
+    if (pending && deal.mine(placed) != 0ull) pending = false;
+}
+
+// values == NULL: key number i gets the value i.  few: at most kHashFewBuilt keys
 __global__ __launch_bounds__(kThreads) void grid_hash_build_kernel(const int *__restrict__ keys,
                                                                    const int *__restrict__ values,
                                                                    unsigned long long *__restrict__ table,
-                                                                   int table_size, long n, int *__restrict__ fail) {
-    // neighbouring keys (those with long sequences are, where the keys are in order) go to different waves
+                                                                   int table_size, long n, bool few, int *__restrict__ fail) {
     const int lane = threadIdx.x & 63;
-    const long i = (long)lane * gridDim.x * (kThreads / 64) + (long)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+    const long wave = (long)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6), waves = (long)gridDim.x * (kThreads / 64);
+    // keys next to each other (those with long sequences are, where the keys are in order, and slots too) stay so
+    // by four only, where they are few: a wave with many long sequences is what the call waits for
+    const int near = few ? 2 : 6;
+    const long i = (((lane >> near) * waves + wave) << near) + (lane & ((1 << near) - 1));
     const int key = i < n ? keys[i] : -1;
     const unsigned value = i < n ? (unsigned)(values ? values[i] : (int)i) : 0u;
     const unsigned long long word = ((unsigned long long)value << 32) | (unsigned long long)(unsigned)key;
-    const unsigned long long empty = ~0ull;  // (-1, -1)
-    bool pending = i < n && key >= 0, failed = i < n && key < 0;
-    if (pending) pending = atomicCAS(table + grid_hash_slot(key, 0, table_size), empty, word) != empty;
-    for (int t = 1; t < kHashOwn && pending; t += kHashStep) {
-        unsigned long long *slot[kHashStep], seen[kHashStep];
-#pragma unroll
-        for (int k = 0; k < kHashStep; ++k) {
-            slot[k] = table + grid_hash_slot(key, min(t + k, table_size - 1), table_size);
-            seen[k] = grid_hash_peek(slot[k]);
+    bool pending = i < n && key >= 0;
+    const bool refused = i < n && key < 0;
+    int t = 0;  // (uniform in a wave, as is all that is decided by the ballots)
+    for (unsigned long long looking = __ballot(pending); looking != 0ull && t < table_size; looking = __ballot(pending)) {
+        if (few ? t < kHashCrowd && __popcll(looking) > 16 : t < kHashOwnMany && __popcll(looking) > 8) {
+            if (pending) pending = atomicCAS(table + grid_hash_slot(key, t, table_size), ~0ull, word) != ~0ull;
+            ++t;
+            continue;
         }
-#pragma unroll
-        for (int k = 0; k < kHashStep; ++k)
-            if (pending && t + k < table_size && seen[k] == empty) pending = atomicCAS(slot[k], empty, word) != empty;
-    }
-    for (unsigned long long left = __ballot(pending); left != 0ull; left &= left - 1ull) {
-        const int owner = __builtin_ctzll(left);
-        const int k = __shfl(key, owner, 64);
-        const unsigned long long w = ((unsigned long long)(unsigned)__shfl((int)value, owner, 64) << 32) | (unsigned)k;
-        bool placed = false;  // (uniform)
-        for (int t0 = kHashOwn; t0 < table_size && !placed; t0 += 64) {
-            const int t = t0 + lane;
-            unsigned long long *slot = table + grid_hash_slot(k, min(t, table_size - 1), table_size);
-            unsigned long long free = __ballot(t < table_size && grid_hash_peek(slot) == empty);
-            // the first empty slot, or the next one if that was taken in between
-            for (; free != 0ull && !placed; free &= free - 1ull) {
-                const int first = __builtin_ctzll(free);
-                placed = __ballot(lane == first && atomicCAS(slot, empty, w) == empty) != 0ull;
-            }
+        const HashDeal deal(looking);
+        if (t < kHashLong && deal.log2 >= 2) {
+            hash_place<1>(deal, t, key, word, table, table_size, pending);
+            t += 1 << deal.log2;
+        } else {
+            hash_place<kHashAhead>(deal, t, key, word, table, table_size, pending);
+            t += kHashAhead << deal.log2;
         }
-        if (!placed && lane == owner) failed = true;
     }
-    if (failed && fail) fail[0] = 1;  // table full or key negative (the reference asserts)
+    if ((pending || refused) && fail) fail[0] = 1;  // table full or key negative (the reference asserts)
 }
 
-// Value of the lane's key (-1: absent); a wave at a time, `in`: the lane has a key.
-__device__ __forceinline__ int grid_hash_find(int key, bool in, const unsigned long long *__restrict__ table, int table_size) {
-    const int lane = threadIdx.x & 63;
+// Slots number t0 + k of a group's key, for k < AHEAD << deal.log2, up to the key or an empty slot.  An empty
+// slot on the probe sequence proves the key was never inserted (no deletions).  The reference keeps scanning
+// all table_size slots before giving up (functions.cuh:54-63), with the same answer.
+template <int AHEAD>
+__device__ __forceinline__ void hash_look(const HashDeal &deal, int t0, int key, const unsigned long long *__restrict__ table,
+                                          int table_size, bool &pending, int &found) {
+    const int lane = threadIdx.x & 63, step = 1 << deal.log2;
+    const int k = __shfl(key, deal.from, 64);
+    unsigned long long word[AHEAD];
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a)
+        word[a] = table[grid_hash_slot(k, min(t0 + a * step + (lane & (step - 1)), table_size - 1), table_size)];
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a) {
+        const int slot_key = (int)(unsigned)(word[a] & 0xffffffffull);
+        const bool ends = deal.works && t0 + a * step + (lane & (step - 1)) < table_size && (slot_key == k || slot_key == -1);
+        const unsigned long long mine = deal.mine(__ballot(ends));
+        const int at = pending && mine != 0ull ? (deal.rank << deal.log2) + __builtin_ctzll(mine) : lane;
+        const int at_key = __shfl(slot_key, at, 64), at_value = __shfl((int)(unsigned)(word[a] >> 32), at, 64);
+        if (pending && mine != 0ull) {
+            if (at_key == key) found = at_value;
+            pending = false;
+        }
+    }
+}
+
+// Value of the lane's key (-1: absent); a wave at a time, `in`: the lane has a key, and its own lane for `own` slots.
+__device__ __forceinline__ int grid_hash_find(int key, bool in, const unsigned long long *__restrict__ table, int table_size,
+                                              int own) {
     int found = -1;
     bool pending = in && key >= 0;
-    // An empty slot on the probe sequence proves the key was never inserted (no deletions).  The
-    // reference keeps scanning all table_size slots before giving up (functions.cuh:54-63), with the
-    // same answer.
-    auto look = [&](int t, unsigned long long word) {
-        const int slot_key = (int)(unsigned)(word & 0xffffffffull);
-        if (!pending || t >= table_size) return;
-        if (slot_key == key) found = (int)(unsigned)(word >> 32);
-        pending = slot_key != key && slot_key != -1;
-    };
-    if (pending) look(0, table[grid_hash_slot(key, 0, table_size)]);
-    for (int t = 1; t < kHashOwn && pending; t += kHashStep) {
-        unsigned long long word[kHashStep];
-#pragma unroll
-        for (int k = 0; k < kHashStep; ++k) word[k] = table[grid_hash_slot(key, min(t + k, table_size - 1), table_size)];
-#pragma unroll
-        for (int k = 0; k < kHashStep; ++k) look(t + k, word[k]);
-    }
-    for (unsigned long long left = __ballot(pending); left != 0ull; left &= left - 1ull) {
-        const int owner = __builtin_ctzll(left), k = __shfl(key, owner, 64);
-        for (int t0 = kHashOwn; t0 < table_size; t0 += 64) {
-            const int t = t0 + lane;
-            const unsigned long long word = table[grid_hash_slot(k, min(t, table_size - 1), table_size)];
-            const int slot_key = (int)(unsigned)(word & 0xffffffffull);
-            const unsigned long long ends = __ballot(t < table_size && (slot_key == k || slot_key == -1));
-            if (ends == 0ull) continue;
-            const int first = __builtin_ctzll(ends);
-            const int value = __shfl((int)(unsigned)(word >> 32), first, 64), at = __shfl(slot_key, first, 64);
-            if (lane == owner && at == k) found = value;
-            break;
+    int t = 0;  // (uniform, as above)
+    for (unsigned long long looking = __ballot(pending); looking != 0ull && t < table_size; looking = __ballot(pending)) {
+        if (t < own || __popcll(looking) > 32) {
+            if (pending) {
+                const unsigned long long word = table[grid_hash_slot(key, t, table_size)];
+                const int slot_key = (int)(unsigned)(word & 0xffffffffull);
+                if (slot_key == key) found = (int)(unsigned)(word >> 32);
+                pending = slot_key != key && slot_key != -1;
+            }
+            ++t;
+            continue;
+        }
+        const HashDeal deal(looking);
+        if (t < kHashLong) {
+            hash_look<1>(deal, t, key, table, table_size, pending, found);
+            t += 1 << deal.log2;
+        } else {
+            hash_look<kHashAhead>(deal, t, key, table, table_size, pending, found);
+            t += kHashAhead << deal.log2;
         }
     }
     return found;
 }
 
+inline int hash_own(long n) { return n <= kHashFewProbes ? 1 : kHashOwn; }
+
 template <class Keys>
 __global__ void grid_hash_probe_kernel(Keys keys, const unsigned long long *__restrict__ table, int table_size,
-                                       long n, int *__restrict__ out) {
+                                       long n, int own, int *__restrict__ out) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int value = grid_hash_find(i < n ? (int)keys(i) : -1, i < n, table, table_size);
+    const int value = grid_hash_find(i < n ? (int)keys(i) : -1, i < n, table, table_size, own);
     if (i < n) out[i] = value;
 }
 
@@ -1142,7 +1232,7 @@ int txs_grid_hash_index(const int32_t *bitmap_ws, int64_t key_bound, int64_t num
     const KeyMap m = key_map(b, nullptr, 0, key_bound, nullptr, unq_keys, num_unq);
     grid_hash_prepare_kernel<<<dim3((unsigned)map_parts(m)), dim3(kThreads), 0, st>>>(m, slots, table_size);
     grid_hash_build_kernel<<<dim3(blocks_for(num_unq)), dim3(kThreads), 0, st>>>(unq_keys, nullptr, slots,
-                                                                                (int)table_size, num_unq, nullptr);
+                                                                                (int)table_size, num_unq, num_unq <= kHashFewBuilt, nullptr);
     const long tiles = (table_size + kValidTile - 1) / kValidTile;
     grid_hash_valid_kernel<<<dim3((unsigned)tiles), dim3(kThreads), 0, st>>>(slots, table_size, valid, tile_sums);
     const bool few = tiles <= kValidSumTiles;
@@ -1317,7 +1407,7 @@ int txs_grid_hash_build(const int32_t *keys, const int32_t *values, int64_t num_
     if (num_keys > 0) {
         if (!keys || !values || num_keys > table_size) return TXS_ERR_INVALID_ARG;
         grid_hash_build_kernel<<<dim3(blocks_for(num_keys)), dim3(kThreads), 0, st>>>(
-            keys, values, (unsigned long long *)table, (int)table_size, num_keys, fail_flag);
+            keys, values, (unsigned long long *)table, (int)table_size, num_keys, num_keys <= kHashFewBuilt, fail_flag);
     }
     return status_of(hipGetLastError());
 }
@@ -1329,7 +1419,8 @@ int txs_grid_hash_probe(const int32_t *keys, int64_t num_keys, const int32_t *ta
     if (num_keys == 0) return TXS_OK;
     if (!keys || !out_values) return TXS_ERR_INVALID_ARG;
     grid_hash_probe_kernel<<<dim3(blocks_for(num_keys)), dim3(kThreads), 0, (hipStream_t)stream>>>(
-        FlatKeys<int>{keys}, (const unsigned long long *)table, (int)table_size, num_keys, out_values);
+        FlatKeys<int>{keys}, (const unsigned long long *)table, (int)table_size, num_keys, hash_own(num_keys),
+        out_values);
     return status_of(hipGetLastError());
 }
 
@@ -1343,12 +1434,13 @@ int txs_grid_hash_probe_coors(const void *coors, int coor_is_int64, int64_t num_
     const dim3 grid(blocks_for(num_coors)), blk(kThreads);
     const long s0 = (long)(dim1 * dim2), s1 = (long)dim2;
     auto slots = (const unsigned long long *)table;
+    const int own = hash_own(num_coors);
     if (coor_is_int64)
         grid_hash_probe_kernel<<<grid, blk, 0, st>>>(CoorKeys<long long>{static_cast<const long long *>(coors), s0, s1},
-                                                     slots, (int)table_size, num_coors, out_values);
+                                                     slots, (int)table_size, num_coors, own, out_values);
     else
         grid_hash_probe_kernel<<<grid, blk, 0, st>>>(CoorKeys<int>{static_cast<const int *>(coors), s0, s1}, slots,
-                                                     (int)table_size, num_coors, out_values);
+                                                     (int)table_size, num_coors, own, out_values);
     return status_of(hipGetLastError());
 }
 
