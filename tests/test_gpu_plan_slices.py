@@ -112,7 +112,8 @@ def test_an_overfull_bucket_leaves_the_rows_alone(N):
 
 
 @pytest.mark.parametrize("N,U", [
-    (1, 1), (2, 5000), (1023, 2), (1024, 3), (1025, 1 << 20), (3000, (1 << 22) - 1), (1 << 18, 700), ((1 << 18) + 1, 90_000),
+    (1, 1), (2, 5000), (1023, 2), (1024, 3), (1025, 1 << 20), (3000, (1 << 22) - 1),
+    (1 << 17, 1500), ((1 << 17) + 1, 1500), (350_000, 1500), (1 << 18, 700), ((1 << 18) + 1, 90_000),
     (5 << 18, 2048), ((5 << 18) + 1, 2049), (1 << 21, 1 << 20), ((1 << 21) + 1, 1_000_003),
     (1 << 24, 1 << 22), (1 << 24, 1500), ((1 << 24) + 1, 1 << 21), ((1 << 24) + 1, 1500), ((1 << 24) + 4097, 70_000)])
 def test_plan_at_the_edges_of_tiles(N, U):

@@ -466,8 +466,10 @@ TileSplit tile_split(long n, int bits) {
 }
 // Threads of the workgroups that serve a slice of kBktItems rows per thread: 256 while they can look at all tiles
 // (256 of them; 2^19 rows) and at all of a bucket's voxels (four a thread).  256 / 512: 60k rows in 1500 voxels 47 / 56 us a
-// plan, grouped 51 / 61; 262k in 1500 voxels 52 / 60, a sweep 53 / 50; 2^19 rows 62 / 63 and 56 / 63.
-int slice_threads_for(long n, int low_bits) { return n > (1L << 19) || low_bits > 10 ? 512 : 256; }
+// plan, grouped 51 / 61; 262k in 1500 voxels 52 / 60, a sweep 53 / 50; 2^19 rows 62 / 63 and 56 / 63.  Ranks come with the
+// number of rows for a bound, so that few groups crowd one bucket, whose slices each look at all others' counts: 2000
+// rows 35 - 40 / 36 - 48 us, 100k 40 - 52 / 41 - 49, 200k in 64 groups 72 / 55, in 66,000 46 / 45, 350k in 1500 113 / 69.
+int slice_threads_for(long n, int low_bits, bool ranks) { return n > (ranks ? 1L << 17 : 1L << 19) || low_bits > 10 ? 512 : 256; }
 
 // exclusive scan of one int per thread across a workgroup of WAVES wavefronts
 template <int WAVES>
@@ -1490,7 +1492,8 @@ struct PlanLayout {
     int64_t hist, scan_ws;               // otherwise
     int64_t tile_flags, bucket_start, ctl, part_hist, len;
 };
-PlanLayout plan_layout(int64_t n, int bits) {
+// ranks: for the ranks alone (which need no more than the plan does)
+PlanLayout plan_layout(int64_t n, int bits, bool ranks) {
     PlanLayout l = {};
     l.tiled = n <= kTiledRows;
     int64_t at = 0;
@@ -1521,7 +1524,7 @@ PlanLayout plan_layout(int64_t n, int bits) {
     l.bucket_start = take(((int64_t)1 << l.high_bits) + 1);
     l.ctl = take(1);
     const int low_bits = bits - l.high_bits;
-    l.slice_threads = slice_threads_for((long)n, low_bits);
+    l.slice_threads = slice_threads_for((long)n, low_bits, ranks);
     l.slices_more = n / (l.slice_threads * kBktItems);
     l.part_hist = take(low_bits > 0 ? (((int64_t)1 << l.high_bits) + l.slices_more) << low_bits : 0);
     l.len = at;
@@ -1659,7 +1662,7 @@ int64_t txs_plan_workspace_len(int64_t num_total, int64_t num_unq) {
     const int64_t general = txs_sort_workspace_len(num_total, num_unq);
     const int bits = radix_bits((int)(num_unq > 1 ? num_unq : 1));
     if (bits > kBucketBitsMax) return general;
-    const PlanLayout l = plan_layout(num_total, bits);
+    const PlanLayout l = plan_layout(num_total, bits, false);
     return general > l.len ? general : l.len;
 }
 
@@ -1773,7 +1776,7 @@ int build(const int32_t *unq_inv, int64_t num_total, int64_t num_unq, int32_t he
                 return TXS_ERR_LAUNCH;
         lds_allowed[dev].store(true, std::memory_order_release);
     }
-    const PlanLayout l = plan_layout(n, bits);
+    const PlanLayout l = plan_layout(n, bits, ranks != nullptr);
     const int low_most = bits - l.high_bits;  // (of the voxels there are at most; the kernels know their number)
     int *bucket_start = plan_ws + l.bucket_start;
     const int threads = l.slice_threads;
