@@ -360,6 +360,14 @@ __device__ __forceinline__ int dpp_test(const DppBox &bx, float x, float y, floa
     return in_box ? 2 : (in_large ? 1 : 0);
 }
 
+// What a lane of the wave has written to LDS in front of this, every other lane sees behind it (the hardware keeps
+// a wave's LDS accesses in order by itself; this holds the compiler to it).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // A workgroup takes 1024 points, four per lane, and kDppGroup boxes.  It lays a grid of kDppCells x kDppCells
 // cells over its boxes and marks in every cell the boxes whose circle may reach it; a point looks its
 // cell up and meets those boxes alone.  The pairs are queued by wave and tested 64 at a time, whatever their

@@ -218,14 +218,6 @@ __device__ __forceinline__ float from_ordered_bits(unsigned r) {
     return __uint_as_float((r & 0x80000000u) ? (r ^ 0x80000000u) : ~r);
 }
 
-// What a lane of the wave has written to LDS in front of this, every other lane sees behind it (the hardware keeps
-// a wave's LDS accesses in order by itself; this holds the compiler to it).
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ----------------------------------------------------------- workgroup scan --
 
 __device__ __forceinline__ int wave_inclusive_scan(int x) {
