@@ -33,7 +33,7 @@ def test_keys_of_one_sequence(n, shuffled):
 
 
 @pytest.mark.parametrize("n,probes", [(1000, 5000), (30_000, 70_001), (65_536, 100_000), (3 << 17, 1 << 20),
-                                      ((3 << 17) + 1, (1 << 20) + 1)])
+                                      ((3 << 17) + 1, (1 << 20) + 1), ((1 << 20) + 1, (1 << 20) + 1)])
 def test_one_long_sequence_among_many_short_ones(n, probes):
     """Numbers of keys on either side of where fewer of them get the lanes of others; 300 keys of one sequence, next to
     each other and then anywhere, among keys that find a slot soon (or, in a table that is nearly full, do not)."""

@@ -744,15 +744,14 @@ __device__ __forceinline__ int grid_hash_slot(int key, int probe_i, int table_si
 // a line for each: 16 / 27, and 1M keys in order 50 us against 17 now and with a lane to a key, 3M probes 115 against 86.)
 //
 // How long a key keeps its own lane, us a call with it / with lanes dealt out at once:
-//   placing, up to kHashFewBuilt keys, which wait for trips to memory: while more than 16 keys of the wave look.  A key
-//     tries its slot at once, where a group looks first: a trip more.  In a crowd of long sequences that lasts
-//     kHashCrowd slots, as looking ahead is cheaper than trying: 262k keys in 2^18 slots 3010 / 1210, then 1440;
-//     262k keys 448 apart 404 / 723.
-//   placing, more keys: kHashOwnMany slots while more than 8 keys look.  600k keys 55 / 88, 3M 234 / 361, 1M keys 448 apart
-//     1240 (no end to it) / 668.
-//   looking, up to kHashFewProbes keys: while more than 32 keys look.  1M absent keys in a table 0.95 full 290, 397 as above.
-//   looking, more keys, which wait for the memory itself, so that what is looked at behind a sequence's end costs
-//     time: kHashOwn slots.  3M coordinates 86 / 146, 3M absent keys 194 / 275, 2M in a table 0.95 full 646 / 834.
+//   placing: while more than 8 keys of the wave look.  A key tries its slot at once, where a group looks first, a trip
+//     more: 600k keys 55 / 88, 3M 234 / 361.  In a crowd of long sequences looking ahead is cheaper than trying, the
+//     more so the more keys there are: up to kHashFewBuilt keys that lasts kHashCrowd slots (262k keys in 2^18 slots 3010
+//     to the end / 1210, so 1230; 30,000 keys 448 apart 88 / 192), above kHashOwnMany (1M keys 448 apart 1240 / 616, so 667).
+//   looking: while more than 32 keys look (1M absent keys in a table 0.95 full 290, one by one 272; 300k probes of a frame
+//     above).  More than kHashFewProbes keys in as many slots wait for the memory itself, so that what is looked
+//     at behind a sequence's end costs time: kHashOwn slots there (3M coordinates 86 / 146, 3M absent keys 194 / 275, 2M
+//     in a table 0.95 full 646 / 834; but 1.4M probes of 2^19 slots 43 / 20, of 2^17 47 / 23).
 // From kHashLong slots on, the sequences left are long ones, and a lane asks for kHashAhead slots at a time.
 constexpr int kHashLong = 32, kHashAhead = 4;
 constexpr long kHashFewBuilt = 3L << 17, kHashFewProbes = 1L << 20;
@@ -847,7 +846,7 @@ __global__ __launch_bounds__(kThreads) void grid_hash_build_kernel(const int *__
     const bool refused = i < n && key < 0;
     int t = 0;  // (uniform in a wave, as is all that is decided by the ballots)
     for (unsigned long long looking = __ballot(pending); looking != 0ull && t < table_size; looking = __ballot(pending)) {
-        if (few ? t < kHashCrowd && __popcll(looking) > 16 : t < kHashOwnMany && __popcll(looking) > 8) {
+        if (t < (few ? kHashCrowd : kHashOwnMany) && __popcll(looking) > 8) {
             if (pending) pending = atomicCAS(table + grid_hash_slot(key, t, table_size), ~0ull, word) != ~0ull;
             ++t;
             continue;
@@ -919,7 +918,7 @@ __device__ __forceinline__ int grid_hash_find(int key, bool in, const unsigned l
     return found;
 }
 
-inline int hash_own(long n) { return n <= kHashFewProbes ? 1 : kHashOwn; }
+inline int hash_own(long n, long table_size) { return n > kHashFewProbes && table_size > kHashFewProbes ? kHashOwn : 1; }
 
 template <class Keys>
 __global__ void grid_hash_probe_kernel(Keys keys, const unsigned long long *__restrict__ table, int table_size,
@@ -1427,7 +1426,7 @@ int txs_grid_hash_probe(const int32_t *keys, int64_t num_keys, const int32_t *ta
     if (num_keys == 0) return TXS_OK;
     if (!keys || !out_values) return TXS_ERR_INVALID_ARG;
     grid_hash_probe_kernel<<<dim3(blocks_for(num_keys)), dim3(kThreads), 0, (hipStream_t)stream>>>(
-        FlatKeys<int>{keys}, (const unsigned long long *)table, (int)table_size, num_keys, hash_own(num_keys),
+        FlatKeys<int>{keys}, (const unsigned long long *)table, (int)table_size, num_keys, hash_own(num_keys, table_size),
         out_values);
     return status_of(hipGetLastError());
 }
@@ -1442,7 +1441,7 @@ int txs_grid_hash_probe_coors(const void *coors, int coor_is_int64, int64_t num_
     const dim3 grid(blocks_for(num_coors)), blk(kThreads);
     const long s0 = (long)(dim1 * dim2), s1 = (long)dim2;
     auto slots = (const unsigned long long *)table;
-    const int own = hash_own(num_coors);
+    const int own = hash_own(num_coors, table_size);
     if (coor_is_int64)
         grid_hash_probe_kernel<<<grid, blk, 0, st>>>(CoorKeys<long long>{static_cast<const long long *>(coors), s0, s1},
                                                      slots, (int)table_size, num_coors, own, out_values);
